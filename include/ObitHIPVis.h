@@ -104,7 +104,10 @@ int ObitHIPSkyModelDFTGraphLaunch(GPUInfo *gpuInfo);
  * full and only its selected channels written; for a subtraction with a
  * Gaussian table on such channels, its components without Gaussian terms,
  * the rest on the VALU kernel; other launches run the 32-channel VALU
- * kernel), which ignores tile and wgPerCU.  Autotune times
+ * kernel), which ignores tile and wgPerCU.  Until SetVariant or Autotune is
+ * called, a point model runs on whichever of the matrix-core kernel and the
+ * default VALU shape (32, 64, 2) takes fewer rounds of workgroups, by their
+ * measured cost; GetVariant then reports the VALU shape.  Autotune times
  * every shape on a copy of the first resident rows and keeps the fastest:
  * sampleRows rows, raised where needed so that the widest grid gets at
  * least 8 rounds of work items, and capped at the resident rows. */

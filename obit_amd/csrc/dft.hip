@@ -920,8 +920,10 @@ struct State {
   size_t partCap = 0;
   std::vector<hipEvent_t> events;                 // per-buffer segment events
   std::unordered_map<const void *, int> occ;      // resident workgroups per CU of a kernel
-  // kernel shape
+  // kernel shape; chosen: set by SetVariant or Autotune (until then the
+  // resident launch picks between the two kernels itself)
   int cpt = 32, tile = 64, wgPerCU = 2, prec = 1;
+  bool chosen = false;
   // graph
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -1307,6 +1309,26 @@ int launch_fp64(State *st, const Desc &d) {
   return kOK;
 }
 
+// The kernel of a resident launch whose variant the caller has not set: 64
+// (k_dft_mfma) or st->cpt (k_dft_split).  Both run in rounds of their
+// resident workgroups, and the last round of a short launch costs as much as
+// a full one, so the whole rounds are compared: a round of k_dft_mfma (a row
+// quad a workgroup, 256 channel slots a pass) takes 59 ns a component, one
+// of k_dft_split (256 rows x 32 channels) 550 ns, measured on full launches of
+// 4 IF x 64 channels (13.4e12 and 7.65e12 evaluations/s).  Both sides
+// measured with 3,000 points: 4 x 64 channels, 60,000 rows 3.6 against 6.0 ms;
+// 3 x 37, 20,000 rows 1.17 against 1.5; 1 x 64, 2,000 rows 0.16 against 1.2;
+// 1 x 64, 70,201 rows 4.1 against 2.3 (a quarter of the slots filled).
+int resident_cpt(State *st, const Desc &d) {
+  if (st->chosen || !mfma_ok(st, d)) return st->cpt;
+  const long long nquad = (d.nrow + 3) / 4, npass = (d.nIFsel * ((d.nchsel + 63) / 64) + 3) / 4;
+  const long long slotsM = (long long)st->nCU * occupancy_of(st, (const void *)mfma_fn(st));
+  const long long slotsV = (long long)st->nCU * st->wgPerCU;
+  const double tM = 59.0 * (double)npass * (double)((nquad + slotsM - 1) / slotsM);
+  const double tV = 550.0 * (double)((d.nitems + slotsV - 1) / slotsV);
+  return tM < tV ? 64 : st->cpt;
+}
+
 // Run the operation over nrow rows at a device pointer.
 int run_device(State *st, const GPUInfo *gi, float *vis, long long nrow, bool fp64) {
   Desc d;
@@ -1322,7 +1344,7 @@ int run_device(State *st, const GPUInfo *gi, float *vis, long long nrow, bool fp
   }
   st->lastPath = (fp64 || !st->uniform) ? 1 : 0;
   if (fp64 || !st->uniform) return launch_fp64(st, d);
-  return launch_split(st, d, st->cpt, st->tile, st->wgPerCU);
+  return launch_split(st, d, resident_cpt(st, d), st->tile, st->wgPerCU);
 }
 
 // ---- the per-buffer launch plan (ObitCUDASkyModelDFTCalc) ----
@@ -1990,15 +2012,16 @@ int ObitHIPSkyModelDFTGraphLaunch(GPUInfo *gpuInfo) {
   if (!st || !st->dvis) return obit::fail(obit::kState, "no resident visibilities");
   OBIT_HIP_TRY(hipSetDevice(st->device));
   const long long key = (long long)(size_t)st->dvis ^ (st->nres << 20) ^ ((long long)st->cpt << 8) ^
-                        ((long long)st->tile << 12) ^ ((long long)st->wgPerCU << 4) ^ st->prec;
+                        ((long long)st->tile << 12) ^ ((long long)st->wgPerCU << 4) ^ ((long long)st->chosen << 16) ^ st->prec;
   if (!st->gexec || st->graphKey != key) {
     obit::dft::destroy_graph(st);
     obit::dft::Desc d;
     int rc = obit::dft::make_desc(st, gpuInfo, st->dvis, st->nres, st->cpt, d);
     if (rc) return rc;
     OBIT_HIP_TRY(hipStreamSynchronize(st->stream));
+    const int cpt = obit::dft::resident_cpt(st, d);  // asks for the occupancy: before the capture
     OBIT_HIP_TRY(hipStreamBeginCapture(st->stream, hipStreamCaptureModeThreadLocal));
-    rc = st->uniform ? obit::dft::launch_split(st, d, st->cpt, st->tile, st->wgPerCU)
+    rc = st->uniform ? obit::dft::launch_split(st, d, cpt, st->tile, st->wgPerCU)
                      : obit::dft::launch_fp64(st, d);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(st->stream, &g);
@@ -2020,6 +2043,7 @@ int ObitHIPSkyModelDFTSetVariant(GPUInfo *gpuInfo, int cpt, int tile, int wgPerC
   if (tile != 32 && tile != 64 && tile != 128) return obit::fail(obit::kInvalid, "tile must be 32, 64 or 128");
   if (wgPerCU < 1 || wgPerCU > 8) return obit::fail(obit::kInvalid, "wgPerCU must be 1..8");
   st->cpt = cpt; st->tile = tile; st->wgPerCU = wgPerCU;
+  st->chosen = true;
   return obit::kOK;
 }
 
@@ -2115,6 +2139,7 @@ int ObitHIPSkyModelDFTAutotune(GPUInfo *gpuInfo, long long sampleRows, int reps)
   (void)hipFree(tmp);
   if (rc) return rc;
   st->cpt = bc; st->tile = bt; st->wgPerCU = bw;
+  st->chosen = true;
   obit::dft::destroy_graph(st);
   return obit::kOK;
 }
