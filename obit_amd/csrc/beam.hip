@@ -27,6 +27,7 @@
 #include "ObitHIPBeam.h"
 #include "ObitHIPBeamModel.h"
 #include "ObitHIPVis.h"
+#include "mfma_dft.h"
 #include "phasor.h"
 
 #include <algorithm>
@@ -70,21 +71,11 @@ struct Desc {
   int chanb, chane, IFb, IFe;  // the selection the model is applied to
 };
 
-// One product per (pair, component, beam channel): beam1 * P * beam2^H,
-// in the CPU's order (model * beam2^H, then beam1 * that;
-// src/ObitSkyModelVMBeamMF.c:2752-2755).
-__global__ __launch_bounds__(256) void k_beam_coh(const float *__restrict__ jones,
-                                                  float2 *__restrict__ coh, int ntype, int ncomp,
-                                                  int njchan, int stokType, float c, float s) {
-  const long long n = (long long)ntype * ntype * ncomp * njchan;
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int jc = (int)(i % njchan);
-  const int k = (int)((i / njchan) % ncomp);
-  const int p = (int)(i / ((long long)njchan * ncomp));
-  const int t1 = p / ntype, t2 = p - t1 * ntype;
-  const float *A = jones + (((long long)t1 * ncomp + k) * njchan + jc) * 8;
-  const float *B = jones + (((long long)t2 * ncomp + k) * njchan + jc) * 8;
+// beam1 * P * beam2^H of the Jones matrices A, B (8 floats each) and the
+// model's Stokes parameter, in the CPU's order (model * beam2^H, then beam1 *
+// that; src/ObitSkyModelVMBeamMF.c:2752-2755): XX, XY, YX, YY.
+__device__ __forceinline__ void coh_product(const float *__restrict__ A, const float *__restrict__ B, int stokType,
+                                            float c, float s, float2 (&out)[4]) {
   // coherency P of the model's Stokes parameter, linear feeds
   float Pr[4] = {1.0f, 0.0f, 0.0f, 1.0f}, Pi[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   if (stokType == 2) {
@@ -114,7 +105,6 @@ __global__ __launch_bounds__(256) void k_beam_coh(const float *__restrict__ jone
     }
   }
   // M = A * T
-  float2 *out = coh + i * 4;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
 #pragma unroll
@@ -129,6 +119,25 @@ __global__ __launch_bounds__(256) void k_beam_coh(const float *__restrict__ jone
       out[2 * r + q] = make_float2(re, im);
     }
   }
+}
+
+// One product per (pair, component, beam channel), for k_beam_dft.
+__global__ __launch_bounds__(256) void k_beam_coh(const float *__restrict__ jones,
+                                                  float2 *__restrict__ coh, int ntype, int ncomp,
+                                                  int njchan, int stokType, float c, float s) {
+  const long long n = (long long)ntype * ntype * ncomp * njchan;
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int jc = (int)(i % njchan);
+  const int k = (int)((i / njchan) % ncomp);
+  const int p = (int)(i / ((long long)njchan * ncomp));
+  const int t1 = p / ntype, t2 = p - t1 * ntype;
+  float2 m[4];
+  coh_product(jones + (((long long)t1 * ncomp + k) * njchan + jc) * 8,
+              jones + (((long long)t2 * ncomp + k) * njchan + jc) * 8, stokType, c, s, m);
+  float2 *out = coh + i * 4;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) out[e] = m[e];
 }
 
 // Antenna numbers (0-rel) from BASELINE = 256 a1 + a2 (+ subarray
@@ -401,6 +410,452 @@ __global__ __launch_bounds__(kRows, kBlocksPerCU) void k_beam_dft(Desc d) {
   }
 }
 
+// ---- the matrix-core beam DFT (point components) ----
+//
+// k_beam_dft spends 13 (2 correlations) or 21 (4) FMAs an evaluation on the
+// VALU.  Here the sum over components runs on the FP16 matrix units.  The
+// selected channels are cut into blocks of up to 16 channels of one IF and one
+// beam channel; channel t = -8 .. 7 of block b is at frequency f_b + t df, and
+// correlation e of one row is
+//   M_e[t][b] = sum_k X_k[t] Y_ke[b],
+//   X_k[t] = e(psi df t),  Y_ke[b] = C_keb e(psi f_b),  e(x) = exp(2 pi i x),
+// with C the component's amplitude times its coherency product (k_beam_prod).
+// X is shared by the blocks and the correlations, so a wave forms 16 X and 16
+// Y per correlation for 256 channels of a row.  The product layout is
+// k_dft_mfma's (dft.hip): real 16 x 16 tiles, rows (Re, Im) of 8 t, columns
+// 16 blocks, K = (component, Re / Im), every operand split into FP16 parts
+// x_h + x_l and A_h B_h + A_h B_l + A_l B_h summed in FP32, folded into FP64
+// every 2 tiles of 32 components (every 4 left 2.5e-7 of the model's norm, more
+// than k_beam_dft's 2.3e-7; every tile 1.7e-7 and 4 % slower); conj Y in B.  Y is scaled by a power of two
+// (the largest |C| to [2^13, 2^14)), taken out exactly at the end.
+//
+// A spectrum (AMP) makes the amplitude a_k(t, b) of a channel depend on t and
+// b.  k_beam_fit writes it as A_kb G_k(t) (1 + kappa_k tau(t) s_b): G goes into
+// X, A into C, and the last term, of order 1e-4 (the curvature of ln nu over
+// a block), is one more product of the high parts alone, (kappa X_h) Y_h, with
+// tau and s applied to its sums.  A table that this does not reproduce to
+// 3e-7 of the component's largest amplitude (bins that jump inside a block, a
+// slope that differs from bin to bin) stays on k_beam_dft.
+//
+// A block of threads is 4 waves with a row each; an item is (pass of 16
+// channel blocks, correlation pair, row quad), so 4 correlations are two
+// items that share nothing.  Lane j forms, for component j mod 32 of a tile,
+// the X of 8 t (lanes 0..31: t = -1 .. -8, lanes 32..63: t = 0 .. 7) and the Y
+// of 8 blocks; e(psi df) and e(6 psi df) come from one half-wave each and the
+// other powers from at most two products (of the pairs 1 and n, 6 leaves the
+// least of the two phasors' rounding in the powers up to 8).
+// Bound by VALU issue (330 instructions a tile, 400 with a spectrum; 24 or 32
+// matrix steps beside them).  The second correlation's Y wait in registers for
+// the first's operand area, so a wave needs 13 KB of LDS and three blocks fit
+// a CU at 168 registers; with an area for each (17 KB, two blocks) the VALU
+// was busy 68 % of the time.  With a spectrum two blocks: at 168 registers
+// it spills.  Measured: 20,160 rows x 256 channels x 2,000 points, XX/YY, 8
+// beam channels: 5.59 ms on k_beam_dft, 1.35 with two blocks, 1.20 with three;
+// 7,020 rows x 128 channels x 700 components, 4 correlations, spectra: 888 us
+// on k_beam_dft, 450 here.
+constexpr int kMmTile = 32;          // components a tile
+// slots of a 4-component block: 32 rows (A) or 16 columns (B) + 1 (k_dft_mfma's
+// layout); 16-byte slots of one operand part
+constexpr int kMmRA = 33, kMmRB = 17;
+constexpr int kMmSlotsA = 8 * kMmRA, kMmSlotsB = 8 * kMmRB;
+constexpr int kMmT = 16;             // channels of a block
+constexpr int kMmPass = 16;          // blocks of a pass
+
+struct Blk {
+  double fc;            // nu/nu0 of channel ch0 + 8
+  int IF, ch0;          // first channel (t = -8)
+  int vlo, vhi;         // channels the block writes
+  int jc;               // beam channel
+  float s;              // df (1 / fc - 1 / f0), f0 the pass's reference
+};
+
+struct MmTab {
+  const Blk *blk;
+  int nblk, npass, ncpad;     // ncpad: components padded with zeros (a whole tile of them at least)
+  const float4 *prod;         // [2][npair][npass * 16][ncpad]: conj C of a correlation pair, scaled
+  const unsigned *amax;       // largest |C| (float bits)
+  const float *G;             // [npass][16][ncpad], or null: no spectrum
+  const unsigned *kap;        // [npass][ncpad]: (kappa, kappa) in FP16
+  const float *r0;            // [npass]: df / f0
+};
+
+// exponent that brings amax to [2^13, 2^14)
+__device__ __forceinline__ int mm_shift(unsigned bits) {
+  const int e = (int)((bits >> 23) & 255u) - 126;
+  return bits == 0u ? 0 : 14 - e;
+}
+
+// C of every (correlation pair, type pair, block, component): the largest
+// finite part to amax (WRITE false), then the scaled conjugates to prod.
+template <bool WRITE>
+__global__ __launch_bounds__(256) void k_beam_prod(const float *__restrict__ jones, const float *__restrict__ camp,
+                                                   const float *__restrict__ Ab, const Blk *__restrict__ blk,
+                                                   int nblk, int nblkPad, int ntype, int ncomp, int ncpad, int njchan,
+                                                   int nep, int stokType, float c, float s,
+                                                   unsigned *__restrict__ amax, float4 *__restrict__ prod) {
+  const int npair = ntype * ntype;
+  const long long n = (long long)npair * nblk * ncpad;
+  float big = 0.0f;
+  const float sc = WRITE ? ldexpf(1.0f, mm_shift(*amax)) : 1.0f;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x) {
+    const int k = (int)(i % ncpad);
+    const long long q = i / ncpad;
+    const int b = (int)(q % nblk), p = (int)(q / nblk);
+    float2 m[4];
+    if (k < ncomp) {
+      const int t1 = p / ntype, t2 = p - t1 * ntype, jc = blk[b].jc;
+      coh_product(jones + (((long long)t1 * ncomp + k) * njchan + jc) * 8,
+                  jones + (((long long)t2 * ncomp + k) * njchan + jc) * 8, stokType, c, s, m);
+      const float a = Ab ? Ab[(long long)b * ncpad + k] : camp[k];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m[e] = make_float2(a * m[e].x, a * m[e].y);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m[e] = make_float2(0.0f, 0.0f);
+    }
+    if (WRITE) {
+      for (int ep = 0; ep < nep; ++ep) {
+        const float2 u = m[ep ? 1 : 0], v = m[ep ? 2 : 3];  // (XX, YY) or (XY, YX)
+        prod[(((long long)ep * npair + p) * nblkPad + b) * ncpad + k] =
+            make_float4(sc * u.x, -sc * u.y, sc * v.x, -sc * v.y);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = fabsf(m[e].x), y = fabsf(m[e].y);
+        if (x < INFINITY) big = fmaxf(big, x);
+        if (y < INFINITY) big = fmaxf(big, y);
+      }
+    }
+  }
+  if (!WRITE) {
+    for (int o = 32; o > 0; o >>= 1) big = fmaxf(big, __shfl_xor(big, o));
+    if ((threadIdx.x & 63) == 0 && big > 0.0f) atomicMax(amax, __float_as_uint(big));
+  }
+}
+
+__global__ void k_beam_zero(unsigned *a) { *a = 0u; }
+
+// The factors A_kb G_k(t) (1 + kappa_k tau(t) s_b) of the amplitude table
+// (see above), one thread a component and pass; resid: the largest relative
+// residual (float bits).  G is the shape of the pass's reference block, the
+// first from its middle with an amplitude there; A and the slope of each block
+// are taken at two channels 0.7 of the way to its ends, which halves the error
+// of the linear term at them; kappa is the slopes' least-squares fit to s_b.
+__global__ __launch_bounds__(64) void k_beam_fit(const float *__restrict__ tab, int nchan, long long ldk,
+                                                 const Blk *__restrict__ blk, int nblk, const float *__restrict__ r0,
+                                                 int ncomp, int ncpad, float *__restrict__ Ab, float *__restrict__ G,
+                                                 unsigned *__restrict__ kap, unsigned *__restrict__ resid) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x, ps = blockIdx.y;
+  float worst = 0.0f;
+  if (k < ncomp) {
+    const float *row = tab + (long long)k * ldk;
+    const int b0 = ps * kMmPass, nb = min(kMmPass, nblk - b0);
+    auto amp = [&](int b, int t) {
+      const int ch = min(max(blk[b].ch0 + 8 + t, 0), nchan - 1);
+      return (double)row[(long long)blk[b].IF * nchan + ch];
+    };
+    int ref = b0 + nb / 2;
+    for (int i = 0; i < nb && amp(ref, 0) == 0.0; ++i) ref = b0 + i;
+    const double a0 = amp(ref, 0);
+    double g[kMmT];
+    for (int t = -8; t < 8; ++t) {
+      g[t + 8] = a0 != 0.0 ? amp(ref, t) / a0 : 1.0;
+      if (!(fabs(g[t + 8]) > 1e-3 && fabs(g[t + 8]) < 1e3)) g[t + 8] = 1.0;  // the residual tells
+      g[t + 8] = (double)(float)g[t + 8];
+      G[((long long)ps * kMmT + t + 8) * ncpad + k] = (float)g[t + 8];
+    }
+    const double r = r0[ps];
+    auto tau = [&](int t) { return (double)t - (double)t * (double)t * r; };
+    auto ends = [&](int b, int &t1, int &t2) {
+      const double lo = blk[b].vlo - blk[b].ch0 - 8, hi = blk[b].vhi - blk[b].ch0 - 8;
+      const double m = 0.5 * (lo + hi), w = 0.35 * (hi - lo);
+      t1 = (int)rint(m - w);
+      t2 = (int)rint(m + w);
+    };
+    double num = 0.0, den = 0.0, big = 0.0;
+    for (int b = b0; b < b0 + nb; ++b) {
+      int t1, t2;
+      ends(b, t1, t2);
+      const double p1 = amp(b, t1) / g[t1 + 8], p2 = amp(b, t2) / g[t2 + 8];
+      const double d = p1 * tau(t2) - p2 * tau(t1), s = blk[b].s;
+      if (t2 > t1 && d != 0.0 && s != 0.0) {
+        num += (p2 - p1) / d * s;
+        den += s * s;
+      }
+    }
+    double ka = den > 0.0 ? num / den : 0.0;
+    if (!(fabs(ka) < 1e3)) ka = 0.0;
+    const _Float16 kh = (_Float16)(float)ka;
+    ka = (double)(float)kh;
+    kap[(long long)ps * ncpad + k] = (unsigned)__builtin_bit_cast(unsigned short, kh) * 0x10001u;
+    double off = 0.0;
+    for (int b = b0; b < b0 + nb; ++b) {
+      int t1, t2;
+      ends(b, t1, t2);
+      const double s = blk[b].s;
+      const double A = 0.5 * (amp(b, t1) / (g[t1 + 8] * (1.0 + ka * tau(t1) * s)) +
+                              amp(b, t2) / (g[t2 + 8] * (1.0 + ka * tau(t2) * s)));
+      Ab[(long long)b * ncpad + k] = (float)A;
+      for (int ch = blk[b].vlo; ch <= blk[b].vhi; ++ch) {
+        const int t = ch - blk[b].ch0 - 8;
+        const double a = amp(b, t), e = fabs(a - (double)(float)A * g[t + 8] * (1.0 + ka * tau(t) * s));
+        big = fmax(big, fabs(a));
+        off = (e >= off) ? e : (e < off ? off : INFINITY);  // a NaN counts as infinite
+      }
+    }
+    worst = big > 0.0 ? (float)(off / big) : (off > 0.0 ? INFINITY : 0.0f);
+    if (!(worst >= 0.0f)) worst = INFINITY;
+  } else if (k < ncpad) {
+    for (int t = 0; t < kMmT; ++t) G[((long long)ps * kMmT + t) * ncpad + k] = 1.0f;
+    kap[(long long)ps * ncpad + k] = 0u;
+  }
+  for (int o = 32; o > 0; o >>= 1) worst = fmaxf(worst, __shfl_xor(worst, o));
+  if ((threadIdx.x & 63) == 0 && worst > 0.0f) atomicMax(resid, __float_as_uint(worst));
+}
+
+// Apply a correlation pair of one channel: ep 0 (XX, YY) or 1 (XY, YX, never
+// for a division), by the rules k_beam_dft applies them.
+__device__ __forceinline__ void apply_pair(const Desc &d, float *p, int ncorr, int ep, const float *vr,
+                                           const float *vi) {
+  const bool repl = d.op == ObitHIPBeamOpRepl;
+  bool allBad = (p[2] <= 0.0f) && (p[5] <= 0.0f);
+  if (ncorr == 4) allBad = allBad && (p[8] <= 0.0f) && (p[11] <= 0.0f);
+  if (allBad && !repl) return;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float f = ep ? d.sf[1 + h] : d.sf[3 * h];
+    float mr = vr[h] * f, mi = vi[h] * f;
+    float *q = p + 6 * ep + 3 * h;
+    if (!(q[2] > 0.0f || repl)) continue;
+    if (d.op == ObitHIPBeamOpDiv) {
+      float wm = mr * mr + mi * mi;
+      mr = mr / wm;
+      mi = mi / wm;
+      wm = sqrtf(wm);
+      const float re = q[0], im = q[1];
+      q[0] = mr * re + mi * im;
+      q[1] = mr * im - mi * re;
+      q[2] = q[2] * wm;
+    } else if (repl) {
+      q[0] = mr;
+      q[1] = mi;
+    } else {
+      q[0] -= mr;
+      q[1] -= mi;
+    }
+  }
+}
+
+template <bool AMP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3, AMP ? 2 : 3))) void k_beam_mm(Desc d, MmTab m, int ncorr,
+                                                                                            int nep) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  __shared__ uint4 s_op[4][2 * kMmSlotsA + 2 * kMmSlotsB];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint4 *sAh = s_op[wv], *sAl = sAh + kMmSlotsA, *sBh = sAl + kMmSlotsA, *sBl = sBh + kMmSlotsB;
+  const int i = lane & 15, qd = lane >> 4;   // matrix-step roles
+  const int kc = lane & 31, h = lane >> 5;   // set-up roles: component, half
+  unsigned *wA = reinterpret_cast<unsigned *>(sAh + (kc >> 2) * kMmRA + 16 * h) + (kc & 3);
+  unsigned *wB = reinterpret_cast<unsigned *>(sBh + (kc >> 2) * kMmRB + 8 * h) + (kc & 3);
+  constexpr int kLoA = 4 * kMmSlotsA, kLoB = 4 * kMmSlotsB;  // words from the _h to the _l array
+  const double df = d.dfIF[d.IFb];           // the same for every selected IF
+  const double wdf = h ? 6.0 * df : df;
+  const long long nquad = (d.nrow + 3) / 4;
+  for (long long it = blockIdx.x; it < nquad * nep * m.npass; it += gridDim.x) {
+    const long long rq = it % nquad;
+    const int q = (int)(it / nquad), ep = q % nep, ps = q / nep;
+    const long long row = rq * 4 + wv;
+    if (row >= d.nrow) continue;
+    const float *rp = d.vis + row * (long long)d.lrec;
+    int a1, a2;
+    row_ants(d, rp, &a1, &a2);
+    a1 = __builtin_amdgcn_readfirstlane(a1);
+    a2 = __builtin_amdgcn_readfirstlane(a2);
+    if (a1 < 0 || a1 >= d.nant || a2 < 0 || a2 >= d.nant) continue;
+    const int pair = d.antType[a1] * d.ntype + d.antType[a2];
+    const double u = rp[d.ilocu], v = rp[d.ilocv], w = rp[d.ilocw];
+    // this lane's 8 blocks (one past the last is worked on as the last: its
+    // columns are not written)
+    double fc[8];
+    unsigned po[8];  // offset of a block's products
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const int g = min(ps * kMmPass + 8 * h + b, m.nblk - 1);
+      fc[b] = -m.blk[g].fc;
+      po[b] = (unsigned)g * (unsigned)m.ncpad;
+    }
+    const float4 *prod = m.prod + ((long long)ep * d.npair + pair) * (long long)m.npass * kMmPass * m.ncpad;
+    const float *G = AMP ? m.G + ((long long)ps * kMmT + (h ? 8 : 7)) * m.ncpad : nullptr;
+    const int gstep = h ? m.ncpad : -m.ncpad;
+    const unsigned *kap = AMP ? m.kap + (long long)ps * m.ncpad : nullptr;
+    double o[2][2][4];
+    f4 d2[2][2];
+#pragma unroll
+    for (int T = 0; T < 2; ++T)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        d2[T][e] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[T][e][r] = 0.0;
+      }
+    // the next tile's positions, read a tile ahead
+    double nx, ny, nz;
+    auto fetch = [&](int k0) {
+      const int k = min(k0 + kc, d.ncomp - 1);
+      nx = d.cx[k];
+      ny = d.cy[k];
+      nz = d.cz[k];
+    };
+    fetch(0);
+    for (int k4 = 0; k4 < d.ncomp; k4 += 2 * kMmTile) {
+      f4 acc[2][2];
+#pragma unroll
+      for (int T = 0; T < 2; ++T)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) acc[T][e] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+      for (int kt = 0; kt < 2; ++kt) {
+        const int k0 = k4 + kt * kMmTile;
+        if (k0 >= d.ncomp) break;
+        // this tile's products and shape, used after the powers below
+        const unsigned kp = (unsigned)(k0 + kc);
+        float4 pr[8];
+#pragma unroll
+        for (int b = 0; b < 8; ++b) pr[b] = prod[po[b] + kp];
+        float g[8];
+        if (AMP) {
+          // slot c of this half: t = c (second half) or -(c + 1)
+#pragma unroll
+          for (int c = 0; c < 8; ++c) g[c] = G[(int)kp + c * gstep];
+        }
+        const double psi = fma(w, nz, fma(v, ny, u * nx));
+        fetch(k0 + kMmTile);
+        {
+          const float2 s1 = eturn<false>(psi * wdf);
+          float2 z[9];
+          swap_halves(s1, z[1], z[6]);
+          z[2] = cmul(z[1], z[1]);
+          z[3] = cmul(z[2], z[1]);
+          auto cjmul = [](float2 a, float2 b) {  // a conj(b)
+            return make_float2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
+          };
+          z[4] = cjmul(z[6], z[2]);
+          z[5] = cjmul(z[6], z[1]);
+          z[7] = cmul(z[6], z[1]);
+          z[8] = cmul(z[6], z[2]);
+          z[0] = make_float2(1.0f, 0.0f);
+#pragma unroll
+          for (int c = 0; c < 8; ++c) {
+            float xr = h ? z[c].x : z[c + 1].x, xi = h ? z[c].y : -z[c + 1].y;
+            if (AMP) { xr *= g[c]; xi *= g[c]; }
+            unsigned xh, xl;
+            split_pair(xr, xi, xh, xl);
+            wA[4 * c] = xh;
+            wA[4 * c + kLoA] = xl;
+            wA[4 * (c + 8)] = swap_neg(xh);
+            wA[4 * (c + 8) + kLoA] = swap_neg(xl);
+          }
+        }
+        // the first correlation's Y into the operand area, the second's kept
+        // until the first's are read
+        unsigned y1h[8], y1l[8];
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+          const float2 pg = eturn<true>(psi * fc[b]);  // conj P
+          const float2 y0 = cmul(pg, make_float2(pr[b].x, pr[b].y)), y1 = cmul(pg, make_float2(pr[b].z, pr[b].w));
+          unsigned yh, yl;
+          split_pair(y0.x, y0.y, yh, yl);
+          wB[4 * b] = yh;
+          wB[4 * b + kLoB] = yl;
+          split_pair(y1.x, y1.y, y1h[b], y1l[b]);
+        }
+        // a wave's LDS accesses complete in order: writes, reads, writes, reads
+        h8 ah[2][2], al[2][2];  // [step][tile]
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          h8 bh[2], bl[2];
+          if (e) {
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+              wB[4 * b] = y1h[b];
+              wB[4 * b + kLoB] = y1l[b];
+            }
+            asm volatile("" ::: "memory");
+          }
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+            if (!e) {
+#pragma unroll
+              for (int T = 0; T < 2; ++T) {
+                const int at = (qd + 4 * s) * kMmRA + 16 * T + i;
+                ah[s][T] = __builtin_bit_cast(h8, sAh[at]);
+                al[s][T] = __builtin_bit_cast(h8, sAl[at]);
+              }
+            }
+            bh[s] = __builtin_bit_cast(h8, sBh[(qd + 4 * s) * kMmRB + i]);
+            bl[s] = __builtin_bit_cast(h8, sBl[(qd + 4 * s) * kMmRB + i]);
+          }
+          asm volatile("" ::: "memory");
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int T = 0; T < 2; ++T)
+              acc[T][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s][T], bh[s], acc[T][e], 0, 0, 0);
+#pragma unroll
+            for (int T = 0; T < 2; ++T)
+              acc[T][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s][T], bl[s], acc[T][e], 0, 0, 0);
+#pragma unroll
+            for (int T = 0; T < 2; ++T)
+              acc[T][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[s][T], bh[s], acc[T][e], 0, 0, 0);
+            if (AMP) {
+              const h8 ks = __builtin_bit_cast(h8, *reinterpret_cast<const uint4 *>(kap + k0 + 4 * (qd + 4 * s)));
+#pragma unroll
+              for (int T = 0; T < 2; ++T)
+                d2[T][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s][T] * ks, bh[s], d2[T][e], 0, 0, 0);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int T = 0; T < 2; ++T)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[T][e][r] += (double)acc[T][e][r];
+    }
+    // lanes 0..31 hold the Re of slots c = 4 (lane / 16) + r of tile T, lane +
+    // 32 the Im of the same; column n = lane mod 16 is block n of the pass
+    const int n = lane & 15, gb = min(ps * kMmPass + n, m.nblk - 1);
+    const Blk bk = m.blk[gb];
+    const double unscale = ldexp(1.0, -mm_shift(*m.amax));
+    const float r0 = AMP ? m.r0[ps] : 0.0f;
+    float *base = d.vis + row * (long long)d.lrec + d.nrparm + (long long)bk.IF * d.incif;
+#pragma unroll
+    for (int T = 0; T < 2; ++T)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int c = 4 * (qd & 1) + r, t = T ? c : -(c + 1);
+        float vr[2], vi[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          double x = o[T][e][r];
+          if (AMP) x += (double)(((float)t - (float)(t * t) * r0) * bk.s * d2[T][e][r]);
+          const double y = __shfl_xor(x, 32);
+          vr[e] = (float)(x * unscale);
+          vi[e] = (float)(y * unscale);
+        }
+        const int ch = bk.ch0 + 8 + t;
+        if (lane < 32 && ps * kMmPass + n < m.nblk && ch >= bk.vlo && ch <= bk.vhi)
+          apply_pair(d, base + (long long)ch * d.incf, ncorr, ep, vr, vi);
+      }
+  }
+}
+
 // ---- Jones matrices from beam images (the reference's GetJonesKernel,
 // ObitCUDABeamModel.cu:1227-1308, with CUDABeamInterpPixel and
 // SetConvKernal, include/CUDABeamInterp.h:81-145, 233-258, and
@@ -575,6 +1030,14 @@ struct ObitHIPBeam {
   float *d_tab = nullptr;     // per-channel amplitudes (ObitHIPBeamDFTSetAmps)
   obit::beam::BeamImg *d_imgs = nullptr;
   float refSizeFact = 0.0f, fblank = 0.0f;
+  // k_beam_mm: channel blocks, and the tables made when it can run (SetMod);
+  // mmAmp: the amplitude table has its factors (SetAmps)
+  int nblk = 0, npass = 0, ncpad = 0;
+  bool mmTables = false, mmAmp = false;
+  obit::beam::Blk *d_blk = nullptr;
+  float *d_r0 = nullptr, *d_Ab = nullptr, *d_G = nullptr;
+  unsigned *d_kap = nullptr, *d_mm = nullptr;  // d_mm: largest |C|, fit residual (float bits)
+  float4 *d_prod = nullptr;
 };
 
 namespace {
@@ -582,10 +1045,102 @@ namespace {
 void release(ObitHIPBeam *h) {
   if (!h) return;
   void *ptrs[] = {h->d_freq, h->d_antType, h->d_jmap, h->d_pos, h->d_amp, h->d_g, h->d_jones, h->d_coh,
-                  h->d_images, h->d_bfreq, h->d_cpos, h->d_imgs, h->d_tab};
+                  h->d_images, h->d_bfreq, h->d_cpos, h->d_imgs, h->d_tab, h->d_blk, h->d_r0, h->d_Ab, h->d_G,
+                  h->d_kap, h->d_mm, h->d_prod};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   delete h;
+}
+
+// Whether the next launch runs on k_beam_mm: its tables are there (SetMod: a
+// point table whose channel blocks fill the kernel's slots well enough), and
+// a spectral table has its factors.
+bool use_mm(const ObitHIPBeam *h) { return h->mmTables && (!h->d_tab || h->mmAmp); }
+
+// The channel blocks of k_beam_mm for the selected channels: runs of one IF
+// and beam channel in blocks of 16; a run's last block is moved back to end
+// with the run (it writes the channels the block before does not), a run
+// shorter than a block is one block.  Empty where the IFs' channel steps
+// differ (the kernel has one).
+void mm_blocks(const ObitHIPBeamDesc &D, const double *fIF, const double *dfIF, const int *jmap,
+               std::vector<obit::beam::Blk> &blk, std::vector<float> &r0) {
+  using namespace obit::beam;
+  blk.clear();
+  r0.clear();
+  const double df = dfIF[D.IFb];
+  for (int i = D.IFb; i <= D.IFe; ++i)
+    if (!(std::fabs(dfIF[i] - df) <= 1e-12 * std::fabs(df))) return;
+  for (int i = D.IFb; i <= D.IFe; ++i) {
+    const int *jm = jmap + (size_t)i * D.nchan;
+    for (int c = D.chanb; c <= D.chane;) {
+      int e = c;
+      while (e < D.chane && jm[e + 1] == jm[c]) ++e;
+      for (int a = c; a <= e; a += kMmT) {
+        Blk b{};
+        b.IF = i;
+        b.ch0 = std::max(c, std::min(a, e - kMmT + 1));
+        b.vlo = a;
+        b.vhi = std::min(e, a + kMmT - 1);
+        b.jc = jm[c];
+        b.fc = fIF[i] + (double)(b.ch0 + 8) * dfIF[i];
+        blk.push_back(b);
+      }
+      c = e + 1;
+    }
+  }
+  for (size_t p = 0; p < blk.size(); p += kMmPass) {
+    const size_t n = std::min<size_t>(kMmPass, blk.size() - p);
+    const double f0 = blk[p + n / 2].fc;
+    r0.push_back((float)(df / f0));
+    for (size_t b = p; b < p + n; ++b) blk[b].s = (float)(df * (1.0 / blk[b].fc - 1.0 / f0));
+  }
+}
+
+// The tables of k_beam_mm (once per handle): taken where the model is points
+// and at least 0.3 of its 256 channel slots a pass are selected channels (the
+// kernel runs at about four times k_beam_dft's rate, measured full), and the
+// products fit 512 MiB.
+int mm_tables(ObitHIPBeam *h) {
+  using namespace obit;
+  const ObitHIPBeamDesc &D = h->desc;
+  h->mmTables = false;
+  if (h->gauss || D.ncomp < 1 || h->nblk < 1) return kOK;
+  const double sel = (double)(D.IFe - D.IFb + 1) * (D.chane - D.chanb + 1);
+  if (sel < 0.3 * 256.0 * h->npass) return kOK;
+  const size_t nbp = (size_t)h->npass * beam::kMmPass, nep = D.ncorr == 4 ? 2 : 1;
+  const size_t ncpad = ((size_t)D.ncomp + 31) / 32 * 32 + 32;
+  const size_t nprod = nep * D.ntype * D.ntype * nbp * ncpad;
+  if (nprod * sizeof(float4) > (size_t(512) << 20) || nbp * ncpad > 0x7fffffffULL) return kOK;
+  if (!h->d_prod) {
+    h->ncpad = (int)ncpad;
+    OBIT_HIP_TRY(hipMalloc(&h->d_mm, 2 * sizeof(unsigned)));
+    OBIT_HIP_TRY(hipMalloc(&h->d_prod, nprod * sizeof(float4)));
+  }
+  h->mmTables = true;
+  return kOK;
+}
+
+// The factors of the amplitude table for k_beam_mm (k_beam_fit), and whether
+// they reproduce it.
+int mm_fit(ObitHIPBeam *h) {
+  using namespace obit;
+  const ObitHIPBeamDesc &D = h->desc;
+  h->mmAmp = false;
+  if (!h->mmTables || !h->d_tab) return kOK;
+  const size_t nbp = (size_t)h->npass * beam::kMmPass, nc = (size_t)h->ncpad;
+  if (!h->d_Ab) OBIT_HIP_TRY(hipMalloc(&h->d_Ab, nbp * nc * sizeof(float)));
+  if (!h->d_G) OBIT_HIP_TRY(hipMalloc(&h->d_G, (size_t)h->npass * beam::kMmT * nc * sizeof(float)));
+  if (!h->d_kap) OBIT_HIP_TRY(hipMalloc(&h->d_kap, (size_t)h->npass * nc * sizeof(unsigned)));
+  hipLaunchKernelGGL(beam::k_beam_zero, dim3(1), dim3(1), 0, h->stream, h->d_mm + 1);
+  hipLaunchKernelGGL(beam::k_beam_fit, dim3((unsigned)((nc + 63) / 64), (unsigned)h->npass), dim3(64), 0, h->stream,
+                     h->d_tab, D.nchan, (long long)D.nif * D.nchan, h->d_blk, h->nblk, h->d_r0, D.ncomp, h->ncpad,
+                     h->d_Ab, h->d_G, h->d_kap, h->d_mm + 1);
+  OBIT_HIP_TRY(hipGetLastError());
+  float worst = 0.0f;
+  OBIT_HIP_TRY(hipStreamSynchronize(h->stream));
+  OBIT_HIP_TRY(hipMemcpy(&worst, h->d_mm + 1, sizeof(float), hipMemcpyDeviceToHost));
+  h->mmAmp = worst <= 3e-7f;
+  return kOK;
 }
 
 // no component with flux: the data are left as they are (the reference
@@ -600,6 +1155,21 @@ int beam_coh(ObitHIPBeam *h, float parAng, hipStream_t stream) {
   using namespace obit;
   const ObitHIPBeamDesc &D = h->desc;
   const double c2 = std::cos(2.0 * (double)parAng), s2 = std::sin(2.0 * (double)parAng);
+  if (use_mm(h)) {
+    const int nep = D.ncorr == 4 ? 2 : 1;
+    const float *Ab = h->d_tab ? h->d_Ab : nullptr;
+    const long long n = (long long)D.ntype * D.ntype * h->nblk * h->ncpad;
+    const dim3 grid((unsigned)std::min<long long>((n + 255) / 256, (long long)std::max(h->ncu, 1) * 16));
+    hipLaunchKernelGGL(beam::k_beam_zero, dim3(1), dim3(1), 0, stream, h->d_mm);
+    hipLaunchKernelGGL((beam::k_beam_prod<false>), grid, dim3(256), 0, stream, h->d_jones, h->d_amp, Ab, h->d_blk,
+                       h->nblk, h->npass * beam::kMmPass, D.ntype, D.ncomp, h->ncpad, D.njchan, nep, D.stokType,
+                       (float)c2, (float)s2, h->d_mm, h->d_prod);
+    hipLaunchKernelGGL((beam::k_beam_prod<true>), grid, dim3(256), 0, stream, h->d_jones, h->d_amp, Ab, h->d_blk,
+                       h->nblk, h->npass * beam::kMmPass, D.ntype, D.ncomp, h->ncpad, D.njchan, nep, D.stokType,
+                       (float)c2, (float)s2, h->d_mm, h->d_prod);
+    OBIT_HIP_TRY(hipGetLastError());
+    return kOK;
+  }
   const long long ncoh = (long long)D.ntype * D.ntype * D.ncomp * D.njchan;
   hipLaunchKernelGGL(beam::k_beam_coh, dim3((unsigned)((ncoh + 255) / 256)), dim3(256), 0, stream,
                      h->d_jones, h->d_coh, D.ntype, D.ncomp, D.njchan, D.stokType, (float)c2, (float)s2);
@@ -636,6 +1206,22 @@ int beam_dft(ObitHIPBeam *h, float *d_vis, long long nrow, hipStream_t stream) {
   d.op = D.opType;
   for (int i = 0; i < 4; ++i) d.sf[i] = D.stokFact[i];
   d.chanb = D.chanb; d.chane = D.chane; d.IFb = D.IFb; d.IFe = D.IFe;
+  if (use_mm(h)) {
+    beam::MmTab m;
+    m.blk = h->d_blk;
+    m.nblk = h->nblk; m.npass = h->npass; m.ncpad = h->ncpad;
+    m.prod = h->d_prod;
+    m.amax = h->d_mm;
+    m.G = h->d_G; m.kap = h->d_kap; m.r0 = h->d_r0;
+    // the cross hands are not divided
+    const int nep = D.ncorr == 4 && D.opType != ObitHIPBeamOpDiv ? 2 : 1;
+    const long long items = ((nrow + 3) / 4) * nep * h->npass;
+    const dim3 grid((unsigned)std::min<long long>(items, (long long)std::max(h->ncu, 1) * (h->d_tab ? 2 : 3)));
+    if (h->d_tab) hipLaunchKernelGGL((beam::k_beam_mm<true>), grid, dim3(256), 0, stream, d, m, D.ncorr, nep);
+    else hipLaunchKernelGGL((beam::k_beam_mm<false>), grid, dim3(256), 0, stream, d, m, D.ncorr, nep);
+    OBIT_HIP_TRY(hipGetLastError());
+    return kOK;
+  }
   long long grid = (long long)std::max(h->ncu, 1) * beam::kBlocksPerCU;
   if (grid > d.nitems) grid = d.nitems;
   void *args[] = {&d};
@@ -719,6 +1305,15 @@ int ObitHIPBeamDFTCreate(ObitHIPBeam **out, const ObitHIPBeamDesc *desc, const d
   if (!rc) rc = up((void **)&h->d_jones, nullptr, (size_t)d.ntype * nc * d.njchan * 8 * sizeof(float));
   if (!rc) rc = up((void **)&h->d_coh, nullptr, (size_t)d.ntype * d.ntype * nc * d.njchan * 4 * sizeof(float2));
   if (!rc) rc = ObitHIPBeamDFTSetJones(h, nullptr);
+  std::vector<beam::Blk> blk;
+  std::vector<float> r0;
+  mm_blocks(d, fIF, dfIF, visJChan, blk, r0);
+  if (!rc && !blk.empty()) {
+    rc = up((void **)&h->d_blk, blk.data(), blk.size() * sizeof(beam::Blk));
+    if (!rc) rc = up((void **)&h->d_r0, r0.data(), r0.size() * sizeof(float));
+    h->nblk = (int)blk.size();
+    h->npass = (int)r0.size();
+  }
   if (rc) { release(h); return rc; }
   *out = h;
   return kOK;
@@ -752,7 +1347,9 @@ int ObitHIPBeamDFTSetMod(ObitHIPBeam *h, const float *comps) {
   h->gauss = gauss;
   h->anyFlux = any;
   h->haveMod = true;
-  return kOK;
+  int rc = mm_tables(h);
+  if (!rc) rc = mm_fit(h);  // a spectral table set before
+  return rc;
 }
 
 int ObitHIPBeamDFTSetJones(ObitHIPBeam *h, const float *jones) {
@@ -787,6 +1384,7 @@ int ObitHIPBeamDFTSetAmps(ObitHIPBeam *h, const float *amp) {
   if (!amp) {
     if (h->d_tab) OBIT_HIP_TRY(hipFree(h->d_tab));
     h->d_tab = nullptr;
+    h->mmAmp = false;
     return kOK;
   }
   const size_t n = (size_t)std::max(h->desc.ncomp, 1) * h->desc.nif * h->desc.nchan;
@@ -795,7 +1393,7 @@ int ObitHIPBeamDFTSetAmps(ObitHIPBeam *h, const float *amp) {
   bool any = false;
   for (size_t i = 0; i < n && !any; ++i) any = amp[i] != 0.0f;
   h->anyTab = any;
-  return kOK;
+  return mm_fit(h);
 }
 
 int ObitHIPBeamDFTGetJones(ObitHIPBeam *h, float *jones) {
