@@ -960,54 +960,44 @@ __device__ __forceinline__ float inv_beam(float fact, float freq, float ang) {
   return div / cosf((float)(3.141592653589793 * (double)arg));
 }
 
-// One thread per (component, antenna type), looping over beam channels.
+// One thread per element of a Jones matrix: (antenna type, beam channel,
+// component, element), element fastest, so a matrix is written whole by 8
+// neighbouring lanes and they gather from the same place of 8 image planes.
+// The latency of the gathers bounds it: a thread that looped over the beam
+// channels and the 8 planes took 216 us for 700 components x 2 types x 4
+// channels, 6 blocks of threads on the whole chip; spread out, 14 us.
 __global__ __launch_bounds__(256) void k_beam_jones(const float *__restrict__ images,
                                                     const BeamImg *__restrict__ imgs,
                                                     const float *__restrict__ pos,
                                                     const float *__restrict__ bfreq, float refSizeFact,
-                                                    int ncomp, int nchan, float parAng, float fblank,
+                                                    int ntype, int ncomp, int nchan, float parAng, float fblank,
                                                     float *__restrict__ jones) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  const int t = blockIdx.y;
-  if (k >= ncomp) return;
-  const BeamImg b = imgs[t];
-  float *J = jones + ((long long)t * ncomp + k) * nchan * 8;
-  const double p0 = -(double)pos[2 * k], p1 = (double)pos[2 * k + 1];
-  float px, py;
-  if (beam_pixel(b, p0, p1, parAng, &px, &py) != 0) {
-    for (int c = 0; c < nchan; ++c) {
-      float *q = J + 8 * c;
-      q[0] = 1.0f; q[1] = 0.0f; q[2] = 0.0f; q[3] = 0.0f;
-      q[4] = 0.0f; q[5] = 0.0f; q[6] = 1.0f; q[7] = 0.0f;
-    }
-    return;
-  }
-  const float ang = sqrtf((float)(p0 * p0 + p1 * p1));
-  const long long planeSz = (long long)b.nx * b.ny, imgSz = planeSz * nchan;
-  for (int c = 0; c < nchan; ++c) {
+  const long long n = (long long)ntype * nchan * ncomp * 8;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x) {
+    const int e = (int)(i & 7);
+    const long long q = i >> 3;
+    const int k = (int)(q % ncomp);
+    const int c = (int)((q / ncomp) % nchan);
+    const int t = (int)(q / ((long long)ncomp * nchan));
+    const BeamImg b = imgs[t];
+    const double p0 = -(double)pos[2 * k], p1 = (double)pos[2 * k + 1];
+    float px, py;
+    const bool placed = beam_pixel(b, p0, p1, parAng, &px, &py) == 0;
+    // images in the reference's order: P1 re, P1 im, P2 re, P2 im, X1 re,
+    // X1 im, X2 re, X2 im; elements P1, X1, X2, P2
+    const int plane = e < 2 ? e : e < 6 ? e + 2 : e - 4;
+    const long long planeSz = (long long)b.nx * b.ny, imgSz = planeSz * nchan;
+    const float ang = sqrtf((float)(p0 * p0 + p1 * p1));
     const float ipb = inv_beam(refSizeFact, bfreq[c], ang);
-    const float *base = images + b.off + (long long)c * planeSz;
-    // images in the reference's order: P1 re, P1 im, P2 re, P2 im,
-    // X1 re, X1 im, X2 re, X2 im
-    float P1r = ipb * beam_interp(base, b, px, py, fblank);
-    float P2r = ipb * beam_interp(base + 2 * imgSz, b, px, py, fblank);
-    float P1i, P2i, X1r, X1i, X2r, X2i;
-    // the reference's sanity test (it tests P1r twice)
-    if (ipb < 10.0f && fabsf(P1r) <= 1.3f && fabsf(P1r) <= 1.3f) {
-      P1i = ipb * beam_interp(base + 1 * imgSz, b, px, py, fblank);
-      P2i = ipb * beam_interp(base + 3 * imgSz, b, px, py, fblank);
-      X1r = ipb * beam_interp(base + 4 * imgSz, b, px, py, fblank);
-      X1i = ipb * beam_interp(base + 5 * imgSz, b, px, py, fblank);
-      X2r = ipb * beam_interp(base + 6 * imgSz, b, px, py, fblank);
-      X2i = ipb * beam_interp(base + 7 * imgSz, b, px, py, fblank);
-    } else {
-      P1r = P2r = 1.0f;
-      P1i = P2i = 0.0f;
-      X1r = X1i = X2r = X2i = 0.0f;
-    }
-    float *q = J + 8 * c;
-    q[0] = P1r; q[1] = P1i; q[2] = X1r; q[3] = X1i;
-    q[4] = X2r; q[5] = X2i; q[6] = P2r; q[7] = P2i;
+    const float val =
+        placed ? ipb * beam_interp(images + b.off + plane * imgSz + (long long)c * planeSz, b, px, py, fblank) : 0.0f;
+    // the reference's sanity test, on the gain and P1r: a matrix that fails it
+    // is the unit matrix (n is a multiple of 8, so the 8 lanes are all here)
+    const float P1r = __shfl(val, (int)(threadIdx.x & 63) & ~7);
+    const bool ok = placed && ipb < 10.0f && fabsf(P1r) <= 1.3f;
+    const float unit = (e == 0 || e == 6) ? 1.0f : 0.0f;
+    jones[(((long long)t * ncomp + k) * nchan + c) * 8 + e] = ok ? val : unit;
   }
 }
 
@@ -1463,9 +1453,10 @@ int ObitHIPBeamDFTJonesFromBeams(ObitHIPBeam *h, const float *pos, float parAng)
   OBIT_HIP_TRY(hipStreamSynchronize(h->stream));
   if (!h->d_cpos) OBIT_HIP_TRY(hipMalloc(&h->d_cpos, (size_t)n * 2 * sizeof(float)));
   OBIT_HIP_TRY(hipMemcpy(h->d_cpos, pos, (size_t)n * 2 * sizeof(float), hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(beam::k_beam_jones, dim3((unsigned)((n + 255) / 256), (unsigned)h->desc.ntype), dim3(256), 0,
-                     h->stream, h->d_images, h->d_imgs, h->d_cpos, h->d_bfreq, h->refSizeFact, n, h->desc.njchan,
-                     parAng, h->fblank, h->d_jones);
+  const long long nel = (long long)h->desc.ntype * h->desc.njchan * n * 8;
+  const dim3 grid((unsigned)std::min<long long>((nel + 255) / 256, (long long)std::max(h->ncu, 1) * 32));
+  hipLaunchKernelGGL(beam::k_beam_jones, grid, dim3(256), 0, h->stream, h->d_images, h->d_imgs, h->d_cpos, h->d_bfreq,
+                     h->refSizeFact, h->desc.ntype, n, h->desc.njchan, parAng, h->fblank, h->d_jones);
   OBIT_HIP_TRY(hipGetLastError());
   return kOK;
 }
