@@ -439,7 +439,10 @@ __global__ __launch_bounds__(kRows, kBlocksPerCU) void k_beam_dft(Desc d) {
 //
 // A block of threads is 4 waves with a row each; an item is (pass of 16
 // channel blocks, correlation pair, row quad), so 4 correlations are two
-// items that share nothing.  Lane j forms, for component j mod 32 of a tile,
+// items that share nothing.  Where the selection has 8 blocks or fewer (128
+// channels), half the columns would be empty: the half-waves then form the Y
+// of the same 8 blocks, for a correlation each (ONE) or a pair each, and 4
+// correlations are one item.  Lane j forms, for component j mod 32 of a tile,
 // the X of 8 t (lanes 0..31: t = -1 .. -8, lanes 32..63: t = 0 .. 7) and the Y
 // of 8 blocks; e(psi df) and e(6 psi df) come from one half-wave each and the
 // other powers from at most two products (of the pairs 1 and n, 6 leaves the
@@ -615,42 +618,43 @@ __global__ __launch_bounds__(64) void k_beam_fit(const float *__restrict__ tab, 
   if ((threadIdx.x & 63) == 0 && worst > 0.0f) atomicMax(resid, __float_as_uint(worst));
 }
 
-// Apply a correlation pair of one channel: ep 0 (XX, YY) or 1 (XY, YX, never
-// for a division), by the rules k_beam_dft applies them.
-__device__ __forceinline__ void apply_pair(const Desc &d, float *p, int ncorr, int ep, const float *vr,
-                                           const float *vi) {
+// Whether any correlation of a channel is unflagged.
+__device__ __forceinline__ bool channel_live(const float *p, int ncorr) {
+  bool live = !(p[2] <= 0.0f) || !(p[5] <= 0.0f);
+  if (ncorr == 4) live = live || !(p[8] <= 0.0f) || !(p[11] <= 0.0f);
+  return live;
+}
+
+// Apply correlation e of pair ep (0: XX, YY; 1: XY, YX, never for a division)
+// of one channel, by the rules k_beam_dft applies them.
+__device__ __forceinline__ void apply_corr(const Desc &d, float *p, int ep, int e, float vr, float vi) {
   const bool repl = d.op == ObitHIPBeamOpRepl;
-  bool allBad = (p[2] <= 0.0f) && (p[5] <= 0.0f);
-  if (ncorr == 4) allBad = allBad && (p[8] <= 0.0f) && (p[11] <= 0.0f);
-  if (allBad && !repl) return;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const float f = ep ? d.sf[1 + h] : d.sf[3 * h];
-    float mr = vr[h] * f, mi = vi[h] * f;
-    float *q = p + 6 * ep + 3 * h;
-    if (!(q[2] > 0.0f || repl)) continue;
-    if (d.op == ObitHIPBeamOpDiv) {
-      float wm = mr * mr + mi * mi;
-      mr = mr / wm;
-      mi = mi / wm;
-      wm = sqrtf(wm);
-      const float re = q[0], im = q[1];
-      q[0] = mr * re + mi * im;
-      q[1] = mr * im - mi * re;
-      q[2] = q[2] * wm;
-    } else if (repl) {
-      q[0] = mr;
-      q[1] = mi;
-    } else {
-      q[0] -= mr;
-      q[1] -= mi;
-    }
+  const float f = ep ? (e ? d.sf[2] : d.sf[1]) : (e ? d.sf[3] : d.sf[0]);
+  float mr = vr * f, mi = vi * f;
+  float *q = p + 6 * ep + 3 * e;
+  if (!(q[2] > 0.0f || repl)) return;
+  if (d.op == ObitHIPBeamOpDiv) {
+    float wm = mr * mr + mi * mi;
+    mr = mr / wm;
+    mi = mi / wm;
+    wm = sqrtf(wm);
+    const float re = q[0], im = q[1];
+    q[0] = mr * re + mi * im;
+    q[1] = mr * im - mi * re;
+    q[2] = q[2] * wm;
+  } else if (repl) {
+    q[0] = mr;
+    q[1] = mi;
+  } else {
+    q[0] -= mr;
+    q[1] -= mi;
   }
 }
 
-template <bool AMP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3, AMP ? 2 : 3))) void k_beam_mm(Desc d, MmTab m, int ncorr,
-                                                                                            int nep) {
+template <bool AMP, bool ONE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3, AMP ? 2 : 3))) void k_beam_mm(
+    Desc d, MmTab m, int ncorr, int nep, int split) {
+  constexpr int NE = ONE ? 1 : 2;  // correlations a column block of a lane has
   typedef float f4 __attribute__((ext_vector_type(4)));
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   __shared__ uint4 s_op[4][2 * kMmSlotsA + 2 * kMmSlotsB];
@@ -678,26 +682,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
     if (a1 < 0 || a1 >= d.nant || a2 < 0 || a2 >= d.nant) continue;
     const int pair = d.antType[a1] * d.ntype + d.antType[a2];
     const double u = rp[d.ilocu], v = rp[d.ilocv], w = rp[d.ilocw];
-    // this lane's 8 blocks (one past the last is worked on as the last: its
+    // this lane's 8 blocks: with split, the first 8 for both halves, which have
+    // a correlation (ONE) or a pair each; else the half's 8 of the pass (one past the last is worked on as the last: its
     // columns are not written)
     double fc[8];
     unsigned po[8];  // offset of a block's products
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-      const int g = min(ps * kMmPass + 8 * h + b, m.nblk - 1);
+      const int g = min(split ? b : ps * kMmPass + 8 * h + b, m.nblk - 1);
       fc[b] = -m.blk[g].fc;
       po[b] = (unsigned)g * (unsigned)m.ncpad;
     }
-    const float4 *prod = m.prod + ((long long)ep * d.npair + pair) * (long long)m.npass * kMmPass * m.ncpad;
+    const float4 *prod = m.prod + ((long long)(split && !ONE ? h : ep) * d.npair + pair) *
+                                      (long long)m.npass * kMmPass * m.ncpad;
     const float *G = AMP ? m.G + ((long long)ps * kMmT + (h ? 8 : 7)) * m.ncpad : nullptr;
     const int gstep = h ? m.ncpad : -m.ncpad;
     const unsigned *kap = AMP ? m.kap + (long long)ps * m.ncpad : nullptr;
-    double o[2][2][4];
-    f4 d2[2][2];
+    double o[2][NE][4];
+    f4 d2[2][NE];
 #pragma unroll
     for (int T = 0; T < 2; ++T)
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
+      for (int e = 0; e < NE; ++e) {
         d2[T][e] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[T][e][r] = 0.0;
@@ -712,11 +718,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
     };
     fetch(0);
     for (int k4 = 0; k4 < d.ncomp; k4 += 2 * kMmTile) {
-      f4 acc[2][2];
+      f4 acc[2][NE];
 #pragma unroll
       for (int T = 0; T < 2; ++T)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) acc[T][e] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int e = 0; e < NE; ++e) acc[T][e] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
       for (int kt = 0; kt < 2; ++kt) {
         const int k0 = k4 + kt * kMmTile;
@@ -725,7 +731,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
         const unsigned kp = (unsigned)(k0 + kc);
         float4 pr[8];
 #pragma unroll
-        for (int b = 0; b < 8; ++b) pr[b] = prod[po[b] + kp];
+        for (int b = 0; b < 8; ++b) {
+          if (ONE) {
+            const float2 x = reinterpret_cast<const float2 *>(prod)[2u * (po[b] + kp) + (unsigned)h];
+            pr[b] = make_float4(x.x, x.y, 0.0f, 0.0f);
+          } else {
+            pr[b] = prod[po[b] + kp];
+          }
+        }
         float g[8];
         if (AMP) {
           // slot c of this half: t = c (second half) or -(c + 1)
@@ -766,18 +779,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
           const float2 pg = eturn<true>(psi * fc[b]);  // conj P
-          const float2 y0 = cmul(pg, make_float2(pr[b].x, pr[b].y)), y1 = cmul(pg, make_float2(pr[b].z, pr[b].w));
+          const float2 y0 = cmul(pg, make_float2(pr[b].x, pr[b].y));
           unsigned yh, yl;
           split_pair(y0.x, y0.y, yh, yl);
           wB[4 * b] = yh;
           wB[4 * b + kLoB] = yl;
-          split_pair(y1.x, y1.y, y1h[b], y1l[b]);
+          if (!ONE) {
+            const float2 y1 = cmul(pg, make_float2(pr[b].z, pr[b].w));
+            split_pair(y1.x, y1.y, y1h[b], y1l[b]);
+          }
         }
         // a wave's LDS accesses complete in order: writes, reads, writes, reads
         h8 ah[2][2], al[2][2];  // [step][tile]
         asm volatile("" ::: "memory");
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
+        for (int e = 0; e < NE; ++e) {
           h8 bh[2], bl[2];
           if (e) {
 #pragma unroll
@@ -824,14 +840,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
 #pragma unroll
       for (int T = 0; T < 2; ++T)
 #pragma unroll
-        for (int e = 0; e < 2; ++e)
+        for (int e = 0; e < NE; ++e)
 #pragma unroll
           for (int r = 0; r < 4; ++r) o[T][e][r] += (double)acc[T][e][r];
     }
     // lanes 0..31 hold the Re of slots c = 4 (lane / 16) + r of tile T, lane +
-    // 32 the Im of the same; column n = lane mod 16 is block n of the pass
-    const int n = lane & 15, gb = min(ps * kMmPass + n, m.nblk - 1);
-    const Blk bk = m.blk[gb];
+    // 32 the Im of the same; column n = lane mod 16 is block n of the pass, or
+    // with split block n mod 8 of correlation or pair n / 8
+    const int n = lane & 15, nb = split ? n & 7 : n, cp = !ONE && split ? n >> 3 : ep;
+    const Blk bk = m.blk[min(ps * kMmPass + nb, m.nblk - 1)];
+    const bool have = lane < 32 && ps * kMmPass + nb < m.nblk;
     const double unscale = ldexp(1.0, -mm_shift(*m.amax));
     const float r0 = AMP ? m.r0[ps] : 0.0f;
     float *base = d.vis + row * (long long)d.lrec + d.nrparm + (long long)bk.IF * d.incif;
@@ -840,9 +858,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int c = 4 * (qd & 1) + r, t = T ? c : -(c + 1);
-        float vr[2], vi[2];
+        float vr[NE], vi[NE];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
+        for (int e = 0; e < NE; ++e) {
           double x = o[T][e][r];
           if (AMP) x += (double)(((float)t - (float)(t * t) * r0) * bk.s * d2[T][e][r]);
           const double y = __shfl_xor(x, 32);
@@ -850,8 +868,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
           vi[e] = (float)(y * unscale);
         }
         const int ch = bk.ch0 + 8 + t;
-        if (lane < 32 && ps * kMmPass + n < m.nblk && ch >= bk.vlo && ch <= bk.vhi)
-          apply_pair(d, base + (long long)ch * d.incf, ncorr, ep, vr, vi);
+        float *p = base + (long long)ch * d.incf;
+        const bool take = have && ch >= bk.vlo && ch <= bk.vhi;
+        // the channel's flags, read before any lane's division changes a weight
+        const bool use = take && (d.op == ObitHIPBeamOpRepl || channel_live(p, ncorr));
+        if (use) {
+#pragma unroll
+          for (int e = 0; e < NE; ++e) apply_corr(d, p, cp, ONE && split ? n >> 3 : e, vr[e], vi[e]);
+        }
       }
   }
 }
@@ -1100,7 +1124,7 @@ int mm_tables(ObitHIPBeam *h) {
   const size_t nbp = (size_t)h->npass * beam::kMmPass, nep = D.ncorr == 4 ? 2 : 1;
   const size_t ncpad = ((size_t)D.ncomp + 31) / 32 * 32 + 32;
   const size_t nprod = nep * D.ntype * D.ntype * nbp * ncpad;
-  if (nprod * sizeof(float4) > (size_t(512) << 20) || nbp * ncpad > 0x7fffffffULL) return kOK;
+  if (nprod * sizeof(float4) > (size_t(512) << 20) || nbp * ncpad > 0x3fffffffULL) return kOK;
   if (!h->d_prod) {
     h->ncpad = (int)ncpad;
     OBIT_HIP_TRY(hipMalloc(&h->d_mm, 2 * sizeof(unsigned)));
@@ -1204,11 +1228,18 @@ int beam_dft(ObitHIPBeam *h, float *d_vis, long long nrow, hipStream_t stream) {
     m.amax = h->d_mm;
     m.G = h->d_G; m.kap = h->d_kap; m.r0 = h->d_r0;
     // the cross hands are not divided
-    const int nep = D.ncorr == 4 && D.opType != ObitHIPBeamOpDiv ? 2 : 1;
+    const bool cross = D.ncorr == 4 && D.opType != ObitHIPBeamOpDiv;
+    // up to 8 blocks leave half the columns free: the half-waves take a
+    // correlation or a pair each, instead of 8 blocks each
+    const int split = h->nblk <= 8;
+    const bool one = split && !cross;
+    const int nep = cross && !split ? 2 : 1;
+    const bool sp = h->d_tab != nullptr;
     const long long items = ((nrow + 3) / 4) * nep * h->npass;
-    const dim3 grid((unsigned)std::min<long long>(items, (long long)std::max(h->ncu, 1) * (h->d_tab ? 2 : 3)));
-    if (h->d_tab) hipLaunchKernelGGL((beam::k_beam_mm<true>), grid, dim3(256), 0, stream, d, m, D.ncorr, nep);
-    else hipLaunchKernelGGL((beam::k_beam_mm<false>), grid, dim3(256), 0, stream, d, m, D.ncorr, nep);
+    const dim3 grid((unsigned)std::min<long long>(items, (long long)std::max(h->ncu, 1) * (sp ? 2 : 3)));
+    auto fn = sp ? (one ? beam::k_beam_mm<true, true> : beam::k_beam_mm<true, false>)
+                 : (one ? beam::k_beam_mm<false, true> : beam::k_beam_mm<false, false>);
+    hipLaunchKernelGGL(fn, grid, dim3(256), 0, stream, d, m, D.ncorr, nep, split);
     OBIT_HIP_TRY(hipGetLastError());
     return kOK;
   }

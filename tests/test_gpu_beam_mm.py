@@ -45,6 +45,9 @@ CASES = [
     (2, 63, 1, 256, 100, 96, 1, "div", -0.7, None),
     (2, 64, 4, 64, 64, 64, 1, "sub", None, ((5, 60), (1, 3))),
     (4, 61, 4, 64, 32, 64, 1, "sub", -0.7, ((0, 55), (0, 2))),
+    (2, 61, 1, 64, 32, 100, 2, "sub", None, None),      # 8 blocks or fewer: a correlation a half-wave
+    (4, 66, 1, 128, 64, 95, 1, "repl", -0.7, None),
+    (2, 61, 1, 128, 128, 70, 1, "div", None, None),
 ]
 
 
