@@ -104,7 +104,9 @@ int ObitHIPSkyModelDFTGraphLaunch(GPUInfo *gpuInfo);
  * full and only its selected channels written; for a subtraction with a
  * Gaussian table on such channels, its components without Gaussian terms,
  * the rest on the VALU kernel; other launches run the 32-channel VALU
- * kernel), which ignores tile and wgPerCU.  Until SetVariant or Autotune is
+ * kernel), which ignores tile and wgPerCU.  A spectral
+ * point model runs on a matrix-core kernel of its own where its amplitudes
+ * factor smoothly over blocks of 16 channels.  Until SetVariant or Autotune is
  * called, a point model runs on whichever of the matrix-core kernel and the
  * default VALU shape (32, 64, 2) takes fewer rounds of workgroups, by their
  * measured cost; GetVariant then reports the VALU shape.  Autotune times

@@ -430,11 +430,11 @@ __global__ __launch_bounds__(kRows, kBlocksPerCU) void k_beam_dft(Desc d) {
 // (the largest |C| to [2^13, 2^14)), taken out exactly at the end.
 //
 // A spectrum (AMP) makes the amplitude a_k(t, b) of a channel depend on t and
-// b.  k_beam_fit writes it as A_kb G_k(t) (1 + kappa_k tau(t) s_b): G goes into
+// b.  mm::k_fit writes it as A_kb G_k(t) (1 + kappa_k tau(t) s_b): G goes into
 // X, A into C, and the last term, of order 1e-4 (the curvature of ln nu over
 // a block), is one more product of the high parts alone, (kappa X_h) Y_h, with
-// tau and s applied to its sums.  A table that this does not reproduce to
-// 3e-7 of the component's largest amplitude (bins that jump inside a block, a
+// tau and s applied to its sums.  A table that this does not reproduce
+// (mm::kFitTol: bins that jump inside a block, a
 // slope that differs from bin to bin) stays on k_beam_dft.
 //
 // A block of threads is 4 waves with a row each; an item is (pass of 16
@@ -456,24 +456,8 @@ __global__ __launch_bounds__(kRows, kBlocksPerCU) void k_beam_dft(Desc d) {
 // beam channels: 5.59 ms on k_beam_dft, 1.35 with two blocks, 1.20 with three;
 // 7,020 rows x 128 channels x 700 components, 4 correlations, spectra: 888 us
 // on k_beam_dft, 450 here.
-constexpr int kMmTile = 32;          // components a tile
-// slots of a 4-component block: 32 rows (A) or 16 columns (B) + 1 (k_dft_mfma's
-// layout); 16-byte slots of one operand part
-constexpr int kMmRA = 33, kMmRB = 17;
-constexpr int kMmSlotsA = 8 * kMmRA, kMmSlotsB = 8 * kMmRB;
-constexpr int kMmT = 16;             // channels of a block
-constexpr int kMmPass = 16;          // blocks of a pass
-
-struct Blk {
-  double fc;            // nu/nu0 of channel ch0 + 8
-  int IF, ch0;          // first channel (t = -8)
-  int vlo, vhi;         // channels the block writes
-  int jc;               // beam channel
-  float s;              // df (1 / fc - 1 / f0), f0 the pass's reference
-};
-
 struct MmTab {
-  const Blk *blk;
+  const mm::Blk *blk;
   int nblk, npass, ncpad;     // ncpad: components padded with zeros (a whole tile of them at least)
   const float4 *prod;         // [2][npair][npass * 16][ncpad]: conj C of a correlation pair, scaled
   const unsigned *amax;       // largest |C| (float bits)
@@ -482,24 +466,18 @@ struct MmTab {
   const float *r0;            // [npass]: df / f0
 };
 
-// exponent that brings amax to [2^13, 2^14)
-__device__ __forceinline__ int mm_shift(unsigned bits) {
-  const int e = (int)((bits >> 23) & 255u) - 126;
-  return bits == 0u ? 0 : 14 - e;
-}
-
 // C of every (correlation pair, type pair, block, component): the largest
 // finite part to amax (WRITE false), then the scaled conjugates to prod.
 template <bool WRITE>
 __global__ __launch_bounds__(256) void k_beam_prod(const float *__restrict__ jones, const float *__restrict__ camp,
-                                                   const float *__restrict__ Ab, const Blk *__restrict__ blk,
+                                                   const float *__restrict__ Ab, const mm::Blk *__restrict__ blk,
                                                    int nblk, int nblkPad, int ntype, int ncomp, int ncpad, int njchan,
                                                    int nep, int stokType, float c, float s,
                                                    unsigned *__restrict__ amax, float4 *__restrict__ prod) {
   const int npair = ntype * ntype;
   const long long n = (long long)npair * nblk * ncpad;
   float big = 0.0f;
-  const float sc = WRITE ? ldexpf(1.0f, mm_shift(*amax)) : 1.0f;
+  const float sc = WRITE ? ldexpf(1.0f, mm::shift_of(*amax)) : 1.0f;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
     const int k = (int)(i % ncpad);
@@ -536,86 +514,6 @@ __global__ __launch_bounds__(256) void k_beam_prod(const float *__restrict__ jon
     for (int o = 32; o > 0; o >>= 1) big = fmaxf(big, __shfl_xor(big, o));
     if ((threadIdx.x & 63) == 0 && big > 0.0f) atomicMax(amax, __float_as_uint(big));
   }
-}
-
-__global__ void k_beam_zero(unsigned *a) { *a = 0u; }
-
-// The factors A_kb G_k(t) (1 + kappa_k tau(t) s_b) of the amplitude table
-// (see above), one thread a component and pass; resid: the largest relative
-// residual (float bits).  G is the shape of the pass's reference block, the
-// first from its middle with an amplitude there; A and the slope of each block
-// are taken at two channels 0.7 of the way to its ends, which halves the error
-// of the linear term at them; kappa is the slopes' least-squares fit to s_b.
-__global__ __launch_bounds__(64) void k_beam_fit(const float *__restrict__ tab, int nchan, long long ldk,
-                                                 const Blk *__restrict__ blk, int nblk, const float *__restrict__ r0,
-                                                 int ncomp, int ncpad, float *__restrict__ Ab, float *__restrict__ G,
-                                                 unsigned *__restrict__ kap, unsigned *__restrict__ resid) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x, ps = blockIdx.y;
-  float worst = 0.0f;
-  if (k < ncomp) {
-    const float *row = tab + (long long)k * ldk;
-    const int b0 = ps * kMmPass, nb = min(kMmPass, nblk - b0);
-    auto amp = [&](int b, int t) {
-      const int ch = min(max(blk[b].ch0 + 8 + t, 0), nchan - 1);
-      return (double)row[(long long)blk[b].IF * nchan + ch];
-    };
-    int ref = b0 + nb / 2;
-    for (int i = 0; i < nb && amp(ref, 0) == 0.0; ++i) ref = b0 + i;
-    const double a0 = amp(ref, 0);
-    double g[kMmT];
-    for (int t = -8; t < 8; ++t) {
-      g[t + 8] = a0 != 0.0 ? amp(ref, t) / a0 : 1.0;
-      if (!(fabs(g[t + 8]) > 1e-3 && fabs(g[t + 8]) < 1e3)) g[t + 8] = 1.0;  // the residual tells
-      g[t + 8] = (double)(float)g[t + 8];
-      G[((long long)ps * kMmT + t + 8) * ncpad + k] = (float)g[t + 8];
-    }
-    const double r = r0[ps];
-    auto tau = [&](int t) { return (double)t - (double)t * (double)t * r; };
-    auto ends = [&](int b, int &t1, int &t2) {
-      const double lo = blk[b].vlo - blk[b].ch0 - 8, hi = blk[b].vhi - blk[b].ch0 - 8;
-      const double m = 0.5 * (lo + hi), w = 0.35 * (hi - lo);
-      t1 = (int)rint(m - w);
-      t2 = (int)rint(m + w);
-    };
-    double num = 0.0, den = 0.0, big = 0.0;
-    for (int b = b0; b < b0 + nb; ++b) {
-      int t1, t2;
-      ends(b, t1, t2);
-      const double p1 = amp(b, t1) / g[t1 + 8], p2 = amp(b, t2) / g[t2 + 8];
-      const double d = p1 * tau(t2) - p2 * tau(t1), s = blk[b].s;
-      if (t2 > t1 && d != 0.0 && s != 0.0) {
-        num += (p2 - p1) / d * s;
-        den += s * s;
-      }
-    }
-    double ka = den > 0.0 ? num / den : 0.0;
-    if (!(fabs(ka) < 1e3)) ka = 0.0;
-    const _Float16 kh = (_Float16)(float)ka;
-    ka = (double)(float)kh;
-    kap[(long long)ps * ncpad + k] = (unsigned)__builtin_bit_cast(unsigned short, kh) * 0x10001u;
-    double off = 0.0;
-    for (int b = b0; b < b0 + nb; ++b) {
-      int t1, t2;
-      ends(b, t1, t2);
-      const double s = blk[b].s;
-      const double A = 0.5 * (amp(b, t1) / (g[t1 + 8] * (1.0 + ka * tau(t1) * s)) +
-                              amp(b, t2) / (g[t2 + 8] * (1.0 + ka * tau(t2) * s)));
-      Ab[(long long)b * ncpad + k] = (float)A;
-      for (int ch = blk[b].vlo; ch <= blk[b].vhi; ++ch) {
-        const int t = ch - blk[b].ch0 - 8;
-        const double a = amp(b, t), e = fabs(a - (double)(float)A * g[t + 8] * (1.0 + ka * tau(t) * s));
-        big = fmax(big, fabs(a));
-        off = (e >= off) ? e : (e < off ? off : INFINITY);  // a NaN counts as infinite
-      }
-    }
-    worst = big > 0.0 ? (float)(off / big) : (off > 0.0 ? INFINITY : 0.0f);
-    if (!(worst >= 0.0f)) worst = INFINITY;
-  } else if (k < ncpad) {
-    for (int t = 0; t < kMmT; ++t) G[((long long)ps * kMmT + t) * ncpad + k] = 1.0f;
-    kap[(long long)ps * ncpad + k] = 0u;
-  }
-  for (int o = 32; o > 0; o >>= 1) worst = fmaxf(worst, __shfl_xor(worst, o));
-  if ((threadIdx.x & 63) == 0 && worst > 0.0f) atomicMax(resid, __float_as_uint(worst));
 }
 
 // Whether any correlation of a channel is unflagged.
@@ -655,19 +553,11 @@ template <bool AMP, bool ONE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3, AMP ? 2 : 3))) void k_beam_mm(
     Desc d, MmTab m, int ncorr, int nep, int split) {
   constexpr int NE = ONE ? 1 : 2;  // correlations a column block of a lane has
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-  __shared__ uint4 s_op[4][2 * kMmSlotsA + 2 * kMmSlotsB];
+  __shared__ uint4 s_op[4][mm::kSlots];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  uint4 *sAh = s_op[wv], *sAl = sAh + kMmSlotsA, *sBh = sAl + kMmSlotsA, *sBl = sBh + kMmSlotsB;
-  const int i = lane & 15, qd = lane >> 4;   // matrix-step roles
-  const int kc = lane & 31, h = lane >> 5;   // set-up roles: component, half
-  unsigned *wA = reinterpret_cast<unsigned *>(sAh + (kc >> 2) * kMmRA + 16 * h) + (kc & 3);
-  unsigned *wB = reinterpret_cast<unsigned *>(sBh + (kc >> 2) * kMmRB + 8 * h) + (kc & 3);
-  constexpr int kLoA = 4 * kMmSlotsA, kLoB = 4 * kMmSlotsB;  // words from the _h to the _l array
+  const int qd = lane >> 4, h = lane >> 5;   // output rows; set-up half
   const double df = d.dfIF[d.IFb];           // the same for every selected IF
-  const double wdf = h ? 6.0 * df : df;
   const long long nquad = (d.nrow + 3) / 4;
   for (long long it = blockIdx.x; it < nquad * nep * m.npass; it += gridDim.x) {
     const long long rq = it % nquad;
@@ -689,168 +579,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
     unsigned po[8];  // offset of a block's products
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-      const int g = min(split ? b : ps * kMmPass + 8 * h + b, m.nblk - 1);
+      const int g = min(split ? b : ps * mm::kPass + 8 * h + b, m.nblk - 1);
       fc[b] = -m.blk[g].fc;
       po[b] = (unsigned)g * (unsigned)m.ncpad;
     }
     const float4 *prod = m.prod + ((long long)(split && !ONE ? h : ep) * d.npair + pair) *
-                                      (long long)m.npass * kMmPass * m.ncpad;
-    const float *G = AMP ? m.G + ((long long)ps * kMmT + (h ? 8 : 7)) * m.ncpad : nullptr;
+                                      (long long)m.npass * mm::kPass * m.ncpad;
+    const float *G = AMP ? m.G + ((long long)ps * mm::kT + (h ? 8 : 7)) * m.ncpad : nullptr;
     const int gstep = h ? m.ncpad : -m.ncpad;
     const unsigned *kap = AMP ? m.kap + (long long)ps * m.ncpad : nullptr;
     double o[2][NE][4];
-    f4 d2[2][NE];
-#pragma unroll
-    for (int T = 0; T < 2; ++T)
-#pragma unroll
-      for (int e = 0; e < NE; ++e) {
-        d2[T][e] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[T][e][r] = 0.0;
-      }
-    // the next tile's positions, read a tile ahead
-    double nx, ny, nz;
-    auto fetch = [&](int k0) {
-      const int k = min(k0 + kc, d.ncomp - 1);
-      nx = d.cx[k];
-      ny = d.cy[k];
-      nz = d.cz[k];
-    };
-    fetch(0);
-    for (int k4 = 0; k4 < d.ncomp; k4 += 2 * kMmTile) {
-      f4 acc[2][NE];
-#pragma unroll
-      for (int T = 0; T < 2; ++T)
-#pragma unroll
-        for (int e = 0; e < NE; ++e) acc[T][e] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-      for (int kt = 0; kt < 2; ++kt) {
-        const int k0 = k4 + kt * kMmTile;
-        if (k0 >= d.ncomp) break;
-        // this tile's products and shape, used after the powers below
-        const unsigned kp = (unsigned)(k0 + kc);
-        float4 pr[8];
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-          if (ONE) {
-            const float2 x = reinterpret_cast<const float2 *>(prod)[2u * (po[b] + kp) + (unsigned)h];
-            pr[b] = make_float4(x.x, x.y, 0.0f, 0.0f);
-          } else {
-            pr[b] = prod[po[b] + kp];
-          }
-        }
-        float g[8];
-        if (AMP) {
-          // slot c of this half: t = c (second half) or -(c + 1)
-#pragma unroll
-          for (int c = 0; c < 8; ++c) g[c] = G[(int)kp + c * gstep];
-        }
-        const double psi = fma(w, nz, fma(v, ny, u * nx));
-        fetch(k0 + kMmTile);
-        {
-          const float2 s1 = eturn<false>(psi * wdf);
-          float2 z[9];
-          swap_halves(s1, z[1], z[6]);
-          z[2] = cmul(z[1], z[1]);
-          z[3] = cmul(z[2], z[1]);
-          auto cjmul = [](float2 a, float2 b) {  // a conj(b)
-            return make_float2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
-          };
-          z[4] = cjmul(z[6], z[2]);
-          z[5] = cjmul(z[6], z[1]);
-          z[7] = cmul(z[6], z[1]);
-          z[8] = cmul(z[6], z[2]);
-          z[0] = make_float2(1.0f, 0.0f);
-#pragma unroll
-          for (int c = 0; c < 8; ++c) {
-            float xr = h ? z[c].x : z[c + 1].x, xi = h ? z[c].y : -z[c + 1].y;
-            if (AMP) { xr *= g[c]; xi *= g[c]; }
-            unsigned xh, xl;
-            split_pair(xr, xi, xh, xl);
-            wA[4 * c] = xh;
-            wA[4 * c + kLoA] = xl;
-            wA[4 * (c + 8)] = swap_neg(xh);
-            wA[4 * (c + 8) + kLoA] = swap_neg(xl);
-          }
-        }
-        // the first correlation's Y into the operand area, the second's kept
-        // until the first's are read
-        unsigned y1h[8], y1l[8];
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-          const float2 pg = eturn<true>(psi * fc[b]);  // conj P
-          const float2 y0 = cmul(pg, make_float2(pr[b].x, pr[b].y));
-          unsigned yh, yl;
-          split_pair(y0.x, y0.y, yh, yl);
-          wB[4 * b] = yh;
-          wB[4 * b + kLoB] = yl;
-          if (!ONE) {
-            const float2 y1 = cmul(pg, make_float2(pr[b].z, pr[b].w));
-            split_pair(y1.x, y1.y, y1h[b], y1l[b]);
-          }
-        }
-        // a wave's LDS accesses complete in order: writes, reads, writes, reads
-        h8 ah[2][2], al[2][2];  // [step][tile]
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int e = 0; e < NE; ++e) {
-          h8 bh[2], bl[2];
-          if (e) {
-#pragma unroll
-            for (int b = 0; b < 8; ++b) {
-              wB[4 * b] = y1h[b];
-              wB[4 * b + kLoB] = y1l[b];
-            }
-            asm volatile("" ::: "memory");
-          }
-#pragma unroll
-          for (int s = 0; s < 2; ++s) {
-            if (!e) {
-#pragma unroll
-              for (int T = 0; T < 2; ++T) {
-                const int at = (qd + 4 * s) * kMmRA + 16 * T + i;
-                ah[s][T] = __builtin_bit_cast(h8, sAh[at]);
-                al[s][T] = __builtin_bit_cast(h8, sAl[at]);
-              }
-            }
-            bh[s] = __builtin_bit_cast(h8, sBh[(qd + 4 * s) * kMmRB + i]);
-            bl[s] = __builtin_bit_cast(h8, sBl[(qd + 4 * s) * kMmRB + i]);
-          }
-          asm volatile("" ::: "memory");
-#pragma unroll
-          for (int s = 0; s < 2; ++s) {
-#pragma unroll
-            for (int T = 0; T < 2; ++T)
-              acc[T][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s][T], bh[s], acc[T][e], 0, 0, 0);
-#pragma unroll
-            for (int T = 0; T < 2; ++T)
-              acc[T][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s][T], bl[s], acc[T][e], 0, 0, 0);
-#pragma unroll
-            for (int T = 0; T < 2; ++T)
-              acc[T][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[s][T], bh[s], acc[T][e], 0, 0, 0);
-            if (AMP) {
-              const h8 ks = __builtin_bit_cast(h8, *reinterpret_cast<const uint4 *>(kap + k0 + 4 * (qd + 4 * s)));
-#pragma unroll
-              for (int T = 0; T < 2; ++T)
-                d2[T][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s][T] * ks, bh[s], d2[T][e], 0, 0, 0);
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int T = 0; T < 2; ++T)
-#pragma unroll
-        for (int e = 0; e < NE; ++e)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[T][e][r] += (double)acc[T][e][r];
-    }
+    mm::f4 d2[2][NE];
+    mm::sum<AMP, NE, false>(s_op[wv], d.cx, d.cy, d.cz, d.ncomp, 0, d.ncomp, u, v, w, df, fc, po,
+                            ONE ? (const void *)(reinterpret_cast<const float2 *>(prod) + h) : (const void *)prod,
+                            ONE ? 2u : 1u, G, gstep, kap, o, d2);
     // lanes 0..31 hold the Re of slots c = 4 (lane / 16) + r of tile T, lane +
     // 32 the Im of the same; column n = lane mod 16 is block n of the pass, or
     // with split block n mod 8 of correlation or pair n / 8
     const int n = lane & 15, nb = split ? n & 7 : n, cp = !ONE && split ? n >> 3 : ep;
-    const Blk bk = m.blk[min(ps * kMmPass + nb, m.nblk - 1)];
-    const bool have = lane < 32 && ps * kMmPass + nb < m.nblk;
-    const double unscale = ldexp(1.0, -mm_shift(*m.amax));
+    const mm::Blk bk = m.blk[min(ps * mm::kPass + nb, m.nblk - 1)];
+    const bool have = lane < 32 && ps * mm::kPass + nb < m.nblk;
+    const double unscale = ldexp(1.0, -mm::shift_of(*m.amax));
     const float r0 = AMP ? m.r0[ps] : 0.0f;
     float *base = d.vis + row * (long long)d.lrec + d.nrparm + (long long)bk.IF * d.incif;
 #pragma unroll
@@ -1048,7 +797,7 @@ struct ObitHIPBeam {
   // mmAmp: the amplitude table has its factors (SetAmps)
   int nblk = 0, npass = 0, ncpad = 0;
   bool mmTables = false, mmAmp = false;
-  obit::beam::Blk *d_blk = nullptr;
+  obit::mm::Blk *d_blk = nullptr;
   float *d_r0 = nullptr, *d_Ab = nullptr, *d_G = nullptr;
   unsigned *d_kap = nullptr, *d_mm = nullptr;  // d_mm: largest |C|, fit residual (float bits)
   float4 *d_prod = nullptr;
@@ -1077,8 +826,8 @@ bool use_mm(const ObitHIPBeam *h) { return h->mmTables && (!h->d_tab || h->mmAmp
 // shorter than a block is one block.  Empty where the IFs' channel steps
 // differ (the kernel has one).
 void mm_blocks(const ObitHIPBeamDesc &D, const double *fIF, const double *dfIF, const int *jmap,
-               std::vector<obit::beam::Blk> &blk, std::vector<float> &r0) {
-  using namespace obit::beam;
+               std::vector<obit::mm::Blk> &blk, std::vector<float> &r0) {
+  using namespace obit;
   blk.clear();
   r0.clear();
   const double df = dfIF[D.IFb];
@@ -1089,12 +838,12 @@ void mm_blocks(const ObitHIPBeamDesc &D, const double *fIF, const double *dfIF, 
     for (int c = D.chanb; c <= D.chane;) {
       int e = c;
       while (e < D.chane && jm[e + 1] == jm[c]) ++e;
-      for (int a = c; a <= e; a += kMmT) {
-        Blk b{};
+      for (int a = c; a <= e; a += mm::kT) {
+        mm::Blk b{};
         b.IF = i;
-        b.ch0 = std::max(c, std::min(a, e - kMmT + 1));
+        b.ch0 = std::max(c, std::min(a, e - mm::kT + 1));
         b.vlo = a;
-        b.vhi = std::min(e, a + kMmT - 1);
+        b.vhi = std::min(e, a + mm::kT - 1);
         b.jc = jm[c];
         b.fc = fIF[i] + (double)(b.ch0 + 8) * dfIF[i];
         blk.push_back(b);
@@ -1102,8 +851,8 @@ void mm_blocks(const ObitHIPBeamDesc &D, const double *fIF, const double *dfIF, 
       c = e + 1;
     }
   }
-  for (size_t p = 0; p < blk.size(); p += kMmPass) {
-    const size_t n = std::min<size_t>(kMmPass, blk.size() - p);
+  for (size_t p = 0; p < blk.size(); p += mm::kPass) {
+    const size_t n = std::min<size_t>(mm::kPass, blk.size() - p);
     const double f0 = blk[p + n / 2].fc;
     r0.push_back((float)(df / f0));
     for (size_t b = p; b < p + n; ++b) blk[b].s = (float)(df * (1.0 / blk[b].fc - 1.0 / f0));
@@ -1121,7 +870,7 @@ int mm_tables(ObitHIPBeam *h) {
   if (h->gauss || D.ncomp < 1 || h->nblk < 1) return kOK;
   const double sel = (double)(D.IFe - D.IFb + 1) * (D.chane - D.chanb + 1);
   if (sel < 0.3 * 256.0 * h->npass) return kOK;
-  const size_t nbp = (size_t)h->npass * beam::kMmPass, nep = D.ncorr == 4 ? 2 : 1;
+  const size_t nbp = (size_t)h->npass * mm::kPass, nep = D.ncorr == 4 ? 2 : 1;
   const size_t ncpad = ((size_t)D.ncomp + 31) / 32 * 32 + 32;
   const size_t nprod = nep * D.ntype * D.ntype * nbp * ncpad;
   if (nprod * sizeof(float4) > (size_t(512) << 20) || nbp * ncpad > 0x3fffffffULL) return kOK;
@@ -1134,26 +883,26 @@ int mm_tables(ObitHIPBeam *h) {
   return kOK;
 }
 
-// The factors of the amplitude table for k_beam_mm (k_beam_fit), and whether
+// The factors of the amplitude table for k_beam_mm (mm::k_fit), and whether
 // they reproduce it.
 int mm_fit(ObitHIPBeam *h) {
   using namespace obit;
   const ObitHIPBeamDesc &D = h->desc;
   h->mmAmp = false;
   if (!h->mmTables || !h->d_tab) return kOK;
-  const size_t nbp = (size_t)h->npass * beam::kMmPass, nc = (size_t)h->ncpad;
+  const size_t nbp = (size_t)h->npass * mm::kPass, nc = (size_t)h->ncpad;
   if (!h->d_Ab) OBIT_HIP_TRY(hipMalloc(&h->d_Ab, nbp * nc * sizeof(float)));
-  if (!h->d_G) OBIT_HIP_TRY(hipMalloc(&h->d_G, (size_t)h->npass * beam::kMmT * nc * sizeof(float)));
+  if (!h->d_G) OBIT_HIP_TRY(hipMalloc(&h->d_G, (size_t)h->npass * mm::kT * nc * sizeof(float)));
   if (!h->d_kap) OBIT_HIP_TRY(hipMalloc(&h->d_kap, (size_t)h->npass * nc * sizeof(unsigned)));
-  hipLaunchKernelGGL(beam::k_beam_zero, dim3(1), dim3(1), 0, h->stream, h->d_mm + 1);
-  hipLaunchKernelGGL(beam::k_beam_fit, dim3((unsigned)((nc + 63) / 64), (unsigned)h->npass), dim3(64), 0, h->stream,
-                     h->d_tab, D.nchan, (long long)D.nif * D.nchan, h->d_blk, h->nblk, h->d_r0, D.ncomp, h->ncpad,
-                     h->d_Ab, h->d_G, h->d_kap, h->d_mm + 1);
+  hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(64), 0, h->stream, h->d_mm + 1, 1);
+  hipLaunchKernelGGL(mm::k_fit, dim3((unsigned)((nc + 63) / 64), (unsigned)h->npass), dim3(64), 0, h->stream,
+                     h->d_tab, D.nchan, D.nchan, (long long)D.nif * D.nchan, h->d_blk, h->nblk, h->d_r0, D.ncomp, h->ncpad,
+                     h->d_Ab, h->d_G, h->d_kap, h->d_mm + 1, nullptr);
   OBIT_HIP_TRY(hipGetLastError());
   float worst = 0.0f;
   OBIT_HIP_TRY(hipStreamSynchronize(h->stream));
   OBIT_HIP_TRY(hipMemcpy(&worst, h->d_mm + 1, sizeof(float), hipMemcpyDeviceToHost));
-  h->mmAmp = worst <= 3e-7f;
+  h->mmAmp = worst <= mm::kFitTol;
   return kOK;
 }
 
@@ -1174,12 +923,12 @@ int beam_coh(ObitHIPBeam *h, float parAng, hipStream_t stream) {
     const float *Ab = h->d_tab ? h->d_Ab : nullptr;
     const long long n = (long long)D.ntype * D.ntype * h->nblk * h->ncpad;
     const dim3 grid((unsigned)std::min<long long>((n + 255) / 256, (long long)std::max(h->ncu, 1) * 16));
-    hipLaunchKernelGGL(beam::k_beam_zero, dim3(1), dim3(1), 0, stream, h->d_mm);
+    hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(64), 0, stream, h->d_mm, 1);
     hipLaunchKernelGGL((beam::k_beam_prod<false>), grid, dim3(256), 0, stream, h->d_jones, h->d_amp, Ab, h->d_blk,
-                       h->nblk, h->npass * beam::kMmPass, D.ntype, D.ncomp, h->ncpad, D.njchan, nep, D.stokType,
+                       h->nblk, h->npass * mm::kPass, D.ntype, D.ncomp, h->ncpad, D.njchan, nep, D.stokType,
                        (float)c2, (float)s2, h->d_mm, h->d_prod);
     hipLaunchKernelGGL((beam::k_beam_prod<true>), grid, dim3(256), 0, stream, h->d_jones, h->d_amp, Ab, h->d_blk,
-                       h->nblk, h->npass * beam::kMmPass, D.ntype, D.ncomp, h->ncpad, D.njchan, nep, D.stokType,
+                       h->nblk, h->npass * mm::kPass, D.ntype, D.ncomp, h->ncpad, D.njchan, nep, D.stokType,
                        (float)c2, (float)s2, h->d_mm, h->d_prod);
     OBIT_HIP_TRY(hipGetLastError());
     return kOK;
@@ -1326,11 +1075,11 @@ int ObitHIPBeamDFTCreate(ObitHIPBeam **out, const ObitHIPBeamDesc *desc, const d
   if (!rc) rc = up((void **)&h->d_jones, nullptr, (size_t)d.ntype * nc * d.njchan * 8 * sizeof(float));
   if (!rc) rc = up((void **)&h->d_coh, nullptr, (size_t)d.ntype * d.ntype * nc * d.njchan * 4 * sizeof(float2));
   if (!rc) rc = ObitHIPBeamDFTSetJones(h, nullptr);
-  std::vector<beam::Blk> blk;
+  std::vector<mm::Blk> blk;
   std::vector<float> r0;
   mm_blocks(d, fIF, dfIF, visJChan, blk, r0);
   if (!rc && !blk.empty()) {
-    rc = up((void **)&h->d_blk, blk.data(), blk.size() * sizeof(beam::Blk));
+    rc = up((void **)&h->d_blk, blk.data(), blk.size() * sizeof(mm::Blk));
     if (!rc) rc = up((void **)&h->d_r0, r0.data(), r0.size() * sizeof(float));
     h->nblk = (int)blk.size();
     h->npass = (int)r0.size();

@@ -634,6 +634,85 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   }
 }
 
+// ---- spectral models on the matrix units ----
+//
+// k_dft_mfma's factoring with an amplitude a_k(c) of every channel: the
+// selected channels in blocks of 16 of one IF and (tabulated spectra) one
+// coarse bin, the amplitude table as A_kb G_k(t) (1 + kappa_k tau(t) s_b)
+// (mm::k_fit), the sums by mm::sum, a wave a row, 16 blocks a pass.  The items
+// are (component part, pass, row quad).  Taken where the fit reproduces the
+// table (mm::kFitTol).  Bound by VALU issue (303 instructions and 16 matrix
+// steps a tile of 32 components x 256 channels): 10.0e12 evaluations/s at
+// 4 x 256 channels against 5.7e12 on k_dft_split, at half its error (2.2e-7
+// against 4.7e-7 of the model's norm).
+struct SpecTab {
+  const mm::Blk *blk;     // fc, IF (selected), ch0 .. relative to chanb
+  int nblk, npass, ncpad;
+  const float *Ab, *G, *r0;
+  const unsigned *kap;
+  int shift;              // A is scaled by 2^shift
+};
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_dft_spec(Desc d, SpecTab m) {
+  __shared__ uint4 s_op[4][mm::kSlots];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qd = lane >> 4, h = lane >> 5;
+  const double df = d.fdel[0];
+  const long long nquad = (d.nrow + 3) / 4;
+  const int nsplit = max(d.nsplit, 1);
+  for (long long it = blockIdx.x; it < nquad * m.npass * nsplit; it += gridDim.x) {
+    const long long rq = it % nquad;
+    const int q = (int)(it / nquad), ps = q % m.npass, part = q / m.npass;
+    const int kBeg = part * d.kpart, kEnd = nsplit > 1 ? min(d.ncomp, kBeg + d.kpart) : d.ncomp;
+    const long long row = rq * 4 + wv;
+    if (row >= d.nrow) continue;
+    const float *rp = d.vis + row * (long long)d.lrec;
+    const double u = rp[d.ilocu], v = rp[d.ilocv], w = rp[d.ilocw];
+    double fc[8];
+    unsigned po[8];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const int g = min(ps * mm::kPass + 8 * h + b, m.nblk - 1);
+      fc[b] = -m.blk[g].fc;
+      po[b] = (unsigned)g * (unsigned)m.ncpad;
+    }
+    const float *G = m.G + ((long long)ps * mm::kT + (h ? 8 : 7)) * m.ncpad;
+    double o[2][1][4];
+    mm::f4 d2[2][1];
+    mm::sum<true, 1, true>(s_op[wv], d.cx, d.cy, d.cz, d.ncomp, kBeg, kEnd, u, v, w, df, fc, po, m.Ab, 1u, G,
+                           h ? m.ncpad : -m.ncpad, m.kap + (long long)ps * m.ncpad, o, d2);
+    const int n = lane & 15;
+    const mm::Blk bk = m.blk[min(ps * mm::kPass + n, m.nblk - 1)];
+    const bool have = lane < 32 && ps * mm::kPass + n < m.nblk;
+    const double unscale = ldexp(1.0, -m.shift);
+    const float r0 = m.r0[ps];
+    float *base = d.vis + row * (long long)d.lrec + d.nrparm + (d.IFb + bk.IF) * d.incif + d.chanb * d.incf +
+                  d.stokb * d.incs;
+    double2 *pp = d.part ? d.part + (((long long)part * d.nrow + row) * d.nIFsel + bk.IF) * d.nchsel : nullptr;
+#pragma unroll
+    for (int T = 0; T < 2; ++T)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int c = 4 * (qd & 1) + r, t = T ? c : -(c + 1), ch = bk.ch0 + 8 + t;
+        double x = o[T][0][r] + (double)(((float)t - (float)(t * t) * r0) * bk.s * d2[T][0][r]);
+        double y = __shfl_xor(x, 32);
+        x *= unscale;
+        y *= unscale;
+        if (!have || ch < bk.vlo || ch > bk.vhi) continue;
+        if (pp) pp[ch] = make_double2(x, y);
+        else apply_op(d, base + ch * d.incf, (float)x, (float)y);
+      }
+  }
+}
+
+// n amplitudes times 2^shift
+__global__ void k_scale(float *a, long long n, int shift) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x)
+    a[i] = ldexpf(a[i], shift);
+}
+
 // The sums of the nsplit component parts of every (row, IF, channel),
 // added in part order in FP64, applied to the row as k_dft_split applies
 // its own.
@@ -848,6 +927,13 @@ struct State {
   size_t tabCap = 0;
   bool tabReady = false;
   long long tabKey = -1;
+  // the table's factors for k_dft_spec, if they reproduce it
+  bool specMm = false;
+  SpecTab spec{};
+  mm::Blk *sblk = nullptr;
+  float *sbuf = nullptr;     // A [npass * 16][ncpad], G [npass][16][ncpad], kappa [npass][ncpad], r0 [npass]
+  size_t sblkCap = 0, sbufCap = 0;
+  unsigned *smax = nullptr;  // residual, largest |A|
   // frequencies
   std::vector<double> freq64;
   double uvRef = 0.0;
@@ -983,6 +1069,90 @@ int frequency_lines(State *st, const GPUVisInfo *vi, std::vector<double> &fb,
   return kOK;
 }
 
+// The factors of the amplitude table for k_dft_spec: channel blocks (runs of
+// one coarse bin in blocks of 16, a run's last block moved back to end with
+// it), then mm::k_fit and the scale.  Points only, one channel step for every
+// IF, and at least 0.55 of the 256 channel slots a pass selected channels:
+// below that k_dft_split (5.7e12 evaluations/s) is faster than the filled part
+// of k_dft_spec's 10.0e12.
+int spec_factors(State *st, int nIFsel, int nchsel, int nchpad, const std::vector<double> &fb,
+                 const std::vector<double> &fdl, const std::vector<int> &bin) {
+  st->specMm = false;
+  if (st->ncomp < 1 || model_gauss_off(st->type) >= 0 || !st->uniform) return kOK;
+  for (int i = 1; i < nIFsel; ++i)
+    if (!(std::fabs(fdl[i] - fdl[0]) <= 1e-12 * std::fabs(fdl[0]))) return kOK;
+  std::vector<mm::Blk> blk;
+  for (int i = 0; i < nIFsel; ++i)
+    for (int c = 0; c < nchsel;) {
+      int e = c;
+      while (e + 1 < nchsel && bin[(size_t)i * nchsel + e + 1] == bin[(size_t)i * nchsel + c]) ++e;
+      for (int a = c; a <= e; a += mm::kT) {
+        mm::Blk b{};
+        b.IF = i;
+        b.ch0 = std::max(c, std::min(a, e - mm::kT + 1));
+        b.vlo = a;
+        b.vhi = std::min(e, a + mm::kT - 1);
+        b.fc = fb[i] + (double)(b.ch0 + 8) * fdl[i];
+        blk.push_back(b);
+      }
+      c = e + 1;
+    }
+  const size_t npass = (blk.size() + mm::kPass - 1) / mm::kPass;
+  if ((double)nIFsel * nchsel < 0.55 * 256.0 * (double)npass) return kOK;
+  const size_t ncpad = ((size_t)st->ncomp + 31) / 32 * 32 + 32, nA = npass * mm::kPass * ncpad;
+  if (nA > 0x3fffffffULL) return kOK;
+  std::vector<float> r0(npass);
+  for (size_t p = 0; p < npass; ++p) {
+    const size_t b0 = p * mm::kPass, n = std::min<size_t>(mm::kPass, blk.size() - b0);
+    const double f0 = blk[b0 + n / 2].fc;
+    r0[p] = (float)(fdl[0] / f0);
+    for (size_t b = b0; b < b0 + n; ++b) blk[b].s = (float)(fdl[0] * (1.0 / blk[b].fc - 1.0 / f0));
+  }
+  if (blk.size() > st->sblkCap) {
+    destroy_graph(st);  // a captured launch reads the old blocks
+    (void)hipFree(st->sblk);
+    st->sblk = nullptr;
+    st->sblkCap = 0;
+    OBIT_HIP_TRY(hipMalloc(&st->sblk, blk.size() * sizeof(mm::Blk)));
+    st->sblkCap = blk.size();
+  }
+  const size_t need = nA + npass * mm::kT * ncpad + npass * ncpad + npass;
+  if (need > st->sbufCap) {
+    destroy_graph(st);
+    (void)hipFree(st->sbuf);
+    st->sbuf = nullptr;
+    st->sbufCap = 0;
+    if (hipMalloc(&st->sbuf, need * sizeof(float)) != hipSuccess) {
+      (void)hipGetLastError();
+      return kOK;  // no room: k_dft_split
+    }
+    st->sbufCap = need;
+  }
+  if (!st->smax) OBIT_HIP_TRY(hipMalloc(&st->smax, 2 * sizeof(unsigned)));
+  float *Ab = st->sbuf, *G = Ab + nA, *kap = G + npass * mm::kT * ncpad, *dr0 = kap + npass * ncpad;
+  OBIT_HIP_TRY(hipMemcpy(st->sblk, blk.data(), blk.size() * sizeof(mm::Blk), hipMemcpyHostToDevice));
+  OBIT_HIP_TRY(hipMemcpy(dr0, r0.data(), npass * sizeof(float), hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(64), 0, st->stream, st->smax, 2);
+  hipLaunchKernelGGL(mm::k_fit, dim3((unsigned)((ncpad + 63) / 64), (unsigned)npass), dim3(64), 0, st->stream,
+                     st->tab, nchsel, nchpad, (long long)nIFsel * nchpad, st->sblk, (int)blk.size(), dr0, st->ncomp,
+                     (int)ncpad, Ab, G, reinterpret_cast<unsigned *>(kap), st->smax, st->smax + 1);
+  OBIT_HIP_TRY(hipGetLastError());
+  unsigned got[2];
+  OBIT_HIP_TRY(hipMemcpyAsync(got, st->smax, sizeof(got), hipMemcpyDeviceToHost, st->stream));
+  OBIT_HIP_TRY(hipStreamSynchronize(st->stream));
+  float worst, top;
+  std::memcpy(&worst, got, sizeof(float));
+  std::memcpy(&top, got + 1, sizeof(float));
+  if (!(worst <= mm::kFitTol) || !std::isfinite(top)) return kOK;
+  const int shift = mm::shift_of(got[1]);
+  hipLaunchKernelGGL(k_scale, dim3(256), dim3(256), 0, st->stream, Ab, (long long)(blk.size() * ncpad), shift);
+  OBIT_HIP_TRY(hipGetLastError());
+  st->spec = SpecTab{st->sblk, (int)blk.size(), (int)npass, (int)ncpad, Ab, G, dr0,
+                     reinterpret_cast<unsigned *>(kap), shift};
+  st->specMm = true;
+  return kOK;
+}
+
 // Build (or reuse) the spectral amplitude table for the current selection.
 int ensure_spec_table(State *st, const GPUInfo *gi) {
   const GPUVisInfo *vi = gi->h_visInfo;
@@ -1046,6 +1216,8 @@ int ensure_spec_table(State *st, const GPUInfo *gi) {
                        nIFsel, nchsel, nchpad, st->tab);
     OBIT_HIP_TRY(hipGetLastError());
   }
+  rc = spec_factors(st, nIFsel, nchsel, nchpad, fb, fdl, bin);
+  if (rc) return rc;
   OBIT_HIP_TRY(hipStreamSynchronize(st->stream));
   OBIT_HIP_TRY(hipFree(dl));
   OBIT_HIP_TRY(hipFree(db));
@@ -1164,6 +1336,10 @@ bool mixed_ok(const State *st, const Desc &d) {
   return st->type == GPUModTypeGauss && st->npoint > 0 && d.op == kSub && !d.part && channels_ok(st, d);
 }
 
+// A spectral model whose factors k_dft_spec has (for the selection make_desc
+// has just made the table for).
+bool spec_ok(const State *st, const Desc &d) { return d.tab && model_is_spec(st->type) && st->specMm; }
+
 typedef void (*MfmaFn)(Desc, int, int, int);
 MfmaFn mfma_fn(const State *st) {
   return st->prec == 0 ? k_dft_mfma<0> : st->prec == 2 ? k_dft_mfma<2> : k_dft_mfma<1>;
@@ -1199,6 +1375,15 @@ int launch_mfma(State *st, const Desc &d, hipStream_t stream) {
   return kOK;
 }
 
+int launch_spec(State *st, const Desc &d, hipStream_t stream) {
+  const long long items = ((d.nrow + 3) / 4) * st->spec.npass * std::max(d.nsplit, 1);
+  const long long grid = std::min<long long>(items, (long long)st->nCU * occupancy_of(st, (const void *)k_dft_spec));
+  hipLaunchKernelGGL(k_dft_spec, dim3((unsigned)std::max<long long>(grid, 1)), dim3(kRows), 0,
+                     stream ? stream : st->stream, d, st->spec);
+  OBIT_HIP_TRY(hipGetLastError());
+  return kOK;
+}
+
 // The points-first copy of a Gaussian table (SetMod): its points and its
 // Gaussians as two descriptors over d's rows.
 void mixed_descs(const State *st, const Desc &d, Desc &dp, Desc &dg) {
@@ -1222,6 +1407,7 @@ int launch_split(State *st, const Desc &d, int cpt, int tile, int wgPerCU, hipSt
   if (d.nitems <= 0) return kOK;
   if (cpt == 64) {
     if (mfma_ok(st, d)) return launch_mfma(st, d, stream);
+    if (spec_ok(st, d)) return launch_spec(st, d, stream);
     if (mixed_ok(st, d)) {
       Desc dp, dg;
       mixed_descs(st, d, dp, dg);
@@ -1271,13 +1457,20 @@ int launch_fp64(State *st, const Desc &d) {
 // measured with 3,000 points: 4 x 64 channels, 60,000 rows 3.6 against 6.0 ms;
 // 3 x 37, 20,000 rows 1.17 against 1.5; 1 x 64, 2,000 rows 0.16 against 1.2;
 // 1 x 64, 70,201 rows 4.1 against 2.3 (a quarter of the slots filled).
+// A spectral model's rounds: 75 ns for k_dft_spec (a row quad and pass) and
+// 625 ns for k_dft_split with the amplitude table (3,000 components: 4 x 64
+// channels, 20,000 rows 1.56 against 3.75 ms; 4 x 256, 12,000 rows 3.67 against
+// 6.49; 2 x 96, 20,000 rows 1.52 against 2.15).
 int resident_cpt(State *st, const Desc &d) {
-  if (st->chosen || !mfma_ok(st, d)) return st->cpt;
+  const bool spec = spec_ok(st, d);
+  if (st->chosen || !(mfma_ok(st, d) || spec)) return st->cpt;
   const long long nquad = (d.nrow + 3) / 4, npass = (d.nIFsel * ((d.nchsel + 63) / 64) + 3) / 4;
-  const long long slotsM = (long long)st->nCU * occupancy_of(st, (const void *)mfma_fn(st));
+  const void *fn = spec ? (const void *)k_dft_spec : (const void *)mfma_fn(st);
+  const long long slotsM = (long long)st->nCU * occupancy_of(st, fn);
   const long long slotsV = (long long)st->nCU * st->wgPerCU;
-  const double tM = 59.0 * (double)npass * (double)((nquad + slotsM - 1) / slotsM);
-  const double tV = 550.0 * (double)((d.nitems + slotsV - 1) / slotsV);
+  const double tM = spec ? 75.0 * (double)((nquad * st->spec.npass + slotsM - 1) / slotsM)
+                         : 59.0 * (double)npass * (double)((nquad + slotsM - 1) / slotsM);
+  const double tV = (spec ? 625.0 : 550.0) * (double)((d.nitems + slotsV - 1) / slotsV);
   return tM < tV ? 64 : st->cpt;
 }
 
@@ -1356,10 +1549,13 @@ BufPlan plan_buffer(State *st, const Desc &d, size_t rowBytes) {
   const double capParts = double(size_t(1) << 30) / (chans * sizeof(double2));  // parts the scratch holds
   const bool mixed = st->type == GPUModTypeGauss && st->npoint > 0 && st->npoint < d.ncomp &&
                      channels_ok(st, d) && fill >= 0.6 && capParts >= 2.0;
-  if ((mfma_ok(st, d) && fill >= 0.6) || mixed) {
+  const bool spec = spec_ok(st, d);
+  if ((mfma_ok(st, d) && fill >= 0.6) || mixed || spec) {
     p.cpt = 64;
-    const long long slots = (long long)std::max(st->nCU, 1) * occupancy_of(st, (const void *)mfma_fn(st));
-    const long long nquad = (d.nrow + 3) / 4;
+    const void *fn = spec ? (const void *)k_dft_spec : (const void *)mfma_fn(st);
+    const long long slots = (long long)std::max(st->nCU, 1) * occupancy_of(st, fn);
+    const int npass = spec ? st->spec.npass : 1;  // items of a row quad and part
+    const long long nquad = (d.nrow + 3) / 4 * npass;
     const int npt = mixed ? st->npoint : d.ncomp;
     if (mixed) {
       // the Gaussians: VALU items of whole 64-component tiles, about 10
@@ -1384,7 +1580,7 @@ BufPlan plan_buffer(State *st, const Desc &d, size_t rowBytes) {
         p.kpart = kpt;
       }
     }
-    const long long perBlock = (long long)(kRows / 4) * p.nsplit;  // items of one row block
+    const long long perBlock = (long long)(kRows / 4) * npass * p.nsplit;  // items of one row block
     const int round = (int)std::max<long long>(1, slots / perBlock);
     const int mid = std::max(2 * round, (d.nrowblk + 5) / 6);
     int b = 0;
@@ -1799,7 +1995,7 @@ void ObitCUDASkyModelDFTShutdown(GPUInfo *gpuInfo) {
   obit::dft::destroy_graph(st);
   (void)hipFree(st->cx); (void)hipFree(st->cy); (void)hipFree(st->cz); (void)hipFree(st->camp); (void)hipFree(st->cg);
   (void)hipFree(st->tab); (void)hipFree(st->dfreq); (void)hipFree(st->stage); (void)hipFree(st->part);
-  (void)hipFree(st->dAmax);
+  (void)hipFree(st->dAmax); (void)hipFree(st->sblk); (void)hipFree(st->sbuf); (void)hipFree(st->smax);
   (void)hipFree(st->mbuf);
   for (hipEvent_t e : st->events) (void)hipEventDestroy(e);
   if (st->hfreq) (void)hipHostFree(st->hfreq);
@@ -2073,7 +2269,7 @@ int ObitHIPSkyModelDFTAutotune(GPUInfo *gpuInfo, long long sampleRows, int reps)
     obit::dft::Desc d, dw;
     rc = obit::dft::make_desc(st, gpuInfo, tmp, n, 64, d);
     if (!rc) rc = obit::dft::make_desc(st, gpuInfo, tmp, std::min(n, (long long)obit::dft::kRows), 64, dw);
-    if (!rc && (obit::dft::mfma_ok(st, d) || obit::dft::mixed_ok(st, d))) {
+    if (!rc && (obit::dft::mfma_ok(st, d) || obit::dft::spec_ok(st, d) || obit::dft::mixed_ok(st, d))) {
       rc = obit::dft::launch_split(st, dw, 64, bt, bw);
       if (!rc) {
         (void)hipEventRecord(e0, st->stream);
