@@ -47,7 +47,8 @@
 namespace obit {
 namespace dft {
 
-constexpr int kRows = 256;  // rows (threads) per workgroup
+constexpr int kRows = 256;  // threads per workgroup; rows of a k_dft_split item
+constexpr int kShareRows = 64;  // rows of a k_dft_share item
 
 enum Op { kSub = 0, kDiv = 1, kRepl = 2 };
 
@@ -371,6 +372,347 @@ __global__ __launch_bounds__(kRows, 2) void k_dft_split(Desc d) {
   }
 }
 
+// apply_op for N channels of a row at base + p[j] (those with ok), every load of a
+// Stokes issued before the first is waited on: one at a time, each channel's
+// read costs the latency of HBM (60,000 rows x 256 channels x 100 points on
+// k_dft_mfma 0.47 -> 0.44 ms).
+template <int N>
+__device__ __forceinline__ void apply_ops(const Desc &d, float *base, const int (&p)[N], const bool (&ok)[N],
+                                          float (&mr)[N], float (&mi)[N]) {
+  float wm[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    if (d.doSwap) { const float t = mr[j]; mr[j] = -mi[j]; mi[j] = t; }
+    wm[j] = 1.0f;
+    if (d.op == kDiv) {
+      wm[j] = mr[j] * mr[j] + mi[j] * mi[j];
+      mr[j] = mr[j] / wm[j];
+      mi[j] = mi[j] / wm[j];
+      wm[j] = sqrtf(wm[j]);
+    }
+  }
+  for (int s = 0; s < d.nstoksel; ++s) {
+    const int o = s * d.incs;
+    float re[N], im[N], wt[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) re[j] = im[j] = wt[j] = 0.0f;
+    if (d.op != kRepl) {
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if (ok[j]) {
+          const float *q = base + (p[j] + o);
+          re[j] = q[0]; im[j] = q[1]; wt[j] = q[2];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (!ok[j] || (wt[j] <= 0.0f && d.op != kRepl)) continue;
+      float *pp = base + (p[j] + o);
+      if (d.op == kDiv) {
+        pp[0] = mr[j] * re[j] + mi[j] * im[j];
+        pp[1] = mr[j] * im[j] - mi[j] * re[j];
+        pp[2] = wt[j] * wm[j];
+      } else if (d.op == kRepl) {
+        pp[0] = mr[j];
+        pp[1] = mi[j];
+      } else {
+        pp[0] = re[j] - mr[j];
+        pp[1] = im[j] - mi[j];
+      }
+      mr[j] *= d.stokFactor;
+      mi[j] *= d.stokFactor;
+    }
+  }
+}
+
+// k_dft_split for launches of few items: a workgroup is 64 rows, its four waves
+// take a quarter of the components each, stage their own tiles and add their
+// FP64 sums through LDS at the end.  Four times the items in flight: a
+// launch of 351 rows x 64 channels fills 12 workgroups instead of 4 quarter
+// as long, and 70,201 rows (550 items of k_dft_split on 512 resident
+// workgroups) 4.3 rounds instead of 2 whole ones.  k_dft_split keeps the
+// launches that fill their rounds: its tiles are staged once for four waves and
+// nothing is added at the end (4 x 256 channels, 12,000 rows x 3,000 components
+// with Gaussians and spectra: 9.0 against 9.9 ms here).  70,201 rows x 64
+// channels, a fifth Gaussians: 100 components 0.30 -> 0.18 ms, 6,000 5.2 -> 3.6
+// ms; 351 rows x 6,000 components 2.45 -> 0.61 ms.
+template <int CPT, bool GAUSS, bool SPEC, int PREC>
+__global__ __launch_bounds__(kRows, 2) void k_dft_share(Desc d) {
+  constexpr int TILE = 64;
+  static_assert(CPT % 2 == 0, "CPT must be even");
+  constexpr bool kMirror = !SPEC;
+  constexpr int H = CPT / 2;
+  struct Tile {
+    double x[TILE], y[TILE], z[TILE];
+    float a[TILE];
+    float g[GAUSS ? 3 * TILE : 2];
+    float t[SPEC ? TILE * CPT : 2];
+  };
+  // a wave's tile, or (the tiles done) the sums on their way to the wave that
+  // applies them: a quarter of the channels from three waves
+  constexpr int kQ = CPT / 4;
+  union Lds {
+    Tile tile[4];
+    double red[3][2 * kQ][64];
+  };
+  __shared__ Lds s_lds;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Tile &tl = s_lds.tile[wv];
+  double *s_x = tl.x, *s_y = tl.y, *s_z = tl.z;
+  float *s_a = tl.a, *s_g = tl.g, *s_t = tl.t;
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+
+  for (long long item = blockIdx.x; item < d.nitems; item += gridDim.x) {
+    const int rb = (int)(item % d.nrowblk);
+    const int ic = (int)(item / d.nrowblk);
+    // this wave's quarter
+    const int per = (d.ncomp + 3) / 4;
+    const int kBeg = min(d.ncomp, wv * per), kEnd = min(d.ncomp, kBeg + per);
+    const int isel = ic / d.nchunk;
+    const int c0 = (ic - isel * d.nchunk) * CPT;
+    const long long row = (long long)rb * kShareRows + lane;
+    const bool valid = row < d.nrow;
+    const float *rp = d.vis + (valid ? row : 0LL) * (long long)d.lrec;
+    const float uf = valid ? rp[d.ilocu] : 0.0f;
+    const float vf = valid ? rp[d.ilocv] : 0.0f;
+    const float wf = valid ? rp[d.ilocw] : 0.0f;
+    const double u = uf, v = vf, w = wf;
+    const double fd = d.fdel[isel];
+    const double fm = d.fbase[isel] + (double)(c0 + H) * fd;
+    const float fmf = (float)fm, fdf = (float)fd;
+    const float uu = uf * uf, vv = vf * vf, uv = uf * vf;
+
+    float accr[CPT], acci[CPT];
+    double outr[CPT], outi[CPT];
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) { accr[j] = acci[j] = 0.0f; outr[j] = outi[j] = 0.0; }
+
+    // the centre phasor (cm, sm) of component kk and its step as three
+    // shears (tau, sig), the step reduced to |pd| <= 1/4 turn; flip: an odd
+    // count of half turns was taken out, every odd offset changes sign
+    auto phasors = [&](int kk, float &cm, float &sm, float &tau, float &sig, bool &flip) {
+      const double psi = fma(w, s_z[kk], fma(v, s_y[kk], u * s_x[kk]));
+      double pm = psi * fm, pd = psi * fd;
+      pm -= rint(pm);
+      const double h2 = rint(2.0 * pd);
+      pd -= 0.5 * h2;
+      flip = ((int)h2) & 1;
+      float sh, ch;
+      sincos_turns<PREC == 2 ? 1 : 0>((float)pm, &sm, &cm);
+      if (PREC == 0) sincos_turns_hw((float)(0.5 * pd), &sh, &ch);
+      else sincos_halfturns_small((float)pd, &sh, &ch);
+      tau = sh * __builtin_amdgcn_rcpf(ch);
+      sig = 2.0f * sh * ch;
+    };
+
+    for (int k0 = kBeg; k0 < kEnd; k0 += TILE) {
+      wave_sync();
+      const int kn = min(TILE, kEnd - k0);
+      int ntile = 0;  // components of the tile that take the mirrored walk
+      if (GAUSS && kMirror) {
+        // the tile's points in front (both kinds in table order)
+        unsigned long long mp[(TILE + 63) / 64];
+#pragma unroll
+        for (int t0 = 0; t0 < TILE; t0 += 64) {
+          const int k = k0 + min(t0 + lane, kn - 1);
+          const bool pt = d.cg[k] == 0.0f && d.cg[d.ncomp + k] == 0.0f && d.cg[2 * d.ncomp + k] == 0.0f;
+          mp[t0 / 64] = __ballot(t0 + lane < min(kn, TILE) && pt);
+          ntile += (int)__popcll(mp[t0 / 64]);
+        }
+        int nb = 0, gb = ntile;  // places taken in front and behind
+#pragma unroll
+        for (int t0 = 0; t0 < TILE; t0 += 64) {
+          const bool ok = t0 + lane < min(kn, TILE);
+          const int k = k0 + min(t0 + lane, kn - 1);
+          const unsigned long long p = mp[t0 / 64], g = __ballot(ok) & ~p;
+          const unsigned long long below = (1ull << lane) - 1ull;
+          const int at = ((p >> lane) & 1) ? nb + (int)__popcll(p & below) : gb + (int)__popcll(g & below);
+          if (ok) {
+            s_x[at] = d.cx[k];
+            s_y[at] = d.cy[k];
+            s_z[at] = d.cz[k];
+            s_a[at] = d.camp[k];
+            s_g[3 * at + 0] = d.cg[k];
+            s_g[3 * at + 1] = d.cg[d.ncomp + k];
+            s_g[3 * at + 2] = d.cg[2 * d.ncomp + k];
+          }
+          nb += (int)__popcll(p);
+          gb += (int)__popcll(g);
+        }
+      } else {
+        for (int t = lane; t < kn; t += 64) {
+          const int k = k0 + t;
+          s_x[t] = d.cx[k];
+          s_y[t] = d.cy[k];
+          s_z[t] = d.cz[k];
+          s_a[t] = d.camp[k];
+          if (GAUSS) {
+            s_g[3 * t + 0] = d.cg[k];
+            s_g[3 * t + 1] = d.cg[d.ncomp + k];
+            s_g[3 * t + 2] = d.cg[2 * d.ncomp + k];
+          }
+        }
+      }
+      if (SPEC) {
+        for (int t = lane; t < kn * CPT; t += 64) {
+          const int kk = t / CPT, cc = t - kk * CPT;
+          s_t[t] = d.tab[(size_t)(k0 + kk) * d.tab_ldk + (size_t)isel * d.tab_nchpad + c0 + cc];
+        }
+      }
+      wave_sync();
+      const int np = !kMirror ? 0 : GAUSS ? __builtin_amdgcn_readfirstlane(ntile) : kn;
+      if (kMirror) {
+        for (int kk = 0; kk < np; ++kk) {
+          float cm, sm, tau, sig;
+          bool flip;
+          phasors(kk, cm, sm, tau, sig, flip);
+          const float a0 = s_a[kk], ao = flip ? -a0 : a0;
+          const float ce = a0 * cm, se = a0 * sm, co = ao * cm, so = ao * sm;
+          accr[H] += ce;
+          acci[H] += se;
+          float x = 1.0f, y = 0.0f;  // W^q
+#pragma unroll
+          for (int q1 = 1; q1 <= H; ++q1) {
+            const float x1 = fmaf(-tau, y, x);
+            y = fmaf(sig, x1, y);
+            x = fmaf(-tau, y, x1);
+            const float c = (q1 & 1) ? co : ce, s = (q1 & 1) ? so : se;
+            if (q1 < H) {
+              accr[H + q1] = fmaf(x, c, accr[H + q1]);  // C c
+              accr[H - q1] = fmaf(y, s, accr[H - q1]);  // S s
+              acci[H + q1] = fmaf(x, s, acci[H + q1]);  // C s
+              acci[H - q1] = fmaf(y, c, acci[H - q1]);  // S c
+            } else {  // the one channel without a mirror
+              accr[0] = fmaf(x, c, fmaf(y, s, accr[0]));
+              acci[0] = fmaf(x, s, fmaf(-y, c, acci[0]));
+            }
+          }
+        }
+        // the tile's channel sums
+#pragma unroll
+        for (int q1 = 1; q1 < H; ++q1) {
+          const float cc = accr[H + q1], ss = accr[H - q1], cs = acci[H + q1], sc = acci[H - q1];
+          accr[H + q1] = cc - ss;
+          accr[H - q1] = cc + ss;
+          acci[H + q1] = cs + sc;
+          acci[H - q1] = cs - sc;
+        }
+      }
+      if (GAUSS || SPEC) {
+        for (int kk = np; kk < kn; ++kk) {
+          float cm, sm, tau, sig;
+          bool flip;
+          phasors(kk, cm, sm, tau, sig, flip);
+          const float a0 = s_a[kk];
+          const float sgn = flip ? -1.0f : 1.0f;
+          float gf = a0, rf = 0.0f, rbk = 0.0f, qg = 0.0f;
+          if (GAUSS) {
+            const float G = fmaf(s_g[3 * kk + 2], uv, fmaf(s_g[3 * kk + 1], vv, s_g[3 * kk] * uu));
+            const float e0 = G * fmf * fmf;
+            const float Gd = G * fdf;
+            const bool live = e0 > -60.0f;
+            gf = live ? (SPEC ? 1.0f : a0) * __expf(e0) : 0.0f;
+            // the per-step ratios carry the sign of the odd offsets
+            rf = live ? sgn * __expf(Gd * (2.0f * fmf + fdf)) : 0.0f;
+            rbk = live ? sgn * __expf(Gd * (fdf - 2.0f * fmf)) : 0.0f;
+            qg = live ? __expf(2.0f * Gd * fdf) : 0.0f;
+          }
+          // forward from the centre channel
+          float x = cm, y = sm, g = gf, r = rf;
+#pragma unroll
+          for (int j = H; j < CPT; ++j) {
+            const bool odd = (j - H) & 1;
+            float amp;
+            if (GAUSS) amp = SPEC ? s_t[kk * CPT + j] * g : g;
+            else amp = odd ? s_t[kk * CPT + j] * sgn : s_t[kk * CPT + j];
+            accr[j] = fmaf(amp, x, accr[j]);
+            acci[j] = fmaf(amp, y, acci[j]);
+            if (j + 1 < CPT) {
+              const float x1 = fmaf(-tau, y, x);
+              y = fmaf(sig, x1, y);
+              x = fmaf(-tau, y, x1);
+              if (GAUSS) { g *= r; r *= qg; }
+            }
+          }
+          // backward from the centre channel
+          x = cm; y = sm;
+          float gb = gf * rbk, rb2 = rbk * qg;
+#pragma unroll
+          for (int j = H - 1; j >= 0; --j) {
+            const bool odd = (H - j) & 1;
+            const float x1 = fmaf(tau, y, x);
+            y = fmaf(-sig, x1, y);
+            x = fmaf(tau, y, x1);
+            float amp;
+            if (GAUSS) amp = SPEC ? s_t[kk * CPT + j] * gb : gb;
+            else amp = odd ? s_t[kk * CPT + j] * sgn : s_t[kk * CPT + j];
+            accr[j] = fmaf(amp, x, accr[j]);
+            acci[j] = fmaf(amp, y, acci[j]);
+            if (GAUSS && j > 0) { gb *= rb2; rb2 *= qg; }
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < CPT; ++j) {
+        outr[j] += (double)accr[j];
+        outi[j] += (double)acci[j];
+        accr[j] = acci[j] = 0.0f;
+      }
+    }
+
+    // the four waves' sums: wave r adds channels r kQ .. r kQ + kQ - 1 (kept in
+    // FP32, as they are applied), then all apply theirs at once: applied in turn
+    // inside the loop, 100 components took 0.28 ms instead of 0.21
+    float fr[kQ], fi[kQ];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      __syncthreads();  // the tiles, or the quarter before, are read
+      if (wv != r) {
+        const int at = wv < r ? wv : wv - 1;
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+          s_lds.red[at][2 * j][lane] = outr[r * kQ + j];
+          s_lds.red[at][2 * j + 1][lane] = outi[r * kQ + j];
+        }
+      }
+      __syncthreads();
+      if (wv == r) {
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+          double mr = r == 0 ? outr[j] : s_lds.red[0][2 * j][lane];
+          double mi = r == 0 ? outi[j] : s_lds.red[0][2 * j + 1][lane];
+#pragma unroll
+          for (int o = 1; o < 4; ++o) {
+            mr += o == r ? outr[r * kQ + j] : s_lds.red[o < r ? o : o - 1][2 * j][lane];
+            mi += o == r ? outi[r * kQ + j] : s_lds.red[o < r ? o : o - 1][2 * j + 1][lane];
+          }
+          fr[j] = (float)mr;
+          fi[j] = (float)mi;
+        }
+      }
+    }
+    if (valid) {
+      const int cb = c0 + wv * kQ;
+      float *p = d.vis + row * (long long)d.lrec + d.nrparm + (d.IFb + isel) * d.incif + (d.chanb + cb) * d.incf +
+                 d.stokb * d.incs;
+      int pj[kQ];
+      bool ok[kQ];
+#pragma unroll
+      for (int j = 0; j < kQ; ++j) {
+        pj[j] = j * d.incf;
+        ok[j] = cb + j < d.nchsel;
+      }
+      apply_ops<kQ>(d, p, pj, ok, fr, fi);
+    }
+    __syncthreads();  // the last quarter is read before the next item's tiles
+  }
+}
+
 // ---- the matrix-core DFT (point components) ----
 //
 // Channel c = c1 + 8 c2 (c1, c2 < 8) of a 64-channel group g (an IF's
@@ -610,25 +952,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       if (valid && lane < 32) {
         const double unscale = ldexp(1.0, -ashift);
         const int n = lane & 15, c2 = n & 7;
+        float *base = d.vis + row * (long long)d.lrec + d.nrparm + d.chanb * d.incf + d.stokb * d.incs;
+        float mr[8], mi[8];
+        int pj[8];
+        bool ok[8];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const int g = 4 * tg + 2 * t + (n >> 3);
-          if (g >= ngrp) continue;
           const int isel = g / nchunk64, cbase = (g - isel * nchunk64) * 64;
-          float *p = d.vis + row * (long long)d.lrec + d.nrparm + (d.IFb + isel) * d.incif +
-                     (d.chanb + cbase) * d.incf + d.stokb * d.incs;
+          const int p = (d.IFb + isel) * d.incif + cbase * d.incf;
           double2 *pp = d.part ? d.part + (((long long)part * d.nrow + row) * d.nIFsel + isel) * d.nchsel + cbase
                                : nullptr;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int c1 = 4 * (lane >> 4) + r;
-            const int c = c1 + 8 * c2;
-            if (cbase + c >= d.nchsel) continue;  // past a ragged selection's last channel
-            const double re = t ? o1[r] : o0[r], imv = t ? im1[r] : im0[r];
-            if (pp) pp[c] = make_double2(re * unscale, imv * unscale);
-            else apply_op(d, p + c * d.incf, (float)(re * unscale), (float)(imv * unscale));
+            const int c = c1 + 8 * c2, j = 4 * t + r;
+            // not past a ragged selection's last channel
+            ok[j] = g < ngrp && cbase + c < d.nchsel;
+            const double re = (t ? o1[r] : o0[r]) * unscale, imv = (t ? im1[r] : im0[r]) * unscale;
+            if (pp && ok[j]) pp[c] = make_double2(re, imv);
+            pj[j] = p + c * d.incf;
+            mr[j] = (float)re;
+            mi[j] = (float)imv;
           }
         }
+        if (!d.part) apply_ops<8>(d, base, pj, ok, mr, mi);
       }
     }
   }
@@ -687,22 +1035,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const bool have = lane < 32 && ps * mm::kPass + n < m.nblk;
     const double unscale = ldexp(1.0, -m.shift);
     const float r0 = m.r0[ps];
-    float *base = d.vis + row * (long long)d.lrec + d.nrparm + (d.IFb + bk.IF) * d.incif + d.chanb * d.incf +
-                  d.stokb * d.incs;
+    float *base = d.vis + row * (long long)d.lrec + d.nrparm + d.chanb * d.incf + d.stokb * d.incs;
     double2 *pp = d.part ? d.part + (((long long)part * d.nrow + row) * d.nIFsel + bk.IF) * d.nchsel : nullptr;
+    float mr[8], mi[8];
+    int pj[8];
+    bool ok[8];
 #pragma unroll
     for (int T = 0; T < 2; ++T)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int c = 4 * (qd & 1) + r, t = T ? c : -(c + 1), ch = bk.ch0 + 8 + t;
+        const int c = 4 * (qd & 1) + r, t = T ? c : -(c + 1), ch = bk.ch0 + 8 + t, j = 4 * T + r;
         double x = o[T][0][r] + (double)(((float)t - (float)(t * t) * r0) * bk.s * d2[T][0][r]);
         double y = __shfl_xor(x, 32);
         x *= unscale;
         y *= unscale;
-        if (!have || ch < bk.vlo || ch > bk.vhi) continue;
-        if (pp) pp[ch] = make_double2(x, y);
-        else apply_op(d, base + ch * d.incf, (float)x, (float)y);
+        ok[j] = have && ch >= bk.vlo && ch <= bk.vhi;
+        if (pp && ok[j]) pp[ch] = make_double2(x, y);
+        pj[j] = (d.IFb + bk.IF) * d.incif + ch * d.incf;
+        mr[j] = (float)x;
+        mi[j] = (float)y;
       }
+    if (!pp) apply_ops<8>(d, base, pj, ok, mr, mi);
   }
 }
 
@@ -888,6 +1241,16 @@ KernelFn pick_shape(int cpt, int tile, bool g, bool s) {
   if (tile == 32) return pick_gs<32, 32, P>(g, s);
   if (tile == 128) return pick_gs<32, 128, P>(g, s);
   return pick_gs<32, 64, P>(g, s);
+}
+
+template <int P>
+KernelFn pick_share(bool c16, bool g, bool s) {
+  if (c16) {
+    if (g) return s ? k_dft_share<16, true, true, P> : k_dft_share<16, true, false, P>;
+    return s ? k_dft_share<16, false, true, P> : k_dft_share<16, false, false, P>;
+  }
+  if (g) return s ? k_dft_share<32, true, true, P> : k_dft_share<32, true, false, P>;
+  return s ? k_dft_share<32, false, true, P> : k_dft_share<32, false, false, P>;
 }
 
 KernelFn pick_split(int cpt, int tile, bool g, bool s, int prec) {
@@ -1447,31 +1810,58 @@ int launch_fp64(State *st, const Desc &d) {
   return kOK;
 }
 
-// The kernel of a resident launch whose variant the caller has not set: 64
-// (k_dft_mfma) or st->cpt (k_dft_split).  Both run in rounds of their
-// resident workgroups, and the last round of a short launch costs as much as
-// a full one, so the whole rounds are compared: a round of k_dft_mfma (a row
-// quad a workgroup, 256 channel slots a pass) takes 59 ns a component, one
-// of k_dft_split (256 rows x 32 channels) 550 ns, measured on full launches of
-// 4 IF x 64 channels (13.4e12 and 7.65e12 evaluations/s).  Both sides
-// measured with 3,000 points: 4 x 64 channels, 60,000 rows 3.6 against 6.0 ms;
-// 3 x 37, 20,000 rows 1.17 against 1.5; 1 x 64, 2,000 rows 0.16 against 1.2;
-// 1 x 64, 70,201 rows 4.1 against 2.3 (a quarter of the slots filled).
-// A spectral model's rounds: 75 ns for k_dft_spec (a row quad and pass) and
-// 625 ns for k_dft_split with the amplitude table (3,000 components: 4 x 64
-// channels, 20,000 rows 1.56 against 3.75 ms; 4 x 256, 12,000 rows 3.67 against
-// 6.49; 2 x 96, 20,000 rows 1.52 against 2.15).
-int resident_cpt(State *st, const Desc &d) {
-  const bool spec = spec_ok(st, d);
-  if (st->chosen || !(mfma_ok(st, d) || spec)) return st->cpt;
+// k_dft_share at cpt channels a thread, a workgroup an item.
+int launch_share(State *st, const Desc &d, int cpt, hipStream_t stream) {
+  const bool g = model_gauss_off(st->type) >= 0, s = model_is_spec(st->type);
+  Desc dd = d;
+  dd.nchunk = (d.nchsel + cpt - 1) / cpt;
+  dd.nrowblk = (int)((d.nrow + kShareRows - 1) / kShareRows);
+  dd.nitems = (long long)dd.nrowblk * d.nIFsel * dd.nchunk;
+  if (dd.nitems <= 0) return kOK;
+  const KernelFn fn = st->prec == 0 ? pick_share<0>(cpt == 16, g, s)
+                      : st->prec == 2 ? pick_share<2>(cpt == 16, g, s) : pick_share<1>(cpt == 16, g, s);
+  void *args[] = {&dd};
+  const long long grid = std::min<long long>(dd.nitems, INT_MAX);
+  OBIT_HIP_TRY(hipLaunchKernel((const void *)fn, dim3((unsigned)grid), dim3(kRows), args, 0,
+                               stream ? stream : st->stream));
+  return kOK;
+}
+
+// The launch over resident rows.  A variant that the caller has set is taken;
+// otherwise the kernel that takes the least rounds of its resident
+// workgroups, since the last round of a short launch costs as much as a full
+// one.  A round takes, for each component,
+//   k_dft_mfma   59 ns (a row quad, 256 channel slots a pass)
+//   k_dft_spec   75 ns (a row quad and pass)
+//   k_dft_split  500 ns (256 rows x 32 channels), 625 with spectra or Gaussians
+//   k_dft_share  a quarter of that and 8 % (64 rows)
+// measured on full launches.  Both sides measured with 3,000 components: points
+// of 4 x 64 channels, 60,000 rows 3.4 ms on k_dft_mfma, 6.0 on k_dft_split;
+// 3 x 37, 20,000 rows 1.1 against 1.5; 1 x 64, 2,000 rows 0.14 against 1.2;
+// 1 x 64, 70,201 rows 4.0 against 2.2 and 1.55 on k_dft_share; spectra of
+// 4 x 64, 20,000 rows 1.56 against 3.75; 2 x 96, 20,000 rows 1.52 against 2.15;
+// Gaussians of 1 x 64, 5,000 rows x 6,000 components 3.5 ms against 0.63 on
+// k_dft_share.
+int launch_resident(State *st, const Desc &d, bool matrix) {
+  if (st->chosen) return launch_split(st, d, matrix ? st->cpt : (st->cpt == 64 ? 32 : st->cpt), st->tile, st->wgPerCU);
+  auto rounds = [&](long long items, int perCU) {
+    const long long slots = (long long)st->nCU * perCU;
+    return (double)((items + slots - 1) / slots);
+  };
+  const bool spec = matrix && spec_ok(st, d), g = model_gauss_off(st->type) >= 0, s = model_is_spec(st->type);
+  const double tItem = g || s ? 625.0 : 500.0;
+  const int n16 = (d.nchsel + 15) / 16, n32 = (d.nchsel + 31) / 32;
+  const int cs = (n16 * 16 / 0.9 < n32 * 32.0) ? 16 : 32;  // as plan_buffer
+  const long long blk = (d.nrow + kShareRows - 1) / kShareRows * d.nIFsel;
+  const double tSplit = tItem * rounds(d.nitems, 2);
+  const double tShare = tItem * 0.27 * (cs == 16 ? 0.55 * rounds(blk * n16, 2) : rounds(blk * n32, 2));
+  double tM = 1e300;
   const long long nquad = (d.nrow + 3) / 4, npass = (d.nIFsel * ((d.nchsel + 63) / 64) + 3) / 4;
-  const void *fn = spec ? (const void *)k_dft_spec : (const void *)mfma_fn(st);
-  const long long slotsM = (long long)st->nCU * occupancy_of(st, fn);
-  const long long slotsV = (long long)st->nCU * st->wgPerCU;
-  const double tM = spec ? 75.0 * (double)((nquad * st->spec.npass + slotsM - 1) / slotsM)
-                         : 59.0 * (double)npass * (double)((nquad + slotsM - 1) / slotsM);
-  const double tV = (spec ? 625.0 : 550.0) * (double)((d.nitems + slotsV - 1) / slotsV);
-  return tM < tV ? 64 : st->cpt;
+  if (spec) tM = 75.0 * rounds(nquad * st->spec.npass, occupancy_of(st, (const void *)k_dft_spec));
+  else if (matrix && mfma_ok(st, d)) tM = 59.0 * npass * rounds(nquad, occupancy_of(st, (const void *)mfma_fn(st)));
+  if (tM < tSplit && tM < tShare) return launch_split(st, d, 64, st->tile, st->wgPerCU);
+  if (tShare < tSplit) return launch_share(st, d, cs, nullptr);
+  return launch_split(st, d, st->cpt, st->tile, st->wgPerCU);
 }
 
 // Run the operation over nrow rows at a device pointer.
@@ -1489,7 +1879,7 @@ int run_device(State *st, const GPUInfo *gi, float *vis, long long nrow, bool fp
   }
   st->lastPath = (fp64 || !st->uniform) ? 1 : 0;
   if (fp64 || !st->uniform) return launch_fp64(st, d);
-  return launch_split(st, d, resident_cpt(st, d), st->tile, st->wgPerCU);
+  return launch_resident(st, d, true);
 }
 
 // ---- the per-buffer launch plan (ObitCUDASkyModelDFTCalc) ----
@@ -2090,7 +2480,7 @@ int ObitHIPSkyModelDFTCalcNoAlloc(GPUInfo *gpuInfo, const float *d_model, int nc
   st->lastPath = 0;
   // the VALU kernel (the matrix-core kernel's eligibility reads the host
   // copy of the lines, which this call does not make)
-  return launch_split(st, d, st->cpt == 64 ? 32 : st->cpt, st->tile, st->wgPerCU);
+  return launch_resident(st, d, false);
 }
 
 int ObitHIPSkyModelDFTSetSpecRef(GPUInfo *gpuInfo, const double *refFreq, int n) {
@@ -2167,9 +2557,11 @@ int ObitHIPSkyModelDFTGraphLaunch(GPUInfo *gpuInfo) {
     int rc = obit::dft::make_desc(st, gpuInfo, st->dvis, st->nres, st->cpt, d);
     if (rc) return rc;
     OBIT_HIP_TRY(hipStreamSynchronize(st->stream));
-    const int cpt = obit::dft::resident_cpt(st, d);  // asks for the occupancy: before the capture
+    // the kernels' occupancies, asked for before the capture
+    (void)obit::dft::occupancy_of(st, (const void *)obit::dft::k_dft_spec);
+    (void)obit::dft::occupancy_of(st, (const void *)obit::dft::mfma_fn(st));
     OBIT_HIP_TRY(hipStreamBeginCapture(st->stream, hipStreamCaptureModeThreadLocal));
-    rc = st->uniform ? obit::dft::launch_split(st, d, cpt, st->tile, st->wgPerCU)
+    rc = st->uniform ? obit::dft::launch_resident(st, d, true)
                      : obit::dft::launch_fp64(st, d);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(st->stream, &g);
