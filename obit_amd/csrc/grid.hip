@@ -29,6 +29,7 @@
 #include <hipfft/hipfft.h>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
+#include <rocprim/iterator/counting_iterator.hpp>
 #include <rocprim/iterator/transform_iterator.hpp>
 #include "ObitCUDAUtil.h"
 #include "ObitHIPVis.h"
@@ -216,29 +217,38 @@ __device__ Sample prep_sample(const FacetDev &f, const Common &cm, const float *
 
 // ---------------- binning ----------------
 
-// Clear two int arrays with a kernel (kept out of memset nodes so the
-// sequence stays capturable in a hipGraph).
-__global__ void k_zero2(int *a, int *b, long long n) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) { a[i] = 0; b[i] = 0; }
+// Everything a pass starts from zero, in one launch (a kernel, kept out of
+// memset nodes so the sequence stays capturable in a hipGraph): the walk
+// statistics, the count after the last track, the uvw checksum and the lists'
+// first and last entries.
+__global__ void k_pass_clear(unsigned long long *walk, unsigned *lastCount, unsigned long long *hash, long long *first,
+                             long long *last, long long n) {
+  const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i0 == 0) {
+    walk[0] = walk[1] = 0;
+    *hash = 0;
+    if (lastCount) *lastCount = 0;
+  }
+  for (long long i = i0; i < n; i += (long long)gridDim.x * blockDim.x) { first[i] = 0; last[i] = 0; }
 }
 
 // Order-independent checksum of the rows' u, v, w bit patterns: the track
 // lists of a pass may be reused only for rows with the same uvw.
+__device__ __forceinline__ unsigned long long row_hash(const float *row, long long r) {
+  const unsigned long long a = __float_as_uint(row[0]), b = __float_as_uint(row[1]), c = __float_as_uint(row[2]);
+  unsigned long long x = (a * 0x9E3779B97F4A7C15ULL) ^ (b * 0xC2B2AE3D27D4EB4FULL) ^
+                         (c * 0x165667B19E3779F9ULL) ^ ((unsigned long long)r * 0xD6E8FEB86659FD93ULL);
+  x ^= x >> 29;
+  x *= 0xBF58476D1CE4E5B9ULL;
+  x ^= x >> 32;
+  return x;
+}
+
 __global__ void k_uvw_hash(const float *vis, long long nrow, int lenvis, unsigned long long *out) {
   unsigned long long h = 0;
   for (long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x; r < nrow;
-       r += (long long)gridDim.x * blockDim.x) {
-    const float *row = vis + r * (long long)lenvis;
-    const unsigned long long a = __float_as_uint(row[0]), b = __float_as_uint(row[1]),
-                             c = __float_as_uint(row[2]);
-    unsigned long long x = (a * 0x9E3779B97F4A7C15ULL) ^ (b * 0xC2B2AE3D27D4EB4FULL) ^
-                           (c * 0x165667B19E3779F9ULL) ^ ((unsigned long long)r * 0xD6E8FEB86659FD93ULL);
-    x ^= x >> 29;
-    x *= 0xBF58476D1CE4E5B9ULL;
-    x ^= x >> 32;
-    h += x;
-  }
+       r += (long long)gridDim.x * blockDim.x)
+    h += row_hash(vis + r * (long long)lenvis, r);
   for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
   if ((threadIdx.x & 63) == 0 && h) atomicAdd(out, h);
 }
@@ -258,9 +268,9 @@ __global__ void k_uvw_hash(const float *vis, long long nrow, int lenvis, unsigne
 // column, < 80).
 template <typename Fn>
 __device__ __forceinline__ void track_tiles(const FacetDev &f, const Common &cm, float uu, float vv,
-                                            Fn fn) {
+                                            int p0, int p1, Fn fn) {
   const int ncol = f.lrow / 2;
-  for (int p = 0; p < cm.nplane; ++p) {
+  for (int p = p0; p < p1; ++p) {
     const int npc = cm.pcount[p];
     if (npc <= 0) continue;
     int iu0, iv0, iu1, iv1;
@@ -325,22 +335,41 @@ __device__ __forceinline__ void track_tiles(const FacetDev &f, const Common &cm,
   }
 }
 
-// Binning, pass 1: the number of (plane, tile) entries of every track of
-// every facet, one thread per (row, facet), facet fastest.
-__global__ void k_bin_count(const float *vis, long long nrow, const FacetDev *facets, int nf, Common cm,
-                            unsigned *cnt) {
-  const long long total = nrow * (long long)nf;
+// A thread of the binning passes: (row, facet, planes p0 .. p1 - 1), the planes
+// fastest, in nsplit <= nplane parts (see grid_device), so the entries of a
+// tile's list come in row order whatever the parts.
+struct BinTrack { long long r; int fi, p0, p1; };
+__device__ __forceinline__ BinTrack bin_track(long long it, int nf, int nsplit, int nplane) {
+  BinTrack b;
+  const long long rf = it / nsplit;
+  const int part = (int)(it - rf * nsplit);
+  b.r = rf / nf;
+  b.fi = (int)(rf - b.r * nf);
+  b.p0 = part * nplane / nsplit;
+  b.p1 = (part + 1) * nplane / nsplit;
+  return b;
+}
+
+// Binning, pass 1: the number of (plane, tile) entries of every thread's track;
+// the first thread of a row adds it to the uvw checksum.
+__global__ void k_bin_count(const float *vis, long long nrow, const FacetDev *facets, int nf, int nsplit, Common cm,
+                            unsigned *cnt, unsigned long long *hash) {
+  const long long total = nrow * (long long)nf * nsplit;
+  unsigned long long h = 0;
   for (long long it = (long long)blockIdx.x * blockDim.x + threadIdx.x; it < total;
        it += (long long)gridDim.x * blockDim.x) {
-    const int fi = (int)(it % nf);
-    const long long r = it / nf;
-    const FacetDev &f = facets[fi];
+    const BinTrack b = bin_track(it, nf, nsplit, cm.nplane);
+    const FacetDev &f = facets[b.fi];
+    const float *row = vis + b.r * (long long)cm.lenvis;
     float uu, vv, ww;
-    rotate_uvw(f, vis + r * (long long)cm.lenvis, uu, vv, ww);
+    rotate_uvw(f, row, uu, vv, ww);
     unsigned n = 0;
-    track_tiles(f, cm, uu, vv, [&](long long, unsigned, int, int) { ++n; });
+    track_tiles(f, cm, uu, vv, b.p0, b.p1, [&](long long, unsigned, int, int) { ++n; });
     cnt[it] = n;
+    if (b.fi == 0 && b.p0 == 0) h += row_hash(row, b.r);
   }
+  for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
+  if ((threadIdx.x & 63) == 0 && h) atomicAdd(hash, h);
 }
 
 // Binning, pass 2: every entry as a sort key (list << 7 | window block)
@@ -348,18 +377,19 @@ __global__ void k_bin_count(const float *vis, long long nrow, const FacetDev *fa
 // scanned offset.  Sorting the pairs by key gives each tile's list ordered
 // by the window its tracks enter first, then by row (the sort is stable
 // and the emission ordered).
-// The entries of a block's 256 (row, facet) tracks are one contiguous
+// The entries of a block's 256 threads are one contiguous
 // range of the output ([off[it0], off[it1])): where it fits, the block
 // stages it in LDS and writes it out whole (the tracks' own runs are short
 // and scattered); a larger range is written run by run.
 constexpr int kEmitCap = 4096;  // entries a block stages (48 KB)
 
 __global__ __launch_bounds__(256) void k_bin_emit(const float *vis, long long nrow, const FacetDev *facets,
-                                                  int nf, Common cm, const unsigned long long *off,
+                                                  int nf, int nsplit, Common cm,
+                                                  const unsigned long long *off,
                                                   unsigned *keys, int2 *rows) {
   __shared__ unsigned s_key[kEmitCap];
   __shared__ int2 s_row[kEmitCap];
-  const long long total = nrow * (long long)nf;
+  const long long total = nrow * (long long)nf * nsplit;
   const long long nchunk = (total + 255) / 256;
   for (long long ch = blockIdx.x; ch < nchunk; ch += gridDim.x) {
     const long long it0 = ch * 256, it1 = min(total, it0 + 256);
@@ -367,15 +397,14 @@ __global__ __launch_bounds__(256) void k_bin_emit(const float *vis, long long nr
     const bool stage = span <= (unsigned long long)kEmitCap;  // the same for the whole block
     const long long it = it0 + threadIdx.x;
     if (it < total) {
-      const int fi = (int)(it % nf);
-      const long long r = it / nf;
-      const FacetDev &f = facets[fi];
+      const BinTrack b = bin_track(it, nf, nsplit, cm.nplane);
+      const FacetDev &f = facets[b.fi];
       float uu, vv, ww;
-      rotate_uvw(f, vis + r * (long long)cm.lenvis, uu, vv, ww);
+      rotate_uvw(f, vis + b.r * (long long)cm.lenvis, uu, vv, ww);
       unsigned long long o = off[it];
-      track_tiles(f, cm, uu, vv, [&](long long L, unsigned wkey, int lo, int hi) {
+      track_tiles(f, cm, uu, vv, b.p0, b.p1, [&](long long L, unsigned wkey, int lo, int hi) {
         const unsigned k = ((unsigned)L << 7) | wkey;
-        const int2 v = make_int2((int)r, lo | (hi << 16));
+        const int2 v = make_int2((int)b.r, lo | (hi << 16));
         if (stage) {
           s_key[o - base] = k;
           s_row[o - base] = v;
@@ -408,21 +437,11 @@ __global__ void k_list_bounds(const unsigned *keys, long long n, long long *firs
   }
 }
 
-__global__ void k_list_counts(const long long *first, const long long *last, long long nl, int *counts) {
-  for (long long L = (long long)blockIdx.x * blockDim.x + threadIdx.x; L < nl;
-       L += (long long)gridDim.x * blockDim.x)
-    counts[L] = (int)(last[L] - first[L]);
-}
-
-__global__ void k_zero64(long long *a, long long *b, long long n) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) { a[i] = 0; b[i] = 0; }
-}
-
 // ---------------- tile gridding ----------------
 
 constexpr int kW = 7;          // GCF support in cells (checked on the host)
-constexpr int kChunk = 128;    // tracks per work item (swept 64..2048 on workload 4: 128 best)
+constexpr int kChunk = 128;    // most tracks of a work item (swept 64..2048 on workload 4: 128 best)
+constexpr int kMinChunk = 16;  // least (see grid_device)
 constexpr int kWaves = 4;      // waves per workgroup, each with a private tile
 // A sample's footprint is accumulated through a 16 (u) x 8 (v) window of
 // cells whose origin is its base cell rounded down to a multiple of 8 in u
@@ -491,8 +510,8 @@ __device__ __forceinline__ float keep_lanes(float a, unsigned long long m) {
 // atomics.
 __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, const FacetDev *facets,
                                                            const int *listFacet, const int2 *items,
-                                                           long long nitems, Common cm,
-                                                           const int *counts, const long long *offsets,
+                                                           const long long *nitemsPtr, int chunk, Common cm,
+                                                           const long long *offsets, const long long *lend,
                                                            const int2 *lists,
                                                            unsigned long long *stats) {
   __shared__ float4 s_tile4[kWaves][2 * kPlane / 4];  // re plane, then im plane
@@ -525,14 +544,16 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
   const float *svl = reinterpret_cast<const float *>(sv) + 2 * mk + (mm >= 8 ? 1 : 0);
   int *scell = s_cell[wv];
   int *flag = s_flag[wv];
+  const long long nitems = *nitemsPtr;
   for (long long w = (long long)blockIdx.x * kWaves + wv; w < nitems;
        w += (long long)gridDim.x * kWaves) {
     const int2 item = items[w];
     const long long L = __builtin_amdgcn_readfirstlane(item.x);
-    const int n = counts[L];
-    const int e0 = __builtin_amdgcn_readfirstlane(item.y) * kChunk;
-    const int e1 = min(n, e0 + kChunk);
-    const bool multi = n > kChunk;
+    const long long l0 = offsets[L];
+    const int n = (int)(lend[L] - l0);
+    const int e0 = __builtin_amdgcn_readfirstlane(item.y) * chunk;
+    const int e1 = min(n, e0 + chunk);
+    const bool multi = n > chunk;
     const int fi = listFacet[L];
     // a register copy: the wave fences below would otherwise make every
     // pass reload the descriptor from memory and wait on the row prefetch
@@ -544,7 +565,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
     const int tv = t / f.ntu, tu = t - tv * f.ntu;
     const int col0 = tu * TU, row0 = tv * TV;
     for (int i = lane; i < 2 * kPlane / 4; i += 64) s_tile4[wv][i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const int2 *lst = lists + offsets[L];
+    const int2 *lst = lists + l0;
     const int npc = cm.pcount[p];
     if (npc <= 0) continue;  // planes without channels have no tracks
     const int *pch = cm.pchan + (size_t)p * cm.maxpc;
@@ -1213,7 +1234,6 @@ struct GpuState {
   std::vector<FacetDev> h_facets;
   int *d_listFacet = nullptr;
   long long nlist = 0;
-  int *d_counts = nullptr;
   int2 *d_lists = nullptr;          // per list entry: row, lo | hi << 16 (channels of the plane list)
   long long *d_offsets = nullptr;  // first entry of every list (64-bit: passes may exceed 2^31 entries)
   long long *d_lend = nullptr;     // one past the last entry of every list
@@ -1229,11 +1249,12 @@ struct GpuState {
   void *d_scanTmp = nullptr;       // scan scratch
   size_t scanTmpBytes = 0;
   long long *h_tot = nullptr;      // pinned: list entries and work items of the last pass
-  long long nitems = 0;
+  long long nitems = 0, itemBound = 0;  // work items of the last pass; at most this many
+  int chunk = kChunk;              // tracks per work item of the last pass
+  bool anyBeam = false;            // a facet is gridded as a beam
   bool listsValid = false;         // the lists of the last pass, for ...
   long long listsRows = 0;         // ... a pass over as many rows ...
-  unsigned long long listsHash = 0;  // ... with the same uvw (k_uvw_hash)
-  unsigned long long *d_hash = nullptr;
+  unsigned long long *d_hash = nullptr;  // ... with the same uvw: their checksum, and another pass's
   unsigned long long *d_walk = nullptr;  // staged samples, base-cell moves of the last pass
   // FFT to images: C2R plan for (nx, ny, nplane), complex scratch, corrections
   hipfftHandle fftPlan = 0;
@@ -1327,6 +1348,7 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
   gs->h_facets.assign(nf, FacetDev{});
   long long listBase = 0;
   std::vector<int> listFacet;
+  gs->anyBeam = false;
   for (int k = 0; k < nf; ++k) {
     const FacetInfo *fi = in->h_facetInfo[gs->facets[k]];
     FacetDev &f = gs->h_facets[k];
@@ -1361,6 +1383,7 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
     f.ntu = (f.lrow / 2 + TU - 1) / TU;
     f.ntv = (f.ny + TV - 1) / TV;
     f.listBase = listBase;
+    gs->anyBeam = gs->anyBeam || f.doBeam;
     const long long nl = (long long)nplane * f.ntu * f.ntv;
     listFacet.insert(listFacet.end(), (size_t)nl, k);
     listBase += nl;
@@ -1456,39 +1479,35 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
   // 25 bits above the 7-bit window block
   if (gs->nlist >= (1LL << 25))
     return fail(kInvalid, "%lld tile lists (facets x planes x tiles) exceed 2^25", gs->nlist);
-  (void)hipFree(gs->d_counts); (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets);
-  gs->d_counts = nullptr; gs->d_lend = nullptr; gs->d_offsets = nullptr;
-  OBIT_HIP_TRY(hipMalloc(&gs->d_counts, sizeof(int) * (gs->nlist + 1)));
+  (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets);
+  gs->d_lend = nullptr; gs->d_offsets = nullptr;
   OBIT_HIP_TRY(hipMalloc(&gs->d_lend, sizeof(long long) * (gs->nlist + 1)));
   OBIT_HIP_TRY(hipMalloc(&gs->d_offsets, sizeof(long long) * (gs->nlist + 1)));
   (void)hipFree(gs->d_itemOff);
   OBIT_HIP_TRY(hipMalloc(&gs->d_itemOff, sizeof(long long) * (gs->nlist + 1)));
-  if (!gs->h_tot) OBIT_HIP_TRY(hipHostMalloc(&gs->h_tot, 2 * sizeof(long long), hipHostMallocDefault));
+  if (!gs->h_tot) OBIT_HIP_TRY(hipHostMalloc(&gs->h_tot, 4 * sizeof(long long), hipHostMallocDefault));
   gs->ready = true;
   return kOK;
 }
 
-// Bin and grid nrow rows at a device pointer into every facet on gs.
-// List sizes as 64-bit entry counts and as kChunk-track work-item counts.
-struct ToEntries {
-  __host__ __device__ long long operator()(int n) const { return (long long)n; }
-};
 struct ToEntriesU {
   __host__ __device__ unsigned long long operator()(unsigned n) const { return (unsigned long long)n; }
 };
+// Work items of a list: its entries in chunks.
 struct ToChunks {
-  __host__ __device__ long long operator()(int n) const { return (long long)((n + kChunk - 1) / kChunk); }
+  const long long *first, *last;
+  int chunk;
+  __host__ __device__ long long operator()(long long L) const { return (last[L] - first[L] + chunk - 1) / chunk; }
 };
 
 // Work items (list, chunk) of every list, in list order, at the list's
 // scanned item offset.
-__global__ __launch_bounds__(256) void k_items(const int *counts, const long long *itemOff, long long nl,
-                                               int2 *items) {
+__global__ __launch_bounds__(256) void k_items(const long long *first, const long long *last, int chunk,
+                                               const long long *itemOff, long long nl, int2 *items) {
   for (long long L = (long long)blockIdx.x * blockDim.x + threadIdx.x; L < nl;
        L += (long long)gridDim.x * blockDim.x) {
-    const int n = counts[L];
-    const long long base = itemOff[L];
-    for (int c = 0; c * kChunk < n; ++c) items[base + c] = make_int2((int)L, c);
+    const long long n = (last[L] - first[L] + chunk - 1) / chunk, base = itemOff[L];
+    for (long long c = 0; c < n; ++c) items[base + c] = make_int2((int)L, (int)c);
   }
 }
 
@@ -1505,19 +1524,12 @@ hipError_t ensure_tmp(GpuState *gs, size_t need) {
   return e;
 }
 
-// Checksum of the uvw of nrow rows (k_uvw_hash), read back.
-int uvw_hash(GpuState *gs, const float *vis, long long nrow, unsigned long long &h) {
-  if (!gs->d_hash) OBIT_HIP_TRY(hipMalloc(&gs->d_hash, sizeof(unsigned long long)));
-  hipLaunchKernelGGL(k_zero2, dim3(1), dim3(64), 0, gs->stream, (int *)gs->d_hash, (int *)gs->d_hash + 1, 1LL);
-  const int nb = (int)std::min<long long>((nrow + 255) / 256, (long long)gs->nCU * 4);
-  hipLaunchKernelGGL(k_uvw_hash, dim3(std::max(nb, 1)), dim3(256), 0, gs->stream, vis, nrow, gs->cm.lenvis,
-                     gs->d_hash);
-  OBIT_HIP_TRY(hipGetLastError());
-  OBIT_HIP_TRY(hipMemcpyAsync(&h, gs->d_hash, sizeof(h), hipMemcpyDeviceToHost, gs->stream));
-  OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));
-  return kOK;
-}
+// Sort of the entries: radix passes from 16,384 entries up, where the default
+// merge sort of up to 2^20 entries launches two kernels for every doubling.
+using SortConfig = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
+                                              rocprim::default_config, 16384>;
 
+// Bin and grid nrow rows at a device pointer into every facet on gs.
 int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   if (!gs->ready) return fail(kState, "gridder not initialised");
   if (nrow > (long long)INT_MAX)
@@ -1528,24 +1540,38 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   const int nf = (int)gs->facets.size();
   const long long nl = gs->nlist;
   if (reuse) {
-    unsigned long long h = 0;
-    int rc = uvw_hash(gs, vis, nrow, h);
-    if (rc) return rc;
-    if (h != gs->listsHash)
-      return fail(kState, "cannot reuse the track lists: these rows' u, v, w differ from the last pass's");
-    // the lists, offsets and work items of the last pass stand: only the
-    // walk statistics restart
-    hipLaunchKernelGGL(k_zero2, dim3(1), dim3(64), 0, gs->stream, (int *)gs->d_walk, (int *)gs->d_walk + 2, 2LL);
+    // the rows' checksum beside the lists'; the lists, offsets and work items of
+    // the last pass stand: only the walk statistics restart
+    hipLaunchKernelGGL(k_pass_clear, dim3(1), dim3(64), 0, gs->stream, gs->d_walk, (unsigned *)nullptr, gs->d_hash + 1,
+                       (long long *)nullptr, (long long *)nullptr, 0LL);
+    const int nb = (int)std::min<long long>((nrow + 255) / 256, (long long)gs->nCU * 4);
+    hipLaunchKernelGGL(k_uvw_hash, dim3(std::max(nb, 1)), dim3(256), 0, gs->stream, vis, nrow, gs->cm.lenvis,
+                       gs->d_hash + 1);
     OBIT_HIP_TRY(hipGetLastError());
+    OBIT_HIP_TRY(hipMemcpyAsync(gs->h_tot + 2, gs->d_hash, 2 * sizeof(long long), hipMemcpyDeviceToHost, gs->stream));
+    OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));
+    if (gs->h_tot[2] != gs->h_tot[3])
+      return fail(kState, "cannot reuse the track lists: these rows' u, v, w differ from the last pass's");
     return launch_taps(gs, vis);
+  }
+  if (!gs->d_walk) OBIT_HIP_TRY(hipMalloc(&gs->d_walk, 2 * sizeof(unsigned long long)));
+  if (!gs->d_hash) OBIT_HIP_TRY(hipMalloc(&gs->d_hash, 2 * sizeof(unsigned long long)));
+  if (gs->tapsPerCU <= 0) {
+    int nb = 0;
+    OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_grid_taps, 64 * kWaves, 0));
+    gs->tapsPerCU = std::max(nb, 1);
   }
   gs->listsValid = false;
   if ((long long)nrow * gs->cm.nplane * nf > (1LL << 40)) return fail(kInvalid, "too many tracks");
-  if (!gs->d_walk) OBIT_HIP_TRY(hipMalloc(&gs->d_walk, 2 * sizeof(unsigned long long)));
-  hipLaunchKernelGGL(k_zero2, dim3(1), dim3(64), 0, gs->stream, (int *)gs->d_walk,
-                     (int *)gs->d_walk + 2, 2LL);
-  OBIT_HIP_TRY(hipGetLastError());
-  const long long ntr = nrow * (long long)nf;
+  // Threads of the binning: one per (row, facet), or where those fill less than 4
+  // waves of every SIMD, with the planes divided to about as many.  A thread's
+  // time is a chain of binary searches, the longer the more planes it takes, and
+  // a small pass waits for the chain; a large pass gains nothing by it and would
+  // scan more counts.
+  const long long nrf = nrow * (long long)nf;
+  const long long fill = (long long)gs->nCU * 4 * 64 * 4;
+  const int nsplit = (int)std::min<long long>(gs->cm.nplane, (fill + nrf - 1) / nrf);
+  const long long ntr = nrf * nsplit;
   if (ntr + 1 > gs->tcap) {
     (void)hipFree(gs->d_tcnt); (void)hipFree(gs->d_toff);
     gs->d_tcnt = nullptr; gs->d_toff = nullptr;
@@ -1556,10 +1582,11 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   const int nbB = (int)std::min<long long>((ntr + 255) / 256, (long long)gs->nCU * 32);
   // pass 1: entries per track; the slot after the last track is zero so
   // the scan's last element is the total
-  hipLaunchKernelGGL(k_zero2, dim3(1), dim3(64), 0, gs->stream, (int *)gs->d_tcnt + ntr,
-                     (int *)gs->d_tcnt + ntr, 1LL);
-  hipLaunchKernelGGL(k_bin_count, dim3(nbB), dim3(256), 0, gs->stream, vis, nrow, gs->d_facets, nf, gs->cm,
-                     gs->d_tcnt);
+  const int nbz = (int)std::min<long long>((nl + 1 + 255) / 256, (long long)gs->nCU * 16);
+  hipLaunchKernelGGL(k_pass_clear, dim3(nbz), dim3(256), 0, gs->stream, gs->d_walk, gs->d_tcnt + ntr, gs->d_hash,
+                     gs->d_offsets, gs->d_lend, nl + 1);
+  hipLaunchKernelGGL(k_bin_count, dim3(nbB), dim3(256), 0, gs->stream, vis, nrow, gs->d_facets, nf, nsplit,
+                     gs->cm, gs->d_tcnt, gs->d_hash);
   OBIT_HIP_TRY(hipGetLastError());
   {
     size_t need = 0;
@@ -1588,84 +1615,89 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     gs->listCap = total;
   }
   // pass 2: keys and rows, then the stable sort by (list, window block)
-  hipLaunchKernelGGL(k_bin_emit, dim3(nbB), dim3(256), 0, gs->stream, vis, nrow, gs->d_facets, nf, gs->cm,
+  hipLaunchKernelGGL(k_bin_emit, dim3(nbB), dim3(256), 0, gs->stream, vis, nrow, gs->d_facets, nf, nsplit, gs->cm,
                      gs->d_toff, gs->d_keys, gs->d_rows);
   OBIT_HIP_TRY(hipGetLastError());
   int endBit = 7;
   while ((1LL << (endBit - 7)) < nl) ++endBit;
   if (total > 0) {
     size_t need = 0;
-    OBIT_HIP_TRY(rocprim::radix_sort_pairs(nullptr, need, gs->d_keys, gs->d_keys2, gs->d_rows, gs->d_lists,
+    OBIT_HIP_TRY(rocprim::radix_sort_pairs<SortConfig>(nullptr, need, gs->d_keys, gs->d_keys2, gs->d_rows, gs->d_lists,
                                            (size_t)total, 0, endBit, gs->stream));
     OBIT_HIP_TRY(ensure_tmp(gs, need));
-    OBIT_HIP_TRY(rocprim::radix_sort_pairs(gs->d_scanTmp, need, gs->d_keys, gs->d_keys2, gs->d_rows,
+    OBIT_HIP_TRY(rocprim::radix_sort_pairs<SortConfig>(gs->d_scanTmp, need, gs->d_keys, gs->d_keys2, gs->d_rows,
                                            gs->d_lists, (size_t)total, 0, endBit, gs->stream));
   }
-  // list extents and sizes, then the work items: an exclusive scan of the
-  // lists' kChunk-track chunk counts (the entry after the last list is
-  // zero, so the scan's last element is the number of items)
-  {
-    const int nbz = (int)std::min<long long>((nl + 1 + 255) / 256, 65535);
-    hipLaunchKernelGGL(k_zero64, dim3(nbz), dim3(256), 0, gs->stream, gs->d_offsets, gs->d_lend, nl + 1);
+  // Tracks per work item.  A wave walks its item's samples one after the other,
+  // so a pass takes at least as long as an item, which goes with its tracks; and
+  // each item costs a tile cleared and added to the grid, which goes with the
+  // number of items a wave has, entries / (tracks x waves).  The two balance
+  // where the tracks go with sqrt(entries / waves): tracks are halved from 128
+  // while 80 entries / waves stays under their square (calls of 8,192 rows x 64
+  // channels into 512^2, 11,000 entries: 128 tracks 383 us, 16 tracks 169; 20,000
+  // x 256 ch into 8 planes of 2048^2, 243,000: 776, 64 tracks 727, 16 tracks 956;
+  // from 650,000 entries 128 is the fastest).  Passes with a beam keep 128: its
+  // samples add equal terms, whose FP32 rounding does not average out (3e-4 of
+  // the peak where a cell takes 12,000), so that its sums would move with the
+  // grouping.
+  const long long waves = (long long)gs->nCU * gs->tapsPerCU * kWaves;
+  gs->chunk = kChunk;
+  if (!gs->anyBeam)
+    while (gs->chunk > kMinChunk && 80 * total < waves * gs->chunk * gs->chunk) gs->chunk /= 2;
+  gs->itemBound = std::min(total, nl + total / gs->chunk + 1);
+  if (gs->itemBound > gs->itemCap) {
+    (void)hipFree(gs->d_items);
+    gs->d_items = nullptr;
+    gs->itemCap = 0;
+    OBIT_HIP_TRY(hipMalloc(&gs->d_items, sizeof(int2) * (size_t)gs->itemBound));
+    gs->itemCap = gs->itemBound;
+  }
+  // list extents, then the work items: an exclusive scan of the lists' chunk
+  // counts (the list after the last is empty, so the scan's last element is the
+  // number of items, which the gridding kernel reads where it is)
+  if (total > 0) {
     const int nbk = (int)std::min<long long>((total + 255) / 256, (long long)gs->nCU * 32);
-    if (total > 0)
-      hipLaunchKernelGGL(k_list_bounds, dim3(nbk), dim3(256), 0, gs->stream, gs->d_keys2, total, gs->d_offsets,
-                         gs->d_lend);
-    hipLaunchKernelGGL(k_list_counts, dim3(nbz), dim3(256), 0, gs->stream, gs->d_offsets, gs->d_lend, nl + 1,
-                       gs->d_counts);
+    hipLaunchKernelGGL(k_list_bounds, dim3(nbk), dim3(256), 0, gs->stream, gs->d_keys2, total, gs->d_offsets,
+                       gs->d_lend);
     OBIT_HIP_TRY(hipGetLastError());
-    const auto chunks = rocprim::make_transform_iterator(gs->d_counts, ToChunks());
+    const auto chunks = rocprim::make_transform_iterator(rocprim::counting_iterator<long long>(0),
+                                                         ToChunks{gs->d_offsets, gs->d_lend, gs->chunk});
     size_t need = 0;
     OBIT_HIP_TRY(rocprim::exclusive_scan(nullptr, need, chunks, gs->d_itemOff, 0LL, (size_t)nl + 1,
                                          rocprim::plus<long long>(), gs->stream));
     OBIT_HIP_TRY(ensure_tmp(gs, need));
     OBIT_HIP_TRY(rocprim::exclusive_scan(gs->d_scanTmp, need, chunks, gs->d_itemOff, 0LL, (size_t)nl + 1,
                                          rocprim::plus<long long>(), gs->stream));
+    const int nbI = (int)std::min<long long>((nl + 255) / 256, (long long)gs->nCU * 16);
+    hipLaunchKernelGGL(k_items, dim3(nbI), dim3(256), 0, gs->stream, gs->d_offsets, gs->d_lend, gs->chunk,
+                       gs->d_itemOff, nl, gs->d_items);
+    OBIT_HIP_TRY(hipGetLastError());
     OBIT_HIP_TRY(hipMemcpyAsync(gs->h_tot + 1, gs->d_itemOff + nl, sizeof(long long), hipMemcpyDeviceToHost,
                                 gs->stream));
-    OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));
+  } else {
+    gs->h_tot[1] = 0;
   }
-  const long long nitems = gs->h_tot[1];
-  gs->nitems = nitems;
-  if (nitems < 0 || nitems > total) return fail(kHipError, "list scan gave %lld entries, %lld items", total, nitems);
-  if (nitems > gs->itemCap) {
-    (void)hipFree(gs->d_items);
-    gs->d_items = nullptr;
-    OBIT_HIP_TRY(hipMalloc(&gs->d_items, sizeof(int2) * (size_t)std::max<long long>(nitems, 1)));
-    gs->itemCap = nitems;
-  }
-  if (nitems) {
-    const int nbI = (int)std::min<long long>((nl + 255) / 256, (long long)gs->nCU * 16);
-    hipLaunchKernelGGL(k_items, dim3(nbI), dim3(256), 0, gs->stream, gs->d_counts, gs->d_itemOff, nl,
-                       gs->d_items);
-    OBIT_HIP_TRY(hipGetLastError());
-  }
-  {
-    int rc = uvw_hash(gs, vis, nrow, gs->listsHash);
-    if (rc) return rc;
-  }
+  int rc = launch_taps(gs, vis);  // the pass is complete when it returns
+  if (rc) return rc;
+  gs->nitems = gs->h_tot[1];
+  if (gs->nitems < 0 || gs->nitems > gs->itemBound)
+    return fail(kHipError, "list scan gave %lld entries, %lld items", total, gs->nitems);
   gs->listsValid = true;
   gs->listsRows = nrow;
-  return launch_taps(gs, vis);
+  return kOK;
 }
 
 // The tile-gridding launch over the current work items; the pass is
 // complete when it returns.
 int launch_taps(GpuState *gs, const float *vis) {
-  const long long nitems = gs->nitems;
-  if (nitems) {
+  if (gs->itemBound) {
     // persistent grid of exactly the resident blocks: more would queue a
     // second round of blocks behind the first and idle CUs at the end
-    if (gs->tapsPerCU <= 0) {
-      int nb = 0;
-      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_grid_taps, 64 * kWaves, 0));
-      gs->tapsPerCU = std::max(nb, 1);
-    }
     const long long nbG =
-        std::min<long long>((nitems + kWaves - 1) / kWaves, (long long)gs->nCU * gs->tapsPerCU);
+        std::min<long long>((gs->itemBound + kWaves - 1) / kWaves, (long long)gs->nCU * gs->tapsPerCU);
     hipLaunchKernelGGL(k_grid_taps, dim3((unsigned)nbG), dim3(64 * kWaves), 0, gs->stream, vis,
-                       gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items, nitems, gs->cm,
-                       gs->d_counts, gs->d_offsets, gs->d_lists, gs->d_walk);
+                       gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items, gs->d_itemOff + gs->nlist, gs->chunk,
+                       gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists, gs->d_walk);
     OBIT_HIP_TRY(hipGetLastError());
   }
   // the pass is complete when the call returns
@@ -1837,7 +1869,7 @@ void ObitCUDAGridShutdown(CUDAGridInfo *cudaInfo, long iGPU) {
     (void)hipFree(gs->d_gcf); (void)hipFree(gs->d_freq); (void)hipFree(gs->d_sig); (void)hipFree(gs->d_pf);
     (void)hipFree(gs->d_pfreq); (void)hipFree(gs->d_pmono);
     (void)hipFree(gs->d_pchan); (void)hipFree(gs->d_pcount); (void)hipFree(gs->d_facets); (void)hipFree(gs->d_listFacet);
-    (void)hipFree(gs->d_counts); (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets); (void)hipFree(gs->d_lists);
+    (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets); (void)hipFree(gs->d_lists);
     (void)hipFree(gs->d_tcnt); (void)hipFree(gs->d_toff); (void)hipFree(gs->d_keys); (void)hipFree(gs->d_keys2);
     (void)hipFree(gs->d_rows);
     (void)hipFree(gs->d_items); (void)hipFree(gs->d_vis); (void)hipFree(gs->d_walk); (void)hipFree(gs->d_hash);
@@ -2145,16 +2177,18 @@ int ObitHIPGridListStats(CUDAGridInfo *in, long iGPU, long long *stats) {
   GpuState *gs = obit::grid::get_gpu(in, iGPU, false);
   if (!gs || !stats) return obit::fail(obit::kState, "gridder not allocated");
   long long nonEmpty = 0, entries = 0, maxc = 0, multi = 0;
-  std::vector<int> counts((size_t)gs->nlist);
-  if (gs->nlist > 0 && gs->d_counts) {
+  std::vector<long long> first((size_t)gs->nlist), last((size_t)gs->nlist);
+  if (gs->nlist > 0 && gs->d_offsets) {
     OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));
-    OBIT_HIP_TRY(hipMemcpy(counts.data(), gs->d_counts, sizeof(int) * gs->nlist, hipMemcpyDeviceToHost));
+    OBIT_HIP_TRY(hipMemcpy(first.data(), gs->d_offsets, sizeof(long long) * gs->nlist, hipMemcpyDeviceToHost));
+    OBIT_HIP_TRY(hipMemcpy(last.data(), gs->d_lend, sizeof(long long) * gs->nlist, hipMemcpyDeviceToHost));
   }
-  for (int c : counts) {
+  for (long long i = 0; i < gs->nlist; ++i) {
+    const long long c = last[i] - first[i];
     if (c > 0) ++nonEmpty;
     entries += c;
     if (c > maxc) maxc = c;
-    if (c > obit::grid::kChunk) ++multi;
+    if (c > gs->chunk) ++multi;
   }
   stats[0] = gs->nlist;
   stats[1] = nonEmpty;
