@@ -783,6 +783,19 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
   }
 }
 
+// The grids of every facet set to zero in one launch (a memset a facet took two
+// or three launches each: 2 facets x 3 planes of 1200^2 32 us).  Write bound.
+__global__ __launch_bounds__(256) void k_grid_clear(const FacetDev *facets, int nf, int nplane) {
+  for (int fi = blockIdx.y; fi < nf; fi += gridDim.y) {
+    float *g = facets[fi].grid;
+    const long long n = (long long)facets[fi].sizeGrid * nplane, n4 = n >> 2;
+    float4 *g4 = reinterpret_cast<float4 *>(g);
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n4; i += (long long)gridDim.x * 256)
+      g4[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) g[4 * n4 + threadIdx.x] = 0.0f;
+  }
+}
+
 // ThreadFlip (src/ObitThreadGrid.c:998-1045) as a parallel update: thread
 // (facet plane, vrow in 1..ny/2, iu in 0..hw).  Each thread reads the
 // cells at hw-iu (never written) and hw+iu (written only by itself).
@@ -1230,10 +1243,10 @@ struct GpuState {
   int nCU = 256;
   int tapsPerCU = 0;        // resident k_grid_taps blocks per CU (0: not queried yet)
   std::vector<int> facets;  // facet indices on this GPU
-  FacetDev *d_facets = nullptr;
+  FacetDev *d_facets = nullptr;  // in d_tab
   std::vector<FacetDev> h_facets;
   int *d_listFacet = nullptr;
-  long long nlist = 0;
+  long long nlist = 0, nlistCap = 0;  // tile lists; room in the arrays with an element for each
   int2 *d_lists = nullptr;          // per list entry: row, lo | hi << 16 (channels of the plane list)
   long long *d_offsets = nullptr;  // first entry of every list (64-bit: passes may exceed 2^31 entries)
   long long *d_lend = nullptr;     // one past the last entry of every list
@@ -1270,9 +1283,8 @@ struct GpuState {
   std::vector<float> h_corr;  // xCorr, yCorr of the last (nx, ny) (GridCorrFn)
   int corrNx = 0, corrNy = 0;
   // tables
-  float *d_gcf = nullptr, *d_freq = nullptr, *d_sig = nullptr, *d_pf = nullptr, *d_pfreq = nullptr;
-  int *d_pmono = nullptr;
-  int *d_pchan = nullptr, *d_pcount = nullptr;
+  char *d_tab = nullptr, *h_tab = nullptr;  // tables (refresh), device and pinned
+  size_t tabCap = 0;
   Common cm{};
   bool ready = false;
   // staging for host buffers
@@ -1327,6 +1339,19 @@ void build_gcf(const float *convfn, int W, int N, std::vector<float> &gcf) {
     }
 }
 
+// The facet of every tile list: the last whose first list is not after it.
+__global__ __launch_bounds__(256) void k_list_facet(const FacetDev *facets, int nf, long long nl, int *listFacet) {
+  for (long long L = (long long)blockIdx.x * blockDim.x + threadIdx.x; L < nl;
+       L += (long long)gridDim.x * blockDim.x) {
+    int a = 0, b = nf;  // listBase of a <= L, of b > L
+    while (b - a > 1) {
+      const int m = (a + b) >> 1;
+      if (facets[m].listBase <= L) a = m; else b = m;
+    }
+    listFacet[L] = a;
+  }
+}
+
 // Upload tables and facet parameters from the host descriptors.
 int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
   gs->listsValid = false;
@@ -1347,7 +1372,6 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
   const int nf = (int)gs->facets.size();
   gs->h_facets.assign(nf, FacetDev{});
   long long listBase = 0;
-  std::vector<int> listFacet;
   gs->anyBeam = false;
   for (int k = 0; k < nf; ++k) {
     const FacetInfo *fi = in->h_facetInfo[gs->facets[k]];
@@ -1385,7 +1409,6 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
     f.listBase = listBase;
     gs->anyBeam = gs->anyBeam || f.doBeam;
     const long long nl = (long long)nplane * f.ntu * f.ntv;
-    listFacet.insert(listFacet.end(), (size_t)nl, k);
     listBase += nl;
   }
   gs->nlist = listBase;
@@ -1430,61 +1453,89 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
   bool hasSigma = false;
   if (gi->h_sigma1)
     for (int c = 0; c < nchan; ++c) hasSigma = hasSigma || gi->h_sigma1[c] != 0.0f;
-  // (re)allocate device tables
-  (void)hipFree(gs->d_gcf); (void)hipFree(gs->d_freq); (void)hipFree(gs->d_sig); (void)hipFree(gs->d_pf);
-  (void)hipFree(gs->d_pchan); (void)hipFree(gs->d_pcount); (void)hipFree(gs->d_facets); (void)hipFree(gs->d_listFacet);
-  (void)hipFree(gs->d_pfreq); (void)hipFree(gs->d_pmono);
-  OBIT_HIP_TRY(hipMalloc(&gs->d_pfreq, sizeof(float) * hpfreq.size()));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_pmono, sizeof(int) * nplane));
-  OBIT_HIP_TRY(hipMemcpy(gs->d_pfreq, hpfreq.data(), sizeof(float) * hpfreq.size(), hipMemcpyHostToDevice));
-  OBIT_HIP_TRY(hipMemcpy(gs->d_pmono, hmono.data(), sizeof(int) * nplane, hipMemcpyHostToDevice));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_gcf, sizeof(float) * kGcf8));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_freq, sizeof(float) * nchan));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_sig, sizeof(float) * 3 * nchan));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_pf, sizeof(float) * 2 * nplane));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_pchan, sizeof(int) * hpch.size()));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_pcount, sizeof(int) * nplane));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_facets, sizeof(FacetDev) * std::max(nf, 1)));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_listFacet, sizeof(int) * std::max<long long>(gs->nlist, 1)));
-  // rows of 8 (seven taps and a zero) so a row loads as two float4
-  std::vector<float> gcf8(kGcf8, 0.0f);
-  for (int it = 0; it <= N; ++it)
-    for (int c = 0; c < W; ++c) gcf8[8 * it + c] = gcf[(size_t)W * it + c];
-  OBIT_HIP_TRY(hipMemcpy(gs->d_gcf, gcf8.data(), sizeof(float) * kGcf8, hipMemcpyHostToDevice));
-  OBIT_HIP_TRY(hipMemcpy(gs->d_freq, gi->h_freqArr, sizeof(float) * nchan, hipMemcpyHostToDevice));
-  std::vector<float> sig(3 * (size_t)nchan, 0.0f);
-  if (gi->h_sigma1) std::memcpy(sig.data(), gi->h_sigma1, sizeof(float) * nchan);
-  if (gi->h_sigma2) std::memcpy(sig.data() + nchan, gi->h_sigma2, sizeof(float) * nchan);
-  if (gi->h_sigma3) std::memcpy(sig.data() + 2 * nchan, gi->h_sigma3, sizeof(float) * nchan);
-  OBIT_HIP_TRY(hipMemcpy(gs->d_sig, sig.data(), sizeof(float) * 3 * nchan, hipMemcpyHostToDevice));
-  OBIT_HIP_TRY(hipMemcpy(gs->d_pf, pf.data(), sizeof(float) * 2 * nplane, hipMemcpyHostToDevice));
-  OBIT_HIP_TRY(hipMemcpy(gs->d_pchan, hpch.data(), sizeof(int) * hpch.size(), hipMemcpyHostToDevice));
-  OBIT_HIP_TRY(hipMemcpy(gs->d_pcount, hpcount.data(), sizeof(int) * nplane, hipMemcpyHostToDevice));
-  if (nf) OBIT_HIP_TRY(hipMemcpy(gs->d_facets, gs->h_facets.data(), sizeof(FacetDev) * nf, hipMemcpyHostToDevice));
-  if (gs->nlist)
-    OBIT_HIP_TRY(hipMemcpy(gs->d_listFacet, listFacet.data(), sizeof(int) * gs->nlist, hipMemcpyHostToDevice));
-  Common &cm = gs->cm;
-  cm.nrparm = gi->nrparm; cm.lenvis = gi->lenvis; cm.nchan = nchan; cm.nplane = nplane;
-  cm.convWidth = W; cm.convNperCell = N;
-  cm.freq = gs->d_freq;
-  cm.sig1 = gs->d_sig; cm.sig2 = gs->d_sig + nchan; cm.sig3 = gs->d_sig + 2 * nchan;
-  cm.hasSigma = hasSigma ? 1 : 0;
-  cm.pchan = gs->d_pchan; cm.pcount = gs->d_pcount;
-  cm.pfmin = gs->d_pf; cm.pfmax = gs->d_pf + nplane;
-  cm.maxpc = maxpc;
-  cm.pfreq = gs->d_pfreq;
-  cm.pmono = gs->d_pmono;
-  cm.gcf = gs->d_gcf;
   // list buffers sized for the lists; sort keys hold the list index in
   // 25 bits above the 7-bit window block
   if (gs->nlist >= (1LL << 25))
     return fail(kInvalid, "%lld tile lists (facets x planes x tiles) exceed 2^25", gs->nlist);
-  (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets);
-  gs->d_lend = nullptr; gs->d_offsets = nullptr;
-  OBIT_HIP_TRY(hipMalloc(&gs->d_lend, sizeof(long long) * (gs->nlist + 1)));
-  OBIT_HIP_TRY(hipMalloc(&gs->d_offsets, sizeof(long long) * (gs->nlist + 1)));
-  (void)hipFree(gs->d_itemOff);
-  OBIT_HIP_TRY(hipMalloc(&gs->d_itemOff, sizeof(long long) * (gs->nlist + 1)));
+  // The tables lie one after the other in one device block, packed in pinned
+  // memory and sent in one copy on the stream: each image starts with a refresh,
+  // and an allocation, a free and a blocking copy for each of 15 tables took 190 us
+  // (the lists' facets, 2.8 MB for 20 facets x 8 planes of 2048^2, 750 us).
+  // Both blocks and the list arrays are kept until a larger layout or Shutdown.
+  size_t tab = 0;
+  auto room = [&](size_t bytes) {
+    const size_t at = tab;
+    tab += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t oGcf = room(sizeof(float) * kGcf8), oFreq = room(sizeof(float) * nchan),
+               oSig = room(sizeof(float) * 3 * nchan), oPf = room(sizeof(float) * 2 * nplane),
+               oPchan = room(sizeof(int) * hpch.size()), oPcount = room(sizeof(int) * nplane),
+               oPfreq = room(sizeof(float) * hpfreq.size()), oPmono = room(sizeof(int) * nplane),
+               oFacets = room(sizeof(FacetDev) * std::max(nf, 1));
+  // the last refresh's copy and every launch that reads the tables have ended
+  OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));
+  gs->ready = false;
+  if (tab > gs->tabCap) {
+    (void)hipFree(gs->d_tab);
+    if (gs->h_tab) (void)hipHostFree(gs->h_tab);
+    gs->d_tab = gs->h_tab = nullptr;
+    gs->tabCap = 0;
+    OBIT_HIP_TRY(hipMalloc(&gs->d_tab, tab));
+    OBIT_HIP_TRY(hipHostMalloc(&gs->h_tab, tab, hipHostMallocDefault));
+    gs->tabCap = tab;
+  }
+  // rows of 8 (seven taps and a zero) so a row loads as two float4
+  float *gcf8 = reinterpret_cast<float *>(gs->h_tab + oGcf);
+  std::memset(gcf8, 0, sizeof(float) * kGcf8);
+  for (int it = 0; it <= N; ++it)
+    for (int c = 0; c < W; ++c) gcf8[8 * it + c] = gcf[(size_t)W * it + c];
+  std::memcpy(gs->h_tab + oFreq, gi->h_freqArr, sizeof(float) * nchan);
+  float *sig = reinterpret_cast<float *>(gs->h_tab + oSig);
+  std::memset(sig, 0, sizeof(float) * 3 * nchan);
+  if (gi->h_sigma1) std::memcpy(sig, gi->h_sigma1, sizeof(float) * nchan);
+  if (gi->h_sigma2) std::memcpy(sig + nchan, gi->h_sigma2, sizeof(float) * nchan);
+  if (gi->h_sigma3) std::memcpy(sig + 2 * nchan, gi->h_sigma3, sizeof(float) * nchan);
+  std::memcpy(gs->h_tab + oPf, pf.data(), sizeof(float) * 2 * nplane);
+  std::memcpy(gs->h_tab + oPchan, hpch.data(), sizeof(int) * hpch.size());
+  std::memcpy(gs->h_tab + oPcount, hpcount.data(), sizeof(int) * nplane);
+  std::memcpy(gs->h_tab + oPfreq, hpfreq.data(), sizeof(float) * hpfreq.size());
+  std::memcpy(gs->h_tab + oPmono, hmono.data(), sizeof(int) * nplane);
+  if (nf) std::memcpy(gs->h_tab + oFacets, gs->h_facets.data(), sizeof(FacetDev) * nf);
+  OBIT_HIP_TRY(hipMemcpyAsync(gs->d_tab, gs->h_tab, tab, hipMemcpyHostToDevice, gs->stream));
+  gs->d_facets = reinterpret_cast<FacetDev *>(gs->d_tab + oFacets);
+  Common &cm = gs->cm;
+  cm.nrparm = gi->nrparm; cm.lenvis = gi->lenvis; cm.nchan = nchan; cm.nplane = nplane;
+  cm.convWidth = W; cm.convNperCell = N;
+  cm.freq = reinterpret_cast<float *>(gs->d_tab + oFreq);
+  cm.sig1 = reinterpret_cast<float *>(gs->d_tab + oSig);
+  cm.sig2 = cm.sig1 + nchan; cm.sig3 = cm.sig1 + 2 * nchan;
+  cm.hasSigma = hasSigma ? 1 : 0;
+  cm.pchan = reinterpret_cast<int *>(gs->d_tab + oPchan);
+  cm.pcount = reinterpret_cast<int *>(gs->d_tab + oPcount);
+  cm.pfmin = reinterpret_cast<float *>(gs->d_tab + oPf);
+  cm.pfmax = cm.pfmin + nplane;
+  cm.maxpc = maxpc;
+  cm.pfreq = reinterpret_cast<float *>(gs->d_tab + oPfreq);
+  cm.pmono = reinterpret_cast<int *>(gs->d_tab + oPmono);
+  cm.gcf = reinterpret_cast<float *>(gs->d_tab + oGcf);
+  if (gs->nlist + 1 > gs->nlistCap) {
+    (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets); (void)hipFree(gs->d_itemOff); (void)hipFree(gs->d_listFacet);
+    gs->d_lend = gs->d_offsets = gs->d_itemOff = nullptr;
+    gs->d_listFacet = nullptr;
+    gs->nlistCap = 0;
+    OBIT_HIP_TRY(hipMalloc(&gs->d_lend, sizeof(long long) * (gs->nlist + 1)));
+    OBIT_HIP_TRY(hipMalloc(&gs->d_offsets, sizeof(long long) * (gs->nlist + 1)));
+    OBIT_HIP_TRY(hipMalloc(&gs->d_itemOff, sizeof(long long) * (gs->nlist + 1)));
+    OBIT_HIP_TRY(hipMalloc(&gs->d_listFacet, sizeof(int) * (gs->nlist + 1)));
+    gs->nlistCap = gs->nlist + 1;
+  }
+  if (gs->nlist) {
+    const int nbL = (int)std::min<long long>((gs->nlist + 255) / 256, (long long)gs->nCU * 16);
+    hipLaunchKernelGGL(k_list_facet, dim3(nbL), dim3(256), 0, gs->stream, gs->d_facets, nf, gs->nlist,
+                       gs->d_listFacet);
+    OBIT_HIP_TRY(hipGetLastError());
+  }
   if (!gs->h_tot) OBIT_HIP_TRY(hipHostMalloc(&gs->h_tot, 4 * sizeof(long long), hipHostMallocDefault));
   gs->ready = true;
   return kOK;
@@ -1792,13 +1843,22 @@ void ObitCUDAGridInit(CUDAGridInfo *cudaInfo, long iGPU) {
     if (cudaInfo->FacetGPU && cudaInfo->FacetGPU[i] != iGPU) continue;
     FacetInfo *fi = cudaInfo->h_facetInfo[i];
     const size_t bytes = (size_t)fi->sizeGrid * nplane * sizeof(float);
-    if (!fi->d_grid) OBIT_HIP_CHECK(hipMalloc(&fi->d_grid, bytes));
     // the pinned host copy (h_grid) is allocated by ObitCUDAGrid2CPU on
     // first use, so grids that stay on the device cost no host memory
-    OBIT_HIP_CHECK(hipMemsetAsync(fi->d_grid, 0, bytes, gs->stream));
+    if (!fi->d_grid) OBIT_HIP_CHECK(hipMalloc(&fi->d_grid, bytes));
+  }
+  if (obit::grid::refresh(cudaInfo, iGPU, gs)) grid_abort("ObitCUDAGridInit");
+  const int nf = (int)gs->facets.size();
+  if (nf) {
+    long long most = 0;
+    for (auto &f : gs->h_facets) most = std::max(most, (long long)f.sizeGrid * nplane);
+    const int ny = std::min(nf, 65535);
+    const long long nx = std::min<long long>((most + 4095) / 4096, std::max(1, gs->nCU * 16 / ny));
+    hipLaunchKernelGGL(obit::grid::k_grid_clear, dim3((unsigned)nx, ny), dim3(256), 0, gs->stream, gs->d_facets, nf,
+                       nplane);
+    OBIT_HIP_CHECK(hipGetLastError());
   }
   OBIT_HIP_CHECK(hipStreamSynchronize(gs->stream));
-  if (obit::grid::refresh(cudaInfo, iGPU, gs)) grid_abort("ObitCUDAGridInit");
 }
 
 void ObitCUDAGridGrid(CUDAGridInfo *cudaInfo, long iGPU, int init) {
@@ -1866,9 +1926,8 @@ void ObitCUDAGridShutdown(CUDAGridInfo *cudaInfo, long iGPU) {
       FacetInfo *fi = cudaInfo->h_facetInfo ? cudaInfo->h_facetInfo[i] : nullptr;
       if (fi && fi->d_grid) { (void)hipFree(fi->d_grid); fi->d_grid = nullptr; }
     }
-    (void)hipFree(gs->d_gcf); (void)hipFree(gs->d_freq); (void)hipFree(gs->d_sig); (void)hipFree(gs->d_pf);
-    (void)hipFree(gs->d_pfreq); (void)hipFree(gs->d_pmono);
-    (void)hipFree(gs->d_pchan); (void)hipFree(gs->d_pcount); (void)hipFree(gs->d_facets); (void)hipFree(gs->d_listFacet);
+    (void)hipFree(gs->d_tab); (void)hipFree(gs->d_listFacet);
+    if (gs->h_tab) (void)hipHostFree(gs->h_tab);
     (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets); (void)hipFree(gs->d_lists);
     (void)hipFree(gs->d_tcnt); (void)hipFree(gs->d_toff); (void)hipFree(gs->d_keys); (void)hipFree(gs->d_keys2);
     (void)hipFree(gs->d_rows);
