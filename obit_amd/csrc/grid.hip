@@ -86,10 +86,29 @@ struct Common {
 
 // ---------------- device: CPU-exact sample arithmetic ----------------
 
+// (int)floor(x + 0.5) with the sum exact, in one instruction.
+__device__ __forceinline__ int round_up(float x) {
+  int r;
+  asm("v_cvt_rpi_i32_f32_e32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+}
+
+// The CPU's lround, (int)((double)x +- 0.5): half away from zero.  Its FP64 sum
+// and conversions issue at a quarter of the rate of FP32 instructions, and a
+// sample is rounded four times; the conversion above gives the same for every
+// float below 2^31 (all bit patterns compared).
 __device__ __forceinline__ int lround_obit(float in) {
-#pragma clang fp contract(off)
-  if (in >= 0.0f) return (int)((double)in + 0.5);
-  return (int)((double)in - 0.5);
+  int r;
+  asm("v_cvt_rpi_i32_f32_e64 %0, |%1|" : "=v"(r) : "v"(in));
+  const int s = __float_as_int(in) >> 31;
+  return (r ^ s) - s;
+}
+
+// (int)((double)u + 0.5), u not negative but for frequencies that are not
+// positive.
+__device__ __forceinline__ int column_of(float u) {
+  if (u >= 0.0f) return round_up(u);
+  return (int)((double)u + 0.5);
 }
 
 struct Sample {
@@ -111,6 +130,13 @@ __device__ __forceinline__ void rotate_uvw(const FacetDev &f, const float *row, 
   rotate3(f, row[0], row[1], row[2], uu, vv, ww);
 }
 
+// Rotated uvw with the sign that makes u positive (the conjugate sample's where
+// it was not), and that sign.
+__device__ __forceinline__ float4 signed_uvw(float uu, float vv, float ww) {
+  const float s = (uu <= 0.0f) ? -1.0f : 1.0f;
+  return make_float4(s * uu, s * vv, s * ww, s);
+}
+
 // Cells of a channel at FP32 frequency factor freq (no validity test):
 // used by the binning pass to bound a track's footprint.
 __device__ __forceinline__ void cells_at(const FacetDev &f, float uu, float vv, float freq,
@@ -121,7 +147,7 @@ __device__ __forceinline__ void cells_at(const FacetDev &f, float uu, float vv, 
   float u = uu * ff, v = vv * ff;
   u = u * f.uscale;
   v = v * f.vscale;
-  iu = (int)((double)u + 0.5);
+  iu = column_of(u);
   ivrow = lround_obit(v) - f.hw + f.ny / 2;
 }
 
@@ -153,13 +179,15 @@ __device__ __forceinline__ Sample prep_cells(const FacetDev &f, const Common &cm
   s.vi = vi * vw;
   u = u * f.uscale;
   v = v * f.vscale;
-  const int iu = (int)((double)u + 0.5);
+  const int iu = column_of(u);
   const int iv = lround_obit(v);
   const float N = (float)cm.convNperCell, hN = 0.5f * N;
   const float du = (float)iu - u;
   const float dv = (float)iv - v;
-  s.itu = cm.convNperCell + lround_obit(fmaf(N, du, -hN));
-  s.itv = cm.convNperCell + lround_obit(fmaf(N, dv, -hN));
+  // lround of N d - N/2, which is not positive but for such frequencies (and
+  // never half an odd number where it is)
+  s.itu = cm.convNperCell - round_up(fmaf(-N, du, hN));
+  s.itv = cm.convNperCell - round_up(fmaf(-N, dv, hN));
   if (s.itu < 0 || s.itu > cm.convNperCell || s.itv < 0 || s.itv > cm.convNperCell) {
     // only for non-positive frequencies
     s.iu = f.hw; s.iv = f.ny / 2; s.itu = 0; s.itv = 0; s.vr = 0.0f; s.vi = 0.0f;
@@ -184,15 +212,13 @@ __device__ __forceinline__ Sample prep_cells(const FacetDev &f, const Common &cm
 // rounded to FP32 and goes through a quadrant reduction and Taylor
 // series, so the weighted value differs from the CPU's by a few FP32
 // ulps of the phase, within both evaluations' own error.
-__device__ __forceinline__ Sample prep_vals(const FacetDev &f, const Common &cm, float uu, float vv,
-                                            float ww, int ich, float fsc, float vre, float vim,
-                                            float vwt) {
+__device__ __forceinline__ Sample prep_vals(const FacetDev &f, const Common &cm, float4 q, int ich, float fsc,
+                                            float vre, float vim, float vwt) {
+  // q: signed_uvw; the sign times the frequency times u is that times u
   float u, v, w;
   {
 #pragma clang fp contract(off)
-    const float phaseSign = (uu <= 0.0f) ? -1.0f : 1.0f;
-    const float freqFact = phaseSign * fsc;
-    u = uu * freqFact; v = vv * freqFact; w = ww * freqFact;
+    u = q.x * fsc; v = q.y * fsc; w = q.z * fsc;
   }
   // fast_rot: phase shift of the facet
   float vr, vi;
@@ -202,7 +228,7 @@ __device__ __forceinline__ Sample prep_vals(const FacetDev &f, const Common &cm,
     const double t = (double)u * f.sturn[0] + (double)v * f.sturn[1] + (double)w * f.sturn[2];
     float sn, cs;
     sincos_turns_poly((float)(t - rint(t)), &sn, &cs);
-    const float vvi = (uu <= 0.0f) ? -vim : vim;
+    const float vvi = vim * q.w;
     vr = vre * cs - vvi * sn;
     vi = vre * sn + vvi * cs;
   }
@@ -212,18 +238,22 @@ __device__ __forceinline__ Sample prep_vals(const FacetDev &f, const Common &cm,
 __device__ Sample prep_sample(const FacetDev &f, const Common &cm, const float *row, float uu,
                               float vv, float ww, int ich) {
   const float *vis = row + cm.nrparm + ich * 3;
-  return prep_vals(f, cm, uu, vv, ww, ich, cm.freq[ich], vis[0], vis[1], vis[2]);
+  return prep_vals(f, cm, signed_uvw(uu, vv, ww), ich, cm.freq[ich], vis[0], vis[1], vis[2]);
 }
 
 // ---------------- binning ----------------
 
+constexpr int kParts = 8;        // counters of work items, one an XCD,
+constexpr int kNextStride = 32;  // 128 bytes apart
+
 // Everything a pass starts from zero, in one launch (a kernel, kept out of
 // memset nodes so the sequence stays capturable in a hipGraph): the walk
-// statistics, the count after the last track, the uvw checksum and the lists'
-// first and last entries.
-__global__ void k_pass_clear(unsigned long long *walk, unsigned *lastCount, unsigned long long *hash, long long *first,
-                             long long *last, long long n) {
+// statistics and the counters of work items, the count after the last track,
+// the uvw checksum and the lists' first and last entries.
+__global__ void k_pass_clear(unsigned long long *walk, unsigned *next, unsigned *lastCount, unsigned long long *hash,
+                             long long *first, long long *last, long long n) {
   const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i0 < kParts) next[kNextStride * i0] = 0;
   if (i0 == 0) {
     walk[0] = walk[1] = 0;
     *hash = 0;
@@ -351,9 +381,10 @@ __device__ __forceinline__ BinTrack bin_track(long long it, int nf, int nsplit, 
 }
 
 // Binning, pass 1: the number of (plane, tile) entries of every thread's track;
-// the first thread of a row adds it to the uvw checksum.
+// the first thread of a (row, facet) keeps its rotated uvw for the gridding, that
+// of a row adds it to the uvw checksum.
 __global__ void k_bin_count(const float *vis, long long nrow, const FacetDev *facets, int nf, int nsplit, Common cm,
-                            unsigned *cnt, unsigned long long *hash) {
+                            unsigned *cnt, float4 *rot, unsigned long long *hash) {
   const long long total = nrow * (long long)nf * nsplit;
   unsigned long long h = 0;
   for (long long it = (long long)blockIdx.x * blockDim.x + threadIdx.x; it < total;
@@ -366,6 +397,7 @@ __global__ void k_bin_count(const float *vis, long long nrow, const FacetDev *fa
     unsigned n = 0;
     track_tiles(f, cm, uu, vv, b.p0, b.p1, [&](long long, unsigned, int, int) { ++n; });
     cnt[it] = n;
+    if (b.p0 == 0) rot[b.fi * nrow + b.r] = signed_uvw(uu, vv, ww);
     if (b.fi == 0 && b.p0 == 0) h += row_hash(row, b.r);
   }
   for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
@@ -508,11 +540,12 @@ __device__ __forceinline__ float keep_lanes(float a, unsigned long long m) {
 // grid with plain stores when the item is the tile's whole list; the
 // halo, and every cell of an item of a longer list, add with device
 // atomics.
-__global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, const FacetDev *facets,
+__global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, const float4 *rot, long long nrow,
+                                                           const FacetDev *facets,
                                                            const int *listFacet, const int2 *items,
                                                            const long long *nitemsPtr, int chunk, Common cm,
                                                            const long long *offsets, const long long *lend,
-                                                           const int2 *lists,
+                                                           const int2 *lists, unsigned *next,
                                                            unsigned long long *stats) {
   __shared__ float4 s_tile4[kWaves][2 * kPlane / 4];  // re plane, then im plane
   __shared__ int2 s_si[kWaves][kHalf];      // staged sample: u and v tap-row offsets in s_gcfp
@@ -545,9 +578,20 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
   int *scell = s_cell[wv];
   int *flag = s_flag[wv];
   const long long nitems = *nitemsPtr;
+  // Each wave starts with the item of its number; the others are taken as waves
+  // get free, the next one's number fetched while an item is gridded.  Items
+  // differ in samples: dealt out in turn they left the last wave 20 % behind the
+  // mean after 88 rounds (the pass of 105,300 rows x 256 channels into 20 facets
+  // x 8 planes of 2048^2 13.35 ms, so 11.56).  One counter costs 10 ns an item
+  // whatever the waves (12.36 ms, and 30 us more on a pass of 400); so every XCD
+  // has its own, for each eighth of the items.
+  const unsigned parts = min((unsigned)kParts, gridDim.x), part = blockIdx.x % parts;
+  const long long nwaves = (long long)gridDim.x * kWaves;
+  unsigned taken = 0;
   for (long long w = (long long)blockIdx.x * kWaves + wv; w < nitems;
-       w += (long long)gridDim.x * kWaves) {
+       w = nwaves + (long long)(unsigned)__builtin_amdgcn_readfirstlane((int)taken) * parts + part) {
     const int2 item = items[w];
+    if (lane == 0) taken = atomicAdd(next + kNextStride * part, 1u);
     const long long L = __builtin_amdgcn_readfirstlane(item.x);
     const long long l0 = offsets[L];
     const int n = (int)(lend[L] - l0);
@@ -640,14 +684,15 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       const int c = (int)__popcll(starts);
       jA += c + (__builtin_amdgcn_readlane(pos, c) == 64 ? 1 : 0);
     };
-    float xu, xv, xw, xre, xim, xwt, xfs;
+    const float4 *rotf = rot + fi * nrow;
+    float4 xq;
+    float xre, xim, xwt, xfs;
     int xch;
     auto fetch = [&](int r, int ch) {
-      const float *row = vis + (long long)r * cm.lenvis;
       xch = ch;
       xfs = cm.freq[ch];
-      xu = row[0]; xv = row[1]; xw = row[2];
-      const float *x = row + cm.nrparm + 3 * ch;
+      xq = rotf[r];
+      const float *x = vis + (long long)r * cm.lenvis + cm.nrparm + 3 * ch;
       xre = x[0]; xim = x[1]; xwt = x[2];
     };
     // the row and channel of a slot are read two passes ahead and its data
@@ -664,7 +709,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
     const int npass = (nslot + 63) / 64;
     for (int pass = 0; pass < npass; ++pass) {
       const bool live = liveCur;
-      const float u0 = xu, v0 = xv, w0 = xw, re0 = xre, im0 = xim, wt0 = xwt, fs0 = xfs;
+      const float4 q0 = xq;
+      const float re0 = xre, im0 = xim, wt0 = xwt, fs0 = xfs;
       const int ch0 = xch;
       // the slot after next: its row and channel; then the next pass's data
       int rc, cic;
@@ -675,11 +721,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       bool keep = false;
       Sample sm;
       if (live) {
-        float uu, vv, ww;
-        rotate3(f, u0, v0, w0, uu, vv, ww);
-        sm = prep_vals(f, cm, uu, vv, ww, ch0, fs0, re0, im0, wt0);
-        keep = (sm.vr != 0.0f || sm.vi != 0.0f) && sm.iu >= col0 && sm.iu < col0 + TU &&
-               sm.iv >= row0 && sm.iv < row0 + TV;
+        sm = prep_vals(f, cm, q0, ch0, fs0, re0, im0, wt0);
+        keep = (sm.vr != 0.0f || sm.vi != 0.0f) && (unsigned)(sm.iu - col0) < (unsigned)TU &&
+               (unsigned)(sm.iv - row0) < (unsigned)TV;
       }
       liveCur = liveNext; liveNext = liveC; rb = rc; chb = chc;
       const unsigned long long mask = __ballot(keep);
@@ -768,8 +812,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       float *q = g + (size_t)gr * f.lrow + 2 * gc;
       // the windows of the tiles to the left and above reach kWin - kBlk
       // cells into this one
-      const bool own = !multi && rr >= kWinV - kBlkV && rr < TV && cc >= kWinU - kBlkU && cc < TU;
-      if (own) {
+      const bool inner = !multi && rr >= kWinV - kBlkV && rr < TV && cc >= kWinU - kBlkU && cc < TU;
+      if (inner) {
         q[0] += vr;
         q[1] += vi;
       } else {
@@ -1254,6 +1298,8 @@ struct GpuState {
   unsigned *d_tcnt = nullptr;      // entries per (row, facet) track
   unsigned long long *d_toff = nullptr;  // their exclusive scan
   long long tcap = 0;
+  float4 *d_rot = nullptr;         // rotated uvw [facet][row] of the last pass (signed_uvw)
+  long long rotCap = 0;
   unsigned *d_keys = nullptr, *d_keys2 = nullptr;  // sort keys, in and out
   int2 *d_rows = nullptr;          // (row, channel range) before the sort (d_lists after it)
   int2 *d_items = nullptr;
@@ -1269,6 +1315,7 @@ struct GpuState {
   long long listsRows = 0;         // ... a pass over as many rows ...
   unsigned long long *d_hash = nullptr;  // ... with the same uvw: their checksum, and another pass's
   unsigned long long *d_walk = nullptr;  // staged samples, base-cell moves of the last pass
+  unsigned *d_next = nullptr;            // its counters of work items
   // FFT to images: C2R plan for (nx, ny, nplane), complex scratch, corrections
   hipfftHandle fftPlan = 0;
   int fftNx = 0, fftNy = 0, fftNplane = 0, fftPitch = 0, fftDist = 0;
@@ -1562,7 +1609,7 @@ __global__ __launch_bounds__(256) void k_items(const long long *first, const lon
   }
 }
 
-int launch_taps(GpuState *gs, const float *vis);
+int launch_taps(GpuState *gs, const float *vis, long long nrow);
 
 // Scan / sort scratch of at least need bytes.
 hipError_t ensure_tmp(GpuState *gs, size_t need) {
@@ -1593,8 +1640,8 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   if (reuse) {
     // the rows' checksum beside the lists'; the lists, offsets and work items of
     // the last pass stand: only the walk statistics restart
-    hipLaunchKernelGGL(k_pass_clear, dim3(1), dim3(64), 0, gs->stream, gs->d_walk, (unsigned *)nullptr, gs->d_hash + 1,
-                       (long long *)nullptr, (long long *)nullptr, 0LL);
+    hipLaunchKernelGGL(k_pass_clear, dim3(1), dim3(64), 0, gs->stream, gs->d_walk, gs->d_next,
+                       (unsigned *)nullptr, gs->d_hash + 1, (long long *)nullptr, (long long *)nullptr, 0LL);
     const int nb = (int)std::min<long long>((nrow + 255) / 256, (long long)gs->nCU * 4);
     hipLaunchKernelGGL(k_uvw_hash, dim3(std::max(nb, 1)), dim3(256), 0, gs->stream, vis, nrow, gs->cm.lenvis,
                        gs->d_hash + 1);
@@ -1603,9 +1650,10 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));
     if (gs->h_tot[2] != gs->h_tot[3])
       return fail(kState, "cannot reuse the track lists: these rows' u, v, w differ from the last pass's");
-    return launch_taps(gs, vis);
+    return launch_taps(gs, vis, nrow);
   }
   if (!gs->d_walk) OBIT_HIP_TRY(hipMalloc(&gs->d_walk, 2 * sizeof(unsigned long long)));
+  if (!gs->d_next) OBIT_HIP_TRY(hipMalloc(&gs->d_next, kParts * kNextStride * sizeof(unsigned)));
   if (!gs->d_hash) OBIT_HIP_TRY(hipMalloc(&gs->d_hash, 2 * sizeof(unsigned long long)));
   if (gs->tapsPerCU <= 0) {
     int nb = 0;
@@ -1630,14 +1678,21 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     OBIT_HIP_TRY(hipMalloc(&gs->d_toff, sizeof(unsigned long long) * (size_t)(ntr + 1)));
     gs->tcap = ntr + 1;
   }
+  if (nrf > gs->rotCap) {
+    (void)hipFree(gs->d_rot);
+    gs->d_rot = nullptr;
+    gs->rotCap = 0;
+    OBIT_HIP_TRY(hipMalloc(&gs->d_rot, sizeof(float4) * (size_t)nrf));
+    gs->rotCap = nrf;
+  }
   const int nbB = (int)std::min<long long>((ntr + 255) / 256, (long long)gs->nCU * 32);
   // pass 1: entries per track; the slot after the last track is zero so
   // the scan's last element is the total
   const int nbz = (int)std::min<long long>((nl + 1 + 255) / 256, (long long)gs->nCU * 16);
-  hipLaunchKernelGGL(k_pass_clear, dim3(nbz), dim3(256), 0, gs->stream, gs->d_walk, gs->d_tcnt + ntr, gs->d_hash,
-                     gs->d_offsets, gs->d_lend, nl + 1);
+  hipLaunchKernelGGL(k_pass_clear, dim3(nbz), dim3(256), 0, gs->stream, gs->d_walk, gs->d_next, gs->d_tcnt + ntr,
+                     gs->d_hash, gs->d_offsets, gs->d_lend, nl + 1);
   hipLaunchKernelGGL(k_bin_count, dim3(nbB), dim3(256), 0, gs->stream, vis, nrow, gs->d_facets, nf, nsplit,
-                     gs->cm, gs->d_tcnt, gs->d_hash);
+                     gs->cm, gs->d_tcnt, gs->d_rot, gs->d_hash);
   OBIT_HIP_TRY(hipGetLastError());
   {
     size_t need = 0;
@@ -1728,7 +1783,7 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   } else {
     gs->h_tot[1] = 0;
   }
-  int rc = launch_taps(gs, vis);  // the pass is complete when it returns
+  int rc = launch_taps(gs, vis, nrow);  // the pass is complete when it returns
   if (rc) return rc;
   gs->nitems = gs->h_tot[1];
   if (gs->nitems < 0 || gs->nitems > gs->itemBound)
@@ -1740,15 +1795,16 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
 
 // The tile-gridding launch over the current work items; the pass is
 // complete when it returns.
-int launch_taps(GpuState *gs, const float *vis) {
+int launch_taps(GpuState *gs, const float *vis, long long nrow) {
   if (gs->itemBound) {
     // persistent grid of exactly the resident blocks: more would queue a
     // second round of blocks behind the first and idle CUs at the end
     const long long nbG =
         std::min<long long>((gs->itemBound + kWaves - 1) / kWaves, (long long)gs->nCU * gs->tapsPerCU);
     hipLaunchKernelGGL(k_grid_taps, dim3((unsigned)nbG), dim3(64 * kWaves), 0, gs->stream, vis,
-                       gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items, gs->d_itemOff + gs->nlist, gs->chunk,
-                       gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists, gs->d_walk);
+                       gs->d_rot, nrow, gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items,
+                       gs->d_itemOff + gs->nlist, gs->chunk, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
+                       gs->d_next, gs->d_walk);
     OBIT_HIP_TRY(hipGetLastError());
   }
   // the pass is complete when the call returns
@@ -1930,8 +1986,9 @@ void ObitCUDAGridShutdown(CUDAGridInfo *cudaInfo, long iGPU) {
     if (gs->h_tab) (void)hipHostFree(gs->h_tab);
     (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets); (void)hipFree(gs->d_lists);
     (void)hipFree(gs->d_tcnt); (void)hipFree(gs->d_toff); (void)hipFree(gs->d_keys); (void)hipFree(gs->d_keys2);
-    (void)hipFree(gs->d_rows);
-    (void)hipFree(gs->d_items); (void)hipFree(gs->d_vis); (void)hipFree(gs->d_walk); (void)hipFree(gs->d_hash);
+    (void)hipFree(gs->d_rows); (void)hipFree(gs->d_rot);
+    (void)hipFree(gs->d_items); (void)hipFree(gs->d_vis); (void)hipFree(gs->d_walk);
+    (void)hipFree(gs->d_hash); (void)hipFree(gs->d_next);
     (void)hipFree(gs->d_itemOff); (void)hipFree(gs->d_scanTmp);
     if (gs->h_tot) (void)hipHostFree(gs->h_tot);
     if (gs->fftPlan) (void)hipfftDestroy(gs->fftPlan);
