@@ -474,7 +474,6 @@ __global__ void k_list_bounds(const unsigned *keys, long long n, long long *firs
 constexpr int kW = 7;          // GCF support in cells (checked on the host)
 constexpr int kChunk = 128;    // most tracks of a work item (swept 64..2048 on workload 4: 128 best)
 constexpr int kMinChunk = 16;  // least (see grid_device)
-constexpr int kWaves = 4;      // waves per workgroup, each with a private tile
 // A sample's footprint is accumulated through a 16 (u) x 8 (v) window of
 // cells whose origin is its base cell rounded down to a multiple of 8 in u
 // and of 2 in v, so a window serves the 8x2 base cells of an aligned
@@ -489,7 +488,8 @@ constexpr int kTC = TU + kWinU - kBlkU;            // tile columns with the halo
 constexpr int kPlane = ((kTR * kS + 31) / 64) * 64 + 32;  // floats per re / im plane
 constexpr int kHalf = 64;      // kept samples staged at a time (one pass)
 constexpr int kGrp = kHalf / 4;  // 4-sample groups of a pass (K of one matrix step)
-constexpr int kGcfRow = 24;    // padded GCF row: 7 zeros, 7 taps, 10 zeros
+constexpr int kGcfRow = 16;    // GCF row in LDS: 7 taps and the 9 zeros after them
+constexpr int kGcfLds = 101 * kGcfRow + 7;
 static_assert(kBlkU + kW - 1 <= kWinU && kBlkV + kW - 1 <= kWinV, "the window holds every footprint");
 static_assert(TU % kBlkU == 0 && TV % kBlkV == 0, "windows are aligned within the tile");
 static_assert(kS >= kTC && (4 * kS) % 64 == 48, "tile stride: room for the halo, 4 rows = 48 banks");
@@ -540,6 +540,13 @@ __device__ __forceinline__ float keep_lanes(float a, unsigned long long m) {
 // grid with plain stores when the item is the tile's whole list; the
 // halo, and every cell of an item of a longer list, add with device
 // atomics.
+//
+// What bounds it is the issue of its 400 vector instructions a pass and 20 matrix
+// steps, which exclude each other on a SIMD where they are FP32 (34 cycles each).
+// kWaves waves, each with its own tile, share a workgroup and its table; kGather
+// groups are gathered together.  4 and 16: 3 waves a SIMD; 16 and 8: the one
+// table leaves LDS for 4, in 128 registers (launch_taps).
+template <int kWaves, int kGather>
 __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, const float4 *rot, long long nrow,
                                                            const FacetDev *facets,
                                                            const int *listFacet, const int2 *items,
@@ -548,16 +555,18 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
                                                            const int2 *lists, unsigned *next,
                                                            unsigned long long *stats) {
   __shared__ float4 s_tile4[kWaves][2 * kPlane / 4];  // re plane, then im plane
-  __shared__ int2 s_si[kWaves][kHalf];      // staged sample: u and v tap-row offsets in s_gcfp
   __shared__ float2 s_sv[kWaves][kHalf];    // staged sample: weighted visibility
-  __shared__ int s_cell[kWaves][64];
-  __shared__ int s_flag[kWaves][64];        // entry starts within a window of slots
-  // padded GCF rows: 7 zeros, the 7 taps of fractional offset it, 10 zeros,
-  // so every window column or row reads its tap (or a zero) with no test
-  __shared__ float s_gcfp[101 * kGcfRow];
-  for (int i = threadIdx.x; i < 101 * kGcfRow; i += blockDim.x) {
-    const int it = i / kGcfRow, j = i - it * kGcfRow - 7;
-    s_gcfp[i] = (j >= 0 && j < kW) ? cm.gcf[8 * it + j] : 0.0f;
+  // staged sample: u and v tap-row offsets in s_gcfp (u | v << 16); before that
+  // the kept samples' windows, and before that the entry starts of a window of
+  // slots, each read before the next is written
+  __shared__ int s_si[kWaves][kHalf];
+  // GCF rows: 7 zeros, then for each fractional offset its 7 taps and 9 zeros, so
+  // that any window column or row (up to 7 before and 15 after a row's start less
+  // 7) reads its tap or a zero with no test
+  __shared__ float s_gcfp[kGcfLds];
+  for (int i = threadIdx.x; i < kGcfLds; i += blockDim.x) {
+    const int it = (i - 7) >> 4, j = (i - 7) & 15;  // kGcfRow = 16
+    s_gcfp[i] = (i >= 7 && j < kW) ? cm.gcf[8 * it + j] : 0.0f;
   }
   __syncthreads();
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -570,13 +579,12 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
   const int mm7 = mm & 7;
   float *re = reinterpret_cast<float *>(s_tile4[wv]);
   float *im = re + kPlane;
-  int2 *si = s_si[wv];
+  int *si = s_si[wv];
   float2 *sv = s_sv[wv];
   // this lane's part of a staged visibility: sample mk of a group, real
   // part for window rows (mm < 8), imaginary for the rest
   const float *svl = reinterpret_cast<const float *>(sv) + 2 * mk + (mm >= 8 ? 1 : 0);
-  int *scell = s_cell[wv];
-  int *flag = s_flag[wv];
+  int *scell = si, *flag = si;
   const long long nitems = *nitemsPtr;
   // Each wave starts with the item of its number; the others are taken as waves
   // get free, the next one's number fetched while an item is gridded.  Items
@@ -588,7 +596,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
   const unsigned parts = min((unsigned)kParts, gridDim.x), part = blockIdx.x % parts;
   const long long nwaves = (long long)gridDim.x * kWaves;
   unsigned taken = 0;
-  for (long long w = (long long)blockIdx.x * kWaves + wv; w < nitems;
+  for (long long w = (long long)wv * gridDim.x + blockIdx.x; w < nitems;
        w = nwaves + (long long)(unsigned)__builtin_amdgcn_readfirstlane((int)taken) * parts + part) {
     const int2 item = items[w];
     if (lane == 0) taken = atomicAdd(next + kNextStride * part, 1u);
@@ -749,43 +757,47 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       // the GCF table and walk the groups.
       if (keep) {
         const int cu = sm.iu - col0, cv = sm.iv - row0;
-        si[pos] = make_int2(kGcfRow * sm.itu + 7 - (cu & (kBlkU - 1)), kGcfRow * sm.itv + 7 - (cv & (kBlkV - 1)));
+        si[pos] = (kGcfRow * sm.itu + 7 - (cu & (kBlkU - 1))) | (kGcfRow * sm.itv + 7 - (cv & (kBlkV - 1))) << 16;
         sv[pos] = make_float2(sm.vr, sm.vi);
       }
       if (lane >= nv) {
-        si[lane] = make_int2(0, 0);  // any tap row: the visibility is zero
+        si[lane] = 0;  // any tap row: the visibility is zero
         sv[lane] = make_float2(0.0f, 0.0f);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      float A[kGrp], B[kGrp];
 #pragma unroll
-      for (int g = 0; g < kGrp; ++g) {
-        const int2 q = si[4 * g + mk];
-        B[g] = gcf[q.x + mm];
-        A[g] = gcf[q.y + mm7] * svl[8 * g];
-      }
+      for (int h = 0; h < kGrp; h += kGather) {
+        if (h && 4 * h >= nv) break;
+        float A[kGather], B[kGather];
 #pragma unroll
-      for (int g = 0; g < kGrp; ++g) {
-        if (4 * g >= nv) break;
-        unsigned mg = (unsigned)(moves >> (4 * g)) & 15u;  // moves at the group's samples
-        int s0 = 0;
-        while (mg) {
-          const int p1 = __builtin_ctz(mg);
-          if (p1 > s0) {
-            // samples s0 .. p1 - 1 of the group (p1 <= 3)
-            const unsigned long long m = (~0ull << (16 * s0)) ^ (~0ull << (16 * p1));
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(keep_lanes(A[g], m), B[g], acc, 0, 0, 0);
-          }
-          handover();
-          cur = __builtin_amdgcn_readlane(cellq, 4 * g + p1);
-          acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
-          s0 = p1;
-          mg &= mg - 1;
+        for (int g = 0; g < kGather; ++g) {
+          const int q = si[4 * (h + g) + mk];
+          B[g] = gcf[(q & 0xFFFF) + mm];
+          A[g] = gcf[(q >> 16) + mm7] * svl[8 * (h + g)];
         }
-        // samples s0 .. 3 of the group
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(keep_lanes(A[g], ~0ull << (16 * s0)), B[g], acc, 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < kGather; ++g) {
+          if (4 * (h + g) >= nv) break;
+          unsigned mg = (unsigned)(moves >> (4 * (h + g))) & 15u;  // moves at the group's samples
+          int s0 = 0;
+          while (mg) {
+            const int p1 = __builtin_ctz(mg);
+            if (p1 > s0) {
+              // samples s0 .. p1 - 1 of the group (p1 <= 3)
+              const unsigned long long m = (~0ull << (16 * s0)) ^ (~0ull << (16 * p1));
+              acc = __builtin_amdgcn_mfma_f32_16x16x4f32(keep_lanes(A[g], m), B[g], acc, 0, 0, 0);
+            }
+            handover();
+            cur = __builtin_amdgcn_readlane(cellq, 4 * (h + g) + p1);
+            acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
+            s0 = p1;
+            mg &= mg - 1;
+          }
+          // samples s0 .. 3 of the group
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(keep_lanes(A[g], ~0ull << (16 * s0)), B[g], acc, 0, 0, 0);
+        }
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -1285,7 +1297,7 @@ struct GpuState {
   int device = 0;
   hipStream_t stream = nullptr;
   int nCU = 256;
-  int tapsPerCU = 0;        // resident k_grid_taps blocks per CU (0: not queried yet)
+  int tapsPerCU = 0;        // resident k_grid_taps<4, 16> blocks per CU (0: not queried yet)
   std::vector<int> facets;  // facet indices on this GPU
   FacetDev *d_facets = nullptr;  // in d_tab
   std::vector<FacetDev> h_facets;
@@ -1308,7 +1320,8 @@ struct GpuState {
   void *d_scanTmp = nullptr;       // scan scratch
   size_t scanTmpBytes = 0;
   long long *h_tot = nullptr;      // pinned: list entries and work items of the last pass
-  long long nitems = 0, itemBound = 0;  // work items of the last pass; at most this many
+  // work items of the last pass; at most this many; that many if all were full
+  long long nitems = 0, itemBound = 0, fullItems = 0;
   int chunk = kChunk;              // tracks per work item of the last pass
   bool anyBeam = false;            // a facet is gridded as a beam
   bool listsValid = false;         // the lists of the last pass, for ...
@@ -1657,7 +1670,7 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   if (!gs->d_hash) OBIT_HIP_TRY(hipMalloc(&gs->d_hash, 2 * sizeof(unsigned long long)));
   if (gs->tapsPerCU <= 0) {
     int nb = 0;
-    OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_grid_taps, 64 * kWaves, 0));
+    OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_grid_taps<4, 16>, 64 * 4, 0));
     gs->tapsPerCU = std::max(nb, 1);
   }
   gs->listsValid = false;
@@ -1746,11 +1759,12 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   // samples add equal terms, whose FP32 rounding does not average out (3e-4 of
   // the peak where a cell takes 12,000), so that its sums would move with the
   // grouping.
-  const long long waves = (long long)gs->nCU * gs->tapsPerCU * kWaves;
+  const long long waves = (long long)gs->nCU * gs->tapsPerCU * 4;
   gs->chunk = kChunk;
   if (!gs->anyBeam)
     while (gs->chunk > kMinChunk && 80 * total < waves * gs->chunk * gs->chunk) gs->chunk /= 2;
-  gs->itemBound = std::min(total, nl + total / gs->chunk + 1);
+  gs->fullItems = total / gs->chunk;
+  gs->itemBound = std::min(total, nl + gs->fullItems + 1);
   if (gs->itemBound > gs->itemCap) {
     (void)hipFree(gs->d_items);
     gs->d_items = nullptr;
@@ -1799,12 +1813,25 @@ int launch_taps(GpuState *gs, const float *vis, long long nrow) {
   if (gs->itemBound) {
     // persistent grid of exactly the resident blocks: more would queue a
     // second round of blocks behind the first and idle CUs at the end
-    const long long nbG =
-        std::min<long long>((gs->itemBound + kWaves - 1) / kWaves, (long long)gs->nCU * gs->tapsPerCU);
-    hipLaunchKernelGGL(k_grid_taps, dim3((unsigned)nbG), dim3(64 * kWaves), 0, gs->stream, vis,
-                       gs->d_rot, nrow, gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items,
-                       gs->d_itemOff + gs->nlist, gs->chunk, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
-                       gs->d_next, gs->d_walk);
+    //
+    // 16 waves a workgroup, 4 a SIMD, from 16 items a wave up (105,300 rows x 256
+    // channels into 20 facets x 8 planes of 2048^2, 66 items a wave: 11.50 -> 10.83
+    // ms).  Below, where the time is that of a wave's last items, 4 waves a
+    // workgroup with their longer gathers are as fast (60,000 x 256 into 2 facets,
+    // 4 items a wave: 1.12 ms both) or faster (60,000 x 64 into a 512^2 beam, less
+    // than one: 427 us against 457).
+    const bool wide = gs->fullItems >= 16LL * 16 * gs->nCU;
+    const long long nbG = std::min<long long>(gs->itemBound, (long long)gs->nCU * (wide ? 1 : gs->tapsPerCU));
+    if (wide)
+      hipLaunchKernelGGL((k_grid_taps<16, 8>), dim3((unsigned)nbG), dim3(64 * 16), 0, gs->stream, vis, gs->d_rot,
+                         nrow, gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items,
+                         gs->d_itemOff + gs->nlist, gs->chunk, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
+                         gs->d_next, gs->d_walk);
+    else
+      hipLaunchKernelGGL((k_grid_taps<4, 16>), dim3((unsigned)nbG), dim3(64 * 4), 0, gs->stream, vis, gs->d_rot,
+                         nrow, gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items,
+                         gs->d_itemOff + gs->nlist, gs->chunk, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
+                         gs->d_next, gs->d_walk);
     OBIT_HIP_TRY(hipGetLastError());
   }
   // the pass is complete when the call returns
