@@ -51,6 +51,8 @@ constexpr int TU = 64;        // tile width in grid columns (complex cells)
 // measured on workload 4: 50.0 ms a pass, against 58.3 at 20 rows and 58.9
 // at 12 with 8 waves, 59.9 at 6 rows)
 constexpr int TV = 8;
+constexpr int kLogTU = 6, kLogTV = 3;
+static_assert(TU == 1 << kLogTU && TV == 1 << kLogTV, "the cell of a tile is a shift");
 constexpr int kGcf = 708;     // tabulated GCF, CPU gridding order
 constexpr int kGcf8 = 101 * 8; // the same, rows padded to 8 on the device
 
@@ -245,6 +247,8 @@ __device__ Sample prep_sample(const FacetDev &f, const Common &cm, const float *
 
 constexpr int kParts = 8;        // counters of work items, one an XCD,
 constexpr int kNextStride = 32;  // 128 bytes apart
+constexpr int kHashParts = 16;   // partial sums of the uvw checksum,
+constexpr int kHashStride = 16;  // 128 bytes apart
 
 // Everything a pass starts from zero, in one launch (a kernel, kept out of
 // memset nodes so the sequence stays capturable in a hipGraph): the walk
@@ -254,9 +258,9 @@ __global__ void k_pass_clear(unsigned long long *walk, unsigned *next, unsigned 
                              long long *first, long long *last, long long n) {
   const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i0 < kParts) next[kNextStride * i0] = 0;
+  if (i0 < kHashParts) hash[kHashStride * i0] = 0;
   if (i0 == 0) {
     walk[0] = walk[1] = 0;
-    *hash = 0;
     if (lastCount) *lastCount = 0;
   }
   for (long long i = i0; i < n; i += (long long)gridDim.x * blockDim.x) { first[i] = 0; last[i] = 0; }
@@ -274,27 +278,40 @@ __device__ __forceinline__ unsigned long long row_hash(const float *row, long lo
   return x;
 }
 
-__global__ void k_uvw_hash(const float *vis, long long nrow, int lenvis, unsigned long long *out) {
+// The block's share (256 threads) into its partial sum.  A wave's atomic on one
+// sum costs 10 ns whatever the waves: 33,000 waves took 330 us.
+__device__ __forceinline__ void add_hash(unsigned long long h, unsigned long long *out) {
+  __shared__ unsigned long long s_h[4];
+  for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
+  if ((threadIdx.x & 63) == 0) s_h[threadIdx.x >> 6] = h;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    h = s_h[0] + s_h[1] + s_h[2] + s_h[3];
+    if (h) atomicAdd(out + kHashStride * (blockIdx.x % kHashParts), h);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_uvw_hash(const float *vis, long long nrow, int lenvis, unsigned long long *out) {
   unsigned long long h = 0;
   for (long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x; r < nrow;
        r += (long long)gridDim.x * blockDim.x)
     h += row_hash(vis + r * (long long)lenvis, r);
-  for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
-  if ((threadIdx.x & 63) == 0 && h) atomicAdd(out, h);
+  add_hash(h, out);
 }
 
 // Every (plane, tile of base cells) a track's samples have base cells in,
 // with the channels that do and the window block where they enter:
 // fn(L, wkey, lo, hi) for channels lo <= i < hi of the plane's channel list.
 // A track's base cells are bounded by the cells at the plane's lowest and
-// highest frequency (cells are monotonic in frequency), which gives the
-// candidate tiles.  Where the plane's frequencies are monotonic along its
+// highest frequency (cells are monotonic in frequency); a track outside the
+// grid has none.  Where the plane's frequencies are monotonic along its
 // channel list, so are the cells (the same FP32 arithmetic as prep_cells,
-// each operation monotonic), and a binary search over the list finds
-// exactly the channels whose base cell lies in the tile; a tile no channel
-// lands in is left out.  Other planes give every channel to every
-// candidate tile.  wkey is the 8x2 block of the tile holding the cell of
-// the first channel given (clamped into the tile; block row * 8 + block
+// each operation monotonic), so a track passes through its tiles one after
+// the other and a binary search over the channels that are left finds where
+// it leaves each (half the time of searching every tile of the track's
+// bounding box for its entry and exit).  Other planes give every channel to
+// every tile of the box.  wkey is the 8x2 block of the tile holding the cell
+// of the first channel given (clamped into the tile; block row * 8 + block
 // column, < 80).
 template <typename Fn>
 __device__ __forceinline__ void track_tiles(const FacetDev &f, const Common &cm, float uu, float vv,
@@ -312,56 +329,40 @@ __device__ __forceinline__ void track_tiles(const FacetDev &f, const Common &cm,
     cB = min(cB, ncol - 1); rB = min(rB, f.ny - 1);
     if (cA > cB || rA > rB) continue;
     const float *pf = cm.pfreq + (size_t)p * cm.maxpc;
-    const bool mono = cm.pmono[p] != 0;
-    // cells of the first and last channel of the list: the directions in
-    // which the cells move along it
-    int iuF, ivF, iuL, ivL;
-    cells_at(f, uu, vv, pf[0], iuF, ivF);
-    cells_at(f, uu, vv, pf[npc - 1], iuL, ivL);
-    const int tu0 = cA / TU, tu1 = cB / TU, tv0 = rA / TV, tv1 = rB / TV;
     const long long base = f.listBase + (long long)p * f.ntu * f.ntv;
-    for (int tv = tv0; tv <= tv1; ++tv)
-      for (int tu = tu0; tu <= tu1; ++tu) {
-        const int C0 = tu * TU, C1 = C0 + TU, R0 = tv * TV, R1 = R0 + TV;
-        int lo = 0, hi = npc;
-        if (mono) {
-          // first index in [a, b) where pred holds (pred false, then true)
-          auto first = [&](auto pred) {
-            int a = 0, b = npc;
-            while (a < b) {
-              const int m = (a + b) >> 1;
-              int iu, iv;
-              cells_at(f, uu, vv, pf[m], iu, iv);
-              if (pred(iu, iv)) b = m; else a = m + 1;
-            }
-            return a;
-          };
-          if (min(iuF, iuL) < C0 || max(iuF, iuL) >= C1) {
-            if (iuF <= iuL) {
-              lo = max(lo, first([&](int iu, int) { return iu >= C0; }));
-              hi = min(hi, first([&](int iu, int) { return iu >= C1; }));
-            } else {
-              lo = max(lo, first([&](int iu, int) { return iu < C1; }));
-              hi = min(hi, first([&](int iu, int) { return iu < C0; }));
-            }
+    auto emit = [&](int tu, int tv, int iue, int ive, int lo, int hi) {
+      const int cu = min(max(iue - tu * TU, 0), TU - 1);
+      const int cv = min(max(ive - tv * TV, 0), TV - 1);
+      fn(base + (long long)tv * f.ntu + tu, (unsigned)((cv >> 1) * (TU / 8) + (cu >> 3)), lo, hi);
+    };
+    if (cm.pmono[p] != 0) {
+      // along the track: the tile of channel lo holds it and the channels up to
+      // where the column or the row leaves the tile
+      int iuL, ivL;
+      cells_at(f, uu, vv, pf[npc - 1], iuL, ivL);
+      for (int lo = 0; lo < npc;) {
+        int iu, iv;
+        cells_at(f, uu, vv, pf[lo], iu, iv);
+        const int tu = iu >> kLogTU, tv = iv >> kLogTV;
+        const bool uOut = (iuL >> kLogTU) != tu, vOut = (ivL >> kLogTV) != tv;
+        int a = lo + 1, e = npc;  // channels before a are in the tile, those from e on are not
+        if (uOut || vOut) {
+          while (a < e) {
+            const int m = (a + e) >> 1;
+            int ium, ivm;
+            cells_at(f, uu, vv, pf[m], ium, ivm);
+            if ((ium >> kLogTU) != tu || (ivm >> kLogTV) != tv) e = m; else a = m + 1;
           }
-          if (min(ivF, ivL) < R0 || max(ivF, ivL) >= R1) {
-            if (ivF <= ivL) {
-              lo = max(lo, first([&](int, int iv) { return iv >= R0; }));
-              hi = min(hi, first([&](int, int iv) { return iv >= R1; }));
-            } else {
-              lo = max(lo, first([&](int, int iv) { return iv < R1; }));
-              hi = min(hi, first([&](int, int iv) { return iv < R0; }));
-            }
-          }
-          if (lo >= hi) continue;
         }
-        int iue, ive;
-        cells_at(f, uu, vv, pf[lo], iue, ive);
-        const int cu = min(max(iue - C0, 0), TU - 1);
-        const int cv = min(max(ive - R0, 0), TV - 1);
-        fn(base + (long long)tv * f.ntu + tu, (unsigned)((cv >> 1) * (TU / 8) + (cu >> 3)), lo, hi);
+        if (tu >= 0 && tu <= (ncol - 1) / TU && tv >= 0 && tv <= (f.ny - 1) / TV) emit(tu, tv, iu, iv, lo, e);
+        lo = e;
       }
+    } else {
+      int iuF, ivF;
+      cells_at(f, uu, vv, pf[0], iuF, ivF);
+      for (int tv = rA / TV; tv <= rB / TV; ++tv)
+        for (int tu = cA / TU; tu <= cB / TU; ++tu) emit(tu, tv, iuF, ivF, 0, npc);
+    }
   }
 }
 
@@ -383,7 +384,7 @@ __device__ __forceinline__ BinTrack bin_track(long long it, int nf, int nsplit, 
 // Binning, pass 1: the number of (plane, tile) entries of every thread's track;
 // the first thread of a (row, facet) keeps its rotated uvw for the gridding, that
 // of a row adds it to the uvw checksum.
-__global__ void k_bin_count(const float *vis, long long nrow, const FacetDev *facets, int nf, int nsplit, Common cm,
+__global__ __launch_bounds__(256) void k_bin_count(const float *vis, long long nrow, const FacetDev *facets, int nf, int nsplit, Common cm,
                             unsigned *cnt, float4 *rot, unsigned long long *hash) {
   const long long total = nrow * (long long)nf * nsplit;
   unsigned long long h = 0;
@@ -400,8 +401,7 @@ __global__ void k_bin_count(const float *vis, long long nrow, const FacetDev *fa
     if (b.p0 == 0) rot[b.fi * nrow + b.r] = signed_uvw(uu, vv, ww);
     if (b.fi == 0 && b.p0 == 0) h += row_hash(row, b.r);
   }
-  for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
-  if ((threadIdx.x & 63) == 0 && h) atomicAdd(hash, h);
+  add_hash(h, hash);
 }
 
 // Binning, pass 2: every entry as a sort key (list << 7 | window block)
@@ -1319,7 +1319,7 @@ struct GpuState {
   long long *d_itemOff = nullptr;  // first work item of every list (exclusive scan of chunk counts)
   void *d_scanTmp = nullptr;       // scan scratch
   size_t scanTmpBytes = 0;
-  long long *h_tot = nullptr;      // pinned: list entries and work items of the last pass
+  long long *h_tot = nullptr;      // pinned: list entries and work items of the last pass, checksums to compare
   // work items of the last pass; at most this many; that many if all were full
   long long nitems = 0, itemBound = 0, fullItems = 0;
   int chunk = kChunk;              // tracks per work item of the last pass
@@ -1596,7 +1596,7 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
                        gs->d_listFacet);
     OBIT_HIP_TRY(hipGetLastError());
   }
-  if (!gs->h_tot) OBIT_HIP_TRY(hipHostMalloc(&gs->h_tot, 4 * sizeof(long long), hipHostMallocDefault));
+  if (!gs->h_tot) OBIT_HIP_TRY(hipHostMalloc(&gs->h_tot, (2 + 2 * kHashParts * kHashStride) * sizeof(long long), hipHostMallocDefault));
   gs->ready = true;
   return kOK;
 }
@@ -1654,20 +1654,27 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     // the rows' checksum beside the lists'; the lists, offsets and work items of
     // the last pass stand: only the walk statistics restart
     hipLaunchKernelGGL(k_pass_clear, dim3(1), dim3(64), 0, gs->stream, gs->d_walk, gs->d_next,
-                       (unsigned *)nullptr, gs->d_hash + 1, (long long *)nullptr, (long long *)nullptr, 0LL);
+                       (unsigned *)nullptr, gs->d_hash + kHashParts * kHashStride, (long long *)nullptr, (long long *)nullptr, 0LL);
     const int nb = (int)std::min<long long>((nrow + 255) / 256, (long long)gs->nCU * 4);
     hipLaunchKernelGGL(k_uvw_hash, dim3(std::max(nb, 1)), dim3(256), 0, gs->stream, vis, nrow, gs->cm.lenvis,
-                       gs->d_hash + 1);
+                       gs->d_hash + kHashParts * kHashStride);
     OBIT_HIP_TRY(hipGetLastError());
-    OBIT_HIP_TRY(hipMemcpyAsync(gs->h_tot + 2, gs->d_hash, 2 * sizeof(long long), hipMemcpyDeviceToHost, gs->stream));
+    constexpr int kSums = kHashParts * kHashStride;
+    OBIT_HIP_TRY(hipMemcpyAsync(gs->h_tot + 2, gs->d_hash, 2 * kSums * sizeof(long long), hipMemcpyDeviceToHost,
+                                gs->stream));
     OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));
-    if (gs->h_tot[2] != gs->h_tot[3])
+    unsigned long long lists = 0, rows = 0;
+    for (int i = 0; i < kSums; i += kHashStride) {
+      lists += (unsigned long long)gs->h_tot[2 + i];
+      rows += (unsigned long long)gs->h_tot[2 + kSums + i];
+    }
+    if (lists != rows)
       return fail(kState, "cannot reuse the track lists: these rows' u, v, w differ from the last pass's");
     return launch_taps(gs, vis, nrow);
   }
   if (!gs->d_walk) OBIT_HIP_TRY(hipMalloc(&gs->d_walk, 2 * sizeof(unsigned long long)));
   if (!gs->d_next) OBIT_HIP_TRY(hipMalloc(&gs->d_next, kParts * kNextStride * sizeof(unsigned)));
-  if (!gs->d_hash) OBIT_HIP_TRY(hipMalloc(&gs->d_hash, 2 * sizeof(unsigned long long)));
+  if (!gs->d_hash) OBIT_HIP_TRY(hipMalloc(&gs->d_hash, 2 * kHashParts * kHashStride * sizeof(unsigned long long)));
   if (gs->tapsPerCU <= 0) {
     int nb = 0;
     OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_grid_taps<4, 16>, 64 * 4, 0));
