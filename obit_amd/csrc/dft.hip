@@ -1893,6 +1893,7 @@ struct BufPlan {
   // sums added by k_dft_combine
   bool mixed = false;
   int nsplitG = 0, kpartG = 1;
+  bool share = false;       // k_dft_share at cpt channels a thread, in one part
   bool serial = false;      // each segment's kernel waits for the one before
   std::vector<int> segBlk;  // row blocks of each segment
 };
@@ -2002,6 +2003,19 @@ BufPlan plan_buffer(State *st, const Desc &d, size_t rowBytes) {
       p.kpart = kpt;
       break;
     }
+  }
+  // A buffer of less than one round of resident workgroups takes as long as one
+  // item.  k_dft_share's items are a quarter of the rows and components (costs a
+  // component as in launch_resident); taken where its rounds of them take less
+  // than half of that, so that the parts of a longer list, whose uploads overlap,
+  // stay: 351 rows x 64 channels x 100 components 88 us on k_dft_split.
+  const int cs = p.cpt;
+  const long long shareItems = (d.nrow + kShareRows - 1) / kShareRows * perBlock;
+  const double tShare = (cs == 16 ? 0.55 : 1.0) * 0.27 * (double)((shareItems + slots - 1) / slots);
+  if (d.ncomp > 0 && items * p.nsplit <= slots && tShare < 0.5 * (cs == 16 ? 0.55 : 1.0) / p.nsplit) {
+    p.share = true;
+    p.nsplit = 1;
+    p.kpart = d.ncomp;
   }
   const int round = (int)std::max<long long>(1, slots / (perBlock * p.nsplit));  // row blocks per round
   const int mid = std::max(2 * round, (d.nrowblk + 15) / 16);                     // at most ~17 segments
@@ -2354,6 +2368,8 @@ void ObitCUDASkyModelDFTCalc(GPUInfo *gpuInfo) {
       dg.nitems = (long long)dg.nrowblk * dg.nIFsel * dg.nchunk * plan.nsplitG;
       if (!rc) rc = launch_split(st, dg, 32, plan.tile, 0, s);
       ds.nsplit = ntot;
+    } else if (plan.share) {
+      rc = launch_share(st, ds, cpt, s);
     } else {
       rc = launch_split(st, ds, cpt, plan.tile, 0, s);
     }

@@ -66,3 +66,28 @@ def test_shared_rows(oracle, kind, nif, nchan, rows, ncomp):
     assert np.abs(got - ref).max() <= TOL * peak + 4e-7 * np.abs(d0[..., :2]).max()
     div = run("div", "resident")[:, 5:].reshape(d0.shape)
     assert np.abs(div[..., 2] - d0[..., 2] * np.abs(ref)[..., None]).max() <= 2 * TOL * peak
+
+
+@pytest.mark.parametrize("kind,nif,nchan,rows,ncomp", [
+    ("point", 1, 64, 1, 1), ("point", 1, 64, 351, 100), ("point", 1, 37, 65, 255), ("point", 2, 16, 700, 257),
+    ("gauss0", 1, 64, 351, 100), ("gauss", 2, 33, 64, 63), ("gaussspec", 1, 48, 129, 5),
+])
+def test_shared_rows_buffer(oracle, kind, nif, nchan, rows, ncomp):
+    """Host buffers of less than a round of workgroups, every operation."""
+    from obit_amd.skymodel import SkyModelDFT
+    uv, sky = _case("gauss0" if kind == "point" else kind, nif, nchan, rows, ncomp)
+    if kind == "point":
+        sky = synth.SkyModel(comps=np.ascontiguousarray(sky.comps[:, :4]), modType=0)
+    ref = oracle.dft_model_fp64(uv, sky, nthreads=8)
+    peak = np.abs(ref).max()
+    d0 = uv.data_view()
+    out = {}
+    for op in ("repl", "sub"):
+        with SkyModelDFT(uv, sky, op=op) as sm:
+            out[op] = sm.calc(uv.buffer.copy())[:, 5:].reshape(d0.shape)
+    for st in range(2):
+        got = out["repl"][..., st, 0] + 1j * out["repl"][..., st, 1]
+        assert np.abs(got - ref).max() <= TOL * peak
+        left = d0[..., st, 0] + 1j * d0[..., st, 1] - (out["sub"][..., st, 0] + 1j * out["sub"][..., st, 1])
+        assert np.abs(left - ref).max() <= TOL * peak + 4e-7 * np.abs(d0[..., :2]).max()
+    assert np.array_equal(out["sub"][..., 2], d0[..., 2])
