@@ -1035,28 +1035,42 @@ __device__ __forceinline__ void stockham_pass(float2 *lds, int Ns, const float2 
 // through LDS; the columns are written back in place.  tw[m] = exp(+2 pi
 // i m / N), formed in FP64 on the host.
 //
-// The same transform, 8 columns at a time by persistent blocks of 512
+// The same transform, 8 columns at a time by persistent blocks of NT
 // threads, so each row's 64-byte segment is read and written whole by one
-// wave: wave w, lane L takes rows q + 256 r (q = 32 w + L mod 32) and,
-// with h = L / 32, columns 2h, 2h+1 (bytes 16h..16h+15 of the segment) and
-// 4+2h, 5+2h, so each 16-byte access instruction covers 32 contiguous
-// bytes of 32 rows.  The work is the (plane, 8-column block) list of
-// columns c0 .. c0 + 8 nfull - 1 (c0 even) of nplane planes: the blocks of
-// XCD x (blockIdx mod 8; gridDim.x a multiple of 8) take its x-th eighth,
-// so an XCD works through neighbouring column blocks.  A block loads its
-// next column block into registers as soon as the current one's first
-// pass is in LDS, so the loads run under the LDS passes and the write-back.  The half twiddle table is copied to LDS, so the passes make
-// no global loads that would wait behind those.  Then the blocks take the
-// column side of every plane, one plane at a time.
-template <int N, int R1, int R2, int R3>
-__global__ __launch_bounds__(512) void k_fft_cols8(float2 *grid, int pitchC, long long planeC, int c0, int nplane,
+// wave.  With kC columns a thread and kG = 8 kC, wave w, lane L takes rows
+// q + 256 r (q = kG w + L mod kG) and, with h = L / kG, columns 2h, 2h+1
+// (bytes 16h..16h+15 of the segment) and, at kC = 4, 4+2h, 5+2h: each
+// 16-byte access instruction covers 1024 / kG contiguous bytes of kG rows.
+// The work is the (plane, 8-column block) list of columns c0 .. c0 + 8 nfull
+// - 1 (c0 even) of nplane planes: the blocks of XCD x (blockIdx mod 8;
+// gridDim.x a multiple of 8) take its x-th eighth, so an XCD works through
+// neighbouring column blocks.  A block loads its next column block into
+// registers as soon as the current one's first pass is in LDS, so the loads
+// run under the LDS passes and the write-back.  The half twiddle table is
+// copied to LDS, so the passes make no global loads that would wait behind
+// those.  Then the blocks take the column side of every plane, one plane at
+// a time.
+//
+// A column block of zeros is its own transform: it is read and left (the
+// guard band keeps a fifth of the columns empty, and the data's longest
+// baseline often more).  At 2048, 16 waves of 2 columns a thread instead of 8
+// of 4, which leaves more of them to run while others wait at a barrier.  8
+// planes of 2048^2 with 65-70 % of the columns used: 110 us, 96 without the
+// empty blocks' passes and 92 with 16 waves, 2.4 TB/s; with 4 columns a block
+// (32-byte segments, two blocks a CU) 104.
+template <int N, int R1, int R2, int R3, int NT>
+__global__ __launch_bounds__(NT) void k_fft_cols8(float2 *grid, int pitchC, long long planeC, int c0, int nplane,
                                                    int nfull, int side, const float2 *__restrict__ tw) {
-  constexpr int CB = 8, NT = 512;
+  constexpr int CB = 8;
+  constexpr int kC = CB * 256 / NT, kG = 64 * kC / CB;  // columns of a thread, rows of a wave
   static_assert(R1 * R2 * R3 == N && N / R1 == 256, "radices: the first pass has one item a thread");
   __shared__ float2 lds[CB * kColStride<N>];
   __shared__ float2 twl[N / 2];
+  __shared__ int s_any[3];  // whether the column block of an iteration (mod 3) has a value that is not zero
   const int t = threadIdx.x;
   for (int i = t; i < N / 2; i += NT) twl[i] = tw[i];
+  if (t < 3) s_any[t] = 0;
+  __syncthreads();
   const int total = nplane * nfull, span = (total + 7) / 8, nper = (int)(gridDim.x >> 3);
   const int x = (int)(blockIdx.x & 7);
   const int eEnd = min(total, (x + 1) * span);
@@ -1064,38 +1078,55 @@ __global__ __launch_bounds__(512) void k_fft_cols8(float2 *grid, int pitchC, lon
     const int p = e / nfull, blk = e - p * nfull;
     return grid + (long long)p * planeC + c0 + (long long)blk * CB;
   };
-  float2 v[4][R1];
+  float2 v[kC][R1];
   // rows r0 <= r < r1 of column block e into v, for thread tl
   auto load = [&](int e, int r0, int r1, int tl) {
     const float2 *g = base(e);
-    const int h = (tl >> 5) & 1, q = (tl >> 6) * 32 + (tl & 31);
+    const int h = (tl & 63) / kG, q = (tl >> 6) * kG + (tl & (kG - 1));
 #pragma unroll
     for (int r = r0; r < r1; ++r) {
-      const float2 *row = g + (long long)(q + 256 * r) * pitchC;
-      const float4 a = *reinterpret_cast<const float4 *>(row + 2 * h);
-      const float4 b = *reinterpret_cast<const float4 *>(row + 4 + 2 * h);
-      v[0][r] = make_float2(a.x, a.y);
-      v[1][r] = make_float2(a.z, a.w);
-      v[2][r] = make_float2(b.x, b.y);
-      v[3][r] = make_float2(b.z, b.w);
+      const float2 *row = g + (long long)(q + 256 * r) * pitchC + 2 * h;
+#pragma unroll
+      for (int c = 0; c < kC; c += 2) {
+        const float4 a = *reinterpret_cast<const float4 *>(row + c * (CB / kC));
+        v[c][r] = make_float2(a.x, a.y);
+        v[c + 1][r] = make_float2(a.z, a.w);
+      }
     }
   };
   int e = x * span + (int)(blockIdx.x >> 3);
   if (e < eEnd) load(e, 0, R1, t);
-  for (; e < eEnd; e += nper) {
+  int slot = 0;
+  for (; e < eEnd; e += nper, slot = slot == 2 ? 0 : slot + 1) {
     // the thread index through an empty asm, so the compiler forms the
     // addresses and twiddle indices in each iteration instead of keeping
     // them all in registers across the loop
     int tl = t;
     asm volatile("" : "+v"(tl));
-    const int h = (tl >> 5) & 1, q = (tl >> 6) * 32 + (tl & 31);
-    const int cid[4] = {2 * h, 2 * h + 1, 4 + 2 * h, 5 + 2 * h};
+    const int h = (tl & 63) / kG, q = (tl >> 6) * kG + (tl & (kG - 1));
+    int cid[kC];
+#pragma unroll
+    for (int c = 0; c < kC; ++c) cid[c] = 2 * h + (c >> 1) * (2 * CB / kC) + (c & 1);
+    unsigned bits = 0;
+#pragma unroll
+    for (int c = 0; c < kC; ++c)
+#pragma unroll
+      for (int r = 0; r < R1; ++r) bits |= __float_as_uint(v[c][r].x) | __float_as_uint(v[c][r].y);
+    if ((bits << 1) != 0) s_any[slot] = 1;
+    __syncthreads();  // and the last column block's write-back has read the LDS
+    const bool any = __builtin_amdgcn_readfirstlane(s_any[slot]) != 0;
+    // the slot of the iteration before (read by all before this barrier) for
+    // the one after the next (written after the next barrier)
+    if (t == 0) s_any[slot == 0 ? 2 : slot - 1] = 0;
+    if (!any) {
+      if (e + nper < eEnd) load(e + nper, 0, R1, tl);
+      continue;
+    }
     // the first pass (transforms of length 1 so far: no twiddles)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) dft_small<R1>(v[c]);
-    __syncthreads();  // the last column block's write-back has read the LDS
+    for (int c = 0; c < kC; ++c) dft_small<R1>(v[c]);
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < kC; ++c)
 #pragma unroll
       for (int r = 0; r < R1; ++r) lds[cid[c] * kColStride<N> + lidx(q * R1 + r)] = v[c][r];
     // the next column block's rows, in flight under the passes
@@ -1109,10 +1140,11 @@ __global__ __launch_bounds__(512) void k_fft_cols8(float2 *grid, int pitchC, lon
       const int row = q + 256 * i;
       float2 *dst = g + (long long)row * pitchC;
       const int l = lidx(row);
-      const float2 x0 = lds[cid[0] * kColStride<N> + l], x1 = lds[cid[1] * kColStride<N> + l];
-      const float2 x2 = lds[cid[2] * kColStride<N> + l], x3 = lds[cid[3] * kColStride<N> + l];
-      *reinterpret_cast<float4 *>(dst + 2 * h) = make_float4(x0.x, x0.y, x1.x, x1.y);
-      *reinterpret_cast<float4 *>(dst + 4 + 2 * h) = make_float4(x2.x, x2.y, x3.x, x3.y);
+#pragma unroll
+      for (int c = 0; c < kC; c += 2) {
+        const float2 x0 = lds[cid[c] * kColStride<N> + l], x1 = lds[cid[c + 1] * kColStride<N> + l];
+        *reinterpret_cast<float4 *>(dst + cid[c]) = make_float4(x0.x, x0.y, x1.x, x1.y);
+      }
     }
   }
   // column side of plane sp: threads t < 256 hold rows t + 256 r
@@ -2207,9 +2239,9 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
     const int nfull = nx / 16;
     if (gs->colsPerCU <= 0) {
       int nb = 0;
-      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_cols8<2048, 8, 16, 16>, 512, 0));
+      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_cols8<2048, 8, 16, 16, 1024>, 1024, 0));
       gs->colsPerCU = std::max(nb, 1);
-      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_cols8<1024, 4, 16, 16>, 512, 0));
+      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_cols8<1024, 4, 16, 16, 512>, 512, 0));
       gs->colsPerCU1024 = std::max(nb, 1);
     }
     const long long resident = (long long)gs->nCU * (nx == 2048 ? gs->colsPerCU : gs->colsPerCU1024);
@@ -2219,10 +2251,10 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
     // with 2 rows, 8.4 with 4 and 9.35 with 8), 4 at 1024
     const dim3 grow((unsigned)(ny / 4), (unsigned)nplane), grow2048((unsigned)ny, (unsigned)nplane);
     if (nx == 2048)
-      hipLaunchKernelGGL((obit::grid::k_fft_cols8<2048, 8, 16, 16>), gcol, dim3(512), 0, gs->stream, g2, pitchC,
+      hipLaunchKernelGGL((obit::grid::k_fft_cols8<2048, 8, 16, 16, 1024>), gcol, dim3(1024), 0, gs->stream, g2, pitchC,
                          planeC, c0, nplane, nfull, side, twN);
     else
-      hipLaunchKernelGGL((obit::grid::k_fft_cols8<1024, 4, 16, 16>), gcol, dim3(512), 0, gs->stream, g2, pitchC,
+      hipLaunchKernelGGL((obit::grid::k_fft_cols8<1024, 4, 16, 16, 512>), gcol, dim3(512), 0, gs->stream, g2, pitchC,
                          planeC, c0, nplane, nfull, side, twN);
     OBIT_HIP_TRY(hipGetLastError());
     if (isBeam) {

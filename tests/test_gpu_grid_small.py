@@ -66,3 +66,35 @@ def test_channel_orders(oracle, order, nx):
         assert peak > 0
         # FP32 sums of up to some 10^3 samples a cell (a lost one is 1e-3 of the peak)
         assert np.abs(got[p] - ref).max() < 4e-6 * peak
+
+
+@pytest.mark.parametrize("nx", [1024, 2048])
+@pytest.mark.parametrize("scale", [0.0, 1e-3, 1.0])
+def test_image_of_few_columns(oracle, nx, scale):
+    """Transforms of planes whose column blocks are almost all empty (one row at
+    the origin or near it, or three somewhere), and of a plane without channels."""
+    import ctypes as C
+    from obit_amd import _lib
+    from obit_amd.gridder import GPUGrid
+    uv, _, _ = synth.workload(4, rows=3 if scale == 1.0 else 1)
+    uv.buffer[:, :3] *= np.float32(scale)
+    f = synth.make_facets(1, nx, 0.4 / 3600.0, 0.0)
+    cf = oracle.convfunc()[0]
+    corr = np.zeros(nx, np.float32)
+    _lib.load().ObitHostGridCorrFn(nx, nx // 2 + 1, cf.ctypes.data_as(C.POINTER(C.c_float)), 7, 100,
+                                   corr.ctypes.data_as(C.POINTER(C.c_float)))
+    poc = np.zeros(256, np.int32)
+    poc[1::2] = 2  # the even channels in plane 0, none in 1, the odd ones in 2
+    norm = np.ones(3, np.float32)
+    with GPUGrid(uv, f, nplane=3, plane_of_chan=poc) as gg:
+        gg.grid(uv.buffer)
+        gg.flip()
+        planes = gg.to_host(0)
+        img, _ = gg.fft_image(0, False, norm)
+    assert np.abs(planes[0]).max() > 0 and not planes[1].any() and not img[1].any()
+    ref, _ = oracle.fft2image(planes, cf, False, norm, corr=(corr, corr))
+    taper = (corr[:, None] * corr[None, :]).astype(np.float64)
+    for p in (0, 2):
+        peak = np.abs(ref[p] / taper).max()
+        # FP32 transform of 2^22 points: 22 butterflies of 6e-8, on the uncorrected scale
+        assert np.abs((img[p] - ref[p]) / taper).max() < 1e-6 * peak
