@@ -556,7 +556,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
                                                            unsigned long long *stats) {
   __shared__ float4 s_tile4[kWaves][2 * kPlane / 4];  // re plane, then im plane
   __shared__ float2 s_sv[kWaves][kHalf];    // staged sample: weighted visibility
-  // staged sample: u and v tap-row offsets in s_gcfp (u | v << 16); before that
+  // staged sample: u and v tap-row byte offsets in s_gcfp (u | v << 16); before that
   // the kept samples' windows, and before that the entry starts of a window of
   // slots, each read before the next is written
   __shared__ int s_si[kWaves][kHalf];
@@ -575,8 +575,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
   typedef float f4 __attribute__((ext_vector_type(4)));
   const int mk = lane >> 4, mm = lane & 15;
   const int laneOff = (mk >> 1) * kPlane + 4 * (mk & 1) * kS + mm;
-  const float *gcf = s_gcfp;
-  const int mm7 = mm & 7;
+  // byte offsets of this lane's column and row in the taps, one in each half
+  const char *gcf = reinterpret_cast<const char *>(s_gcfp);
+  const unsigned lanePos = 4 * mm | (4 * (mm & 7)) << 16;
   float *re = reinterpret_cast<float *>(s_tile4[wv]);
   float *im = re + kPlane;
   int *si = s_si[wv];
@@ -681,15 +682,29 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const unsigned long long starts = __ballot(flag[lane] != 0);
-      const int k = min(jA + (int)__popcll(starts & (~0ull >> (63 - lane))), ne - 1);
-      const int ra = __shfl(rowA, k & 63), rb2 = __shfl(rowB, k & 63);
-      const int ba = __shfl(baseA, k & 63), bb = __shfl(baseB, k & 63);
-      row = k < 64 ? ra : rb2;
-      ci = min((k < 64 ? ba : bb) + S + lane, npc - 1);
+      const int mine = flag[lane];
+      const unsigned long long starts = __ballot(mine != 0);
+      const int c = (int)__popcll(starts);
+      // the starts at or before this lane's slot
+      const int k = min((int)__builtin_amdgcn_mbcnt_hi((unsigned)(starts >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((unsigned)starts, jA)) + mine,
+                        ne - 1);
+      int bs;
+      if (jA + c < 64) {  // every entry of the window in the lanes' first ones
+        row = __shfl(rowA, k);
+        bs = __shfl(baseA, k);
+      } else if (jA >= 64) {
+        row = __shfl(rowB, k & 63);
+        bs = __shfl(baseB, k & 63);
+      } else {
+        const int ra = __shfl(rowA, k & 63), rb2 = __shfl(rowB, k & 63);
+        const int ba = __shfl(baseA, k & 63), bb = __shfl(baseB, k & 63);
+        row = k < 64 ? ra : rb2;
+        bs = k < 64 ? ba : bb;
+      }
+      ci = min(bs + S + lane, npc - 1);
       live = S + lane < nslot;
       // the entry holding slot S + 64: one more if an entry starts there
-      const int c = (int)__popcll(starts);
       jA += c + (__builtin_amdgcn_readlane(pos, c) == 64 ? 1 : 0);
     };
     const float4 *rotf = rot + fi * nrow;
@@ -757,7 +772,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       // the GCF table and walk the groups.
       if (keep) {
         const int cu = sm.iu - col0, cv = sm.iv - row0;
-        si[pos] = (kGcfRow * sm.itu + 7 - (cu & (kBlkU - 1))) | (kGcfRow * sm.itv + 7 - (cv & (kBlkV - 1))) << 16;
+        si[pos] = 4 * (kGcfRow * sm.itu + 7 - (cu & (kBlkU - 1))) |
+                  (4 * (kGcfRow * sm.itv + 7 - (cv & (kBlkV - 1)))) << 16;
         sv[pos] = make_float2(sm.vr, sm.vi);
       }
       if (lane >= nv) {
@@ -773,9 +789,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
         float A[kGather], B[kGather];
 #pragma unroll
         for (int g = 0; g < kGather; ++g) {
-          const int q = si[4 * (h + g) + mk];
-          B[g] = gcf[(q & 0xFFFF) + mm];
-          A[g] = gcf[(q >> 16) + mm7] * svl[8 * (h + g)];
+          const unsigned q = (unsigned)si[4 * (h + g) + mk] + lanePos;
+          B[g] = *reinterpret_cast<const float *>(gcf + (q & 0xFFFFu));
+          A[g] = *reinterpret_cast<const float *>(gcf + (q >> 16)) * svl[8 * (h + g)];
         }
 #pragma unroll
         for (int g = 0; g < kGather; ++g) {
