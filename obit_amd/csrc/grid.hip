@@ -913,6 +913,17 @@ __global__ void k_trim_centre(const FacetDev *facets, int fi, int nplane, float 
   }
 }
 
+// The planes' reciprocal norms: in the kernel's arguments for up to 32 planes
+// of an image, whose norms the caller hands in (their copy to the device and the
+// wait for its staging took 10 us of a 190 us transform of 8 planes of 2048^2),
+// else on the device, where a beam's are formed.
+constexpr int kArgNorms = 32;
+struct InvNorm {
+  const float *dev;  // NULL: v
+  float v[kArgNorms];
+};
+__device__ __forceinline__ float inv_norm(const InvNorm &n, int p) { return n.dev ? n.dev[p] : n.v[p]; }
+
 // ObitFArray2DCenter's quadrant swap and ObitFArrayMulColRow's correction
 // (src/ObitFArray.c:3116-3123) of a C2R of the planes as they lie in the
 // gridder (v halves not swapped): a cyclic shift of the v axis by ny/2 before the transform
@@ -921,7 +932,7 @@ __global__ void k_trim_centre(const FacetDev *facets, int fi, int nplane, float 
 // times xCorr[y]/norm and yCorr[x].  One thread per 4 pixels of a row
 // (nx a multiple of 8, so the 4 source pixels are contiguous).
 __global__ void k_center_correct4(const float *fft, int nx, int ny, const float *xc, const float *yc,
-                                  const float *invNorm, float *img) {
+                                  InvNorm invNorm, float *img) {
   const int x0 = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
   const int y = blockIdx.y, p = blockIdx.z;
   if (x0 >= nx) return;
@@ -931,7 +942,7 @@ __global__ void k_center_correct4(const float *fft, int nx, int ny, const float 
   if (xs >= nx) xs -= nx;
   const float4 v = *reinterpret_cast<const float4 *>(fft + ((size_t)p * ny + ys) * nx + xs);
   const float4 c = *reinterpret_cast<const float4 *>(yc + x0);
-  const float r = ((ys & 1) ? -xc[y] : xc[y]) * invNorm[p];
+  const float r = ((ys & 1) ? -xc[y] : xc[y]) * inv_norm(invNorm, p);
   *reinterpret_cast<float4 *>(img + ((size_t)p * ny + y) * nx + x0) =
       make_float4(v.x * r * c.x, v.y * r * c.y, v.z * r * c.z, v.w * r * c.w);
 }
@@ -1199,7 +1210,7 @@ template <int N, int R1, int R2, int R3, int RW = 4, int NT = 256>
 __global__ __launch_bounds__(NT) void k_fft_rows_c2r(const float2 *grid, int pitchC, long long planeC, int hw,
                                                       int ny, const float2 *__restrict__ twN,
                                                       const float2 *__restrict__ twM, const float *xc,
-                                                      const float *yc, const float *invNorm, float *img) {
+                                                      const float *yc, InvNorm invNorm, float *img) {
   constexpr int M = N / 2;
   static_assert(R1 * R2 * R3 == M, "radices");
   __shared__ float2 lds[RW * kColStride<M>];
@@ -1264,7 +1275,7 @@ __global__ __launch_bounds__(NT) void k_fft_rows_c2r(const float2 *grid, int pit
   stockham_pass<M, R2, RW, NT>(lds, R1, twM);
   stockham_pass<M, R3, RW, NT>(lds, R1 * R2, twM);
   // centre, correct, store: thread takes output column pairs
-  const float inv = invNorm[p];
+  const float inv = inv_norm(invNorm, p);
 #pragma unroll
   for (int i = 0; i < RW * M / NT; ++i) {
     const int q = t + NT * i;
@@ -2208,11 +2219,18 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
   if (!gs->h_norm) OBIT_HIP_TRY(hipHostMalloc(&gs->h_norm, sizeof(float) * 2 * 1024, hipHostMallocCoherent));
   float *d_norm = gs->d_corr + nx + ny, *d_inv = d_norm + 1024;
   const float *xc = gs->d_corr, *yc = gs->d_corr + nx;
+  obit::grid::InvNorm inv{d_inv, {}};
   if (!isBeam) {
     // an image takes its beam's norms
-    OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));  // the pinned staging is free
-    for (int p = 0; p < nplane; ++p) gs->h_norm[p] = (float)(1.0 / std::max(1.0e-20, (double)beamNorm[p]));
-    OBIT_HIP_TRY(hipMemcpyAsync(d_inv, gs->h_norm, sizeof(float) * nplane, hipMemcpyHostToDevice, gs->stream));
+    auto recip = [&](int p) { return (float)(1.0 / std::max(1.0e-20, (double)beamNorm[p])); };
+    if (nplane <= obit::grid::kArgNorms) {
+      inv.dev = nullptr;
+      for (int p = 0; p < nplane; ++p) inv.v[p] = recip(p);
+    } else {
+      OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));  // the pinned staging is free
+      for (int p = 0; p < nplane; ++p) gs->h_norm[p] = recip(p);
+      OBIT_HIP_TRY(hipMemcpyAsync(d_inv, gs->h_norm, sizeof(float) * nplane, hipMemcpyHostToDevice, gs->stream));
+    }
   }
   // FFTW's unnormalised backward transform of the gridder's padded half
   // planes (row pitch lrow/2 complex, the u = 0 column hw complex into each
@@ -2280,12 +2298,10 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
     }
     if (nx == 2048)
       hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<2048, 4, 16, 16, 1>), grow2048, dim3(256), 0, gs->stream,
-                         (const float2 *)g2, pitchC, planeC, f.hw, ny, twN, twM, xc, yc, (const float *)d_inv,
-                         d_image);
+                         (const float2 *)g2, pitchC, planeC, f.hw, ny, twN, twM, xc, yc, inv, d_image);
     else
       hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<1024, 8, 8, 8>), grow, dim3(256), 0, gs->stream,
-                         (const float2 *)g2, pitchC, planeC, f.hw, ny, twN, twM, xc, yc, (const float *)d_inv,
-                         d_image);
+                         (const float2 *)g2, pitchC, planeC, f.hw, ny, twN, twM, xc, yc, inv, d_image);
     OBIT_HIP_TRY(hipGetLastError());
   } else {
     // real output of the C2R for every plane
@@ -2323,7 +2339,7 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
     }
     dim3 grid((unsigned)((nx / 4 + 255) / 256), (unsigned)ny, (unsigned)nplane);
     hipLaunchKernelGGL(obit::grid::k_center_correct4, grid, dim3(256), 0, gs->stream, gs->d_fft, nx, ny, xc, yc,
-                       d_inv, d_image);
+                       inv, d_image);
     OBIT_HIP_TRY(hipGetLastError());
   }
   OBIT_HIP_TRY(hipStreamSynchronize(gs->stream));

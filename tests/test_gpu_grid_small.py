@@ -98,3 +98,29 @@ def test_image_of_few_columns(oracle, nx, scale):
         peak = np.abs(ref[p] / taper).max()
         # FP32 transform of 2^22 points: 22 butterflies of 6e-8, on the uncorrected scale
         assert np.abs((img[p] - ref[p]) / taper).max() < 1e-6 * peak
+
+
+@pytest.mark.parametrize("nx,nplane", [(128, 32), (128, 33), (1024, 32), (1024, 33)])
+def test_image_norms(oracle, nx, nplane):
+    """Images of as many planes as take their norms in the kernel's arguments,
+    and of one more, each plane by its own norm."""
+    import ctypes as C
+    from obit_amd import _lib
+    from obit_amd.gridder import GPUGrid
+    uv, _, _ = synth.workload(4, rows=5)
+    f = synth.make_facets(1, nx, 0.4 / 3600.0 * 1024 / nx, 0.0)
+    cf = oracle.convfunc()[0]
+    corr = np.zeros(nx, np.float32)
+    _lib.load().ObitHostGridCorrFn(nx, nx // 2 + 1, cf.ctypes.data_as(C.POINTER(C.c_float)), 7, 100,
+                                   corr.ctypes.data_as(C.POINTER(C.c_float)))
+    norm = np.linspace(0.5, 9.0, nplane).astype(np.float32)
+    with GPUGrid(uv, f, nplane=nplane, plane_of_chan=(np.arange(256) % nplane).astype(np.int32)) as gg:
+        gg.grid(uv.buffer)
+        gg.flip()
+        planes = gg.to_host(0)
+        img, _ = gg.fft_image(0, False, norm)
+    look = [0, 1, nplane - 1]
+    ref, _ = oracle.fft2image(planes[look], cf, False, norm[look], corr=(corr, corr))
+    taper = (corr[:, None] * corr[None, :]).astype(np.float64)
+    for k, p in enumerate(look):
+        assert np.abs((img[p] - ref[k]) / taper).max() < 1e-6 * np.abs(ref[k] / taper).max()
