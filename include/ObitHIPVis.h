@@ -107,9 +107,11 @@ int ObitHIPSkyModelDFTGraphLaunch(GPUInfo *gpuInfo);
  * kernel), which ignores tile and wgPerCU.  A spectral
  * point model runs on a matrix-core kernel of its own where its amplitudes
  * factor smoothly over blocks of 16 channels.  Until SetVariant or Autotune is
- * called, a point model runs on whichever of the matrix-core kernel and the
- * default VALU shape (32, 64, 2) takes fewer rounds of workgroups, by their
- * measured cost; GetVariant then reports the VALU shape.  Autotune times
+ * called, a launch runs on whichever of the matrix-core kernel (where it can
+ * run the model), the default VALU shape (32, 64, 2) and a VALU kernel of
+ * smaller work items (64 rows, the components divided over its waves) takes the
+ * least time by its rounds of workgroups and their measured cost; GetVariant
+ * then reports the VALU shape.  Autotune times
  * every shape on a copy of the first resident rows and keeps the fastest:
  * sampleRows rows, raised where needed so that the widest grid gets at
  * least 8 rounds of work items, and capped at the resident rows. */

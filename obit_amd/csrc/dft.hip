@@ -1827,10 +1827,9 @@ int launch_share(State *st, const Desc &d, int cpt, hipStream_t stream) {
   return kOK;
 }
 
-// The launch over resident rows.  A variant that the caller has set is taken;
-// otherwise the kernel that takes the least rounds of its resident
-// workgroups, since the last round of a short launch costs as much as a full
-// one.  A round takes, for each component,
+// The kernel of a launch in one part: the one that takes the least rounds of
+// its resident workgroups, since the last round of a short launch costs as
+// much as a full one.  A round takes, for each component,
 //   k_dft_mfma   59 ns (a row quad, 256 channel slots a pass)
 //   k_dft_spec   75 ns (a row quad and pass)
 //   k_dft_split  500 ns (256 rows x 32 channels), 625 with spectra or Gaussians
@@ -1842,8 +1841,12 @@ int launch_share(State *st, const Desc &d, int cpt, hipStream_t stream) {
 // 4 x 64, 20,000 rows 1.56 against 3.75; 2 x 96, 20,000 rows 1.52 against 2.15;
 // Gaussians of 1 x 64, 5,000 rows x 6,000 components 3.5 ms against 0.63 on
 // k_dft_share.
-int launch_resident(State *st, const Desc &d, bool matrix) {
-  if (st->chosen) return launch_split(st, d, matrix ? st->cpt : (st->cpt == 64 ? 32 : st->cpt), st->tile, st->wgPerCU);
+struct Choice {
+  enum { split, matrix, share } kernel;
+  int cpt;      // of k_dft_share
+  double cost;  // ns a component
+};
+Choice choose(State *st, const Desc &d, bool matrix) {
   auto rounds = [&](long long items, int perCU) {
     const long long slots = (long long)st->nCU * perCU;
     return (double)((items + slots - 1) / slots);
@@ -1859,9 +1862,17 @@ int launch_resident(State *st, const Desc &d, bool matrix) {
   const long long nquad = (d.nrow + 3) / 4, npass = (d.nIFsel * ((d.nchsel + 63) / 64) + 3) / 4;
   if (spec) tM = 75.0 * rounds(nquad * st->spec.npass, occupancy_of(st, (const void *)k_dft_spec));
   else if (matrix && mfma_ok(st, d)) tM = 59.0 * npass * rounds(nquad, occupancy_of(st, (const void *)mfma_fn(st)));
-  if (tM < tSplit && tM < tShare) return launch_split(st, d, 64, st->tile, st->wgPerCU);
-  if (tShare < tSplit) return launch_share(st, d, cs, nullptr);
-  return launch_split(st, d, st->cpt, st->tile, st->wgPerCU);
+  if (tM < tSplit && tM < tShare) return {Choice::matrix, 64, tM};
+  if (tShare < tSplit) return {Choice::share, cs, tShare};
+  return {Choice::split, st->cpt, tSplit};
+}
+
+// The launch over resident rows: a variant that the caller has set, else choose.
+int launch_resident(State *st, const Desc &d, bool matrix) {
+  if (st->chosen) return launch_split(st, d, matrix ? st->cpt : (st->cpt == 64 ? 32 : st->cpt), st->tile, st->wgPerCU);
+  const Choice c = choose(st, d, matrix);
+  if (c.kernel == Choice::share) return launch_share(st, d, c.cpt, nullptr);
+  return launch_split(st, d, c.kernel == Choice::matrix ? 64 : st->cpt, st->tile, st->wgPerCU);
 }
 
 // Run the operation over nrow rows at a device pointer.
@@ -2005,17 +2016,18 @@ BufPlan plan_buffer(State *st, const Desc &d, size_t rowBytes) {
     }
   }
   // A buffer of less than one round of resident workgroups takes as long as one
-  // item.  k_dft_share's items are a quarter of the rows and components (costs a
-  // component as in launch_resident); taken where its rounds of them take less
-  // than half of that, so that the parts of a longer list, whose uploads overlap,
-  // stay: 351 rows x 64 channels x 100 components 88 us on k_dft_split.
-  const int cs = p.cpt;
-  const long long shareItems = (d.nrow + kShareRows - 1) / kShareRows * perBlock;
-  const double tShare = (cs == 16 ? 0.55 : 1.0) * 0.27 * (double)((shareItems + slots - 1) / slots);
-  if (d.ncomp > 0 && items * p.nsplit <= slots && tShare < 0.5 * (cs == 16 ? 0.55 : 1.0) / p.nsplit) {
-    p.share = true;
-    p.nsplit = 1;
-    p.kpart = d.ncomp;
+  // item of its parts.  Where the kernel that resident rows would take needs less
+  // than half of that it is taken, in one part (the parts of a longer list, whose
+  // uploads overlap, stay): 351 rows x 64 channels x 100 components 88 us on
+  // k_dft_split, the call with its transfers 215 -> 109.
+  if (d.ncomp > 0 && items * p.nsplit <= slots) {
+    const Choice c = choose(st, d, true);
+    if (c.kernel != Choice::split && c.cost < 0.5 * (g || s ? 625.0 : 500.0) * (p.cpt == 16 ? 0.55 : 1.0) / p.nsplit) {
+      p.share = c.kernel == Choice::share;
+      p.cpt = c.cpt;
+      p.nsplit = 1;
+      p.kpart = d.ncomp;
+    }
   }
   const int round = (int)std::max<long long>(1, slots / (perBlock * p.nsplit));  // row blocks per round
   const int mid = std::max(2 * round, (d.nrowblk + 15) / 16);                     // at most ~17 segments
