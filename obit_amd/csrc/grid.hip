@@ -860,11 +860,14 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
 __global__ __launch_bounds__(256) void k_grid_clear(const FacetDev *facets, int nf, int nplane) {
   for (int fi = blockIdx.y; fi < nf; fi += gridDim.y) {
     float *g = facets[fi].grid;
-    const long long n = (long long)facets[fi].sizeGrid * nplane, n4 = n >> 2;
+    const long long n = (long long)facets[fi].sizeGrid * nplane;
+    // a caller's own grid may start at any float
+    const long long n4 = (reinterpret_cast<size_t>(g) & 15) ? 0 : n >> 2;
     float4 *g4 = reinterpret_cast<float4 *>(g);
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n4; i += (long long)gridDim.x * 256)
       g4[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) g[4 * n4 + threadIdx.x] = 0.0f;
+    for (long long i = 4 * n4 + (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
+      g[i] = 0.0f;
   }
 }
 
