@@ -459,13 +459,31 @@ __global__ __launch_bounds__(256) void k_bin_emit(const float *vis, long long nr
 }
 
 // List extents from the sorted keys: first[L] at a list's first entry and
-// last[L] one past its last (both zero for empty lists).
-__global__ void k_list_bounds(const unsigned *keys, long long n, long long *first, long long *last) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const unsigned L = keys[i] >> 7;
-    if (i == 0 || (keys[i - 1] >> 7) != L) first[L] = i;
-    if (i == n - 1 || (keys[i + 1] >> 7) != L) last[L] = i + 1;
+// last[L] one past its last (both zero for empty lists).  Four keys a thread in
+// one load, with the ones on either side: bound by the read of the keys (26.5 M:
+// one key a thread 74 us, so 36).
+__global__ __launch_bounds__(256) void k_list_bounds(const unsigned *keys, long long n, long long *first,
+                                                     long long *last) {
+  const long long n4 = (n + 3) >> 2;
+  for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < n4; q += (long long)gridDim.x * 256) {
+    const long long i0 = 4 * q;
+    const int m = (int)min(4LL, n - i0);
+    unsigned k[4];
+    if (m == 4) {
+      const uint4 v = reinterpret_cast<const uint4 *>(keys)[q];
+      k[0] = v.x >> 7; k[1] = v.y >> 7; k[2] = v.z >> 7; k[3] = v.w >> 7;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) k[j] = keys[i0 + min(j, m - 1)] >> 7;
+    }
+    if (i0 == 0 || (keys[i0 - 1] >> 7) != k[0]) first[k[0]] = i0;
+#pragma unroll
+    for (int j = 1; j < 4; ++j)
+      if (k[j] != k[j - 1]) {
+        last[k[j - 1]] = i0 + j;
+        first[k[j]] = i0 + j;
+      }
+    if (i0 + m == n || (keys[i0 + m] >> 7) != k[3]) last[k[3]] = i0 + m;
   }
 }
 
@@ -473,7 +491,7 @@ __global__ void k_list_bounds(const unsigned *keys, long long n, long long *firs
 
 constexpr int kW = 7;          // GCF support in cells (checked on the host)
 constexpr int kChunk = 128;    // most tracks of a work item (swept 64..2048 on workload 4: 128 best)
-constexpr int kMinChunk = 16;  // least (see grid_device)
+constexpr int kMinChunk = 16;  // least, both powers of two (see grid_device)
 // A sample's footprint is accumulated through a 16 (u) x 8 (v) window of
 // cells whose origin is its base cell rounded down to a multiple of 8 in u
 // and of 2 in v, so a window serves the 8x2 base cells of an aligned
@@ -1669,17 +1687,19 @@ struct ToEntriesU {
 // Work items of a list: its entries in chunks.
 struct ToChunks {
   const long long *first, *last;
-  int chunk;
-  __host__ __device__ long long operator()(long long L) const { return (last[L] - first[L] + chunk - 1) / chunk; }
+  int logChunk;
+  __host__ __device__ long long operator()(long long L) const {
+    return (last[L] - first[L] + (1 << logChunk) - 1) >> logChunk;
+  }
 };
 
 // Work items (list, chunk) of every list, in list order, at the list's
 // scanned item offset.
-__global__ __launch_bounds__(256) void k_items(const long long *first, const long long *last, int chunk,
+__global__ __launch_bounds__(256) void k_items(const long long *first, const long long *last, int logChunk,
                                                const long long *itemOff, long long nl, int2 *items) {
   for (long long L = (long long)blockIdx.x * blockDim.x + threadIdx.x; L < nl;
        L += (long long)gridDim.x * blockDim.x) {
-    const long long n = (last[L] - first[L] + chunk - 1) / chunk, base = itemOff[L];
+    const long long n = (last[L] - first[L] + (1 << logChunk) - 1) >> logChunk, base = itemOff[L];
     for (long long c = 0; c < n; ++c) items[base + c] = make_int2((int)L, (int)c);
   }
 }
@@ -1832,6 +1852,8 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   gs->chunk = kChunk;
   if (!gs->anyBeam)
     while (gs->chunk > kMinChunk && 80 * total < waves * gs->chunk * gs->chunk) gs->chunk /= 2;
+  int logChunk = 0;
+  while ((1 << logChunk) < gs->chunk) ++logChunk;
   gs->fullItems = total / gs->chunk;
   gs->itemBound = std::min(total, nl + gs->fullItems + 1);
   if (gs->itemBound > gs->itemCap) {
@@ -1845,12 +1867,12 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   // counts (the list after the last is empty, so the scan's last element is the
   // number of items, which the gridding kernel reads where it is)
   if (total > 0) {
-    const int nbk = (int)std::min<long long>((total + 255) / 256, (long long)gs->nCU * 32);
+    const int nbk = (int)std::min<long long>((total + 1023) / 1024, (long long)gs->nCU * 32);
     hipLaunchKernelGGL(k_list_bounds, dim3(nbk), dim3(256), 0, gs->stream, gs->d_keys2, total, gs->d_offsets,
                        gs->d_lend);
     OBIT_HIP_TRY(hipGetLastError());
     const auto chunks = rocprim::make_transform_iterator(rocprim::counting_iterator<long long>(0),
-                                                         ToChunks{gs->d_offsets, gs->d_lend, gs->chunk});
+                                                         ToChunks{gs->d_offsets, gs->d_lend, logChunk});
     size_t need = 0;
     OBIT_HIP_TRY(rocprim::exclusive_scan(nullptr, need, chunks, gs->d_itemOff, 0LL, (size_t)nl + 1,
                                          rocprim::plus<long long>(), gs->stream));
@@ -1858,7 +1880,7 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     OBIT_HIP_TRY(rocprim::exclusive_scan(gs->d_scanTmp, need, chunks, gs->d_itemOff, 0LL, (size_t)nl + 1,
                                          rocprim::plus<long long>(), gs->stream));
     const int nbI = (int)std::min<long long>((nl + 255) / 256, (long long)gs->nCU * 16);
-    hipLaunchKernelGGL(k_items, dim3(nbI), dim3(256), 0, gs->stream, gs->d_offsets, gs->d_lend, gs->chunk,
+    hipLaunchKernelGGL(k_items, dim3(nbI), dim3(256), 0, gs->stream, gs->d_offsets, gs->d_lend, logChunk,
                        gs->d_itemOff, nl, gs->d_items);
     OBIT_HIP_TRY(hipGetLastError());
     OBIT_HIP_TRY(hipMemcpyAsync(gs->h_tot + 1, gs->d_itemOff + nl, sizeof(long long), hipMemcpyDeviceToHost,
