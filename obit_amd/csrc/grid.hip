@@ -1028,9 +1028,9 @@ constexpr int kColStride = N + N / 8 + 1;
 // the length of the transforms already formed and k = j mod Ns, the R
 // points j + r N / R times W_{Ns R}^{r k}, a radix-R DFT, written to
 // (j / Ns) Ns R + k + r Ns.
-// With HALF, tw holds W_N^m for m < N / 2 only (W_N^{m + N/2} = -W_N^m).
+// tw holds W_N^m for m < N / 2 (W_N^{m + N/2} = -W_N^m).
 // tid is the thread's index in the block.
-template <int N, int R, int CB, int NT = 256, bool HALF = false>
+template <int N, int R, int CB, int NT>
 __device__ __forceinline__ void stockham_pass(float2 *lds, int Ns, const float2 *__restrict__ tw,
                                               int tid = (int)threadIdx.x) {
   constexpr int kItems = CB * N / R;
@@ -1050,13 +1050,8 @@ __device__ __forceinline__ void stockham_pass(float2 *lds, int Ns, const float2 
         float2 x = lds[c * kColStride<N> + lidx(j + r * (N / R))];
         if (r) {
           const int m = (r * k * step) & (N - 1);
-          float2 w;
-          if (HALF) {
-            w = tw[m & (N / 2 - 1)];
-            if (m & (N / 2)) w = make_float2(-w.x, -w.y);
-          } else {
-            w = tw[m];
-          }
+          float2 w = tw[m & (N / 2 - 1)];
+          if (m & (N / 2)) w = make_float2(-w.x, -w.y);
           x = make_float2(x.x * w.x - x.y * w.y, x.x * w.y + x.y * w.x);
         }
         v[q][r] = x;
@@ -1180,8 +1175,8 @@ __global__ __launch_bounds__(NT) void k_fft_cols8(float2 *grid, int pitchC, long
     // the next column block's rows, in flight under the passes
     if (e + nper < eEnd) load(e + nper, 0, R1, tl);
     __syncthreads();
-    stockham_pass<N, R2, CB, NT, true>(lds, R1, twl, tl);
-    stockham_pass<N, R3, CB, NT, true>(lds, R1 * R2, twl, tl);
+    stockham_pass<N, R2, CB, NT>(lds, R1, twl, tl);
+    stockham_pass<N, R3, CB, NT>(lds, R1 * R2, twl, tl);
     float2 *g = base(e);
 #pragma unroll
     for (int i = 0; i < N / 256; ++i) {
@@ -1208,8 +1203,8 @@ __global__ __launch_bounds__(NT) void k_fft_cols8(float2 *grid, int pitchC, long
       for (int r = 0; r < R1; ++r) lds[lidx(t * R1 + r)] = w[r];
     }
     __syncthreads();
-    stockham_pass<N, R2, 1, NT, true>(lds, R1, twl);
-    stockham_pass<N, R3, 1, NT, true>(lds, R1 * R2, twl);
+    stockham_pass<N, R2, 1, NT>(lds, R1, twl);
+    stockham_pass<N, R3, 1, NT>(lds, R1 * R2, twl);
     for (int i = t; i < N; i += NT) g[(long long)i * pitchC] = lds[lidx(i)];
   }
 }
@@ -1225,91 +1220,92 @@ __global__ __launch_bounds__(NT) void k_fft_cols8(float2 *grid, int pitchC, long
 // Output row y of plane p is input row r = (y + ny/2) mod ny times
 // (-1)^r xc[y] invNorm[p], and column x is sample (x + N/2) mod N times
 // yc[x] (ObitFArray2DCenter and ObitFArrayMulColRow, as k_center_correct4
-// applies them).  Block (RW rows, plane); NT threads.  twN[k] = exp(+2 pi
-// i k / N) and twM = the M-point table (every other entry of twN).
-template <int N, int R1, int R2, int R3, int RW = 4, int NT = 256>
-__global__ __launch_bounds__(NT) void k_fft_rows_c2r(const float2 *grid, int pitchC, long long planeC, int hw,
-                                                      int ny, const float2 *__restrict__ twN,
-                                                      const float2 *__restrict__ twM, const float *xc,
-                                                      const float *yc, InvNorm invNorm, float *img) {
-  constexpr int M = N / 2;
-  static_assert(R1 * R2 * R3 == M, "radices");
-  __shared__ float2 lds[RW * kColStride<M>];
-  const int t = threadIdx.x, p = blockIdx.y;
-  const int r0 = blockIdx.x * RW;
-  const float2 *g = grid + (long long)p * planeC + hw;
-  // rows r0 .. r0+3, samples 0 .. M (row c at lds[c * kColStride<M>]):
-  // every load issued before the first is waited on
-  static_assert(M % NT == 0 && NT >= RW, "whole sample blocks per thread");
-  constexpr int kPerRow = M / NT;
-  float2 xin[RW][kPerRow];
-  float2 xlast = make_float2(0.0f, 0.0f);
-#pragma unroll
-  for (int c = 0; c < RW; ++c)
-#pragma unroll
-    for (int i = 0; i < kPerRow; ++i) xin[c][i] = g[(long long)(r0 + c) * pitchC + t + NT * i];
-  if (t < RW) xlast = g[(long long)(r0 + t) * pitchC + M];
-#pragma unroll
-  for (int c = 0; c < RW; ++c)
-#pragma unroll
-    for (int i = 0; i < kPerRow; ++i) lds[c * kColStride<M> + lidx(t + NT * i)] = xin[c][i];
-  if (t < RW) lds[t * kColStride<M> + lidx(M)] = xlast;
+// applies them).
+//
+// One wave a row, with no barriers between the passes: M = 64 RA points, lane l
+// holds the points l + 64 r; radices RA, RA and R3, two exchanges through the
+// wave's own LDS (point p at p + p / RA, so neither way has bank conflicts).
+// Z[k] takes X[k] and X[M - k] from memory (the second read hits the cache) and
+// the last pass's points go straight to the image, so a row crosses LDS twice
+// instead of five times.  The persistent blocks keep the twiddle table
+// (exp(+2 pi i m / N)) in LDS.  Bound by HBM: 8 planes of 2048^2 74 us with a
+// workgroup a row and barriers, so 52, 5.2 TB/s (the whole call 182 -> 158; of
+// 1024^2 55 -> 47).  Held to 168 registers, for a third wave a SIMD, it spills and
+// takes 93.
+template <int RA, int R3>
+__global__ __launch_bounds__(256) void k_fft_rows_c2r(const float2 *grid, int pitchC, long long planeC, int hw, int ny,
+                                                      int nplane, const float2 *__restrict__ twN,
+                                                      const float *__restrict__ xc, const float *__restrict__ yc,
+                                                      InvNorm invNorm, float *img) {
+  constexpr int M = 64 * RA, N = 2 * M, Ns = RA * RA;
+  static_assert(Ns * R3 == M && RA % R3 == 0, "radices");
+  __shared__ float2 s_lds[4][M + M / RA];
+  __shared__ float2 s_tw[N];
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  float2 *lds = s_lds[wv];
+  auto at = [](int p) { return p + p / RA; };
+  auto settle = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  auto mul = [](float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); };
+  for (int i = threadIdx.x; i < N; i += 256) s_tw[i] = twN[i];
   __syncthreads();
-  // Z in place: the pair (k, M - k) by one thread; all of a thread's
-  // loads first
-  constexpr int kPairs = RW * (M / 2 + 1), kPP = (kPairs + NT - 1) / NT;
-  float2 za[kPP], zb[kPP], wa[kPP], wb[kPP];
+  const long long total = (long long)nplane * ny;
+  for (long long g = (long long)blockIdx.x * 4 + wv; g < total; g += (long long)gridDim.x * 4) {
+    const int p = (int)(g / ny), r0 = (int)(g - (long long)p * ny);
+    const float2 *x = grid + (long long)p * planeC + hw + (long long)r0 * pitchC;
+    float2 a[RA], b[RA], v[RA];
 #pragma unroll
-  for (int i = 0; i < kPP; ++i) {
-    const int q = t + NT * i;
-    const int c = q / (M / 2 + 1), k = q - c * (M / 2 + 1);
-    if (q < kPairs) {
-      const float2 *row = lds + c * kColStride<M>;
-      za[i] = row[lidx(k)];
-      zb[i] = row[lidx(M - k)];
-      wa[i] = twN[k];
-      wb[i] = twN[(M - k) & (N - 1)];
+    for (int r = 0; r < RA; ++r) {
+      a[r] = x[l + 64 * r];
+      b[r] = x[M - l - 64 * r];
     }
-  }
-  __syncthreads();
+    if (l == 0) { a[0].y = 0.0f; b[0].y = 0.0f; }
 #pragma unroll
-  for (int i = 0; i < kPP; ++i) {
-    const int q = t + NT * i;
-    const int c = q / (M / 2 + 1), k = q - c * (M / 2 + 1);
-    if (q < kPairs) {
-      float2 *row = lds + c * kColStride<M>;
-      float2 a = za[i], b = zb[i];
-      if (k == 0) { a.y = 0.0f; b.y = 0.0f; }
-      // Z[k] from X[k], X[M-k] and exp(+2 pi i k / N)
-      auto zk = [](float2 xk, float2 xm, float2 w) {
-        const float2 fe = make_float2(xk.x + xm.x, xk.y - xm.y);
-        const float2 d = make_float2(xk.x - xm.x, xk.y + xm.y);
-        const float2 fo = make_float2(d.x * w.x - d.y * w.y, d.x * w.y + d.y * w.x);
-        return make_float2(fe.x - fo.y, fe.y + fo.x);
-      };
-      row[lidx(k)] = zk(a, b, wa[i]);
-      if (k != 0) row[lidx(M - k)] = zk(b, a, wb[i]);
+    for (int r = 0; r < RA; ++r) {
+      const float2 fe = make_float2(a[r].x + b[r].x, a[r].y - b[r].y);
+      const float2 fo = mul(make_float2(a[r].x - b[r].x, a[r].y + b[r].y), s_tw[l + 64 * r]);
+      v[r] = make_float2(fe.x - fo.y, fe.y + fo.x);
     }
-  }
-  __syncthreads();
-  stockham_pass<M, R1, RW, NT>(lds, 1, twM);
-  stockham_pass<M, R2, RW, NT>(lds, R1, twM);
-  stockham_pass<M, R3, RW, NT>(lds, R1 * R2, twM);
-  // centre, correct, store: thread takes output column pairs
-  const float inv = inv_norm(invNorm, p);
+    dft_small<RA>(v);
+    settle();  // the last row's reads
 #pragma unroll
-  for (int i = 0; i < RW * M / NT; ++i) {
-    const int q = t + NT * i;
-    const int c = q / M, m = q - c * M;
-    const int r = r0 + c;
-    int y = r + ny / 2;
+    for (int r = 0; r < RA; ++r) lds[at(RA * l) + r] = v[r];
+    settle();
+    const int k = l & (RA - 1);
+#pragma unroll
+    for (int r = 0; r < RA; ++r) {
+      v[r] = lds[at(l + 64 * r)];
+      if (r) v[r] = mul(v[r], s_tw[N / Ns * r * k]);  // W_Ns^{r k}
+    }
+    dft_small<RA>(v);
+    settle();
+#pragma unroll
+    for (int r = 0; r < RA; ++r) lds[at((l - k) * RA + k + r * RA)] = v[r];
+    settle();
+    int y = r0 + ny / 2;
     if (y >= ny) y -= ny;
-    const float rs = ((r & 1) ? -xc[y] : xc[y]) * inv;
-    const float2 z = lds[c * kColStride<M> + lidx(m)];
-    int x = 2 * m + N / 2;
-    if (x >= N) x -= N;
-    const float2 yy = *reinterpret_cast<const float2 *>(yc + x);
-    *reinterpret_cast<float2 *>(img + ((long long)p * ny + y) * N + x) = make_float2(z.x * rs * yy.x, z.y * rs * yy.y);
+    const float rs = ((r0 & 1) ? -xc[y] : xc[y]) * inv_norm(invNorm, p);
+    float *out = img + ((long long)p * ny + y) * N;
+#pragma unroll
+    for (int i = 0; i < RA / R3; ++i) {
+      const int j = l + 64 * i;
+      float2 u[R3];
+#pragma unroll
+      for (int r = 0; r < R3; ++r) {
+        u[r] = lds[at(j + Ns * r)];
+        if (r) u[r] = mul(u[r], s_tw[2 * r * j]);  // W_M^{r j}
+      }
+      dft_small<R3>(u);
+#pragma unroll
+      for (int r = 0; r < R3; ++r) {
+        const int xo = (2 * (j + Ns * r) + M) & (N - 1);
+        const float2 yy = *reinterpret_cast<const float2 *>(yc + xo);
+        *reinterpret_cast<float2 *>(out + xo) = make_float2(u[r].x * rs * yy.x, u[r].y * rs * yy.y);
+      }
+    }
   }
 }
 
@@ -1377,6 +1373,7 @@ struct GpuState {
   int device = 0;
   hipStream_t stream = nullptr;
   int nCU = 256;
+  int rowsPerCU = 0, rowsPerCU1024 = 0;  // resident k_fft_rows_c2r blocks per CU (0: not queried yet)
   int tapsPerCU = 0;        // resident k_grid_taps<4, 16> blocks per CU (0: not queried yet)
   std::vector<int> facets;  // facet indices on this GPU
   FacetDev *d_facets = nullptr;  // in d_tab
@@ -2270,14 +2267,13 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
   const int pitchC = f.lrow / 2;
   const bool own = (nx == 1024 || nx == 2048) && pitchC % 4 == 0 && f.sizeGrid % 8 == 0 && ny % 4 == 0;
   if (own) {
-    // exp(+2 pi i m / n) for m < n, and for m < n / 2 at n / 2, in FP64
+    // exp(+2 pi i m / n) for m < n, in FP64
     if (gs->twN != ny) {
-      std::vector<float2> tw((size_t)ny + ny / 2);
+      std::vector<float2> tw((size_t)ny);
       for (int m = 0; m < ny; ++m) {
         const double a = 2.0 * M_PI * (double)m / (double)ny;
         tw[m] = make_float2((float)std::cos(a), (float)std::sin(a));
       }
-      for (int m = 0; m < ny / 2; ++m) tw[ny + m] = tw[2 * m];
       (void)hipFree(gs->d_tw);
       gs->d_tw = nullptr;
       gs->twN = 0;
@@ -2285,7 +2281,7 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
       OBIT_HIP_TRY(hipMemcpy(gs->d_tw, tw.data(), sizeof(float2) * tw.size(), hipMemcpyHostToDevice));
       gs->twN = ny;
     }
-    const float2 *twN = gs->d_tw, *twM = gs->d_tw + ny;
+    const float2 *twN = gs->d_tw;
     float2 *g2 = reinterpret_cast<float2 *>(f.grid);
     const long long planeC = (long long)f.sizeGrid / 2;
     // The nx/2 + 1 columns u = 0 .. nx/2 (hw .. hw + nx/2 of the padded
@@ -2306,9 +2302,6 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
     const long long resident = (long long)gs->nCU * (nx == 2048 ? gs->colsPerCU : gs->colsPerCU1024);
     const long long ncb = 8 * ((std::min<long long>((long long)nplane * nfull, resident) + 7) / 8);
     const dim3 gcol((unsigned)ncb);
-    // rows a block: 1 at 2048 (measured 8.1 ms for 320 planes, against 8.2
-    // with 2 rows, 8.4 with 4 and 9.35 with 8), 4 at 1024
-    const dim3 grow((unsigned)(ny / 4), (unsigned)nplane), grow2048((unsigned)ny, (unsigned)nplane);
     if (nx == 2048)
       hipLaunchKernelGGL((obit::grid::k_fft_cols8<2048, 8, 16, 16, 1024>), gcol, dim3(1024), 0, gs->stream, g2, pitchC,
                          planeC, c0, nplane, nfull, side, twN);
@@ -2321,12 +2314,21 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
                          (const float2 *)g2, planeC, f.hw, nx, xc, yc, ny, d_norm, d_inv, gs->h_norm);
       OBIT_HIP_TRY(hipGetLastError());
     }
+    if (gs->rowsPerCU <= 0) {
+      int nb = 0;
+      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_rows_c2r<16, 4>, 256, 0));
+      gs->rowsPerCU = std::max(nb, 1);
+      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_rows_c2r<8, 8>, 256, 0));
+      gs->rowsPerCU1024 = std::max(nb, 1);
+    }
+    const long long nbR = std::min<long long>(((long long)nplane * ny + 3) / 4,
+                                              (long long)gs->nCU * (nx == 2048 ? gs->rowsPerCU : gs->rowsPerCU1024));
     if (nx == 2048)
-      hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<2048, 4, 16, 16, 1>), grow2048, dim3(256), 0, gs->stream,
-                         (const float2 *)g2, pitchC, planeC, f.hw, ny, twN, twM, xc, yc, inv, d_image);
+      hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<16, 4>), dim3((unsigned)nbR), dim3(256), 0, gs->stream,
+                         (const float2 *)g2, pitchC, planeC, f.hw, ny, nplane, twN, xc, yc, inv, d_image);
     else
-      hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<1024, 8, 8, 8>), grow, dim3(256), 0, gs->stream,
-                         (const float2 *)g2, pitchC, planeC, f.hw, ny, twN, twM, xc, yc, inv, d_image);
+      hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<8, 8>), dim3((unsigned)nbR), dim3(256), 0, gs->stream,
+                         (const float2 *)g2, pitchC, planeC, f.hw, ny, nplane, twN, xc, yc, inv, d_image);
     OBIT_HIP_TRY(hipGetLastError());
   } else {
     // real output of the C2R for every plane
