@@ -1420,7 +1420,7 @@ struct GpuState {
   std::vector<float> h_corr;  // xCorr, yCorr of the last (nx, ny) (GridCorrFn)
   int corrNx = 0, corrNy = 0;
   // tables
-  char *d_tab = nullptr, *h_tab = nullptr;  // tables (refresh), device and pinned
+  char *d_tab = nullptr, *h_tab = nullptr;  // tables (refresh), device and pinned (after h_tot)
   size_t tabCap = 0;
   Common cm{};
   bool ready = false;
@@ -1615,11 +1615,15 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
   gs->ready = false;
   if (tab > gs->tabCap) {
     (void)hipFree(gs->d_tab);
-    if (gs->h_tab) (void)hipHostFree(gs->h_tab);
+    if (gs->h_tot) (void)hipHostFree(gs->h_tot);
     gs->d_tab = gs->h_tab = nullptr;
+    gs->h_tot = nullptr;
     gs->tabCap = 0;
     OBIT_HIP_TRY(hipMalloc(&gs->d_tab, tab));
-    OBIT_HIP_TRY(hipHostMalloc(&gs->h_tab, tab, hipHostMallocDefault));
+    // one pinned block: a pass's totals, then the tables
+    constexpr size_t kTot = ((2 + 2 * kHashParts * kHashStride) * sizeof(long long) + 255) & ~(size_t)255;
+    OBIT_HIP_TRY(hipHostMalloc(&gs->h_tot, kTot + tab, hipHostMallocDefault));
+    gs->h_tab = reinterpret_cast<char *>(gs->h_tot) + kTot;
     gs->tabCap = tab;
   }
   // rows of 8 (seven taps and a zero) so a row loads as two float4
@@ -1673,7 +1677,6 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
                        gs->d_listFacet);
     OBIT_HIP_TRY(hipGetLastError());
   }
-  if (!gs->h_tot) OBIT_HIP_TRY(hipHostMalloc(&gs->h_tot, (2 + 2 * kHashParts * kHashStride) * sizeof(long long), hipHostMallocDefault));
   gs->ready = true;
   return kOK;
 }
@@ -2098,7 +2101,6 @@ void ObitCUDAGridShutdown(CUDAGridInfo *cudaInfo, long iGPU) {
       if (fi && fi->d_grid) { (void)hipFree(fi->d_grid); fi->d_grid = nullptr; }
     }
     (void)hipFree(gs->d_tab); (void)hipFree(gs->d_listFacet);
-    if (gs->h_tab) (void)hipHostFree(gs->h_tab);
     (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets); (void)hipFree(gs->d_lists);
     (void)hipFree(gs->d_tcnt); (void)hipFree(gs->d_toff); (void)hipFree(gs->d_keys); (void)hipFree(gs->d_keys2);
     (void)hipFree(gs->d_rows); (void)hipFree(gs->d_rot);
