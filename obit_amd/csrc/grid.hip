@@ -970,6 +970,14 @@ __global__ void k_center_correct4(const float *fft, int nx, int ny, const float 
 
 // ---- the v transform of FFT2Image: columns of the padded half planes ----
 
+// x w.  Its products and sums, and dft_small's, are written as FMAs: left to the
+// compiler, which product of a sum is fused depends on the code around it and on
+// what it vectorises, and the images' corrections magnify that rounding by 5e4
+// in the corners.
+__device__ __forceinline__ float2 mul_fma(float2 x, float2 w) {
+  return make_float2(fmaf(x.x, w.x, -(x.y * w.y)), fmaf(x.y, w.x, x.x * w.y));
+}
+
 // V[k] = sum_m v[m] exp(+2 pi i m k / R) for R = 4, 8, 16, in natural
 // order: radix-2 stages on a bit-reversed copy, the stage twiddles exact
 // FP32 constants (W16^k).
@@ -1004,7 +1012,8 @@ __device__ __forceinline__ void dft_small(float2 (&v)[R]) {
           t = make_float2(-y.y, y.x);
         } else {
           const float wc = kc[e], ws = kc[(e + 12) & 15];   // cos, sin(2 pi e / 16)
-          t = make_float2(y.x * wc - y.y * ws, y.x * ws + y.y * wc);
+          t = make_float2(fmaf(y.x, wc, -(y.y * ws)),
+                          e == 1 || e == 3 ? fmaf(y.y, wc, y.x * ws) : fmaf(y.x, ws, y.y * wc));
         }
         a[i + j] = make_float2(x.x + t.x, x.y + t.y);
         a[i + j + half] = make_float2(x.x - t.x, x.y - t.y);
@@ -1052,7 +1061,7 @@ __device__ __forceinline__ void stockham_pass(float2 *lds, int Ns, const float2 
           const int m = (r * k * step) & (N - 1);
           float2 w = tw[m & (N / 2 - 1)];
           if (m & (N / 2)) w = make_float2(-w.x, -w.y);
-          x = make_float2(x.x * w.x - x.y * w.y, x.x * w.y + x.y * w.x);
+          x = mul_fma(x, w);
         }
         v[q][r] = x;
       }
@@ -1223,8 +1232,11 @@ __global__ __launch_bounds__(NT) void k_fft_cols8(float2 *grid, int pitchC, long
 // applies them).
 //
 // One wave a row, with no barriers between the passes: M = 64 RA points, lane l
-// holds the points l + 64 r; radices RA, RA and R3, two exchanges through the
-// wave's own LDS (point p at p + p / RA, so neither way has bank conflicts).
+// holds the points l + 64 r; radices R1, RA and RA (R1 = 64 / RA), two
+// exchanges through the wave's own LDS, padded for their writes (strides R1 and
+// 64) to fall on distinct banks.  The smallest radix first: the images'
+// corrections magnify the corners by 5e4, where another order of the radices
+// gives other FP32 roundings of up to 5e-3 of the images' rms.
 // Z[k] takes X[k] and X[M - k] from memory (the second read hits the cache) and
 // the last pass's points go straight to the image, so a row crosses LDS twice
 // instead of five times.  The persistent blocks keep the twiddle table
@@ -1232,24 +1244,24 @@ __global__ __launch_bounds__(NT) void k_fft_cols8(float2 *grid, int pitchC, long
 // workgroup a row and barriers, so 52, 5.2 TB/s (the whole call 182 -> 158; of
 // 1024^2 55 -> 47).  Held to 168 registers, for a third wave a SIMD, it spills and
 // takes 93.
-template <int RA, int R3>
+template <int RA>
 __global__ __launch_bounds__(256) void k_fft_rows_c2r(const float2 *grid, int pitchC, long long planeC, int hw, int ny,
                                                       int nplane, const float2 *__restrict__ twN,
                                                       const float *__restrict__ xc, const float *__restrict__ yc,
                                                       InvNorm invNorm, float *img) {
-  constexpr int M = 64 * RA, N = 2 * M, Ns = RA * RA;
-  static_assert(Ns * R3 == M && RA % R3 == 0, "radices");
-  __shared__ float2 s_lds[4][M + M / RA];
+  constexpr int M = 64 * RA, N = 2 * M, R1 = 64 / RA;
+  static_assert(RA % R1 == 0, "radices");
+  __shared__ float2 s_lds[4][M + M * R1 / 64];
   __shared__ float2 s_tw[N];
   const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
   float2 *lds = s_lds[wv];
-  auto at = [](int p) { return p + p / RA; };
+  auto at1 = [](int p) { return p + p / 32; };
+  auto at2 = [](int p) { return p + p / RA; };
   auto settle = [] {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  auto mul = [](float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); };
   for (int i = threadIdx.x; i < N; i += 256) s_tw[i] = twN[i];
   __syncthreads();
   const long long total = (long long)nplane * ny;
@@ -1266,45 +1278,49 @@ __global__ __launch_bounds__(256) void k_fft_rows_c2r(const float2 *grid, int pi
 #pragma unroll
     for (int r = 0; r < RA; ++r) {
       const float2 fe = make_float2(a[r].x + b[r].x, a[r].y - b[r].y);
-      const float2 fo = mul(make_float2(a[r].x - b[r].x, a[r].y + b[r].y), s_tw[l + 64 * r]);
+      const float2 d = make_float2(a[r].x - b[r].x, a[r].y + b[r].y), w = s_tw[l + 64 * r];
+      // k < M / 2 and the rest with the products' roles exchanged
+      const float2 fo = r < RA / 2 ? make_float2(fmaf(d.x, w.x, -(d.y * w.y)), fmaf(d.x, w.y, d.y * w.x)) : mul_fma(d, w);
       v[r] = make_float2(fe.x - fo.y, fe.y + fo.x);
     }
-    dft_small<RA>(v);
     settle();  // the last row's reads
+    // the lane's RA / R1 transforms of the first pass
 #pragma unroll
-    for (int r = 0; r < RA; ++r) lds[at(RA * l) + r] = v[r];
+    for (int i = 0; i < RA / R1; ++i) {
+      float2 u[R1];
+#pragma unroll
+      for (int r = 0; r < R1; ++r) u[r] = v[i + RA / R1 * r];
+      dft_small<R1>(u);
+#pragma unroll
+      for (int r = 0; r < R1; ++r) lds[at1(R1 * (l + 64 * i) + r)] = u[r];
+    }
     settle();
-    const int k = l & (RA - 1);
+    const int k = l & (R1 - 1);
 #pragma unroll
     for (int r = 0; r < RA; ++r) {
-      v[r] = lds[at(l + 64 * r)];
-      if (r) v[r] = mul(v[r], s_tw[N / Ns * r * k]);  // W_Ns^{r k}
+      v[r] = lds[at1(l + 64 * r)];
+      if (r) v[r] = mul_fma(v[r], s_tw[N / 64 * r * k]);  // W_64^{r k}
     }
     dft_small<RA>(v);
     settle();
 #pragma unroll
-    for (int r = 0; r < RA; ++r) lds[at((l - k) * RA + k + r * RA)] = v[r];
+    for (int r = 0; r < RA; ++r) lds[at2((l - k) * RA + k + r * R1)] = v[r];
     settle();
+#pragma unroll
+    for (int r = 0; r < RA; ++r) {
+      v[r] = lds[at2(l + 64 * r)];
+      if (r) v[r] = mul_fma(v[r], s_tw[2 * r * l]);  // W_M^{r l}
+    }
+    dft_small<RA>(v);
     int y = r0 + ny / 2;
     if (y >= ny) y -= ny;
     const float rs = ((r0 & 1) ? -xc[y] : xc[y]) * inv_norm(invNorm, p);
     float *out = img + ((long long)p * ny + y) * N;
 #pragma unroll
-    for (int i = 0; i < RA / R3; ++i) {
-      const int j = l + 64 * i;
-      float2 u[R3];
-#pragma unroll
-      for (int r = 0; r < R3; ++r) {
-        u[r] = lds[at(j + Ns * r)];
-        if (r) u[r] = mul(u[r], s_tw[2 * r * j]);  // W_M^{r j}
-      }
-      dft_small<R3>(u);
-#pragma unroll
-      for (int r = 0; r < R3; ++r) {
-        const int xo = (2 * (j + Ns * r) + M) & (N - 1);
-        const float2 yy = *reinterpret_cast<const float2 *>(yc + xo);
-        *reinterpret_cast<float2 *>(out + xo) = make_float2(u[r].x * rs * yy.x, u[r].y * rs * yy.y);
-      }
+    for (int r = 0; r < RA; ++r) {
+      const int xo = (2 * (l + 64 * r) + M) & (N - 1);
+      const float2 yy = *reinterpret_cast<const float2 *>(yc + xo);
+      *reinterpret_cast<float2 *>(out + xo) = make_float2(v[r].x * rs * yy.x, v[r].y * rs * yy.y);
     }
   }
 }
@@ -2318,18 +2334,18 @@ int ObitHIPGridFFT2Image(CUDAGridInfo *in, long ifacet, int isBeam, float *beamN
     }
     if (gs->rowsPerCU <= 0) {
       int nb = 0;
-      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_rows_c2r<16, 4>, 256, 0));
+      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_rows_c2r<16>, 256, 0));
       gs->rowsPerCU = std::max(nb, 1);
-      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_rows_c2r<8, 8>, 256, 0));
+      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, obit::grid::k_fft_rows_c2r<8>, 256, 0));
       gs->rowsPerCU1024 = std::max(nb, 1);
     }
     const long long nbR = std::min<long long>(((long long)nplane * ny + 3) / 4,
                                               (long long)gs->nCU * (nx == 2048 ? gs->rowsPerCU : gs->rowsPerCU1024));
     if (nx == 2048)
-      hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<16, 4>), dim3((unsigned)nbR), dim3(256), 0, gs->stream,
+      hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<16>), dim3((unsigned)nbR), dim3(256), 0, gs->stream,
                          (const float2 *)g2, pitchC, planeC, f.hw, ny, nplane, twN, xc, yc, inv, d_image);
     else
-      hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<8, 8>), dim3((unsigned)nbR), dim3(256), 0, gs->stream,
+      hipLaunchKernelGGL((obit::grid::k_fft_rows_c2r<8>), dim3((unsigned)nbR), dim3(256), 0, gs->stream,
                          (const float2 *)g2, pitchC, planeC, f.hw, ny, nplane, twN, xc, yc, inv, d_image);
     OBIT_HIP_TRY(hipGetLastError());
   } else {
