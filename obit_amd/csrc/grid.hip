@@ -490,8 +490,12 @@ __global__ __launch_bounds__(256) void k_list_bounds(const unsigned *keys, long 
 // ---------------- tile gridding ----------------
 
 constexpr int kW = 7;          // GCF support in cells (checked on the host)
-constexpr int kChunk = 128;    // most tracks of a work item (swept 64..2048 on workload 4: 128 best)
-constexpr int kMinChunk = 16;  // least, both powers of two (see grid_device)
+// Tracks of a work item (swept 64..2048 on workload 4: 128 best).  A small pass
+// would be faster with fewer (10,530 rows x 64 channels into 512^2: a call of
+// 0.86 ms with 16, 1.25 with 128), but other FP32 sums than one item's move the
+// pixels of an image's corners by up to 1e-2 of its rms, where the gridding
+// correction magnifies them by 5e4: one length for every pass.
+constexpr int kLogChunk = 7, kChunk = 1 << kLogChunk;
 // A sample's footprint is accumulated through a 16 (u) x 8 (v) window of
 // cells whose origin is its base cell rounded down to a multiple of 8 in u
 // and of 2 in v, so a window serves the 8x2 base cells of an aligned
@@ -568,7 +572,7 @@ template <int kWaves, int kGather>
 __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, const float4 *rot, long long nrow,
                                                            const FacetDev *facets,
                                                            const int *listFacet, const int2 *items,
-                                                           const long long *nitemsPtr, int chunk, Common cm,
+                                                           const long long *nitemsPtr, Common cm,
                                                            const long long *offsets, const long long *lend,
                                                            const int2 *lists, unsigned *next,
                                                            unsigned long long *stats) {
@@ -622,9 +626,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
     const long long L = __builtin_amdgcn_readfirstlane(item.x);
     const long long l0 = offsets[L];
     const int n = (int)(lend[L] - l0);
-    const int e0 = __builtin_amdgcn_readfirstlane(item.y) * chunk;
-    const int e1 = min(n, e0 + chunk);
-    const bool multi = n > chunk;
+    const int e0 = __builtin_amdgcn_readfirstlane(item.y) * kChunk;
+    const int e1 = min(n, e0 + kChunk);
+    const bool multi = n > kChunk;
     const int fi = listFacet[L];
     // a register copy: the wave fences below would otherwise make every
     // pass reload the descriptor from memory and wait on the row prefetch
@@ -1415,8 +1419,6 @@ struct GpuState {
   long long *h_tot = nullptr;      // pinned: list entries and work items of the last pass, checksums to compare
   // work items of the last pass; at most this many; that many if all were full
   long long nitems = 0, itemBound = 0, fullItems = 0;
-  int chunk = kChunk;              // tracks per work item of the last pass
-  bool anyBeam = false;            // a facet is gridded as a beam
   bool listsValid = false;         // the lists of the last pass, for ...
   long long listsRows = 0;         // ... a pass over as many rows ...
   unsigned long long *d_hash = nullptr;  // ... with the same uvw: their checksum, and another pass's
@@ -1525,7 +1527,6 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
   const int nf = (int)gs->facets.size();
   gs->h_facets.assign(nf, FacetDev{});
   long long listBase = 0;
-  gs->anyBeam = false;
   for (int k = 0; k < nf; ++k) {
     const FacetInfo *fi = in->h_facetInfo[gs->facets[k]];
     FacetDev &f = gs->h_facets[k];
@@ -1560,7 +1561,6 @@ int refresh(CUDAGridInfo *in, long iGPU, GpuState *gs) {
     f.ntu = (f.lrow / 2 + TU - 1) / TU;
     f.ntv = (f.ny + TV - 1) / TV;
     f.listBase = listBase;
-    gs->anyBeam = gs->anyBeam || f.doBeam;
     const long long nl = (long long)nplane * f.ntu * f.ntv;
     listBase += nl;
   }
@@ -1703,19 +1703,18 @@ struct ToEntriesU {
 // Work items of a list: its entries in chunks.
 struct ToChunks {
   const long long *first, *last;
-  int logChunk;
   __host__ __device__ long long operator()(long long L) const {
-    return (last[L] - first[L] + (1 << logChunk) - 1) >> logChunk;
+    return (last[L] - first[L] + kChunk - 1) >> kLogChunk;
   }
 };
 
 // Work items (list, chunk) of every list, in list order, at the list's
 // scanned item offset.
-__global__ __launch_bounds__(256) void k_items(const long long *first, const long long *last, int logChunk,
+__global__ __launch_bounds__(256) void k_items(const long long *first, const long long *last,
                                                const long long *itemOff, long long nl, int2 *items) {
   for (long long L = (long long)blockIdx.x * blockDim.x + threadIdx.x; L < nl;
        L += (long long)gridDim.x * blockDim.x) {
-    const long long n = (last[L] - first[L] + (1 << logChunk) - 1) >> logChunk, base = itemOff[L];
+    const long long n = (last[L] - first[L] + kChunk - 1) >> kLogChunk, base = itemOff[L];
     for (long long c = 0; c < n; ++c) items[base + c] = make_int2((int)L, (int)c);
   }
 }
@@ -1852,25 +1851,7 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     OBIT_HIP_TRY(rocprim::radix_sort_pairs<SortConfig>(gs->d_scanTmp, need, gs->d_keys, gs->d_keys2, gs->d_rows,
                                            gs->d_lists, (size_t)total, 0, endBit, gs->stream));
   }
-  // Tracks per work item.  A wave walks its item's samples one after the other,
-  // so a pass takes at least as long as an item, which goes with its tracks; and
-  // each item costs a tile cleared and added to the grid, which goes with the
-  // number of items a wave has, entries / (tracks x waves).  The two balance
-  // where the tracks go with sqrt(entries / waves): tracks are halved from 128
-  // while 80 entries / waves stays under their square (calls of 8,192 rows x 64
-  // channels into 512^2, 11,000 entries: 128 tracks 383 us, 16 tracks 169; 20,000
-  // x 256 ch into 8 planes of 2048^2, 243,000: 776, 64 tracks 727, 16 tracks 956;
-  // from 650,000 entries 128 is the fastest).  Passes with a beam keep 128: its
-  // samples add equal terms, whose FP32 rounding does not average out (3e-4 of
-  // the peak where a cell takes 12,000), so that its sums would move with the
-  // grouping.
-  const long long waves = (long long)gs->nCU * gs->tapsPerCU * 4;
-  gs->chunk = kChunk;
-  if (!gs->anyBeam)
-    while (gs->chunk > kMinChunk && 80 * total < waves * gs->chunk * gs->chunk) gs->chunk /= 2;
-  int logChunk = 0;
-  while ((1 << logChunk) < gs->chunk) ++logChunk;
-  gs->fullItems = total / gs->chunk;
+  gs->fullItems = total / kChunk;
   gs->itemBound = std::min(total, nl + gs->fullItems + 1);
   if (gs->itemBound > gs->itemCap) {
     (void)hipFree(gs->d_items);
@@ -1888,7 +1869,7 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
                        gs->d_lend);
     OBIT_HIP_TRY(hipGetLastError());
     const auto chunks = rocprim::make_transform_iterator(rocprim::counting_iterator<long long>(0),
-                                                         ToChunks{gs->d_offsets, gs->d_lend, logChunk});
+                                                         ToChunks{gs->d_offsets, gs->d_lend});
     size_t need = 0;
     OBIT_HIP_TRY(rocprim::exclusive_scan(nullptr, need, chunks, gs->d_itemOff, 0LL, (size_t)nl + 1,
                                          rocprim::plus<long long>(), gs->stream));
@@ -1896,7 +1877,7 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     OBIT_HIP_TRY(rocprim::exclusive_scan(gs->d_scanTmp, need, chunks, gs->d_itemOff, 0LL, (size_t)nl + 1,
                                          rocprim::plus<long long>(), gs->stream));
     const int nbI = (int)std::min<long long>((nl + 255) / 256, (long long)gs->nCU * 16);
-    hipLaunchKernelGGL(k_items, dim3(nbI), dim3(256), 0, gs->stream, gs->d_offsets, gs->d_lend, logChunk,
+    hipLaunchKernelGGL(k_items, dim3(nbI), dim3(256), 0, gs->stream, gs->d_offsets, gs->d_lend,
                        gs->d_itemOff, nl, gs->d_items);
     OBIT_HIP_TRY(hipGetLastError());
     OBIT_HIP_TRY(hipMemcpyAsync(gs->h_tot + 1, gs->d_itemOff + nl, sizeof(long long), hipMemcpyDeviceToHost,
@@ -1932,12 +1913,12 @@ int launch_taps(GpuState *gs, const float *vis, long long nrow) {
     if (wide)
       hipLaunchKernelGGL((k_grid_taps<16, 8>), dim3((unsigned)nbG), dim3(64 * 16), 0, gs->stream, vis, gs->d_rot,
                          nrow, gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items,
-                         gs->d_itemOff + gs->nlist, gs->chunk, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
+                         gs->d_itemOff + gs->nlist, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
                          gs->d_next, gs->d_walk);
     else
       hipLaunchKernelGGL((k_grid_taps<4, 16>), dim3((unsigned)nbG), dim3(64 * 4), 0, gs->stream, vis, gs->d_rot,
                          nrow, gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items,
-                         gs->d_itemOff + gs->nlist, gs->chunk, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
+                         gs->d_itemOff + gs->nlist, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
                          gs->d_next, gs->d_walk);
     OBIT_HIP_TRY(hipGetLastError());
   }
@@ -2447,7 +2428,7 @@ int ObitHIPGridListStats(CUDAGridInfo *in, long iGPU, long long *stats) {
     if (c > 0) ++nonEmpty;
     entries += c;
     if (c > maxc) maxc = c;
-    if (c > gs->chunk) ++multi;
+    if (c > obit::grid::kChunk) ++multi;
   }
   stats[0] = gs->nlist;
   stats[1] = nonEmpty;

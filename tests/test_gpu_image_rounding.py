@@ -1,7 +1,8 @@
 """Images at the scale of their gridding correction, which magnifies FP32
 rounding by up to 5e4 in the corners, against recorded pixels of the same
-images: another order of a transform's radices moves corner pixels by 1e-3 of
-the images' rms while every test on the uncorrected scale passes."""
+images: regrouped sums of samples or another order of a transform's radices
+move corner pixels by 1e-3 to 1e-2 of the images' rms while every test on the
+uncorrected scale passes."""
 import os
 
 import numpy as np
@@ -13,11 +14,13 @@ pytestmark = pytest.mark.gpu
 
 GOLDEN = os.path.join(os.path.dirname(__file__), "golden", "image_rounding.npz")
 # (side, rows, planes, facets, beam): few rows, whose planes differ between two
-# passes in a few cells at most
+# passes in a few cells at most, and passes of lists of up to 183 tracks
 CASES = {
     "few_1024": (1024, 29, 3, 1, False),
     "few_2048": (2048, 29, 3, 1, False),
     "few_2048_beam": (2048, 29, 3, 1, True),
+    "lists_1200": (1200, 3000, 1, 2, False),
+    "lists_512": (512, 1000, 1, 1, False),
 }
 
 
@@ -50,3 +53,19 @@ def test_recorded_pixels(name):
     # four times what two passes differed by, in the order of their device
     # atomics, and at least 4e-4
     assert d.max() <= 4 * float(g[name + "_own"])
+
+
+@pytest.mark.parametrize("rows", [27, 351, 1000])
+def test_items_of_128_tracks(rows):
+    """A list of up to 128 tracks is one work item, whose sums have one order."""
+    import ctypes as C
+    from obit_amd import _lib
+    from obit_amd.gridder import GPUGrid
+    uv, _, _ = synth.workload(4, rows=rows)
+    with GPUGrid(uv, synth.make_facets(1, 1024, 0.4 / 3600.0, 0.0), nVisPIO=rows) as gg:
+        gg.grid(uv.buffer)
+        st = (C.c_longlong * 8)()
+        _lib.check(gg.lib.ObitHIPGridListStats(gg.c, 0, st))
+    print(f"lists {st[1]}, entries {st[2]}, items {st[3]}, longest {st[4]}, split {st[5]}", flush=True)
+    assert st[4] <= 128
+    assert st[5] == 0 and st[3] == st[1]
