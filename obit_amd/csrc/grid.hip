@@ -245,19 +245,16 @@ __device__ Sample prep_sample(const FacetDev &f, const Common &cm, const float *
 
 // ---------------- binning ----------------
 
-constexpr int kParts = 8;        // counters of work items, one an XCD,
-constexpr int kNextStride = 32;  // 128 bytes apart
 constexpr int kHashParts = 16;   // partial sums of the uvw checksum,
 constexpr int kHashStride = 16;  // 128 bytes apart
 
 // Everything a pass starts from zero, in one launch (a kernel, kept out of
 // memset nodes so the sequence stays capturable in a hipGraph): the walk
-// statistics and the counters of work items, the count after the last track,
-// the uvw checksum and the lists' first and last entries.
-__global__ void k_pass_clear(unsigned long long *walk, unsigned *next, unsigned *lastCount, unsigned long long *hash,
+// statistics, the count after the last track, the uvw checksum and the lists'
+// first and last entries.
+__global__ void k_pass_clear(unsigned long long *walk, unsigned *lastCount, unsigned long long *hash,
                              long long *first, long long *last, long long n) {
   const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i0 < kParts) next[kNextStride * i0] = 0;
   if (i0 < kHashParts) hash[kHashStride * i0] = 0;
   if (i0 == 0) {
     walk[0] = walk[1] = 0;
@@ -382,10 +379,9 @@ __device__ __forceinline__ BinTrack bin_track(long long it, int nf, int nsplit, 
 }
 
 // Binning, pass 1: the number of (plane, tile) entries of every thread's track;
-// the first thread of a (row, facet) keeps its rotated uvw for the gridding, that
-// of a row adds it to the uvw checksum.
+// the first thread of a row adds it to the uvw checksum.
 __global__ __launch_bounds__(256) void k_bin_count(const float *vis, long long nrow, const FacetDev *facets, int nf, int nsplit, Common cm,
-                            unsigned *cnt, float4 *rot, unsigned long long *hash) {
+                            unsigned *cnt, unsigned long long *hash) {
   const long long total = nrow * (long long)nf * nsplit;
   unsigned long long h = 0;
   for (long long it = (long long)blockIdx.x * blockDim.x + threadIdx.x; it < total;
@@ -398,7 +394,6 @@ __global__ __launch_bounds__(256) void k_bin_count(const float *vis, long long n
     unsigned n = 0;
     track_tiles(f, cm, uu, vv, b.p0, b.p1, [&](long long, unsigned, int, int) { ++n; });
     cnt[it] = n;
-    if (b.p0 == 0) rot[b.fi * nrow + b.r] = signed_uvw(uu, vv, ww);
     if (b.fi == 0 && b.p0 == 0) h += row_hash(row, b.r);
   }
   add_hash(h, hash);
@@ -496,6 +491,7 @@ constexpr int kW = 7;          // GCF support in cells (checked on the host)
 // pixels of an image's corners by up to 1e-2 of its rms, where the gridding
 // correction magnifies them by 5e4: one length for every pass.
 constexpr int kLogChunk = 7, kChunk = 1 << kLogChunk;
+constexpr int kWaves = 4;      // waves per workgroup, each with a private tile
 // A sample's footprint is accumulated through a 16 (u) x 8 (v) window of
 // cells whose origin is its base cell rounded down to a multiple of 8 in u
 // and of 2 in v, so a window serves the 8x2 base cells of an aligned
@@ -510,8 +506,7 @@ constexpr int kTC = TU + kWinU - kBlkU;            // tile columns with the halo
 constexpr int kPlane = ((kTR * kS + 31) / 64) * 64 + 32;  // floats per re / im plane
 constexpr int kHalf = 64;      // kept samples staged at a time (one pass)
 constexpr int kGrp = kHalf / 4;  // 4-sample groups of a pass (K of one matrix step)
-constexpr int kGcfRow = 16;    // GCF row in LDS: 7 taps and the 9 zeros after them
-constexpr int kGcfLds = 101 * kGcfRow + 7;
+constexpr int kGcfRow = 24;    // padded GCF row: 7 zeros, 7 taps, 10 zeros
 static_assert(kBlkU + kW - 1 <= kWinU && kBlkV + kW - 1 <= kWinV, "the window holds every footprint");
 static_assert(TU % kBlkU == 0 && TV % kBlkV == 0, "windows are aligned within the tile");
 static_assert(kS >= kTC && (4 * kS) % 64 == 48, "tile stride: room for the halo, 4 rows = 48 banks");
@@ -562,33 +557,23 @@ __device__ __forceinline__ float keep_lanes(float a, unsigned long long m) {
 // grid with plain stores when the item is the tile's whole list; the
 // halo, and every cell of an item of a longer list, add with device
 // atomics.
-//
-// What bounds it is the issue of its 400 vector instructions a pass and 20 matrix
-// steps, which exclude each other on a SIMD where they are FP32 (34 cycles each).
-// kWaves waves, each with its own tile, share a workgroup and its table; kGather
-// groups are gathered together.  4 and 16: 3 waves a SIMD; 16 and 8: the one
-// table leaves LDS for 4, in 128 registers (launch_taps).
-template <int kWaves, int kGather>
-__global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, const float4 *rot, long long nrow,
-                                                           const FacetDev *facets,
+__global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, const FacetDev *facets,
                                                            const int *listFacet, const int2 *items,
                                                            const long long *nitemsPtr, Common cm,
                                                            const long long *offsets, const long long *lend,
-                                                           const int2 *lists, unsigned *next,
+                                                           const int2 *lists,
                                                            unsigned long long *stats) {
   __shared__ float4 s_tile4[kWaves][2 * kPlane / 4];  // re plane, then im plane
+  __shared__ int2 s_si[kWaves][kHalf];      // staged sample: u and v tap-row offsets in s_gcfp
   __shared__ float2 s_sv[kWaves][kHalf];    // staged sample: weighted visibility
-  // staged sample: u and v tap-row byte offsets in s_gcfp (u | v << 16); before that
-  // the kept samples' windows, and before that the entry starts of a window of
-  // slots, each read before the next is written
-  __shared__ int s_si[kWaves][kHalf];
-  // GCF rows: 7 zeros, then for each fractional offset its 7 taps and 9 zeros, so
-  // that any window column or row (up to 7 before and 15 after a row's start less
-  // 7) reads its tap or a zero with no test
-  __shared__ float s_gcfp[kGcfLds];
-  for (int i = threadIdx.x; i < kGcfLds; i += blockDim.x) {
-    const int it = (i - 7) >> 4, j = (i - 7) & 15;  // kGcfRow = 16
-    s_gcfp[i] = (i >= 7 && j < kW) ? cm.gcf[8 * it + j] : 0.0f;
+  __shared__ int s_cell[kWaves][64];
+  __shared__ int s_flag[kWaves][64];        // entry starts within a window of slots
+  // padded GCF rows: 7 zeros, the 7 taps of fractional offset it, 10 zeros,
+  // so every window column or row reads its tap (or a zero) with no test
+  __shared__ float s_gcfp[101 * kGcfRow];
+  for (int i = threadIdx.x; i < 101 * kGcfRow; i += blockDim.x) {
+    const int it = i / kGcfRow, j = i - it * kGcfRow - 7;
+    s_gcfp[i] = (j >= 0 && j < kW) ? cm.gcf[8 * it + j] : 0.0f;
   }
   __syncthreads();
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -597,32 +582,21 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
   typedef float f4 __attribute__((ext_vector_type(4)));
   const int mk = lane >> 4, mm = lane & 15;
   const int laneOff = (mk >> 1) * kPlane + 4 * (mk & 1) * kS + mm;
-  // byte offsets of this lane's column and row in the taps, one in each half
-  const char *gcf = reinterpret_cast<const char *>(s_gcfp);
-  const unsigned lanePos = 4 * mm | (4 * (mm & 7)) << 16;
+  const float *gcf = s_gcfp;
+  const int mm7 = mm & 7;
   float *re = reinterpret_cast<float *>(s_tile4[wv]);
   float *im = re + kPlane;
-  int *si = s_si[wv];
+  int2 *si = s_si[wv];
   float2 *sv = s_sv[wv];
   // this lane's part of a staged visibility: sample mk of a group, real
   // part for window rows (mm < 8), imaginary for the rest
   const float *svl = reinterpret_cast<const float *>(sv) + 2 * mk + (mm >= 8 ? 1 : 0);
-  int *scell = si, *flag = si;
+  int *scell = s_cell[wv];
+  int *flag = s_flag[wv];
   const long long nitems = *nitemsPtr;
-  // Each wave starts with the item of its number; the others are taken as waves
-  // get free, the next one's number fetched while an item is gridded.  Items
-  // differ in samples: dealt out in turn they left the last wave 20 % behind the
-  // mean after 88 rounds (the pass of 105,300 rows x 256 channels into 20 facets
-  // x 8 planes of 2048^2 13.35 ms, so 11.56).  One counter costs 10 ns an item
-  // whatever the waves (12.36 ms, and 30 us more on a pass of 400); so every XCD
-  // has its own, for each eighth of the items.
-  const unsigned parts = min((unsigned)kParts, gridDim.x), part = blockIdx.x % parts;
-  const long long nwaves = (long long)gridDim.x * kWaves;
-  unsigned taken = 0;
-  for (long long w = (long long)wv * gridDim.x + blockIdx.x; w < nitems;
-       w = nwaves + (long long)(unsigned)__builtin_amdgcn_readfirstlane((int)taken) * parts + part) {
+  for (long long w = (long long)blockIdx.x * kWaves + wv; w < nitems;
+       w += (long long)gridDim.x * kWaves) {
     const int2 item = items[w];
-    if (lane == 0) taken = atomicAdd(next + kNextStride * part, 1u);
     const long long L = __builtin_amdgcn_readfirstlane(item.x);
     const long long l0 = offsets[L];
     const int n = (int)(lend[L] - l0);
@@ -704,40 +678,25 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const int mine = flag[lane];
-      const unsigned long long starts = __ballot(mine != 0);
-      const int c = (int)__popcll(starts);
-      // the starts at or before this lane's slot
-      const int k = min((int)__builtin_amdgcn_mbcnt_hi((unsigned)(starts >> 32),
-                                                       __builtin_amdgcn_mbcnt_lo((unsigned)starts, jA)) + mine,
-                        ne - 1);
-      int bs;
-      if (jA + c < 64) {  // every entry of the window in the lanes' first ones
-        row = __shfl(rowA, k);
-        bs = __shfl(baseA, k);
-      } else if (jA >= 64) {
-        row = __shfl(rowB, k & 63);
-        bs = __shfl(baseB, k & 63);
-      } else {
-        const int ra = __shfl(rowA, k & 63), rb2 = __shfl(rowB, k & 63);
-        const int ba = __shfl(baseA, k & 63), bb = __shfl(baseB, k & 63);
-        row = k < 64 ? ra : rb2;
-        bs = k < 64 ? ba : bb;
-      }
-      ci = min(bs + S + lane, npc - 1);
+      const unsigned long long starts = __ballot(flag[lane] != 0);
+      const int k = min(jA + (int)__popcll(starts & (~0ull >> (63 - lane))), ne - 1);
+      const int ra = __shfl(rowA, k & 63), rb2 = __shfl(rowB, k & 63);
+      const int ba = __shfl(baseA, k & 63), bb = __shfl(baseB, k & 63);
+      row = k < 64 ? ra : rb2;
+      ci = min((k < 64 ? ba : bb) + S + lane, npc - 1);
       live = S + lane < nslot;
       // the entry holding slot S + 64: one more if an entry starts there
+      const int c = (int)__popcll(starts);
       jA += c + (__builtin_amdgcn_readlane(pos, c) == 64 ? 1 : 0);
     };
-    const float4 *rotf = rot + fi * nrow;
-    float4 xq;
-    float xre, xim, xwt, xfs;
+    float xu, xv, xw, xre, xim, xwt, xfs;
     int xch;
     auto fetch = [&](int r, int ch) {
+      const float *row = vis + (long long)r * cm.lenvis;
       xch = ch;
       xfs = cm.freq[ch];
-      xq = rotf[r];
-      const float *x = vis + (long long)r * cm.lenvis + cm.nrparm + 3 * ch;
+      xu = row[0]; xv = row[1]; xw = row[2];
+      const float *x = row + cm.nrparm + 3 * ch;
       xre = x[0]; xim = x[1]; xwt = x[2];
     };
     // the row and channel of a slot are read two passes ahead and its data
@@ -754,8 +713,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
     const int npass = (nslot + 63) / 64;
     for (int pass = 0; pass < npass; ++pass) {
       const bool live = liveCur;
-      const float4 q0 = xq;
-      const float re0 = xre, im0 = xim, wt0 = xwt, fs0 = xfs;
+      const float u0 = xu, v0 = xv, w0 = xw, re0 = xre, im0 = xim, wt0 = xwt, fs0 = xfs;
       const int ch0 = xch;
       // the slot after next: its row and channel; then the next pass's data
       int rc, cic;
@@ -766,9 +724,11 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       bool keep = false;
       Sample sm;
       if (live) {
-        sm = prep_vals(f, cm, q0, ch0, fs0, re0, im0, wt0);
-        keep = (sm.vr != 0.0f || sm.vi != 0.0f) && (unsigned)(sm.iu - col0) < (unsigned)TU &&
-               (unsigned)(sm.iv - row0) < (unsigned)TV;
+        float uu, vv, ww;
+        rotate3(f, u0, v0, w0, uu, vv, ww);
+        sm = prep_vals(f, cm, signed_uvw(uu, vv, ww), ch0, fs0, re0, im0, wt0);
+        keep = (sm.vr != 0.0f || sm.vi != 0.0f) && sm.iu >= col0 && sm.iu < col0 + TU &&
+               sm.iv >= row0 && sm.iv < row0 + TV;
       }
       liveCur = liveNext; liveNext = liveC; rb = rc; chb = chc;
       const unsigned long long mask = __ballot(keep);
@@ -794,48 +754,43 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       // the GCF table and walk the groups.
       if (keep) {
         const int cu = sm.iu - col0, cv = sm.iv - row0;
-        si[pos] = 4 * (kGcfRow * sm.itu + 7 - (cu & (kBlkU - 1))) |
-                  (4 * (kGcfRow * sm.itv + 7 - (cv & (kBlkV - 1)))) << 16;
+        si[pos] = make_int2(kGcfRow * sm.itu + 7 - (cu & (kBlkU - 1)), kGcfRow * sm.itv + 7 - (cv & (kBlkV - 1)));
         sv[pos] = make_float2(sm.vr, sm.vi);
       }
       if (lane >= nv) {
-        si[lane] = 0;  // any tap row: the visibility is zero
+        si[lane] = make_int2(0, 0);  // any tap row: the visibility is zero
         sv[lane] = make_float2(0.0f, 0.0f);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      float A[kGrp], B[kGrp];
 #pragma unroll
-      for (int h = 0; h < kGrp; h += kGather) {
-        if (h && 4 * h >= nv) break;
-        float A[kGather], B[kGather];
+      for (int g = 0; g < kGrp; ++g) {
+        const int2 q = si[4 * g + mk];
+        B[g] = gcf[q.x + mm];
+        A[g] = gcf[q.y + mm7] * svl[8 * g];
+      }
 #pragma unroll
-        for (int g = 0; g < kGather; ++g) {
-          const unsigned q = (unsigned)si[4 * (h + g) + mk] + lanePos;
-          B[g] = *reinterpret_cast<const float *>(gcf + (q & 0xFFFFu));
-          A[g] = *reinterpret_cast<const float *>(gcf + (q >> 16)) * svl[8 * (h + g)];
-        }
-#pragma unroll
-        for (int g = 0; g < kGather; ++g) {
-          if (4 * (h + g) >= nv) break;
-          unsigned mg = (unsigned)(moves >> (4 * (h + g))) & 15u;  // moves at the group's samples
-          int s0 = 0;
-          while (mg) {
-            const int p1 = __builtin_ctz(mg);
-            if (p1 > s0) {
-              // samples s0 .. p1 - 1 of the group (p1 <= 3)
-              const unsigned long long m = (~0ull << (16 * s0)) ^ (~0ull << (16 * p1));
-              acc = __builtin_amdgcn_mfma_f32_16x16x4f32(keep_lanes(A[g], m), B[g], acc, 0, 0, 0);
-            }
-            handover();
-            cur = __builtin_amdgcn_readlane(cellq, 4 * (h + g) + p1);
-            acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
-            s0 = p1;
-            mg &= mg - 1;
+      for (int g = 0; g < kGrp; ++g) {
+        if (4 * g >= nv) break;
+        unsigned mg = (unsigned)(moves >> (4 * g)) & 15u;  // moves at the group's samples
+        int s0 = 0;
+        while (mg) {
+          const int p1 = __builtin_ctz(mg);
+          if (p1 > s0) {
+            // samples s0 .. p1 - 1 of the group (p1 <= 3)
+            const unsigned long long m = (~0ull << (16 * s0)) ^ (~0ull << (16 * p1));
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(keep_lanes(A[g], m), B[g], acc, 0, 0, 0);
           }
-          // samples s0 .. 3 of the group
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(keep_lanes(A[g], ~0ull << (16 * s0)), B[g], acc, 0, 0, 0);
+          handover();
+          cur = __builtin_amdgcn_readlane(cellq, 4 * g + p1);
+          acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
+          s0 = p1;
+          mg &= mg - 1;
         }
+        // samples s0 .. 3 of the group
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(keep_lanes(A[g], ~0ull << (16 * s0)), B[g], acc, 0, 0, 0);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -862,8 +817,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, con
       float *q = g + (size_t)gr * f.lrow + 2 * gc;
       // the windows of the tiles to the left and above reach kWin - kBlk
       // cells into this one
-      const bool inner = !multi && rr >= kWinV - kBlkV && rr < TV && cc >= kWinU - kBlkU && cc < TU;
-      if (inner) {
+      const bool own = !multi && rr >= kWinV - kBlkV && rr < TV && cc >= kWinU - kBlkU && cc < TU;
+      if (own) {
         q[0] += vr;
         q[1] += vi;
       } else {
@@ -1394,7 +1349,7 @@ struct GpuState {
   hipStream_t stream = nullptr;
   int nCU = 256;
   int rowsPerCU = 0, rowsPerCU1024 = 0;  // resident k_fft_rows_c2r blocks per CU (0: not queried yet)
-  int tapsPerCU = 0;        // resident k_grid_taps<4, 16> blocks per CU (0: not queried yet)
+  int tapsPerCU = 0;        // resident k_grid_taps blocks per CU (0: not queried yet)
   std::vector<int> facets;  // facet indices on this GPU
   FacetDev *d_facets = nullptr;  // in d_tab
   std::vector<FacetDev> h_facets;
@@ -1407,8 +1362,6 @@ struct GpuState {
   unsigned *d_tcnt = nullptr;      // entries per (row, facet) track
   unsigned long long *d_toff = nullptr;  // their exclusive scan
   long long tcap = 0;
-  float4 *d_rot = nullptr;         // rotated uvw [facet][row] of the last pass (signed_uvw)
-  long long rotCap = 0;
   unsigned *d_keys = nullptr, *d_keys2 = nullptr;  // sort keys, in and out
   int2 *d_rows = nullptr;          // (row, channel range) before the sort (d_lists after it)
   int2 *d_items = nullptr;
@@ -1417,13 +1370,11 @@ struct GpuState {
   void *d_scanTmp = nullptr;       // scan scratch
   size_t scanTmpBytes = 0;
   long long *h_tot = nullptr;      // pinned: list entries and work items of the last pass, checksums to compare
-  // work items of the last pass; at most this many; that many if all were full
-  long long nitems = 0, itemBound = 0, fullItems = 0;
+  long long nitems = 0, itemBound = 0;  // work items of the last pass; at most this many
   bool listsValid = false;         // the lists of the last pass, for ...
   long long listsRows = 0;         // ... a pass over as many rows ...
   unsigned long long *d_hash = nullptr;  // ... with the same uvw: their checksum, and another pass's
   unsigned long long *d_walk = nullptr;  // staged samples, base-cell moves of the last pass
-  unsigned *d_next = nullptr;            // its counters of work items
   // FFT to images: C2R plan for (nx, ny, nplane), complex scratch, corrections
   hipfftHandle fftPlan = 0;
   int fftNx = 0, fftNy = 0, fftNplane = 0, fftPitch = 0, fftDist = 0;
@@ -1719,7 +1670,7 @@ __global__ __launch_bounds__(256) void k_items(const long long *first, const lon
   }
 }
 
-int launch_taps(GpuState *gs, const float *vis, long long nrow);
+int launch_taps(GpuState *gs, const float *vis);
 
 // Scan / sort scratch of at least need bytes.
 hipError_t ensure_tmp(GpuState *gs, size_t need) {
@@ -1750,7 +1701,7 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   if (reuse) {
     // the rows' checksum beside the lists'; the lists, offsets and work items of
     // the last pass stand: only the walk statistics restart
-    hipLaunchKernelGGL(k_pass_clear, dim3(1), dim3(64), 0, gs->stream, gs->d_walk, gs->d_next,
+    hipLaunchKernelGGL(k_pass_clear, dim3(1), dim3(64), 0, gs->stream, gs->d_walk,
                        (unsigned *)nullptr, gs->d_hash + kHashParts * kHashStride, (long long *)nullptr, (long long *)nullptr, 0LL);
     const int nb = (int)std::min<long long>((nrow + 255) / 256, (long long)gs->nCU * 4);
     hipLaunchKernelGGL(k_uvw_hash, dim3(std::max(nb, 1)), dim3(256), 0, gs->stream, vis, nrow, gs->cm.lenvis,
@@ -1767,16 +1718,10 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     }
     if (lists != rows)
       return fail(kState, "cannot reuse the track lists: these rows' u, v, w differ from the last pass's");
-    return launch_taps(gs, vis, nrow);
+    return launch_taps(gs, vis);
   }
   if (!gs->d_walk) OBIT_HIP_TRY(hipMalloc(&gs->d_walk, 2 * sizeof(unsigned long long)));
-  if (!gs->d_next) OBIT_HIP_TRY(hipMalloc(&gs->d_next, kParts * kNextStride * sizeof(unsigned)));
   if (!gs->d_hash) OBIT_HIP_TRY(hipMalloc(&gs->d_hash, 2 * kHashParts * kHashStride * sizeof(unsigned long long)));
-  if (gs->tapsPerCU <= 0) {
-    int nb = 0;
-    OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_grid_taps<4, 16>, 64 * 4, 0));
-    gs->tapsPerCU = std::max(nb, 1);
-  }
   gs->listsValid = false;
   if ((long long)nrow * gs->cm.nplane * nf > (1LL << 40)) return fail(kInvalid, "too many tracks");
   // Threads of the binning: one per (row, facet), or where those fill less than 4
@@ -1795,21 +1740,14 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     OBIT_HIP_TRY(hipMalloc(&gs->d_toff, sizeof(unsigned long long) * (size_t)(ntr + 1)));
     gs->tcap = ntr + 1;
   }
-  if (nrf > gs->rotCap) {
-    (void)hipFree(gs->d_rot);
-    gs->d_rot = nullptr;
-    gs->rotCap = 0;
-    OBIT_HIP_TRY(hipMalloc(&gs->d_rot, sizeof(float4) * (size_t)nrf));
-    gs->rotCap = nrf;
-  }
   const int nbB = (int)std::min<long long>((ntr + 255) / 256, (long long)gs->nCU * 32);
   // pass 1: entries per track; the slot after the last track is zero so
   // the scan's last element is the total
   const int nbz = (int)std::min<long long>((nl + 1 + 255) / 256, (long long)gs->nCU * 16);
-  hipLaunchKernelGGL(k_pass_clear, dim3(nbz), dim3(256), 0, gs->stream, gs->d_walk, gs->d_next, gs->d_tcnt + ntr,
+  hipLaunchKernelGGL(k_pass_clear, dim3(nbz), dim3(256), 0, gs->stream, gs->d_walk, gs->d_tcnt + ntr,
                      gs->d_hash, gs->d_offsets, gs->d_lend, nl + 1);
   hipLaunchKernelGGL(k_bin_count, dim3(nbB), dim3(256), 0, gs->stream, vis, nrow, gs->d_facets, nf, nsplit,
-                     gs->cm, gs->d_tcnt, gs->d_rot, gs->d_hash);
+                     gs->cm, gs->d_tcnt, gs->d_hash);
   OBIT_HIP_TRY(hipGetLastError());
   {
     size_t need = 0;
@@ -1851,8 +1789,7 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
     OBIT_HIP_TRY(rocprim::radix_sort_pairs<SortConfig>(gs->d_scanTmp, need, gs->d_keys, gs->d_keys2, gs->d_rows,
                                            gs->d_lists, (size_t)total, 0, endBit, gs->stream));
   }
-  gs->fullItems = total / kChunk;
-  gs->itemBound = std::min(total, nl + gs->fullItems + 1);
+  gs->itemBound = std::min(total, nl + total / kChunk + 1);
   if (gs->itemBound > gs->itemCap) {
     (void)hipFree(gs->d_items);
     gs->d_items = nullptr;
@@ -1885,7 +1822,7 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
   } else {
     gs->h_tot[1] = 0;
   }
-  int rc = launch_taps(gs, vis, nrow);  // the pass is complete when it returns
+  int rc = launch_taps(gs, vis);  // the pass is complete when it returns
   if (rc) return rc;
   gs->nitems = gs->h_tot[1];
   if (gs->nitems < 0 || gs->nitems > gs->itemBound)
@@ -1897,29 +1834,28 @@ int grid_device(GpuState *gs, const float *vis, long long nrow, bool reuse) {
 
 // The tile-gridding launch over the current work items; the pass is
 // complete when it returns.
-int launch_taps(GpuState *gs, const float *vis, long long nrow) {
+int launch_taps(GpuState *gs, const float *vis) {
   if (gs->itemBound) {
     // persistent grid of exactly the resident blocks: more would queue a
     // second round of blocks behind the first and idle CUs at the end
     //
-    // 16 waves a workgroup, 4 a SIMD, from 16 items a wave up (105,300 rows x 256
-    // channels into 20 facets x 8 planes of 2048^2, 66 items a wave: 11.50 -> 10.83
-    // ms).  Below, where the time is that of a wave's last items, 4 waves a
-    // workgroup with their longer gathers are as fast (60,000 x 256 into 2 facets,
-    // 4 items a wave: 1.12 ms both) or faster (60,000 x 64 into a 512^2 beam, less
-    // than one: 427 us against 457).
-    const bool wide = gs->fullItems >= 16LL * 16 * gs->nCU;
-    const long long nbG = std::min<long long>(gs->itemBound, (long long)gs->nCU * (wide ? 1 : gs->tapsPerCU));
-    if (wide)
-      hipLaunchKernelGGL((k_grid_taps<16, 8>), dim3((unsigned)nbG), dim3(64 * 16), 0, gs->stream, vis, gs->d_rot,
-                         nrow, gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items,
-                         gs->d_itemOff + gs->nlist, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
-                         gs->d_next, gs->d_walk);
-    else
-      hipLaunchKernelGGL((k_grid_taps<4, 16>), dim3((unsigned)nbG), dim3(64 * 4), 0, gs->stream, vis, gs->d_rot,
-                         nrow, gs->d_facets, gs->d_listFacet, (const int2 *)gs->d_items,
-                         gs->d_itemOff + gs->nlist, gs->cm, gs->d_offsets, gs->d_lend, gs->d_lists,
-                         gs->d_next, gs->d_walk);
+    // The items are dealt out in turn, so the adds of neighbouring and split
+    // tiles, which end in the order of their items' lengths, come in much the same
+    // order in every pass.  Items taken from counters as waves get free, 16 waves a
+    // workgroup and shorter per-sample code take the whole call of 105,300 rows x
+    // 256 channels into 20 facets x 8 planes of 2048^2 from 17.5 to 13.8 ms, but
+    // order the adds anew: an image's corner pixels then move by 2 to 10 times
+    // what two passes differ by here (up to 1e-2 of its rms).
+    if (gs->tapsPerCU <= 0) {
+      int nb = 0;
+      OBIT_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_grid_taps, 64 * kWaves, 0));
+      gs->tapsPerCU = std::max(nb, 1);
+    }
+    const long long nbG =
+        std::min<long long>((gs->itemBound + kWaves - 1) / kWaves, (long long)gs->nCU * gs->tapsPerCU);
+    hipLaunchKernelGGL(k_grid_taps, dim3((unsigned)nbG), dim3(64 * kWaves), 0, gs->stream, vis, gs->d_facets,
+                       gs->d_listFacet, (const int2 *)gs->d_items, gs->d_itemOff + gs->nlist, gs->cm, gs->d_offsets,
+                       gs->d_lend, gs->d_lists, gs->d_walk);
     OBIT_HIP_TRY(hipGetLastError());
   }
   // the pass is complete when the call returns
@@ -2100,9 +2036,9 @@ void ObitCUDAGridShutdown(CUDAGridInfo *cudaInfo, long iGPU) {
     (void)hipFree(gs->d_tab); (void)hipFree(gs->d_listFacet);
     (void)hipFree(gs->d_lend); (void)hipFree(gs->d_offsets); (void)hipFree(gs->d_lists);
     (void)hipFree(gs->d_tcnt); (void)hipFree(gs->d_toff); (void)hipFree(gs->d_keys); (void)hipFree(gs->d_keys2);
-    (void)hipFree(gs->d_rows); (void)hipFree(gs->d_rot);
+    (void)hipFree(gs->d_rows);
     (void)hipFree(gs->d_items); (void)hipFree(gs->d_vis); (void)hipFree(gs->d_walk);
-    (void)hipFree(gs->d_hash); (void)hipFree(gs->d_next);
+    (void)hipFree(gs->d_hash);
     (void)hipFree(gs->d_itemOff); (void)hipFree(gs->d_scanTmp);
     if (gs->h_tot) (void)hipHostFree(gs->h_tot);
     if (gs->fftPlan) (void)hipfftDestroy(gs->fftPlan);
