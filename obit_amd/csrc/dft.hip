@@ -1289,7 +1289,8 @@ struct State {
   float *tab = nullptr;
   size_t tabCap = 0;
   bool tabReady = false;
-  long long tabKey = -1;
+  long long tabKey = -1;         // the selection and ...
+  std::vector<double> tabFreq;   // ... channel frequencies it was made for
   // the table's factors for k_dft_spec, if they reproduce it
   bool specMm = false;
   SpecTab spec{};
@@ -1516,18 +1517,19 @@ int spec_factors(State *st, int nIFsel, int nchsel, int nchpad, const std::vecto
   return kOK;
 }
 
-// Build (or reuse) the spectral amplitude table for the current selection.
-int ensure_spec_table(State *st, const GPUInfo *gi) {
+// Build (or reuse) the spectral amplitude table for the current selection and
+// its frequency lines (frequency_lines: the amplitudes and k_dft_spec's block
+// centres are formed from them).
+int ensure_spec_table(State *st, const GPUInfo *gi, const std::vector<double> &fb, const std::vector<double> &fdl,
+                      const std::vector<double> &fch) {
   const GPUVisInfo *vi = gi->h_visInfo;
   const GPUModelInfo *mi = gi->h_modelInfo;
   const int nchsel = vi->chane - vi->chanb + 1, nIFsel = vi->IFe - vi->IFb + 1;
   const int nchpad = (nchsel + 63) / 64 * 64;
   const long long key = ((long long)vi->chanb << 40) ^ ((long long)vi->chane << 28) ^
                         ((long long)vi->IFb << 16) ^ (long long)vi->IFe;
-  if (st->tabReady && st->tabKey == key) return kOK;
-  std::vector<double> fb, fdl, fch;
-  int rc = frequency_lines(st, vi, fb, fdl, &fch);
-  if (rc) return rc;
+  if (st->tabReady && st->tabKey == key && st->tabFreq == fch) return kOK;
+  st->tabReady = false;
   const bool tabulated = model_is_tab(st->type);
   const int coefOff = model_coef_off(st->type);
   if (!tabulated && coefOff + st->nterm > st->size)
@@ -1579,13 +1581,14 @@ int ensure_spec_table(State *st, const GPUInfo *gi) {
                        nIFsel, nchsel, nchpad, st->tab);
     OBIT_HIP_TRY(hipGetLastError());
   }
-  rc = spec_factors(st, nIFsel, nchsel, nchpad, fb, fdl, bin);
+  const int rc = spec_factors(st, nIFsel, nchsel, nchpad, fb, fdl, bin);
   if (rc) return rc;
   OBIT_HIP_TRY(hipStreamSynchronize(st->stream));
   OBIT_HIP_TRY(hipFree(dl));
   OBIT_HIP_TRY(hipFree(db));
   st->tabReady = true;
   st->tabKey = key;
+  st->tabFreq = fch;
   return kOK;
 }
 
@@ -1664,7 +1667,7 @@ int make_desc(State *st, const GPUInfo *gi, float *vis, long long nrow, int cpt,
   d.cx = st->cx; d.cy = st->cy; d.cz = st->cz;
   d.camp = st->camp; d.cg = st->cg;
   if (model_is_spec(st->type)) {
-    rc = ensure_spec_table(st, gi);
+    rc = ensure_spec_table(st, gi, fb, fdl, fch);
     if (rc) return rc;
     d.tab = st->tab;
     d.tab_nchpad = (d.nchsel + 63) / 64 * 64;

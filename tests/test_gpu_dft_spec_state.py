@@ -1,0 +1,75 @@
+"""The spectral matrix-core kernel (k_dft_spec) after what its tables were made
+from has changed: frequencies uploaded again.  Against a handle made for the new
+state, bit for bit, and against the FP64 oracle."""
+import ctypes as C
+import dataclasses
+
+import numpy as np
+import pytest
+
+from obit_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5  # of the model's peak: the split DFT's bound
+
+
+class _Head(C.Structure):
+    """The first fields of a GPUInfo."""
+    _fields_ = [("ints", C.c_int * 10), ("nmodel", C.c_int * 4), ("d_model", C.c_void_p * 4), ("d_freq", C.c_void_p)]
+
+
+def _uv(nif, nchan, rows, step=1e6, scale=1.0):
+    base, _, _ = synth.workload(1, rows=rows)
+    uv = synth.make_uv(base.buffer[:, :5], nif, nchan, 2, base.freq,
+                       synth.freq_table(base.freq, nif, nchan, step), np.random.default_rng(rows))
+    return dataclasses.replace(uv, freqArr=uv.freqArr * scale)
+
+
+def _sky(uv, ncomp, ref):
+    rng = np.random.default_rng(ncomp)
+    l, m = rng.uniform(-0.5, 0.5, (2, ncomp)) * synth.DG2RAD
+    flux = rng.exponential(0.01, ncomp)
+    flux[0] = 0.5
+    c = np.concatenate([synth.point_row(flux, l, m), rng.normal(-0.7, 0.3, (ncomp, 1))], axis=1)
+    return synth.SkyModel(comps=c.astype(np.float32), modType=10, nSpecTerm=1, imgRefFreq=float(ref))
+
+
+def _model(uv, rows):
+    d = rows[:, uv.nrparm:].reshape(uv.nrow, uv.nif, uv.nchan, uv.nstok, 3)
+    return d[..., 0, 0] + 1j * d[..., 0, 1]
+
+
+@pytest.mark.parametrize("path", ["resident", "buffer"])
+@pytest.mark.parametrize("step,scale", [(1e6, 1.01), (1.3e6, 1.0), (1e6, 0.9)])
+def test_frequencies_uploaded_again(oracle, path, step, scale):
+    from obit_amd import _lib
+    from obit_amd.skymodel import SkyModelDFT
+    rows = 100
+    a, b = _uv(1, 256, rows), _uv(1, 256, rows, step, scale)
+    sky = _sky(a, 200, a.freq)
+
+    def apply(sm):
+        if path == "buffer":
+            return sm.calc(a.buffer.copy())
+        sm.set_vis(a.buffer)
+        sm.set_variant(64, 64, 2)
+        sm.calc_resident()
+        return sm.get_vis()
+
+    with SkyModelDFT(a, sky, op="repl", useFreq64=False) as sm:
+        first = apply(sm)
+        fs = np.ascontiguousarray(b.fscale, dtype=np.float32)
+        h = C.cast(sm.g, C.POINTER(_Head)).contents
+        _lib.load().ObitCUDAUtilHost2GPU(h.d_freq, _lib.ptr(fs), fs.nbytes, None)
+        got = apply(sm)
+    with SkyModelDFT(b, sky, op="repl", useFreq64=False) as sm:
+        want = apply(sm)
+    c = np.arange(256.0)
+    fit = np.polyval(np.polyfit(c, b.fscale.astype(np.float64), 1), c)
+    ref = oracle.dft_model_fp64(b, sky, freq_ratio=fit)
+    peak = np.abs(ref).max()
+    e = [np.abs(_model(b, x) - ref).max() / peak for x in (first, got, want)]
+    print(f"of the peak: first table {e[0]:.2e}, uploaded again {e[1]:.2e}, a new handle {e[2]:.2e}", flush=True)
+    assert e[0] > 1e-3 and e[2] <= TOL
+    assert e[1] <= TOL and np.array_equal(got, want)
