@@ -1359,7 +1359,9 @@ int model_coef_off(int type) {
   }
 }
 
+// Drops the captured launch, its last replay ended.
 void destroy_graph(State *st) {
+  if (st->gexec) (void)hipStreamSynchronize(st->stream);
   if (st->gexec) { (void)hipGraphExecDestroy(st->gexec); st->gexec = nullptr; }
   if (st->graph) { (void)hipGraphDestroy(st->graph); st->graph = nullptr; }
   st->graphKey = 0;
@@ -1473,7 +1475,6 @@ int spec_factors(State *st, int nIFsel, int nchsel, int nchpad, const std::vecto
     for (size_t b = b0; b < b0 + n; ++b) blk[b].s = (float)(fdl[0] * (1.0 / blk[b].fc - 1.0 / f0));
   }
   if (blk.size() > st->sblkCap) {
-    destroy_graph(st);  // a captured launch reads the old blocks
     (void)hipFree(st->sblk);
     st->sblk = nullptr;
     st->sblkCap = 0;
@@ -1482,7 +1483,6 @@ int spec_factors(State *st, int nIFsel, int nchsel, int nchpad, const std::vecto
   }
   const size_t need = nA + npass * mm::kT * ncpad + npass * ncpad + npass;
   if (need > st->sbufCap) {
-    destroy_graph(st);
     (void)hipFree(st->sbuf);
     st->sbuf = nullptr;
     st->sbufCap = 0;
@@ -1530,6 +1530,9 @@ int ensure_spec_table(State *st, const GPUInfo *gi, const std::vector<double> &f
                         ((long long)vi->IFb << 16) ^ (long long)vi->IFe;
   if (st->tabReady && st->tabKey == key && st->tabFreq == fch) return kOK;
   st->tabReady = false;
+  // a captured launch reads the old table, or the factors' buffers with the old
+  // factors' scale and counts
+  destroy_graph(st);
   const bool tabulated = model_is_tab(st->type);
   const int coefOff = model_coef_off(st->type);
   if (!tabulated && coefOff + st->nterm > st->size)
@@ -1560,7 +1563,6 @@ int ensure_spec_table(State *st, const GPUInfo *gi, const std::vector<double> &f
   }
   const size_t need = (size_t)st->ncomp * nIFsel * nchpad;
   if (need > st->tabCap) {
-    destroy_graph(st);  // a captured launch reads the old table
     if (st->tab) OBIT_HIP_TRY(hipFree(st->tab));
     st->tab = nullptr;
     hipError_t e = hipMalloc(&st->tab, need * sizeof(float));
@@ -2520,6 +2522,7 @@ int ObitHIPSkyModelDFTSetSpecRef(GPUInfo *gpuInfo, const double *refFreq, int n)
   if (!refFreq || n <= 0) return obit::fail(obit::kInvalid, "bad reference frequencies");
   st->specRef.assign(refFreq, refFreq + n);
   st->tabReady = false;
+  obit::dft::destroy_graph(st);
   return obit::kOK;
 }
 

@@ -1,6 +1,7 @@
 """The spectral matrix-core kernel (k_dft_spec) after what its tables were made
-from has changed: frequencies uploaded again.  Against a handle made for the new
-state, bit for bit, and against the FP64 oracle."""
+from has changed: frequencies uploaded again, other reference frequencies under
+a captured graph.  Each against a handle made for the new state, bit for bit,
+and against the FP64 oracle."""
 import ctypes as C
 import dataclasses
 
@@ -73,3 +74,35 @@ def test_frequencies_uploaded_again(oracle, path, step, scale):
     print(f"of the peak: first table {e[0]:.2e}, uploaded again {e[1]:.2e}, a new handle {e[2]:.2e}", flush=True)
     assert e[0] > 1e-3 and e[2] <= TOL
     assert e[1] <= TOL and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("between", [True, False])
+@pytest.mark.parametrize("factor", [4.0, 0.1])
+def test_graph_after_new_reference(oracle, factor, between):
+    """A launch captured before the reference frequency changed is captured
+    again, whether or not another launch has made the table in between."""
+    from obit_amd import _lib
+    from obit_amd.skymodel import SkyModelDFT
+    uv = _uv(4, 64, 61)
+    sky = _sky(uv, 100, uv.freq)
+    new = dataclasses.replace(sky, imgRefFreq=sky.imgRefFreq * factor)
+    with SkyModelDFT(uv, new, op="repl") as sm:
+        sm.set_variant(64, 64, 2)
+        sm.set_vis(uv.buffer)
+        sm.calc_resident()
+        want = sm.get_vis()
+    with SkyModelDFT(uv, sky, op="repl") as sm:
+        sm.set_variant(64, 64, 2)
+        sm.set_vis(uv.buffer)
+        for _ in range(2):
+            sm.graph_launch()
+        sm.get_vis()
+        f = np.array([new.imgRefFreq])
+        _lib.check(sm.lib.ObitHIPSkyModelDFTSetSpecRef(sm.g, f.ctypes.data_as(C.POINTER(C.c_double)), 1))
+        if between:
+            sm.calc_resident()
+        for _ in range(2):
+            sm.graph_launch()
+            assert np.array_equal(sm.get_vis(), want)
+    ref = oracle.dft_model_fp64(uv, new)
+    assert np.abs(_model(uv, want) - ref).max() <= TOL * np.abs(ref).max()
