@@ -120,8 +120,8 @@ int ObitHIPSkyModelDFTGetVariant(GPUInfo *gpuInfo, int *cpt, int *tile, int *wgP
 int ObitHIPSkyModelDFTAutotune(GPUInfo *gpuInfo, long long sampleRows, int reps);
 /* Sin/cos policy: 0 hardware sin/cos for the centre phasor and the
  * per-channel step; 1 hardware for the centre phasor, Taylor polynomial
- * for the step (default); 2 polynomial for both.  The matrix-core kernel
- * reads its centre phasors P and its steps W, V the same way. */
+ * for the step (default); 2 polynomial for both.  The matrix-core kernels
+ * read their centre phasors P and their steps the same way. */
 int ObitHIPSkyModelDFTSetPrecision(GPUInfo *gpuInfo, int prec);
 /* hipStream_t on which the library launches for this gpuInfo. */
 void *ObitHIPSkyModelDFTStream(GPUInfo *gpuInfo);

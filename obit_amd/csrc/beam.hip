@@ -590,7 +590,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
     const unsigned *kap = AMP ? m.kap + (long long)ps * m.ncpad : nullptr;
     double o[2][NE][4];
     mm::f4 d2[2][NE];
-    mm::sum<AMP, NE, false>(s_op[wv], d.cx, d.cy, d.cz, d.ncomp, 0, d.ncomp, u, v, w, df, fc, po,
+    mm::sum<AMP, NE, false, 1>(s_op[wv], d.cx, d.cy, d.cz, d.ncomp, 0, d.ncomp, u, v, w, df, fc, po,
                             ONE ? (const void *)(reinterpret_cast<const float2 *>(prod) + h) : (const void *)prod,
                             ONE ? 2u : 1u, G, gstep, kap, o, d2);
     // lanes 0..31 hold the Re of slots c = 4 (lane / 16) + r of tile T, lane +

@@ -1001,6 +1001,7 @@ struct SpecTab {
   int shift;              // A is scaled by 2^shift
 };
 
+template <int PREC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_dft_spec(Desc d, SpecTab m) {
   __shared__ uint4 s_op[4][mm::kSlots];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1028,7 +1029,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const float *G = m.G + ((long long)ps * mm::kT + (h ? 8 : 7)) * m.ncpad;
     double o[2][1][4];
     mm::f4 d2[2][1];
-    mm::sum<true, 1, true>(s_op[wv], d.cx, d.cy, d.cz, d.ncomp, kBeg, kEnd, u, v, w, df, fc, po, m.Ab, 1u, G,
+    mm::sum<true, 1, true, PREC>(s_op[wv], d.cx, d.cy, d.cz, d.ncomp, kBeg, kEnd, u, v, w, df, fc, po, m.Ab, 1u, G,
                            h ? m.ncpad : -m.ncpad, m.kap + (long long)ps * m.ncpad, o, d2);
     const int n = lane & 15;
     const mm::Blk bk = m.blk[min(ps * mm::kPass + n, m.nblk - 1)];
@@ -1713,6 +1714,11 @@ MfmaFn mfma_fn(const State *st) {
   return st->prec == 0 ? k_dft_mfma<0> : st->prec == 2 ? k_dft_mfma<2> : k_dft_mfma<1>;
 }
 
+typedef void (*SpecFn)(Desc, SpecTab);
+SpecFn spec_fn(const State *st) {
+  return st->prec == 0 ? k_dft_spec<0> : st->prec == 2 ? k_dft_spec<2> : k_dft_spec<1>;
+}
+
 // Resident workgroups per CU of a kernel (cached).
 int occupancy_of(State *st, const void *fn) {
   auto it = st->occ.find(fn);
@@ -1745,8 +1751,9 @@ int launch_mfma(State *st, const Desc &d, hipStream_t stream) {
 
 int launch_spec(State *st, const Desc &d, hipStream_t stream) {
   const long long items = ((d.nrow + 3) / 4) * st->spec.npass * std::max(d.nsplit, 1);
-  const long long grid = std::min<long long>(items, (long long)st->nCU * occupancy_of(st, (const void *)k_dft_spec));
-  hipLaunchKernelGGL(k_dft_spec, dim3((unsigned)std::max<long long>(grid, 1)), dim3(kRows), 0,
+  SpecFn fn = spec_fn(st);
+  const long long grid = std::min<long long>(items, (long long)st->nCU * occupancy_of(st, (const void *)fn));
+  hipLaunchKernelGGL(fn, dim3((unsigned)std::max<long long>(grid, 1)), dim3(kRows), 0,
                      stream ? stream : st->stream, d, st->spec);
   OBIT_HIP_TRY(hipGetLastError());
   return kOK;
@@ -1865,7 +1872,7 @@ Choice choose(State *st, const Desc &d, bool matrix) {
   const double tShare = tItem * 0.27 * (cs == 16 ? 0.55 * rounds(blk * n16, 2) : rounds(blk * n32, 2));
   double tM = 1e300;
   const long long nquad = (d.nrow + 3) / 4, npass = (d.nIFsel * ((d.nchsel + 63) / 64) + 3) / 4;
-  if (spec) tM = 75.0 * rounds(nquad * st->spec.npass, occupancy_of(st, (const void *)k_dft_spec));
+  if (spec) tM = 75.0 * rounds(nquad * st->spec.npass, occupancy_of(st, (const void *)spec_fn(st)));
   else if (matrix && mfma_ok(st, d)) tM = 59.0 * npass * rounds(nquad, occupancy_of(st, (const void *)mfma_fn(st)));
   if (tM < tSplit && tM < tShare) return {Choice::matrix, 64, tM};
   if (tShare < tSplit) return {Choice::share, cs, tShare};
@@ -1959,7 +1966,7 @@ BufPlan plan_buffer(State *st, const Desc &d, size_t rowBytes) {
   const bool spec = spec_ok(st, d);
   if ((mfma_ok(st, d) && fill >= 0.6) || mixed || spec) {
     p.cpt = 64;
-    const void *fn = spec ? (const void *)k_dft_spec : (const void *)mfma_fn(st);
+    const void *fn = spec ? (const void *)spec_fn(st) : (const void *)mfma_fn(st);
     const long long slots = (long long)std::max(st->nCU, 1) * occupancy_of(st, fn);
     const int npass = spec ? st->spec.npass : 1;  // items of a row quad and part
     const long long nquad = (d.nrow + 3) / 4 * npass;
@@ -2592,7 +2599,7 @@ int ObitHIPSkyModelDFTGraphLaunch(GPUInfo *gpuInfo) {
     if (rc) return rc;
     OBIT_HIP_TRY(hipStreamSynchronize(st->stream));
     // the kernels' occupancies, asked for before the capture
-    (void)obit::dft::occupancy_of(st, (const void *)obit::dft::k_dft_spec);
+    (void)obit::dft::occupancy_of(st, (const void *)obit::dft::spec_fn(st));
     (void)obit::dft::occupancy_of(st, (const void *)obit::dft::mfma_fn(st));
     OBIT_HIP_TRY(hipStreamBeginCapture(st->stream, hipStreamCaptureModeThreadLocal));
     rc = st->uniform ? obit::dft::launch_resident(st, d, true)

@@ -191,10 +191,11 @@ static __global__ __launch_bounds__(64) void k_fit(const float *__restrict__ tab
 // component), REAL floats, or conj C as float2 in steps of pm (NE 1) or
 // float4 (NE 2), zero from ncomp to the end of the last tile.  AMP: G points at
 // the shape of slot 0 of the half (t = 0 or -1), gstep to the next slot's;
-// kap: (kappa, kappa) pairs.  o[T][e][r], d2: lanes 0..31 hold the real parts
+// kap: (kappa, kappa) pairs.  PREC: hardware sin / cos for P and the steps (0), for
+// P (1), for neither (2).  o[T][e][r], d2: lanes 0..31 hold the real parts
 // of slot c = 4 (lane / 16) + r of tile T (t = c, or -(c + 1) for T = 0), lanes 32
 // on the imaginary, of column lane mod 16 (half-wave, block).
-template <bool AMP, int NE, bool REAL>
+template <bool AMP, int NE, bool REAL, int PREC>
 __device__ __forceinline__ void sum(uint4 *lds, const double *__restrict__ cx, const double *__restrict__ cy,
                                     const double *__restrict__ cz, int ncomp, int kBeg, int kEnd, double u, double v,
                                     double w, double df, const double (&fc)[8], const unsigned (&po)[8],
@@ -258,7 +259,7 @@ __device__ __forceinline__ void sum(uint4 *lds, const double *__restrict__ cx, c
       const double psi = fma(w, nz, fma(v, ny, u * nx));
       fetch(k0 + kTile);
       {
-        const float2 s1 = eturn<false>(psi * wdf);
+        const float2 s1 = eturn<PREC == 0>(psi * wdf);
         float2 z[9];
         swap_halves(s1, z[1], z[6]);
         z[2] = cmul(z[1], z[1]);
@@ -288,7 +289,7 @@ __device__ __forceinline__ void sum(uint4 *lds, const double *__restrict__ cx, c
       unsigned y1h[8], y1l[8];
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
-        const float2 pg = eturn<true>(psi * fc[b]);  // conj P
+        const float2 pg = eturn<PREC != 2>(psi * fc[b]);  // conj P
         const float2 y0 = REAL ? make_float2(pr[b].x * pg.x, pr[b].x * pg.y)
                                : cmul(pg, make_float2(pr[b].x, pr[b].y));
         unsigned yh, yl;

@@ -1,7 +1,7 @@
 """The spectral matrix-core kernel (k_dft_spec) after what its tables were made
 from has changed: frequencies uploaded again, other reference frequencies under
-a captured graph.  Each against a handle made for the new state, bit for bit,
-and against the FP64 oracle."""
+a captured graph, the sin/cos policy.  Each against a handle made for the new
+state, bit for bit, and against the FP64 oracle."""
 import ctypes as C
 import dataclasses
 
@@ -106,3 +106,26 @@ def test_graph_after_new_reference(oracle, factor, between):
             assert np.array_equal(sm.get_vis(), want)
     ref = oracle.dft_model_fp64(uv, new)
     assert np.abs(_model(uv, want) - ref).max() <= TOL * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("path", ["resident", "buffer"])
+def test_precision_policies(oracle, path):
+    """Hardware sin/cos for the centre phasors and the steps (0), for the centre
+    phasors (1), for neither (2): each result its own."""
+    from obit_amd.skymodel import SkyModelDFT
+    uv = _uv(4, 64, 61)
+    sky = _sky(uv, 100, uv.freq)
+    ref = oracle.dft_model_fp64(uv, sky)
+    out = []
+    for prec in (0, 1, 2):
+        with SkyModelDFT(uv, sky, op="repl") as sm:
+            sm.set_precision(prec)
+            if path == "buffer":
+                out.append(sm.calc(uv.buffer.copy()))
+            else:
+                sm.set_variant(64, 64, 2)
+                sm.set_vis(uv.buffer)
+                sm.calc_resident()
+                out.append(sm.get_vis())
+        assert np.abs(_model(uv, out[-1]) - ref).max() <= TOL * np.abs(ref).max()
+    assert not np.array_equal(out[1], out[2]) and not np.array_equal(out[0], out[1])
