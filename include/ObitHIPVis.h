@@ -114,7 +114,9 @@ int ObitHIPSkyModelDFTGraphLaunch(GPUInfo *gpuInfo);
  * then reports the VALU shape.  Autotune times
  * every shape on a copy of the first resident rows and keeps the fastest:
  * sampleRows rows, raised where needed so that the widest grid gets at
- * least 8 rounds of work items, and capped at the resident rows. */
+ * least 8 rounds of work items, and capped at the resident rows.  Where an
+ * untuned launch would run on the kernel of smaller work items it is timed too,
+ * and if it is the fastest the launches choose for themselves again. */
 int ObitHIPSkyModelDFTSetVariant(GPUInfo *gpuInfo, int cpt, int tile, int wgPerCU);
 int ObitHIPSkyModelDFTGetVariant(GPUInfo *gpuInfo, int *cpt, int *tile, int *wgPerCU);
 int ObitHIPSkyModelDFTAutotune(GPUInfo *gpuInfo, long long sampleRows, int reps);

@@ -2715,12 +2715,34 @@ int ObitHIPSkyModelDFTAutotune(GPUInfo *gpuInfo, long long sampleRows, int reps)
       }
     }
   }
+  // k_dft_share, where an untuned launch would take it (few rounds of the
+  // resident rows, all of which the sample holds then): if it is the fastest
+  // the launches choose for themselves again
+  bool automatic = false;
+  if (!rc && st->uniform && n == st->nres) {
+    obit::dft::Desc d;
+    rc = obit::dft::make_desc(st, gpuInfo, tmp, n, 32, d);
+    const obit::dft::Choice c = rc ? obit::dft::Choice{} : obit::dft::choose(st, d, true);
+    if (!rc && c.kernel == obit::dft::Choice::share) {
+      rc = obit::dft::launch_share(st, d, c.cpt, nullptr);  // load the code object
+      (void)hipEventRecord(e0, st->stream);
+      for (int r = 0; r < reps && !rc; ++r) rc = obit::dft::launch_share(st, d, c.cpt, nullptr);
+      (void)hipEventRecord(e1, st->stream);
+      (void)hipEventSynchronize(e1);
+      float ms = 0.0f;
+      (void)hipEventElapsedTime(&ms, e0, e1);
+      automatic = !rc && ms < best;
+    }
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   (void)hipFree(tmp);
   if (rc) return rc;
-  st->cpt = bc; st->tile = bt; st->wgPerCU = bw;
-  st->chosen = true;
+  const State def;
+  st->cpt = automatic ? def.cpt : bc;
+  st->tile = automatic ? def.tile : bt;
+  st->wgPerCU = automatic ? def.wgPerCU : bw;
+  st->chosen = !automatic;
   obit::dft::destroy_graph(st);
   return obit::kOK;
 }
