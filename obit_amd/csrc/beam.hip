@@ -859,10 +859,21 @@ void mm_blocks(const ObitHIPBeamDesc &D, const double *fIF, const double *dfIF, 
   }
 }
 
+// Device memory for a table of k_beam_mm, kept until the handle goes; false where
+// there is none: the handle's launches then run on k_beam_dft.
+template <typename T>
+bool mm_alloc(T *&p, size_t n) {
+  if (!p && hipMalloc(&p, n * sizeof(T)) != hipSuccess) {
+    (void)hipGetLastError();
+    p = nullptr;
+  }
+  return p != nullptr;
+}
+
 // The tables of k_beam_mm (once per handle): taken where the model is points
 // and at least 0.3 of its 256 channel slots a pass are selected channels (the
 // kernel runs at about four times k_beam_dft's rate, measured full), and the
-// products fit 512 MiB.
+// products fit 512 MiB and the device's free memory.
 int mm_tables(ObitHIPBeam *h) {
   using namespace obit;
   const ObitHIPBeamDesc &D = h->desc;
@@ -874,12 +885,8 @@ int mm_tables(ObitHIPBeam *h) {
   const size_t ncpad = ((size_t)D.ncomp + 31) / 32 * 32 + 32;
   const size_t nprod = nep * D.ntype * D.ntype * nbp * ncpad;
   if (nprod * sizeof(float4) > (size_t(512) << 20) || nbp * ncpad > 0x3fffffffULL) return kOK;
-  if (!h->d_prod) {
-    h->ncpad = (int)ncpad;
-    OBIT_HIP_TRY(hipMalloc(&h->d_mm, 2 * sizeof(unsigned)));
-    OBIT_HIP_TRY(hipMalloc(&h->d_prod, nprod * sizeof(float4)));
-  }
-  h->mmTables = true;
+  h->ncpad = (int)ncpad;
+  h->mmTables = mm_alloc(h->d_mm, 2) && mm_alloc(h->d_prod, nprod);
   return kOK;
 }
 
@@ -891,9 +898,9 @@ int mm_fit(ObitHIPBeam *h) {
   h->mmAmp = false;
   if (!h->mmTables || !h->d_tab) return kOK;
   const size_t nbp = (size_t)h->npass * mm::kPass, nc = (size_t)h->ncpad;
-  if (!h->d_Ab) OBIT_HIP_TRY(hipMalloc(&h->d_Ab, nbp * nc * sizeof(float)));
-  if (!h->d_G) OBIT_HIP_TRY(hipMalloc(&h->d_G, (size_t)h->npass * mm::kT * nc * sizeof(float)));
-  if (!h->d_kap) OBIT_HIP_TRY(hipMalloc(&h->d_kap, (size_t)h->npass * nc * sizeof(unsigned)));
+  if (!mm_alloc(h->d_Ab, nbp * nc) || !mm_alloc(h->d_G, (size_t)h->npass * mm::kT * nc) ||
+      !mm_alloc(h->d_kap, (size_t)h->npass * nc))
+    return kOK;
   hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(64), 0, h->stream, h->d_mm + 1, 1);
   hipLaunchKernelGGL(mm::k_fit, dim3((unsigned)((nc + 63) / 64), (unsigned)h->npass), dim3(64), 0, h->stream,
                      h->d_tab, D.nchan, D.nchan, (long long)D.nif * D.nchan, h->d_blk, h->nblk, h->d_r0, D.ncomp, h->ncpad,

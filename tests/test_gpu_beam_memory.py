@@ -1,0 +1,45 @@
+"""Beam models on a device whose free memory does not hold the matrix-core
+kernel's products: the calls succeed on the other kernel."""
+import numpy as np
+import pytest
+
+from obit_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def test_no_room_for_products():
+    import torch
+    from obit_amd.beam import BeamDFT
+    nant, nif, nchan, ncomp, ntype = 27, 4, 64, 116000, 3
+    base, _, _ = synth.workload(1, rows=2)
+    rng = np.random.default_rng(1)
+    nf = nif * nchan
+    buf = np.zeros((2, 5 + nf * 3 * 4), np.float32)
+    buf[:, :5] = base.buffer[:, :5]
+    buf[:, 5:].reshape(2, nf * 4, 3)[..., 2] = 1.0
+    fr = (base.freq * (1.0 + 0.05 * np.arange(nif))[:, None] + 1e6 * np.arange(nchan)[None, :]).ravel()
+    uv = synth.UVData(buffer=buf, nchan=nchan, nif=nif, nstok=4, freq=base.freq, freqArr=fr, crval_stokes=-5.0)
+    l, m = rng.uniform(-0.5, 0.5, (2, ncomp)) * synth.DG2RAD
+    comps = synth.point_row(rng.exponential(0.01, ncomp), l, m).astype(np.float32)
+    ant_type = rng.integers(0, ntype, nant)
+
+    def model():
+        # 9 type pairs x 2 correlation pairs x 16 blocks x 116,032 components: 510 MiB of products
+        with BeamDFT(uv, comps, ant_type, np.zeros(nf, np.int32), 1, ntype=ntype, stok_type=1, op="repl") as bm:
+            return bm.calc(uv.buffer, par_ang=0.3)
+    want = model()
+    fill, room = [], 420 << 20
+    try:
+        for _ in range(4):  # the free memory that is reported falls by less than what is taken
+            free = torch.cuda.mem_get_info()[0]
+            if free > room + (4 << 20):
+                fill.append(torch.empty(free - room, dtype=torch.uint8, device="cuda"))
+        got = model()
+    finally:
+        fill.clear()
+        torch.cuda.empty_cache()
+    d = np.abs(got[:, 5:] - want[:, 5:]).max() / np.abs(want[:, 5:]).max()
+    print(f"{free >> 20} MiB left: max |d| / peak {d:.2e}", flush=True)
+    # the split DFT's bound, for either kernel
+    assert 0 < d < 2e-5
