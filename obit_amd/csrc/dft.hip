@@ -1297,7 +1297,7 @@ struct State {
   SpecTab spec{};
   mm::Blk *sblk = nullptr;
   float *sbuf = nullptr;     // A [npass * 16][ncpad], G [npass][16][ncpad], kappa [npass][ncpad], r0 [npass]
-  size_t sblkCap = 0, sbufCap = 0;
+  size_t sblkCap = 0, sbufCap = 0, smaxCap = 0;
   unsigned *smax = nullptr;  // residual, largest |A|
   // frequencies
   std::vector<double> freq64;
@@ -1475,25 +1475,24 @@ int spec_factors(State *st, int nIFsel, int nchsel, int nchpad, const std::vecto
     r0[p] = (float)(fdl[0] / f0);
     for (size_t b = b0; b < b0 + n; ++b) blk[b].s = (float)(fdl[0] * (1.0 / blk[b].fc - 1.0 / f0));
   }
-  if (blk.size() > st->sblkCap) {
-    (void)hipFree(st->sblk);
-    st->sblk = nullptr;
-    st->sblkCap = 0;
-    OBIT_HIP_TRY(hipMalloc(&st->sblk, blk.size() * sizeof(mm::Blk)));
-    st->sblkCap = blk.size();
-  }
-  const size_t need = nA + npass * mm::kT * ncpad + npass * ncpad + npass;
-  if (need > st->sbufCap) {
-    (void)hipFree(st->sbuf);
-    st->sbuf = nullptr;
-    st->sbufCap = 0;
-    if (hipMalloc(&st->sbuf, need * sizeof(float)) != hipSuccess) {
+  // room for n elements of a table; without it the model runs on k_dft_split
+  auto room = [](auto *&p, size_t &cap, size_t n) {
+    if (n <= cap) return true;
+    (void)hipFree(p);
+    p = nullptr;
+    cap = 0;
+    if (hipMalloc(&p, n * sizeof(*p)) != hipSuccess) {
       (void)hipGetLastError();
-      return kOK;  // no room: k_dft_split
+      p = nullptr;
+      return false;
     }
-    st->sbufCap = need;
-  }
-  if (!st->smax) OBIT_HIP_TRY(hipMalloc(&st->smax, 2 * sizeof(unsigned)));
+    cap = n;
+    return true;
+  };
+  const size_t need = nA + npass * mm::kT * ncpad + npass * ncpad + npass;
+  if (!room(st->sblk, st->sblkCap, blk.size()) || !room(st->sbuf, st->sbufCap, need) ||
+      !room(st->smax, st->smaxCap, 2))
+    return kOK;
   float *Ab = st->sbuf, *G = Ab + nA, *kap = G + npass * mm::kT * ncpad, *dr0 = kap + npass * ncpad;
   OBIT_HIP_TRY(hipMemcpy(st->sblk, blk.data(), blk.size() * sizeof(mm::Blk), hipMemcpyHostToDevice));
   OBIT_HIP_TRY(hipMemcpy(dr0, r0.data(), npass * sizeof(float), hipMemcpyHostToDevice));
@@ -1566,14 +1565,21 @@ int ensure_spec_table(State *st, const GPUInfo *gi, const std::vector<double> &f
   if (need > st->tabCap) {
     if (st->tab) OBIT_HIP_TRY(hipFree(st->tab));
     st->tab = nullptr;
+    st->tabCap = 0;
     hipError_t e = hipMalloc(&st->tab, need * sizeof(float));
     if (e != hipSuccess) return fail(kNoMemory, "spectral table (%zu floats): %s", need, hipGetErrorString(e));
     st->tabCap = need;
   }
-  double *dl = nullptr;
-  int *db = nullptr;
-  OBIT_HIP_TRY(hipMalloc(&dl, lnr.size() * sizeof(double)));
-  OBIT_HIP_TRY(hipMalloc(&db, bin.size() * sizeof(int)));
+  // ln(nu / nu_spectrum) and coarse bin of every channel, freed on every way out
+  struct Tmp {
+    double *l = nullptr;
+    int *b = nullptr;
+    ~Tmp() { (void)hipFree(l); (void)hipFree(b); }
+  } tmp;
+  OBIT_HIP_TRY(hipMalloc(&tmp.l, lnr.size() * sizeof(double)));
+  OBIT_HIP_TRY(hipMalloc(&tmp.b, bin.size() * sizeof(int)));
+  double *dl = tmp.l;
+  int *db = tmp.b;
   OBIT_HIP_TRY(hipMemcpy(dl, lnr.data(), lnr.size() * sizeof(double), hipMemcpyHostToDevice));
   OBIT_HIP_TRY(hipMemcpy(db, bin.data(), bin.size() * sizeof(int), hipMemcpyHostToDevice));
   const long long total = (long long)st->ncomp * nIFsel * nchpad;
@@ -1587,8 +1593,6 @@ int ensure_spec_table(State *st, const GPUInfo *gi, const std::vector<double> &f
   const int rc = spec_factors(st, nIFsel, nchsel, nchpad, fb, fdl, bin);
   if (rc) return rc;
   OBIT_HIP_TRY(hipStreamSynchronize(st->stream));
-  OBIT_HIP_TRY(hipFree(dl));
-  OBIT_HIP_TRY(hipFree(db));
   st->tabReady = true;
   st->tabKey = key;
   st->tabFreq = fch;
