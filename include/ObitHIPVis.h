@@ -75,8 +75,11 @@ int ObitHIPSkyModelDFTGetBufferShape(GPUInfo *gpuInfo, int *cpt, int *nsplit);
  * static device scratch of 32 MiB per GPU (838,809 components at most;
  * more is refused with OBIT_HIP_EINVAL, as are spectral model types, more
  * than 64 selected IFs and channel tables that are not a line within each
- * IF).  Asynchronous on ObitHIPSkyModelDFTStream; calls that overlap on one
- * GPU share the scratch and race. */
+ * IF).  It runs on the VALU kernels whatever the model: the result is
+ * CalcResident's bit for bit where that runs on them too, and within both
+ * kernels' error where it takes a matrix-core kernel.  Asynchronous on
+ * ObitHIPSkyModelDFTStream; calls that overlap on one GPU share the scratch
+ * and race. */
 int ObitHIPSkyModelDFTCalcNoAlloc(GPUInfo *gpuInfo, const float *d_model, int ncomp, float *d_vis,
                                   long long nvis);
 /* Reference frequencies of the component spectra in FP64 (Hz): one value

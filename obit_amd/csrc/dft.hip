@@ -2486,8 +2486,11 @@ int ObitHIPSkyModelDFTCalcNoAlloc(GPUInfo *gpuInfo, const float *d_model, int nc
   const int gOff = model_gauss_off(st->type);
   if (gOff >= 0 && st->size < 7) return fail(kInvalid, "Gaussian model needs 7 floats per row");
   if (nvis == 0) return kOK;
+  // the VALU kernels (the matrix-core kernel's eligibility reads the host
+  // copy of the lines, which this call does not make): a handle set to the
+  // matrix-core kernel runs at 32 channels a thread
   Desc d;
-  int rc = desc_layout(gpuInfo, d_vis, nvis, st->cpt, d);
+  int rc = desc_layout(gpuInfo, d_vis, nvis, st->cpt == 64 ? 32 : st->cpt, d);
   if (rc) return rc;
   Lines L;
   rc = lines_fixed(st, gpuInfo->h_visInfo, L);
@@ -2522,8 +2525,6 @@ int ObitHIPSkyModelDFTCalcNoAlloc(GPUInfo *gpuInfo, const float *d_model, int nc
   d.cx = cx; d.cy = cy; d.cz = cz;
   d.camp = camp; d.cg = cg;
   st->lastPath = 0;
-  // the VALU kernel (the matrix-core kernel's eligibility reads the host
-  // copy of the lines, which this call does not make)
   return launch_resident(st, d, false);
 }
 
