@@ -426,8 +426,10 @@ __global__ __launch_bounds__(kRows, kBlocksPerCU) void k_beam_dft(Desc d) {
 // 16 blocks, K = (component, Re / Im), every operand split into FP16 parts
 // x_h + x_l and A_h B_h + A_h B_l + A_l B_h summed in FP32, folded into FP64
 // every 2 tiles of 32 components (every 4 left 2.5e-7 of the model's norm, more
-// than k_beam_dft's 2.3e-7; every tile 1.7e-7 and 4 % slower); conj Y in B.  Y is scaled by a power of two
-// (the largest |C| to [2^13, 2^14)), taken out exactly at the end.
+// than k_beam_dft's 2.3e-7; every tile 1.7e-7 and 4 % slower); conj Y in B.  Y is
+// scaled by a power of two of its correlation, antenna types and block (their
+// largest |C| to [2^13, 2^14)), taken out exactly at the end: with one scale for
+// all, channels or cross hands of 1e-6 of the brightest lost four bits.
 //
 // A spectrum (AMP) makes the amplitude a_k(t, b) of a channel depend on t and
 // b.  mm::k_fit writes it as A_kb G_k(t) (1 + kappa_k tau(t) s_b): G goes into
@@ -460,14 +462,20 @@ struct MmTab {
   const mm::Blk *blk;
   int nblk, npass, ncpad;     // ncpad: components padded with zeros (a whole tile of them at least)
   const float4 *prod;         // [2][npair][npass * 16][ncpad]: conj C of a correlation pair, scaled
-  const unsigned *amax;       // largest |C| (float bits)
+  const unsigned *amax;       // largest |C| (float bits) at scale_at
   const float *G;             // [npass][16][ncpad], or null: no spectrum
   const unsigned *kap;        // [npass][ncpad]: (kappa, kappa) in FP16
   const float *r0;            // [npass]: df / f0
 };
 
+// Where the largest |C| of correlation e of pair ep, type pair p and block b is.
+__device__ __forceinline__ long long scale_at(int ep, int e, int p, int npair, int b, int nblkPad) {
+  return ((long long)(2 * ep + e) * npair + p) * nblkPad + b;
+}
+
 // C of every (correlation pair, type pair, block, component): the largest
-// finite part to amax (WRITE false), then the scaled conjugates to prod.
+// finite part to amax (WRITE false), then the scaled conjugates to prod.  The
+// components of a block are whole half-waves (ncpad is a multiple of 32).
 template <bool WRITE>
 __global__ __launch_bounds__(256) void k_beam_prod(const float *__restrict__ jones, const float *__restrict__ camp,
                                                    const float *__restrict__ Ab, const mm::Blk *__restrict__ blk,
@@ -476,8 +484,6 @@ __global__ __launch_bounds__(256) void k_beam_prod(const float *__restrict__ jon
                                                    unsigned *__restrict__ amax, float4 *__restrict__ prod) {
   const int npair = ntype * ntype;
   const long long n = (long long)npair * nblk * ncpad;
-  float big = 0.0f;
-  const float sc = WRITE ? ldexpf(1.0f, mm::shift_of(*amax)) : 1.0f;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
     const int k = (int)(i % ncpad);
@@ -498,21 +504,23 @@ __global__ __launch_bounds__(256) void k_beam_prod(const float *__restrict__ jon
     if (WRITE) {
       for (int ep = 0; ep < nep; ++ep) {
         const float2 u = m[ep ? 1 : 0], v = m[ep ? 2 : 3];  // (XX, YY) or (XY, YX)
+        const int su = mm::shift_of(amax[scale_at(ep, 0, p, npair, b, nblkPad)]);
+        const int sv = mm::shift_of(amax[scale_at(ep, 1, p, npair, b, nblkPad)]);
         prod[(((long long)ep * npair + p) * nblkPad + b) * ncpad + k] =
-            make_float4(sc * u.x, -sc * u.y, sc * v.x, -sc * v.y);
+            make_float4(ldexpf(u.x, su), -ldexpf(u.y, su), ldexpf(v.x, sv), -ldexpf(v.y, sv));
       }
     } else {
+      for (int ep = 0; ep < nep; ++ep)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float x = fabsf(m[e].x), y = fabsf(m[e].y);
-        if (x < INFINITY) big = fmaxf(big, x);
-        if (y < INFINITY) big = fmaxf(big, y);
-      }
+        for (int e = 0; e < 2; ++e) {
+          const float2 u = ep ? m[1 + e] : m[3 * e];
+          const float x = fabsf(u.x), y = fabsf(u.y);
+          float big = fmaxf(x < INFINITY ? x : 0.0f, y < INFINITY ? y : 0.0f);
+          for (int o = 16; o > 0; o >>= 1) big = fmaxf(big, __shfl_xor(big, o));
+          if ((threadIdx.x & 31) == 0 && big > 0.0f)
+            atomicMax(amax + scale_at(ep, e, p, npair, b, nblkPad), __float_as_uint(big));
+        }
     }
-  }
-  if (!WRITE) {
-    for (int o = 32; o > 0; o >>= 1) big = fmaxf(big, __shfl_xor(big, o));
-    if ((threadIdx.x & 63) == 0 && big > 0.0f) atomicMax(amax, __float_as_uint(big));
   }
 }
 
@@ -597,9 +605,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
     // 32 the Im of the same; column n = lane mod 16 is block n of the pass, or
     // with split block n mod 8 of correlation or pair n / 8
     const int n = lane & 15, nb = split ? n & 7 : n, cp = !ONE && split ? n >> 3 : ep;
-    const mm::Blk bk = m.blk[min(ps * mm::kPass + nb, m.nblk - 1)];
+    const int gb = min(ps * mm::kPass + nb, m.nblk - 1);
+    const mm::Blk bk = m.blk[gb];
     const bool have = lane < 32 && ps * mm::kPass + nb < m.nblk;
-    const double unscale = ldexp(1.0, -mm::shift_of(*m.amax));
+    double unscale[NE];
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+      unscale[e] = ldexp(1.0, -mm::shift_of(m.amax[scale_at(cp, ONE && split ? n >> 3 : e, pair, d.npair, gb,
+                                                            m.npass * mm::kPass)]));
     const float r0 = AMP ? m.r0[ps] : 0.0f;
     float *base = d.vis + row * (long long)d.lrec + d.nrparm + (long long)bk.IF * d.incif;
 #pragma unroll
@@ -613,8 +626,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AMP ? 2 : 3
           double x = o[T][e][r];
           if (AMP) x += (double)(((float)t - (float)(t * t) * r0) * bk.s * d2[T][e][r]);
           const double y = __shfl_xor(x, 32);
-          vr[e] = (float)(x * unscale);
-          vi[e] = (float)(y * unscale);
+          vr[e] = (float)(x * unscale[e]);
+          vi[e] = (float)(y * unscale[e]);
         }
         const int ch = bk.ch0 + 8 + t;
         float *p = base + (long long)ch * d.incf;
@@ -799,7 +812,7 @@ struct ObitHIPBeam {
   bool mmTables = false, mmAmp = false;
   obit::mm::Blk *d_blk = nullptr;
   float *d_r0 = nullptr, *d_Ab = nullptr, *d_G = nullptr;
-  unsigned *d_kap = nullptr, *d_mm = nullptr;  // d_mm: largest |C|, fit residual (float bits)
+  unsigned *d_kap = nullptr, *d_mm = nullptr;  // d_mm: fit residual, then MmTab's amax (float bits)
   float4 *d_prod = nullptr;
 };
 
@@ -886,7 +899,7 @@ int mm_tables(ObitHIPBeam *h) {
   const size_t nprod = nep * D.ntype * D.ntype * nbp * ncpad;
   if (nprod * sizeof(float4) > (size_t(512) << 20) || nbp * ncpad > 0x3fffffffULL) return kOK;
   h->ncpad = (int)ncpad;
-  h->mmTables = mm_alloc(h->d_mm, 2) && mm_alloc(h->d_prod, nprod);
+  h->mmTables = mm_alloc(h->d_mm, 1 + 2 * nep * D.ntype * D.ntype * nbp) && mm_alloc(h->d_prod, nprod);
   return kOK;
 }
 
@@ -901,14 +914,14 @@ int mm_fit(ObitHIPBeam *h) {
   if (!mm_alloc(h->d_Ab, nbp * nc) || !mm_alloc(h->d_G, (size_t)h->npass * mm::kT * nc) ||
       !mm_alloc(h->d_kap, (size_t)h->npass * nc))
     return kOK;
-  hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(64), 0, h->stream, h->d_mm + 1, 1);
+  hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(64), 0, h->stream, h->d_mm, 1);
   hipLaunchKernelGGL(mm::k_fit, dim3((unsigned)((nc + 63) / 64), (unsigned)h->npass), dim3(64), 0, h->stream,
                      h->d_tab, D.nchan, D.nchan, (long long)D.nif * D.nchan, h->d_blk, h->nblk, h->d_r0, D.ncomp, h->ncpad,
-                     h->d_Ab, h->d_G, h->d_kap, h->d_mm + 1, nullptr);
+                     h->d_Ab, h->d_G, h->d_kap, h->d_mm, nullptr);
   OBIT_HIP_TRY(hipGetLastError());
   float worst = 0.0f;
   OBIT_HIP_TRY(hipStreamSynchronize(h->stream));
-  OBIT_HIP_TRY(hipMemcpy(&worst, h->d_mm + 1, sizeof(float), hipMemcpyDeviceToHost));
+  OBIT_HIP_TRY(hipMemcpy(&worst, h->d_mm, sizeof(float), hipMemcpyDeviceToHost));
   h->mmAmp = worst <= mm::kFitTol;
   return kOK;
 }
@@ -930,13 +943,14 @@ int beam_coh(ObitHIPBeam *h, float parAng, hipStream_t stream) {
     const float *Ab = h->d_tab ? h->d_Ab : nullptr;
     const long long n = (long long)D.ntype * D.ntype * h->nblk * h->ncpad;
     const dim3 grid((unsigned)std::min<long long>((n + 255) / 256, (long long)std::max(h->ncu, 1) * 16));
-    hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(64), 0, stream, h->d_mm, 1);
+    hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(256), 0, stream, h->d_mm + 1,
+                       2 * nep * D.ntype * D.ntype * h->npass * mm::kPass);
     hipLaunchKernelGGL((beam::k_beam_prod<false>), grid, dim3(256), 0, stream, h->d_jones, h->d_amp, Ab, h->d_blk,
                        h->nblk, h->npass * mm::kPass, D.ntype, D.ncomp, h->ncpad, D.njchan, nep, D.stokType,
-                       (float)c2, (float)s2, h->d_mm, h->d_prod);
+                       (float)c2, (float)s2, h->d_mm + 1, h->d_prod);
     hipLaunchKernelGGL((beam::k_beam_prod<true>), grid, dim3(256), 0, stream, h->d_jones, h->d_amp, Ab, h->d_blk,
                        h->nblk, h->npass * mm::kPass, D.ntype, D.ncomp, h->ncpad, D.njchan, nep, D.stokType,
-                       (float)c2, (float)s2, h->d_mm, h->d_prod);
+                       (float)c2, (float)s2, h->d_mm + 1, h->d_prod);
     OBIT_HIP_TRY(hipGetLastError());
     return kOK;
   }
@@ -981,7 +995,7 @@ int beam_dft(ObitHIPBeam *h, float *d_vis, long long nrow, hipStream_t stream) {
     m.blk = h->d_blk;
     m.nblk = h->nblk; m.npass = h->npass; m.ncpad = h->ncpad;
     m.prod = h->d_prod;
-    m.amax = h->d_mm;
+    m.amax = h->d_mm + 1;
     m.G = h->d_G; m.kap = h->d_kap; m.r0 = h->d_r0;
     // the cross hands are not divided
     const bool cross = D.ncorr == 4 && D.opType != ObitHIPBeamOpDiv;

@@ -998,7 +998,7 @@ struct SpecTab {
   int nblk, npass, ncpad;
   const float *Ab, *G, *r0;
   const unsigned *kap;
-  int shift;              // A is scaled by 2^shift
+  const unsigned *amax;   // [nblk]: largest |A| of a block (float bits); its A are scaled by 2^shift_of that
 };
 
 template <int PREC>
@@ -1032,9 +1032,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     mm::sum<true, 1, true, PREC>(s_op[wv], d.cx, d.cy, d.cz, d.ncomp, kBeg, kEnd, u, v, w, df, fc, po, m.Ab, 1u, G,
                            h ? m.ncpad : -m.ncpad, m.kap + (long long)ps * m.ncpad, o, d2);
     const int n = lane & 15;
-    const mm::Blk bk = m.blk[min(ps * mm::kPass + n, m.nblk - 1)];
+    const int g = min(ps * mm::kPass + n, m.nblk - 1);
+    const mm::Blk bk = m.blk[g];
     const bool have = lane < 32 && ps * mm::kPass + n < m.nblk;
-    const double unscale = ldexp(1.0, -m.shift);
+    const double unscale = ldexp(1.0, -mm::shift_of(m.amax[g]));
     const float r0 = m.r0[ps];
     float *base = d.vis + row * (long long)d.lrec + d.nrparm + d.chanb * d.incf + d.stokb * d.incs;
     double2 *pp = d.part ? d.part + (((long long)part * d.nrow + row) * d.nIFsel + bk.IF) * d.nchsel : nullptr;
@@ -1060,11 +1061,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   }
 }
 
-// n amplitudes times 2^shift
-__global__ void k_scale(float *a, long long n, int shift) {
+// The amplitudes of nblk blocks of ncpad, the largest of each to [2^13, 2^14): a
+// block of faint channels keeps the FP16 parts' 22 bits.
+__global__ void k_scale(float *a, int nblk, int ncpad, const unsigned *amax) {
+  const long long n = (long long)nblk * ncpad;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x)
-    a[i] = ldexpf(a[i], shift);
+    a[i] = ldexpf(a[i], mm::shift_of(amax[i / ncpad]));
 }
 
 // The sums of the nsplit component parts of every (row, IF, channel),
@@ -1298,7 +1301,7 @@ struct State {
   mm::Blk *sblk = nullptr;
   float *sbuf = nullptr;     // A [npass * 16][ncpad], G [npass][16][ncpad], kappa [npass][ncpad], r0 [npass]
   size_t sblkCap = 0, sbufCap = 0, smaxCap = 0;
-  unsigned *smax = nullptr;  // residual, largest |A|
+  unsigned *smax = nullptr;  // largest |A| of every block, then the residual
   // frequencies
   std::vector<double> freq64;
   double uvRef = 0.0;
@@ -1438,7 +1441,7 @@ int frequency_lines(State *st, const GPUVisInfo *vi, std::vector<double> &fb,
 
 // The factors of the amplitude table for k_dft_spec: channel blocks (runs of
 // one coarse bin in blocks of 16, a run's last block moved back to end with
-// it), then mm::k_fit and the scale.  Points only, one channel step for every
+// it), then mm::k_fit and the scales.  Points only, one channel step for every
 // IF, and at least 0.55 of the 256 channel slots a pass selected channels:
 // below that k_dft_split (5.7e12 evaluations/s) is faster than the filled part
 // of k_dft_spec's 10.0e12.
@@ -1491,28 +1494,31 @@ int spec_factors(State *st, int nIFsel, int nchsel, int nchpad, const std::vecto
   };
   const size_t need = nA + npass * mm::kT * ncpad + npass * ncpad + npass;
   if (!room(st->sblk, st->sblkCap, blk.size()) || !room(st->sbuf, st->sbufCap, need) ||
-      !room(st->smax, st->smaxCap, 2))
+      !room(st->smax, st->smaxCap, blk.size() + 1))
     return kOK;
   float *Ab = st->sbuf, *G = Ab + nA, *kap = G + npass * mm::kT * ncpad, *dr0 = kap + npass * ncpad;
   OBIT_HIP_TRY(hipMemcpy(st->sblk, blk.data(), blk.size() * sizeof(mm::Blk), hipMemcpyHostToDevice));
   OBIT_HIP_TRY(hipMemcpy(dr0, r0.data(), npass * sizeof(float), hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(64), 0, st->stream, st->smax, 2);
+  const int nblk = (int)blk.size();
+  hipLaunchKernelGGL(mm::k_clear, dim3(1), dim3(64), 0, st->stream, st->smax, nblk + 1);
   hipLaunchKernelGGL(mm::k_fit, dim3((unsigned)((ncpad + 63) / 64), (unsigned)npass), dim3(64), 0, st->stream,
-                     st->tab, nchsel, nchpad, (long long)nIFsel * nchpad, st->sblk, (int)blk.size(), dr0, st->ncomp,
-                     (int)ncpad, Ab, G, reinterpret_cast<unsigned *>(kap), st->smax, st->smax + 1);
+                     st->tab, nchsel, nchpad, (long long)nIFsel * nchpad, st->sblk, nblk, dr0, st->ncomp,
+                     (int)ncpad, Ab, G, reinterpret_cast<unsigned *>(kap), st->smax + nblk, st->smax);
   OBIT_HIP_TRY(hipGetLastError());
-  unsigned got[2];
-  OBIT_HIP_TRY(hipMemcpyAsync(got, st->smax, sizeof(got), hipMemcpyDeviceToHost, st->stream));
+  std::vector<unsigned> got(nblk + 1);
+  OBIT_HIP_TRY(hipMemcpyAsync(got.data(), st->smax, got.size() * sizeof(unsigned), hipMemcpyDeviceToHost, st->stream));
   OBIT_HIP_TRY(hipStreamSynchronize(st->stream));
-  float worst, top;
-  std::memcpy(&worst, got, sizeof(float));
-  std::memcpy(&top, got + 1, sizeof(float));
-  if (!(worst <= mm::kFitTol) || !std::isfinite(top)) return kOK;
-  const int shift = mm::shift_of(got[1]);
-  hipLaunchKernelGGL(k_scale, dim3(256), dim3(256), 0, st->stream, Ab, (long long)(blk.size() * ncpad), shift);
+  auto value = [&](int i) {
+    float v;
+    std::memcpy(&v, &got[i], sizeof(float));
+    return v;
+  };
+  if (!(value(nblk) <= mm::kFitTol)) return kOK;
+  for (int i = 0; i < nblk; ++i)
+    if (!std::isfinite(value(i))) return kOK;
+  hipLaunchKernelGGL(k_scale, dim3(256), dim3(256), 0, st->stream, Ab, nblk, (int)ncpad, st->smax);
   OBIT_HIP_TRY(hipGetLastError());
-  st->spec = SpecTab{st->sblk, (int)blk.size(), (int)npass, (int)ncpad, Ab, G, dr0,
-                     reinterpret_cast<unsigned *>(kap), shift};
+  st->spec = SpecTab{st->sblk, nblk, (int)npass, (int)ncpad, Ab, G, dr0, reinterpret_cast<unsigned *>(kap), st->smax};
   st->specMm = true;
   return kOK;
 }

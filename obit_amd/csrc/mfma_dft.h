@@ -74,9 +74,9 @@ constexpr int kSlots = 2 * kSlotsA + 2 * kSlotsB;  // of a wave
 constexpr int kT = 16;             // channels of a block
 constexpr int kPass = 16;          // blocks of a pass
 // Largest residual of the factored amplitudes, relative to the component's
-// largest amplitude, that the matrix-core kernels take.  It is the worst
-// channel's (a steep spectrum at both ends of a pass); the model's error stays
-// below that of the channel walks, whose worst is 1.3e-6 of the peak.
+// largest amplitude in the same block, that the matrix-core kernels take.  It is
+// the worst channel's (a steep spectrum at both ends of a pass); the model's error
+// stays below that of the channel walks, whose worst is 1.3e-6 of the peak.
 constexpr float kFitTol = 1e-6f;
 
 struct Blk {
@@ -94,14 +94,14 @@ __host__ __device__ __forceinline__ int shift_of(unsigned bits) {
 }
 
 static __global__ void k_clear(unsigned *a, int n) {
-  if ((int)threadIdx.x < n) a[threadIdx.x] = 0u;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) a[i] = 0u;
 }
 
 // The factors A_kb G_k(t) (1 + kappa_k tau(t) s_b) of the amplitude table
 // (rows of ldk floats, ldif an IF, of which nchan are channels), one thread a
 // component and pass; resid: the largest relative residual, amax (may be
-// null): the largest |A| (float bits, cleared before).  G is the shape of the
-// pass's reference block, its middle one where it can be; A and the slope of each block
+// null): the largest |A| of every block (float bits, both cleared before).  G is
+// the shape of the pass's reference block, its middle one where it can be; A and the slope of each block
 // are taken at two channels 0.7 of the way to its ends, which halves the error
 // of the linear term at them; kappa is the slopes' least-squares fit to s_b.
 static __global__ __launch_bounds__(64) void k_fit(const float *__restrict__ tab, int nchan, int ldif, long long ldk,
@@ -110,10 +110,10 @@ static __global__ __launch_bounds__(64) void k_fit(const float *__restrict__ tab
                                                  unsigned *__restrict__ kap, unsigned *__restrict__ resid,
                                                  unsigned *__restrict__ amax) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x, ps = blockIdx.y;
-  float worst = 0.0f, top = 0.0f;
+  const int b0 = ps * kPass, nb = min(kPass, nblk - b0);
+  float worst = 0.0f, top[kPass] = {};
   if (k < ncomp) {
     const float *row = tab + (long long)k * ldk;
-    const int b0 = ps * kPass, nb = min(kPass, nblk - b0);
     auto amp = [&](int b, int t) {
       const int ch = min(max(blk[b].ch0 + 8 + t, 0), nchan - 1);
       return (double)row[(long long)blk[b].IF * ldif + ch];
@@ -126,7 +126,8 @@ static __global__ __launch_bounds__(64) void k_fit(const float *__restrict__ tab
     double g[kT];
     for (int t = -8; t < 8; ++t) {
       g[t + 8] = a0 != 0.0 ? amp(ref, t) / a0 : 1.0;
-      if (!(fabs(g[t + 8]) > 1e-3 && fabs(g[t + 8]) < 1e3)) g[t + 8] = 1.0;  // the residual tells
+      // (a shape that varies more would cost X's low FP16 part bits; the residual tells)
+      if (!(fabs(g[t + 8]) > 0.25 && fabs(g[t + 8]) < 4.0)) g[t + 8] = 1.0;
       g[t + 8] = (double)(float)g[t + 8];
       G[((long long)ps * kT + t + 8) * ncpad + k] = (float)g[t + 8];
     }
@@ -138,7 +139,7 @@ static __global__ __launch_bounds__(64) void k_fit(const float *__restrict__ tab
       t1 = (int)rint(m - w);
       t2 = (int)rint(m + w);
     };
-    double num = 0.0, den = 0.0, big = 0.0;
+    double num = 0.0, den = 0.0;
     for (int b = b0; b < b0 + nb; ++b) {
       int t1, t2;
       ends(b, t1, t2);
@@ -154,35 +155,42 @@ static __global__ __launch_bounds__(64) void k_fit(const float *__restrict__ tab
     const _Float16 kh = (_Float16)(float)ka;
     ka = (double)(float)kh;
     kap[(long long)ps * ncpad + k] = (unsigned)__builtin_bit_cast(unsigned short, kh) * 0x10001u;
-    double off = 0.0;
-    for (int b = b0; b < b0 + nb; ++b) {
+#pragma unroll
+    for (int i = 0; i < kPass; ++i) {
+      const int b = b0 + i;
+      if (i >= nb) break;
       int t1, t2;
       ends(b, t1, t2);
       const double s = blk[b].s;
+      double off = 0.0, big = 0.0;
       const double A = 0.5 * (amp(b, t1) / (g[t1 + 8] * (1.0 + ka * tau(t1) * s)) +
                               amp(b, t2) / (g[t2 + 8] * (1.0 + ka * tau(t2) * s)));
       Ab[(long long)b * ncpad + k] = (float)A;
-      top = fmaxf(top, fabsf((float)A));
+      top[i] = fabsf((float)A);
       for (int ch = blk[b].vlo; ch <= blk[b].vhi; ++ch) {
         const int t = ch - blk[b].ch0 - 8;
         const double a = amp(b, t), e = fabs(a - (double)(float)A * g[t + 8] * (1.0 + ka * tau(t) * s));
         big = fmax(big, fabs(a));
         off = (e >= off) ? e : (e < off ? off : INFINITY);  // a NaN counts as infinite
       }
+      const float res = big > 0.0 ? (float)(off / big) : (off > 0.0 ? INFINITY : 0.0f);
+      worst = res >= 0.0f ? fmaxf(worst, res) : INFINITY;
     }
-    worst = big > 0.0 ? (float)(off / big) : (off > 0.0 ? INFINITY : 0.0f);
-    if (!(worst >= 0.0f)) worst = INFINITY;
   } else if (k < ncpad) {
     for (int t = 0; t < kT; ++t) G[((long long)ps * kT + t) * ncpad + k] = 1.0f;
     kap[(long long)ps * ncpad + k] = 0u;
-    for (int b = ps * kPass; b < min(nblk, (ps + 1) * kPass); ++b) Ab[(long long)b * ncpad + k] = 0.0f;
+    for (int b = b0; b < b0 + nb; ++b) Ab[(long long)b * ncpad + k] = 0.0f;
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    worst = fmaxf(worst, __shfl_xor(worst, o));
-    top = fmaxf(top, __shfl_xor(top, o));
-  }
+  for (int o = 32; o > 0; o >>= 1) worst = fmaxf(worst, __shfl_xor(worst, o));
   if ((threadIdx.x & 63) == 0 && worst > 0.0f) atomicMax(resid, __float_as_uint(worst));
-  if ((threadIdx.x & 63) == 0 && amax && top > 0.0f) atomicMax(amax, __float_as_uint(top));
+  if (amax) {
+#pragma unroll
+    for (int i = 0; i < kPass; ++i) {
+      float t = top[i];
+      for (int o = 32; o > 0; o >>= 1) t = fmaxf(t, __shfl_xor(t, o));
+      if ((threadIdx.x & 63) == 0 && i < nb && t > 0.0f) atomicMax(amax + b0 + i, __float_as_uint(t));
+    }
+  }
 }
 
 // The sums over components kBeg .. kEnd - 1 (kBeg a multiple of 32; so is kEnd,
