@@ -248,10 +248,9 @@ __device__ Sample prep_sample(const FacetDev &f, const Common &cm, const float *
 constexpr int kHashParts = 16;   // partial sums of the uvw checksum,
 constexpr int kHashStride = 16;  // 128 bytes apart
 
-// Everything a pass starts from zero, in one launch (a kernel, kept out of
-// memset nodes so the sequence stays capturable in a hipGraph): the walk
-// statistics, the count after the last track, the uvw checksum and the lists'
-// first and last entries.
+// Everything a pass starts from zero, in one launch: the walk statistics, the
+// count after the last track, the uvw checksum and the lists' first and last
+// entries.
 __global__ void k_pass_clear(unsigned long long *walk, unsigned *lastCount, unsigned long long *hash,
                              long long *first, long long *last, long long n) {
   const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
