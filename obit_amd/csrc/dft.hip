@@ -116,6 +116,16 @@ __device__ __forceinline__ void apply_op(const Desc &d, float *p, float mr, floa
   }
 }
 
+// A row's coordinates for the walk of one chunk of channels: fm, fd the frequency
+// of its centre channel and the channel step.
+struct WalkRow {
+  double u, v, w, fm, fd;
+  float fmf, fdf, uu, vv, uv;
+  __device__ __forceinline__ WalkRow(float uf, float vf, float wf, double fm_, double fd_)
+      : u(uf), v(vf), w(wf), fm(fm_), fd(fd_), fmf((float)fm_), fdf((float)fd_), uu(uf * uf), vv(vf * vf),
+        uv(uf * vf) {}
+};
+
 // Components without a spectral table and without Gaussian terms take the
 // mirrored walk: with W^q the step phasor of channel offset q and (c, s) the
 // amplitude times the centre phasor, channels +q and -q are
@@ -132,11 +142,129 @@ __device__ __forceinline__ void apply_op(const Desc &d, float *p, float mr, floa
 // 4 IF x 64 channels, 60,000 rows x 6,000 points: 15.0 -> 12.0 ms (6.16e12 ->
 // 7.65e12 evaluations/s); 40,000 rows x 6,000 components, a fifth of them
 // Gaussian: 10.7 -> 7.4 ms.
-template <int CPT, int TILE, bool GAUSS, bool SPEC, int PREC>
-__global__ __launch_bounds__(kRows, 2) void k_dft_split(Desc d) {
+//
+// The channel sums of a component tile in LDS: components 0 .. np - 1 by the
+// mirrored walk, np .. kn - 1 by the walk of the phasor.
+template <int CPT, bool GAUSS, bool SPEC, int PREC>
+__device__ __forceinline__ void walk_tile(const WalkRow &r, const double *s_x, const double *s_y, const double *s_z,
+                                          const float *s_a, const float *s_g, const float *s_t, int np, int kn,
+                                          float (&accr)[CPT], float (&acci)[CPT]) {
   static_assert(CPT % 2 == 0, "CPT must be even");
   constexpr bool kMirror = !SPEC;
   constexpr int H = CPT / 2;
+  // the centre phasor (cm, sm) of component kk and its step as three
+  // shears (tau, sig), the step reduced to |pd| <= 1/4 turn; flip: an odd
+  // count of half turns was taken out, every odd offset changes sign
+  auto phasors = [&](int kk, float &cm, float &sm, float &tau, float &sig, bool &flip) {
+    const double psi = fma(r.w, s_z[kk], fma(r.v, s_y[kk], r.u * s_x[kk]));
+    double pm = psi * r.fm, pd = psi * r.fd;
+    pm -= rint(pm);
+    const double h2 = rint(2.0 * pd);
+    pd -= 0.5 * h2;
+    flip = ((int)h2) & 1;
+    float sh, ch;
+    sincos_turns<PREC == 2 ? 1 : 0>((float)pm, &sm, &cm);
+    if (PREC == 0) sincos_turns_hw((float)(0.5 * pd), &sh, &ch);
+    else sincos_halfturns_small((float)pd, &sh, &ch);
+    tau = sh * __builtin_amdgcn_rcpf(ch);
+    sig = 2.0f * sh * ch;
+  };
+  if (kMirror) {
+    for (int kk = 0; kk < np; ++kk) {
+      float cm, sm, tau, sig;
+      bool flip;
+      phasors(kk, cm, sm, tau, sig, flip);
+      const float a0 = s_a[kk], ao = flip ? -a0 : a0;
+      const float ce = a0 * cm, se = a0 * sm, co = ao * cm, so = ao * sm;
+      accr[H] += ce;
+      acci[H] += se;
+      float x = 1.0f, y = 0.0f;  // W^q
+#pragma unroll
+      for (int q1 = 1; q1 <= H; ++q1) {
+        const float x1 = fmaf(-tau, y, x);
+        y = fmaf(sig, x1, y);
+        x = fmaf(-tau, y, x1);
+        const float c = (q1 & 1) ? co : ce, s = (q1 & 1) ? so : se;
+        if (q1 < H) {
+          accr[H + q1] = fmaf(x, c, accr[H + q1]);  // C c
+          accr[H - q1] = fmaf(y, s, accr[H - q1]);  // S s
+          acci[H + q1] = fmaf(x, s, acci[H + q1]);  // C s
+          acci[H - q1] = fmaf(y, c, acci[H - q1]);  // S c
+        } else {  // the one channel without a mirror
+          accr[0] = fmaf(x, c, fmaf(y, s, accr[0]));
+          acci[0] = fmaf(x, s, fmaf(-y, c, acci[0]));
+        }
+      }
+    }
+    // the tile's channel sums
+#pragma unroll
+    for (int q1 = 1; q1 < H; ++q1) {
+      const float cc = accr[H + q1], ss = accr[H - q1], cs = acci[H + q1], sc = acci[H - q1];
+      accr[H + q1] = cc - ss;
+      accr[H - q1] = cc + ss;
+      acci[H + q1] = cs + sc;
+      acci[H - q1] = cs - sc;
+    }
+  }
+  if (GAUSS || SPEC) {
+    for (int kk = np; kk < kn; ++kk) {
+      float cm, sm, tau, sig;
+      bool flip;
+      phasors(kk, cm, sm, tau, sig, flip);
+      const float a0 = s_a[kk];
+      const float sgn = flip ? -1.0f : 1.0f;
+      float gf = a0, rf = 0.0f, rbk = 0.0f, qg = 0.0f;
+      if (GAUSS) {
+        const float G = fmaf(s_g[3 * kk + 2], r.uv, fmaf(s_g[3 * kk + 1], r.vv, s_g[3 * kk] * r.uu));
+        const float e0 = G * r.fmf * r.fmf;
+        const float Gd = G * r.fdf;
+        const bool live = e0 > -60.0f;
+        gf = live ? (SPEC ? 1.0f : a0) * __expf(e0) : 0.0f;
+        // the per-step ratios carry the sign of the odd offsets
+        rf = live ? sgn * __expf(Gd * (2.0f * r.fmf + r.fdf)) : 0.0f;
+        rbk = live ? sgn * __expf(Gd * (r.fdf - 2.0f * r.fmf)) : 0.0f;
+        qg = live ? __expf(2.0f * Gd * r.fdf) : 0.0f;
+      }
+      // forward from the centre channel
+      float x = cm, y = sm, g = gf, ra = rf;
+#pragma unroll
+      for (int j = H; j < CPT; ++j) {
+        const bool odd = (j - H) & 1;
+        float amp;
+        if (GAUSS) amp = SPEC ? s_t[kk * CPT + j] * g : g;
+        else amp = odd ? s_t[kk * CPT + j] * sgn : s_t[kk * CPT + j];
+        accr[j] = fmaf(amp, x, accr[j]);
+        acci[j] = fmaf(amp, y, acci[j]);
+        if (j + 1 < CPT) {
+          const float x1 = fmaf(-tau, y, x);
+          y = fmaf(sig, x1, y);
+          x = fmaf(-tau, y, x1);
+          if (GAUSS) { g *= ra; ra *= qg; }
+        }
+      }
+      // backward from the centre channel
+      x = cm; y = sm;
+      float gb = gf * rbk, rb2 = rbk * qg;
+#pragma unroll
+      for (int j = H - 1; j >= 0; --j) {
+        const bool odd = (H - j) & 1;
+        const float x1 = fmaf(tau, y, x);
+        y = fmaf(-sig, x1, y);
+        x = fmaf(tau, y, x1);
+        float amp;
+        if (GAUSS) amp = SPEC ? s_t[kk * CPT + j] * gb : gb;
+        else amp = odd ? s_t[kk * CPT + j] * sgn : s_t[kk * CPT + j];
+        accr[j] = fmaf(amp, x, accr[j]);
+        acci[j] = fmaf(amp, y, acci[j]);
+        if (GAUSS && j > 0) { gb *= rb2; rb2 *= qg; }
+      }
+    }
+  }
+}
+
+template <int CPT, int TILE, bool GAUSS, bool SPEC, int PREC>
+__global__ __launch_bounds__(kRows, 2) void k_dft_split(Desc d) {
+  constexpr bool kMirror = !SPEC;
   __shared__ double s_x[TILE], s_y[TILE], s_z[TILE];
   __shared__ float s_a[TILE];
   __shared__ float s_g[GAUSS ? 3 * TILE : 1];
@@ -160,34 +288,13 @@ __global__ __launch_bounds__(kRows, 2) void k_dft_split(Desc d) {
     const float uf = valid ? rp[d.ilocu] : 0.0f;
     const float vf = valid ? rp[d.ilocv] : 0.0f;
     const float wf = valid ? rp[d.ilocw] : 0.0f;
-    const double u = uf, v = vf, w = wf;
     const double fd = d.fdel[isel];
-    const double fm = d.fbase[isel] + (double)(c0 + H) * fd;
-    const float fmf = (float)fm, fdf = (float)fd;
-    const float uu = uf * uf, vv = vf * vf, uv = uf * vf;
+    const WalkRow wr(uf, vf, wf, d.fbase[isel] + (double)(c0 + CPT / 2) * fd, fd);
 
     float accr[CPT], acci[CPT];
     double outr[CPT], outi[CPT];
 #pragma unroll
     for (int j = 0; j < CPT; ++j) { accr[j] = acci[j] = 0.0f; outr[j] = outi[j] = 0.0; }
-
-    // the centre phasor (cm, sm) of component kk and its step as three
-    // shears (tau, sig), the step reduced to |pd| <= 1/4 turn; flip: an odd
-    // count of half turns was taken out, every odd offset changes sign
-    auto phasors = [&](int kk, float &cm, float &sm, float &tau, float &sig, bool &flip) {
-      const double psi = fma(w, s_z[kk], fma(v, s_y[kk], u * s_x[kk]));
-      double pm = psi * fm, pd = psi * fd;
-      pm -= rint(pm);
-      const double h2 = rint(2.0 * pd);
-      pd -= 0.5 * h2;
-      flip = ((int)h2) & 1;
-      float sh, ch;
-      sincos_turns<PREC == 2 ? 1 : 0>((float)pm, &sm, &cm);
-      if (PREC == 0) sincos_turns_hw((float)(0.5 * pd), &sh, &ch);
-      else sincos_halfturns_small((float)pd, &sh, &ch);
-      tau = sh * __builtin_amdgcn_rcpf(ch);
-      sig = 2.0f * sh * ch;
-    };
 
     for (int k0 = kBeg; k0 < kEnd; k0 += TILE) {
       __syncthreads();
@@ -256,97 +363,7 @@ __global__ __launch_bounds__(kRows, 2) void k_dft_split(Desc d) {
       }
       __syncthreads();
       const int np = !kMirror ? 0 : GAUSS ? __builtin_amdgcn_readfirstlane(s_np) : kn;
-      if (kMirror) {
-        for (int kk = 0; kk < np; ++kk) {
-          float cm, sm, tau, sig;
-          bool flip;
-          phasors(kk, cm, sm, tau, sig, flip);
-          const float a0 = s_a[kk], ao = flip ? -a0 : a0;
-          const float ce = a0 * cm, se = a0 * sm, co = ao * cm, so = ao * sm;
-          accr[H] += ce;
-          acci[H] += se;
-          float x = 1.0f, y = 0.0f;  // W^q
-#pragma unroll
-          for (int q1 = 1; q1 <= H; ++q1) {
-            const float x1 = fmaf(-tau, y, x);
-            y = fmaf(sig, x1, y);
-            x = fmaf(-tau, y, x1);
-            const float c = (q1 & 1) ? co : ce, s = (q1 & 1) ? so : se;
-            if (q1 < H) {
-              accr[H + q1] = fmaf(x, c, accr[H + q1]);  // C c
-              accr[H - q1] = fmaf(y, s, accr[H - q1]);  // S s
-              acci[H + q1] = fmaf(x, s, acci[H + q1]);  // C s
-              acci[H - q1] = fmaf(y, c, acci[H - q1]);  // S c
-            } else {  // the one channel without a mirror
-              accr[0] = fmaf(x, c, fmaf(y, s, accr[0]));
-              acci[0] = fmaf(x, s, fmaf(-y, c, acci[0]));
-            }
-          }
-        }
-        // the tile's channel sums
-#pragma unroll
-        for (int q1 = 1; q1 < H; ++q1) {
-          const float cc = accr[H + q1], ss = accr[H - q1], cs = acci[H + q1], sc = acci[H - q1];
-          accr[H + q1] = cc - ss;
-          accr[H - q1] = cc + ss;
-          acci[H + q1] = cs + sc;
-          acci[H - q1] = cs - sc;
-        }
-      }
-      if (GAUSS || SPEC) {
-        for (int kk = np; kk < kn; ++kk) {
-          float cm, sm, tau, sig;
-          bool flip;
-          phasors(kk, cm, sm, tau, sig, flip);
-          const float a0 = s_a[kk];
-          const float sgn = flip ? -1.0f : 1.0f;
-          float gf = a0, rf = 0.0f, rbk = 0.0f, qg = 0.0f;
-          if (GAUSS) {
-            const float G = fmaf(s_g[3 * kk + 2], uv, fmaf(s_g[3 * kk + 1], vv, s_g[3 * kk] * uu));
-            const float e0 = G * fmf * fmf;
-            const float Gd = G * fdf;
-            const bool live = e0 > -60.0f;
-            gf = live ? (SPEC ? 1.0f : a0) * __expf(e0) : 0.0f;
-            // the per-step ratios carry the sign of the odd offsets
-            rf = live ? sgn * __expf(Gd * (2.0f * fmf + fdf)) : 0.0f;
-            rbk = live ? sgn * __expf(Gd * (fdf - 2.0f * fmf)) : 0.0f;
-            qg = live ? __expf(2.0f * Gd * fdf) : 0.0f;
-          }
-          // forward from the centre channel
-          float x = cm, y = sm, g = gf, r = rf;
-#pragma unroll
-          for (int j = H; j < CPT; ++j) {
-            const bool odd = (j - H) & 1;
-            float amp;
-            if (GAUSS) amp = SPEC ? s_t[kk * CPT + j] * g : g;
-            else amp = odd ? s_t[kk * CPT + j] * sgn : s_t[kk * CPT + j];
-            accr[j] = fmaf(amp, x, accr[j]);
-            acci[j] = fmaf(amp, y, acci[j]);
-            if (j + 1 < CPT) {
-              const float x1 = fmaf(-tau, y, x);
-              y = fmaf(sig, x1, y);
-              x = fmaf(-tau, y, x1);
-              if (GAUSS) { g *= r; r *= qg; }
-            }
-          }
-          // backward from the centre channel
-          x = cm; y = sm;
-          float gb = gf * rbk, rb2 = rbk * qg;
-#pragma unroll
-          for (int j = H - 1; j >= 0; --j) {
-            const bool odd = (H - j) & 1;
-            const float x1 = fmaf(tau, y, x);
-            y = fmaf(-sig, x1, y);
-            x = fmaf(tau, y, x1);
-            float amp;
-            if (GAUSS) amp = SPEC ? s_t[kk * CPT + j] * gb : gb;
-            else amp = odd ? s_t[kk * CPT + j] * sgn : s_t[kk * CPT + j];
-            accr[j] = fmaf(amp, x, accr[j]);
-            acci[j] = fmaf(amp, y, acci[j]);
-            if (GAUSS && j > 0) { gb *= rb2; rb2 *= qg; }
-          }
-        }
-      }
+      walk_tile<CPT, GAUSS, SPEC, PREC>(wr, s_x, s_y, s_z, s_a, s_g, s_t, np, kn, accr, acci);
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
         outr[j] += (double)accr[j];
@@ -439,9 +456,7 @@ __device__ __forceinline__ void apply_ops(const Desc &d, float *base, const int 
 template <int CPT, bool GAUSS, bool SPEC, int PREC>
 __global__ __launch_bounds__(kRows, 2) void k_dft_share(Desc d) {
   constexpr int TILE = 64;
-  static_assert(CPT % 2 == 0, "CPT must be even");
   constexpr bool kMirror = !SPEC;
-  constexpr int H = CPT / 2;
   struct Tile {
     double x[TILE], y[TILE], z[TILE];
     float a[TILE];
@@ -481,34 +496,13 @@ __global__ __launch_bounds__(kRows, 2) void k_dft_share(Desc d) {
     const float uf = valid ? rp[d.ilocu] : 0.0f;
     const float vf = valid ? rp[d.ilocv] : 0.0f;
     const float wf = valid ? rp[d.ilocw] : 0.0f;
-    const double u = uf, v = vf, w = wf;
     const double fd = d.fdel[isel];
-    const double fm = d.fbase[isel] + (double)(c0 + H) * fd;
-    const float fmf = (float)fm, fdf = (float)fd;
-    const float uu = uf * uf, vv = vf * vf, uv = uf * vf;
+    const WalkRow wr(uf, vf, wf, d.fbase[isel] + (double)(c0 + CPT / 2) * fd, fd);
 
     float accr[CPT], acci[CPT];
     double outr[CPT], outi[CPT];
 #pragma unroll
     for (int j = 0; j < CPT; ++j) { accr[j] = acci[j] = 0.0f; outr[j] = outi[j] = 0.0; }
-
-    // the centre phasor (cm, sm) of component kk and its step as three
-    // shears (tau, sig), the step reduced to |pd| <= 1/4 turn; flip: an odd
-    // count of half turns was taken out, every odd offset changes sign
-    auto phasors = [&](int kk, float &cm, float &sm, float &tau, float &sig, bool &flip) {
-      const double psi = fma(w, s_z[kk], fma(v, s_y[kk], u * s_x[kk]));
-      double pm = psi * fm, pd = psi * fd;
-      pm -= rint(pm);
-      const double h2 = rint(2.0 * pd);
-      pd -= 0.5 * h2;
-      flip = ((int)h2) & 1;
-      float sh, ch;
-      sincos_turns<PREC == 2 ? 1 : 0>((float)pm, &sm, &cm);
-      if (PREC == 0) sincos_turns_hw((float)(0.5 * pd), &sh, &ch);
-      else sincos_halfturns_small((float)pd, &sh, &ch);
-      tau = sh * __builtin_amdgcn_rcpf(ch);
-      sig = 2.0f * sh * ch;
-    };
 
     for (int k0 = kBeg; k0 < kEnd; k0 += TILE) {
       wave_sync();
@@ -566,97 +560,7 @@ __global__ __launch_bounds__(kRows, 2) void k_dft_share(Desc d) {
       }
       wave_sync();
       const int np = !kMirror ? 0 : GAUSS ? __builtin_amdgcn_readfirstlane(ntile) : kn;
-      if (kMirror) {
-        for (int kk = 0; kk < np; ++kk) {
-          float cm, sm, tau, sig;
-          bool flip;
-          phasors(kk, cm, sm, tau, sig, flip);
-          const float a0 = s_a[kk], ao = flip ? -a0 : a0;
-          const float ce = a0 * cm, se = a0 * sm, co = ao * cm, so = ao * sm;
-          accr[H] += ce;
-          acci[H] += se;
-          float x = 1.0f, y = 0.0f;  // W^q
-#pragma unroll
-          for (int q1 = 1; q1 <= H; ++q1) {
-            const float x1 = fmaf(-tau, y, x);
-            y = fmaf(sig, x1, y);
-            x = fmaf(-tau, y, x1);
-            const float c = (q1 & 1) ? co : ce, s = (q1 & 1) ? so : se;
-            if (q1 < H) {
-              accr[H + q1] = fmaf(x, c, accr[H + q1]);  // C c
-              accr[H - q1] = fmaf(y, s, accr[H - q1]);  // S s
-              acci[H + q1] = fmaf(x, s, acci[H + q1]);  // C s
-              acci[H - q1] = fmaf(y, c, acci[H - q1]);  // S c
-            } else {  // the one channel without a mirror
-              accr[0] = fmaf(x, c, fmaf(y, s, accr[0]));
-              acci[0] = fmaf(x, s, fmaf(-y, c, acci[0]));
-            }
-          }
-        }
-        // the tile's channel sums
-#pragma unroll
-        for (int q1 = 1; q1 < H; ++q1) {
-          const float cc = accr[H + q1], ss = accr[H - q1], cs = acci[H + q1], sc = acci[H - q1];
-          accr[H + q1] = cc - ss;
-          accr[H - q1] = cc + ss;
-          acci[H + q1] = cs + sc;
-          acci[H - q1] = cs - sc;
-        }
-      }
-      if (GAUSS || SPEC) {
-        for (int kk = np; kk < kn; ++kk) {
-          float cm, sm, tau, sig;
-          bool flip;
-          phasors(kk, cm, sm, tau, sig, flip);
-          const float a0 = s_a[kk];
-          const float sgn = flip ? -1.0f : 1.0f;
-          float gf = a0, rf = 0.0f, rbk = 0.0f, qg = 0.0f;
-          if (GAUSS) {
-            const float G = fmaf(s_g[3 * kk + 2], uv, fmaf(s_g[3 * kk + 1], vv, s_g[3 * kk] * uu));
-            const float e0 = G * fmf * fmf;
-            const float Gd = G * fdf;
-            const bool live = e0 > -60.0f;
-            gf = live ? (SPEC ? 1.0f : a0) * __expf(e0) : 0.0f;
-            // the per-step ratios carry the sign of the odd offsets
-            rf = live ? sgn * __expf(Gd * (2.0f * fmf + fdf)) : 0.0f;
-            rbk = live ? sgn * __expf(Gd * (fdf - 2.0f * fmf)) : 0.0f;
-            qg = live ? __expf(2.0f * Gd * fdf) : 0.0f;
-          }
-          // forward from the centre channel
-          float x = cm, y = sm, g = gf, r = rf;
-#pragma unroll
-          for (int j = H; j < CPT; ++j) {
-            const bool odd = (j - H) & 1;
-            float amp;
-            if (GAUSS) amp = SPEC ? s_t[kk * CPT + j] * g : g;
-            else amp = odd ? s_t[kk * CPT + j] * sgn : s_t[kk * CPT + j];
-            accr[j] = fmaf(amp, x, accr[j]);
-            acci[j] = fmaf(amp, y, acci[j]);
-            if (j + 1 < CPT) {
-              const float x1 = fmaf(-tau, y, x);
-              y = fmaf(sig, x1, y);
-              x = fmaf(-tau, y, x1);
-              if (GAUSS) { g *= r; r *= qg; }
-            }
-          }
-          // backward from the centre channel
-          x = cm; y = sm;
-          float gb = gf * rbk, rb2 = rbk * qg;
-#pragma unroll
-          for (int j = H - 1; j >= 0; --j) {
-            const bool odd = (H - j) & 1;
-            const float x1 = fmaf(tau, y, x);
-            y = fmaf(-sig, x1, y);
-            x = fmaf(tau, y, x1);
-            float amp;
-            if (GAUSS) amp = SPEC ? s_t[kk * CPT + j] * gb : gb;
-            else amp = odd ? s_t[kk * CPT + j] * sgn : s_t[kk * CPT + j];
-            accr[j] = fmaf(amp, x, accr[j]);
-            acci[j] = fmaf(amp, y, acci[j]);
-            if (GAUSS && j > 0) { gb *= rb2; rb2 *= qg; }
-          }
-        }
-      }
+      walk_tile<CPT, GAUSS, SPEC, PREC>(wr, s_x, s_y, s_z, s_a, s_g, s_t, np, kn, accr, acci);
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
         outr[j] += (double)accr[j];
