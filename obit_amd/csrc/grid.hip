@@ -486,7 +486,7 @@ __global__ __launch_bounds__(256) void k_list_bounds(const unsigned *keys, long 
 constexpr int kW = 7;          // GCF support in cells (checked on the host)
 // Tracks of a work item (swept 64..2048 on workload 4: 128 best).  A small pass
 // would be faster with fewer (10,530 rows x 64 channels into 512^2: a call of
-// 0.86 ms with 16, 1.25 with 128), but other FP32 sums than one item's move the
+// 0.86 ms with 16, 1.27 with 128), but other FP32 sums than one item's move the
 // pixels of an image's corners by up to 1e-2 of its rms, where the gridding
 // correction magnifies them by 5e4: one length for every pass.
 constexpr int kLogChunk = 7, kChunk = 1 << kLogChunk;
@@ -1842,7 +1842,7 @@ int launch_taps(GpuState *gs, const float *vis) {
     // tiles, which end in the order of their items' lengths, come in much the same
     // order in every pass.  Items taken from counters as waves get free, 16 waves a
     // workgroup and shorter per-sample code take the whole call of 105,300 rows x
-    // 256 channels into 20 facets x 8 planes of 2048^2 from 17.5 to 13.8 ms, but
+    // 256 channels into 20 facets x 8 planes of 2048^2 from 16.3 to 13.8 ms, but
     // order the adds anew: an image's corner pixels then move by 2 to 10 times
     // what two passes differ by here (up to 1e-2 of its rms).
     if (gs->tapsPerCU <= 0) {
