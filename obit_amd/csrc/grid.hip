@@ -1199,7 +1199,7 @@ __global__ __launch_bounds__(NT) void k_fft_cols8(float2 *grid, int pitchC, long
 // the last pass's points go straight to the image, so a row crosses LDS twice
 // instead of five times.  The persistent blocks keep the twiddle table
 // (exp(+2 pi i m / N)) in LDS.  Bound by HBM: 8 planes of 2048^2 74 us with a
-// workgroup a row and barriers, so 52, 5.2 TB/s (the whole call 182 -> 158; of
+// workgroup a row and barriers, so 50, 5.4 TB/s (the whole call 182 -> 158; of
 // 1024^2 55 -> 47).  Held to 168 registers, for a third wave a SIMD, it spills and
 // takes 93.
 template <int RA>

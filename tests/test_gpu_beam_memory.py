@@ -17,7 +17,7 @@ def test_no_room_for_products():
     # there, and the memory goes back with it
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, os.path.abspath(__file__)], cwd=root, capture_output=True, text=True,
-                       env=dict(os.environ, PYTHONPATH=root), timeout=100)
+                       env=dict(os.environ, PYTHONPATH=root), timeout=240)
     print(r.stdout[-300:], r.stderr[-2000:], flush=True)
     assert r.returncode == 0
 

@@ -2,7 +2,9 @@
 rounding by up to 5e4 in the corners, against recorded pixels of the same
 images: regrouped sums of samples or another order of a transform's radices
 move corner pixels by 1e-3 to 1e-2 of the images' rms while every test on the
-uncorrected scale passes."""
+uncorrected scale passes.  The pixels are those of one pass on an MI355X in
+128-track items dealt out in turn, with transforms of 4, 16, 16 and 8, 8, 8
+points a row; _own is the most that five more passes differed from it."""
 import os
 
 import numpy as np
