@@ -556,6 +556,11 @@ __device__ __forceinline__ float keep_lanes(float a, unsigned long long m) {
 // grid with plain stores when the item is the tile's whole list; the
 // halo, and every cell of an item of a longer list, add with device
 // atomics.
+//
+// What bounds it is the issue of its 430 vector instructions and 20 matrix steps
+// a pass of 64 slots, which exclude each other on a SIMD where they are FP32 (34
+// cycles each); 4 waves and their table leave LDS for 3 workgroups a CU.  105,300
+// rows x 256 channels into 20 facets x 8 planes of 2048^2: 11.1 ms.
 __global__ __launch_bounds__(64 * kWaves) void k_grid_taps(const float *vis, const FacetDev *facets,
                                                            const int *listFacet, const int2 *items,
                                                            const long long *nitemsPtr, Common cm,
@@ -1066,7 +1071,7 @@ __device__ __forceinline__ void stockham_pass(float2 *lds, int Ns, const float2 
 // baseline often more).  At 2048, 16 waves of 2 columns a thread instead of 8
 // of 4, which leaves more of them to run while others wait at a barrier.  8
 // planes of 2048^2 with 65-70 % of the columns used: 110 us, 96 without the
-// empty blocks' passes and 92 with 16 waves, 2.4 TB/s; with 4 columns a block
+// empty blocks' passes and 92-97 with 16 waves, 2.3 TB/s; with 4 columns a block
 // (32-byte segments, two blocks a CU) 104.
 template <int N, int R1, int R2, int R3, int NT>
 __global__ __launch_bounds__(NT) void k_fft_cols8(float2 *grid, int pitchC, long long planeC, int c0, int nplane,
